@@ -129,36 +129,61 @@ __device__ __forceinline__ ExpertScan scan_expert_tiles(const void* offsets, int
     return s;
 }
 
+// The same for the 64 experts from `base` on (any E): a caller with more than 64 experts walks the blocks.
+__device__ __forceinline__ ExpertScan scan_expert_tiles_from(const void* offsets, int off64, int E, int bm, int base)
+{
+    const int lane = threadIdx.x & 63;
+    const int e = base + lane;
+    const int64_t end = load_idx(offsets, e < E ? e : E - 1, off64);
+    int64_t start = __shfl_up(end, 1);
+    if (lane == 0) start = base > 0 ? load_idx(offsets, base - 1, off64) : 0;
+    const int64_t nt = e < E ? (end - start + bm - 1) / bm : 0;
+    int64_t incl = nt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t t = __shfl_up(incl, d);
+        if (lane >= d) incl += t;
+    }
+    ExpertScan s;
+    s.start = start; s.end = end; s.tiles_before = incl - nt; s.tiles_through = incl;
+    return s;
+}
+
 // Maps a linear row-tile id (uniform over the wave) onto (expert, first row, one-past-last row).
 struct RowTile { int expert; int64_t row0; int64_t row1; };
 __device__ __forceinline__ bool find_row_tile(const void* offsets, int off64, int E, int bm, int64_t tile, RowTile* out)
 {
-    if (E <= 64) {
+    for (int base = 0; base < E; base += 64) {   // one memory round trip per 64 experts
         const int lane = threadIdx.x & 63;
-        const ExpertScan s = scan_expert_tiles(offsets, off64, E, bm);
-        const unsigned long long hit = __ballot(lane < E && tile >= s.tiles_before && tile < s.tiles_through);
-        if (hit == 0) return false;
-        const int e = __ffsll(hit) - 1;
-        const int64_t end = __shfl(s.end, e);
-        out->expert = e;
-        out->row0 = __shfl(s.start, e) + (tile - __shfl(s.tiles_before, e)) * bm;
-        out->row1 = (out->row0 + bm < end) ? out->row0 + bm : end;
-        return true;
-    }
-    int64_t start = 0;
-    for (int e = 0; e < E; ++e) {
-        int64_t end = load_idx(offsets, e, off64);
-        int64_t nt = (end - start + bm - 1) / bm;
-        if (tile < nt) {
-            out->expert = e;
-            out->row0 = start + tile * bm;
+        const ExpertScan s = E <= 64 ? scan_expert_tiles(offsets, off64, E, bm) : scan_expert_tiles_from(offsets, off64, E, bm, base);
+        const unsigned long long hit = __ballot(base + lane < E && tile >= s.tiles_before && tile < s.tiles_through);
+        if (hit != 0) {
+            const int l = __ffsll(hit) - 1;
+            const int64_t end = __shfl(s.end, l);
+            out->expert = base + l;
+            out->row0 = __shfl(s.start, l) + (tile - __shfl(s.tiles_before, l)) * bm;
             out->row1 = (out->row0 + bm < end) ? out->row0 + bm : end;
             return true;
         }
-        tile -= nt;
-        start = end;
+        tile -= uniform_i64(__shfl(s.tiles_through, 63));
     }
     return false;
+}
+
+// First and one-past-last row of group e and the number of bm-row tiles of all groups before it.  All 64 lanes active.
+__device__ __forceinline__ void find_group(const void* offsets, int off64, int bm, int e, int64_t* start, int64_t* end, int64_t* tiles_before)
+{
+    const int lane = threadIdx.x & 63;
+    int64_t n = 0;
+    for (int ee = lane; ee < e; ee += 64) {
+        const int64_t s0 = ee > 0 ? load_idx(offsets, ee - 1, off64) : 0;
+        n += (load_idx(offsets, ee, off64) - s0 + bm - 1) / bm;
+    }
+    *start = e > 0 ? load_idx(offsets, e - 1, off64) : 0;
+    *end = load_idx(offsets, e, off64);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d);
+    *tiles_before = n;
 }
 
 #define MOE_DISPATCH_DTYPE(dtype, ...)                                                   \

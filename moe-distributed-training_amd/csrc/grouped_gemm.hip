@@ -110,8 +110,7 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
         sc = scan_expert_tiles(offsets, off64, E, BM);
         T = uniform_i64(__shfl(sc.tiles_through, 63)) * ntiles_n;
     } else {
-        int64_t start = 0;
-        for (int e = 0; e < E; ++e) { const int64_t end = load_idx(offsets, e, off64); T += (end - start + BM - 1) / BM; start = end; }
+        for (int base = 0; base < E; base += 64) T += uniform_i64(__shfl(scan_expert_tiles_from(offsets, off64, E, BM, base).tiles_through, 63));
         T *= ntiles_n;
     }
     const int xcd = blockIdx.x % NXCD;
@@ -174,25 +173,25 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
         w.mt_in_group = __builtin_amdgcn_readfirstlane((int)mt);
         w.valid = true;
     } else {
-        int64_t start = 0, id = t, mtiles_before = 0;
-        for (int e = 0; e < E; ++e) {
-            const int64_t end = load_idx(offsets, e, off64);
+        int64_t mtiles_before = 0;   // row tiles of the experts before `base`
+        for (int base = 0; base < E; base += 64) {
+            sc = scan_expert_tiles_from(offsets, off64, E, BM, base);
+            const int64_t tl = t - mtiles_before * ntiles_n;
+            const unsigned long long hit = __ballot(base + lane < E && tl >= sc.tiles_before * ntiles_n && tl < sc.tiles_through * ntiles_n);
+            if (hit == 0) { mtiles_before += uniform_i64(__shfl(sc.tiles_through, 63)); continue; }
+            const int hl = __ffsll(hit) - 1;
+            const int64_t start = uniform_i64(__shfl(sc.start, hl)), end = uniform_i64(__shfl(sc.end, hl)), before = uniform_i64(__shfl(sc.tiles_before, hl));
             const int64_t mte = (end - start + BM - 1) / BM;
-            const int64_t te = mte * ntiles_n;
-            if (id < te) {
-                w.expert = e;
-                w.nt = (int)(id / mte);
-                const int64_t mt = id % mte;
-                w.mtile = (int)(mtiles_before + mt);
-                w.mt_in_group = (int)mt;
-                w.row0 = start + mt * BM;
-                w.row1 = (w.row0 + BM < end) ? w.row0 + BM : end;
-                w.valid = true;
-                break;
-            }
-            id -= te;
-            mtiles_before += mte;
-            start = end;
+            const int64_t local = tl - before * ntiles_n;
+            const int64_t mt = local % mte;
+            w.expert = base + hl;
+            w.nt = (int)(local / mte);
+            w.row0 = start + mt * BM;
+            w.row1 = (w.row0 + BM < end) ? w.row0 + BM : end;
+            w.mtile = (int)(mtiles_before + before + mt);
+            w.mt_in_group = (int)mt;
+            w.valid = true;
+            break;
         }
     }
     w.part = __builtin_amdgcn_readfirstlane(w.part);

@@ -336,12 +336,8 @@ __global__ void xtp_reduce_kernel(const float* __restrict__ partial, int64_t par
     const int rank = job.rank;
     partial += (int64_t)blockIdx.z * partial_stride;
     const int e = blockIdx.y;
-    int64_t tile0 = 0, start = 0, end = 0;
-    for (int ee = 0; ee <= e; ++ee) {
-        start = end;
-        end = load_idx(offsets, ee, off64);
-        if (ee < e) tile0 += (end - start + XTP_RC - 1) / XTP_RC;
-    }
+    int64_t tile0, start, end;
+    find_group(offsets, off64, XTP_RC, e, &start, &end, &tile0);   // one round trip, not one per expert
     const int64_t ntile = (end - start + XTP_RC - 1) / XTP_RC;
     const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (idx >= K * 16) return;

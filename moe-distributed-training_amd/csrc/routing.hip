@@ -9,15 +9,7 @@
 
 namespace {
 
-constexpr int ROUTER_TOKENS_PER_WAVE = 2;
 constexpr int ROUTER_EXPERT_GROUP = 8;
-
-__device__ __forceinline__ float wave_sum(float v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 
 // 8 consecutive elements as floats; one 16-byte (2-byte types) or two 16-byte (fp32) loads when the row is aligned
 template <typename T>
@@ -39,9 +31,32 @@ __device__ __forceinline__ void load8(const T* p, float* v, int kn, bool vec_ok)
     }
 }
 
-// logits[t][e] = sum_k x[t][k] * wg[e][k], fp32 accumulate.  One wave owns ROUTER_TOKENS_PER_WAVE tokens
-// and walks the hidden dimension 8 elements per lane at a time; experts are processed in groups of 8.
-template <typename T>
+// v[0..N): sums over the 64 lanes, see router_logits_kernel
+template <int N, int O>
+__device__ __forceinline__ void butterfly_sums(float* v, int lane)
+{
+    if constexpr (O > 0) {
+        if constexpr (N > 1) {
+            const bool up = (lane & O) != 0;
+#pragma unroll
+            for (int q = 0; q < N / 2; ++q) {
+                const float keep = up ? v[N / 2 + q] : v[q], send = up ? v[q] : v[N / 2 + q];
+                v[q] = keep + __shfl_xor(send, O, 64);
+            }
+            butterfly_sums<N / 2, O / 2>(v, lane);
+        } else {
+            v[0] += __shfl_xor(v[0], O, 64);
+            butterfly_sums<1, O / 2>(v, lane);
+        }
+    }
+}
+
+// logits[t][e] = sum_k x[t][k] * wg[e][k], fp32 accumulate, for the shapes router_mfma_kernel does not take (more than 8
+// experts, fp32, odd hidden sizes).  One wave owns TOKENS tokens and one group of 8 experts (blockIdx.y) and walks the
+// hidden dimension 8 elements per lane at a time: one wave per expert group keeps every SIMD busy where one wave for all
+// groups did not (2048 tokens x 64 experts x 2048 columns: 83 -> 28 us; bound by the vector ALUs, one FMA per token,
+// expert and column plus the unpacking).  The order of the additions of a logit depends neither on TOKENS nor on the grid.
+template <typename T, int TOKENS>
 __global__ void __launch_bounds__(256) router_logits_kernel(const T* __restrict__ x, int64_t ldx,
                                                             const T* __restrict__ wg, int64_t ldw,
                                                             float* __restrict__ logits, int64_t ntok, int64_t d, int E,
@@ -49,50 +64,140 @@ __global__ void __launch_bounds__(256) router_logits_kernel(const T* __restrict_
 {
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int64_t t0 = wave * ROUTER_TOKENS_PER_WAVE;
+    const int64_t t0 = wave * TOKENS;
     if (t0 >= ntok) return;
-    for (int e0 = 0; e0 < E; e0 += ROUTER_EXPERT_GROUP) {
-        float acc[ROUTER_TOKENS_PER_WAVE][ROUTER_EXPERT_GROUP];
+    const int e0 = blockIdx.y * ROUTER_EXPERT_GROUP;
+    float acc[TOKENS][ROUTER_EXPERT_GROUP];
 #pragma unroll
-        for (int i = 0; i < ROUTER_TOKENS_PER_WAVE; ++i)
+    for (int i = 0; i < TOKENS; ++i)
 #pragma unroll
-            for (int j = 0; j < ROUTER_EXPERT_GROUP; ++j) acc[i][j] = 0.f;
-#pragma unroll 2
-        for (int64_t k0 = (int64_t)lane * 8; k0 < d; k0 += 64 * 8) {
-            const int kn = (d - k0 < 8) ? (int)(d - k0) : 8;
-            float xv[ROUTER_TOKENS_PER_WAVE][8];
+        for (int j = 0; j < ROUTER_EXPERT_GROUP; ++j) acc[i][j] = 0.f;
+#pragma unroll 1
+    for (int64_t k0 = (int64_t)lane * 8; k0 < d; k0 += 64 * 8) {
+        const int kn = (d - k0 < 8) ? (int)(d - k0) : 8;
+        float xv[TOKENS][8];
 #pragma unroll
-            for (int i = 0; i < ROUTER_TOKENS_PER_WAVE; ++i) {
-                const int64_t t = (t0 + i < ntok) ? t0 + i : ntok - 1;
-                load8<T>(x + t * ldx + k0, xv[i], kn, vec_ok);
-            }
-#pragma unroll
-            for (int j = 0; j < ROUTER_EXPERT_GROUP; ++j) {
-                const int e = (e0 + j < E) ? e0 + j : E - 1;
-                float wv[8];
-                load8<T>(wg + (int64_t)e * ldw + k0, wv, kn, vec_ok);
-#pragma unroll
-                for (int i = 0; i < ROUTER_TOKENS_PER_WAVE; ++i)
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) acc[i][j] = fmaf(xv[i][u], wv[u], acc[i][j]);
-            }
+        for (int i = 0; i < TOKENS; ++i) {
+            const int64_t t = (t0 + i < ntok) ? t0 + i : ntok - 1;
+            load8<T>(x + t * ldx + k0, xv[i], kn, vec_ok);
         }
 #pragma unroll
-        for (int i = 0; i < ROUTER_TOKENS_PER_WAVE; ++i)
+        for (int j = 0; j < ROUTER_EXPERT_GROUP; ++j) {
+            const int e = (e0 + j < E) ? e0 + j : E - 1;
+            float wv[8];
+            load8<T>(wg + (int64_t)e * ldw + k0, wv, kn, vec_ok);
 #pragma unroll
-            for (int j = 0; j < ROUTER_EXPERT_GROUP; ++j) {
-                const float s = wave_sum(acc[i][j]);
-                if (lane == 0 && t0 + i < ntok && e0 + j < E) logits[(t0 + i) * E + e0 + j] = s;
-            }
+            for (int i = 0; i < TOKENS; ++i)
+#pragma unroll
+                for (int u = 0; u < 8; ++u) acc[i][j] = fmaf(xv[i][u], wv[u], acc[i][j]);
+        }
+    }
+    // Sums over the 64 lanes of all NV values at once: in each step of the butterfly a lane keeps one half of its values
+    // and sends the other half to its partner, so NV values cost about NV exchanges instead of 6 NV (the additions, and
+    // so the bits, are those of a butterfly per value).  Lane l ends up with value l * NV / 64.
+    constexpr int NV = TOKENS * ROUTER_EXPERT_GROUP;
+    float v[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) v[q] = acc[q / ROUTER_EXPERT_GROUP][q % ROUTER_EXPERT_GROUP];
+    butterfly_sums<NV, 32>(v, lane);
+    const int idx = lane * NV / 64;
+    const bool writer = lane % (64 / NV) == 0;
+    const int i = idx / ROUTER_EXPERT_GROUP, e = e0 + idx % ROUTER_EXPERT_GROUP;
+    if (writer && t0 + i < ntok && e < E) logits[(t0 + i) * E + e] = v[0];
+}
+
+// fp32 softmax over the E logits of one token, k rounds of arg-max (the lowest expert index wins a tie), optional division
+// by the sum of the selected scores.  s / topw / topi point at the token's output rows.  TK_LANES lanes share a token,
+// lane l holding experts l, l + TK_LANES, ..: the score row is read and written coalesced and never read back from memory
+// (one thread per token walking its rows in memory took 347 us for 2048 tokens x 64 experts, top-8; this takes 11).
+// The exponentials are added in expert order, the selected scores in selection order: every lane of the token adds all of
+// them, so the bits do not depend on the number of lanes.  All TK_LANES lanes of a token must be active.
+constexpr int TK_LANES = 16;
+constexpr int TK_MAX_PER_LANE = 16;   // up to TK_LANES * TK_MAX_PER_LANE = 256 experts in registers
+template <int PER_LANE>
+__device__ __forceinline__ void softmax_topk_token(const float* __restrict__ l, float* __restrict__ s,
+                                                   float* __restrict__ topw, int32_t* __restrict__ topi, int E, int k,
+                                                   int renorm, bool store)
+{
+    const int ln = threadIdx.x & (TK_LANES - 1);
+    float v[PER_LANE];
+    float mx = -__builtin_inff();
+#pragma unroll
+    for (int q = 0; q < PER_LANE; ++q) {
+        const int e = q * TK_LANES + ln;
+        v[q] = e < E ? l[e] : -__builtin_inff();
+        mx = fmaxf(mx, v[q]);
+    }
+#pragma unroll
+    for (int o = TK_LANES / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, TK_LANES));
+    float sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < PER_LANE; ++q) {
+        const int e0 = q * TK_LANES;
+        v[q] = e0 + ln < E ? expf(v[q] - mx) : 0.f;
+#pragma unroll
+        for (int i = 0; i < TK_LANES; ++i)
+            if (e0 + i < E) sum += __shfl(v[q], i, TK_LANES);
+    }
+#pragma unroll
+    for (int q = 0; q < PER_LANE; ++q) {
+        const int e = q * TK_LANES + ln;
+        v[q] = v[q] / sum;
+        if (store && e < E) s[e] = v[q];
+        if (e >= E) v[q] = -2.f;                     // never selected
+        else if (!(v[q] >= 0.f)) v[q] = -1.f;        // NaN scores lose to every number and are taken in expert order
+    }
+    float wsum = 0.f, kept_w = 0.f;
+    int kept_e = 0;
+    for (int j = 0; j < k; ++j) {
+        float bv = v[0];
+        int be = ln;
+#pragma unroll
+        for (int q = 1; q < PER_LANE; ++q)
+            if (v[q] > bv) { bv = v[q]; be = q * TK_LANES + ln; }
+#pragma unroll
+        for (int o = TK_LANES / 2; o > 0; o >>= 1) {
+            const float ov = __shfl_xor(bv, o, TK_LANES);
+            const int oe = __shfl_xor(be, o, TK_LANES);
+            if (ov > bv || (ov == bv && oe < be)) { bv = ov; be = oe; }
+        }
+#pragma unroll
+        for (int q = 0; q < PER_LANE; ++q)
+            if (be == q * TK_LANES + ln) v[q] = -2.f;
+        const float w = bv < 0.f ? __builtin_nanf("") : bv;
+        wsum += w;
+        // lane j % TK_LANES keeps selection j until the sum is known; a token with more selections writes them in rounds below
+        if (!renorm) { if (store && ln == 0) { topw[j] = w; topi[j] = be; } }
+        else if (k <= TK_LANES) { if (ln == j) { kept_w = w; kept_e = be; } }
+        else if (store && ln == 0) { topw[j] = w; topi[j] = be; }
+    }
+    if (renorm && store) {
+        if (k <= TK_LANES) { if (ln < k) { topw[ln] = kept_w / wsum; topi[ln] = kept_e; } }
+        else if (ln == 0) for (int j = 0; j < k; ++j) topw[j] = topw[j] / wsum;
     }
 }
 
-// fp32 softmax over the E logits of one token, k rounds of arg-max (strict '>' so the lowest expert index wins a
-// tie), optional division by the sum of the selected scores.  s / topw / topi point at the token's output rows.
-__device__ __forceinline__ void softmax_topk_token(const float* __restrict__ l, float* __restrict__ s,
-                                                   float* __restrict__ topw, int32_t* __restrict__ topi, int E, int k,
-                                                   int renorm)
+template <int PER_LANE>
+__global__ void __launch_bounds__(256) router_topk_kernel(const float* __restrict__ logits, float* __restrict__ scores,
+                                                          float* __restrict__ topw, int32_t* __restrict__ topi, int64_t ntok, int E,
+                                                          int k, int renorm)
 {
+    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / TK_LANES;
+    const int64_t tc = t < ntok ? t : ntok - 1;   // (lanes past the end work on the last token and store nothing)
+    softmax_topk_token<PER_LANE>(logits + tc * E, scores + tc * E, topw + tc * k, topi + tc * k, E, k, renorm, t < ntok);
+}
+
+// More experts than a token's lanes hold in registers: one thread per token, rows walked in memory.
+__global__ void router_topk_wide_kernel(const float* __restrict__ logits, float* __restrict__ scores,
+                                        float* __restrict__ topw, int32_t* __restrict__ topi, int64_t ntok, int E, int k,
+                                        int renorm)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= ntok) return;
+    const float* l = logits + t * E;
+    float* s = scores + t * E;
+    topw += t * k;
+    topi += t * k;
     float mx = l[0];
     for (int e = 1; e < E; ++e) mx = fmaxf(mx, l[e]);
     float sum = 0.f;
@@ -114,16 +219,6 @@ __device__ __forceinline__ void softmax_topk_token(const float* __restrict__ l, 
         wsum += bv;
     }
     if (renorm) for (int j = 0; j < k; ++j) topw[j] = topw[j] / wsum;
-}
-
-// One thread per token.
-__global__ void router_topk_kernel(const float* __restrict__ logits, float* __restrict__ scores,
-                                   float* __restrict__ topw, int32_t* __restrict__ topi, int64_t ntok, int E, int k,
-                                   int renorm)
-{
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntok) return;
-    softmax_topk_token(logits + t * E, scores + t * E, topw + t * k, topi + t * k, E, k, renorm);
 }
 
 // Logits, softmax and top-k in one launch for up to ROUTER_EXPERT_GROUP experts of a 2-byte type, the logits on the
@@ -192,36 +287,65 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_kernel(const T* __r
         if (e < E && t0 + t < ntok) logits[(t0 + t) * E + e] = sum;
     }
     __syncthreads();
-    const int64_t t = t0 + tid;
-    if (tid < RM_TOKENS && t < ntok) softmax_topk_token(s_logits[tid], scores + t * E, topw + t * k, topi + t * k, E, k, renorm);
+    if (tid < RM_TOKENS * TK_LANES) {   // whole waves
+        const int tt = tid / TK_LANES;
+        const int64_t t = t0 + tt;
+        softmax_topk_token<1>(s_logits[tt], scores + t * E, topw + t * k, topi + t * k, E, k, renorm, t < ntok);
+    }
 }
 
 // Backward of softmax -> top-k -> renormalise with respect to the logits.
 // dw (T,k): gradient of the returned weights; w (T,k) the returned weights; scores (T,E) the softmax.
-__global__ void router_bwd_kernel(const float* __restrict__ dw, const float* __restrict__ w,
-                                  const int32_t* __restrict__ topi, const float* __restrict__ scores,
-                                  float* __restrict__ dlogits, int64_t ntok, int E, int k, int renorm)
+// TK_LANES lanes share a token so that its rows move coalesced; every lane computes the token's two sums over the k
+// selected experts itself, in selection order (one thread per token: 59 us for 2048 tokens x 64 experts, top-8; this: 9).
+__global__ void __launch_bounds__(256) router_bwd_kernel(const float* __restrict__ dw, const float* __restrict__ w,
+                                                         const int32_t* __restrict__ topi, const float* __restrict__ scores,
+                                                         float* __restrict__ dlogits, int64_t ntok, int E, int k, int renorm)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntok) return;
+    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / TK_LANES;
+    if (t >= ntok) return;   // (whole groups of TK_LANES lanes)
+    const int ln = threadIdx.x & (TK_LANES - 1);
     const float* s = scores + t * E;
+    const float* dwt = dw + t * k;
+    const float* wt = w + t * k;
+    const int32_t* it = topi + t * k;
     float* dl = dlogits + t * E;
-    for (int e = 0; e < E; ++e) dl[e] = 0.f;
-    // selected scores p_j = s[idx_j]; w_j = p_j / S (S = sum p) when renorm, else w_j = p_j
+    // selected scores p_j = s[idx_j]; w_j = p_j / S (S = sum p) when renorm, else w_j = p_j.  Lane j fetches selection j
+    // (of each TK_LANES selections), the token's other lanes get it by shuffle: one memory round trip for all of them.
+    int my_e = 0;
+    float my_p = 0.f, my_dw = 0.f, my_w = 0.f;
+    auto fetch = [&](int j0) {
+        if (j0 + ln < k) { my_e = it[j0 + ln]; my_dw = dwt[j0 + ln]; my_w = wt[j0 + ln]; my_p = s[my_e]; }
+    };
+    fetch(0);
     float S = 1.f, dot = 0.f;
     if (renorm) {
         S = 0.f;
-        for (int j = 0; j < k; ++j) S += s[topi[t * k + j]];
-        for (int j = 0; j < k; ++j) dot += dw[t * k + j] * w[t * k + j];
+        for (int j = 0; j < k; ++j) {
+            if (j > 0 && j % TK_LANES == 0) fetch(j);
+            S += __shfl(my_p, j % TK_LANES, TK_LANES);
+            dot += __shfl(my_dw, j % TK_LANES, TK_LANES) * __shfl(my_w, j % TK_LANES, TK_LANES);
+        }
+        if (k > TK_LANES) fetch(0);
     }
     float sdot = 0.f;  // sum_e dscore_e * s_e
     for (int j = 0; j < k; ++j) {
-        const int e = topi[t * k + j];
-        const float dp = renorm ? (dw[t * k + j] - dot) / S : dw[t * k + j];
-        dl[e] = dp;  // holds dscore for the selected experts for now
-        sdot += dp * s[e];
+        if (j > 0 && j % TK_LANES == 0) fetch(j);
+        const float d = __shfl(my_dw, j % TK_LANES, TK_LANES);
+        sdot += (renorm ? (d - dot) / S : d) * __shfl(my_p, j % TK_LANES, TK_LANES);
     }
-    for (int e = 0; e < E; ++e) dl[e] = s[e] * (dl[e] - sdot);
+    if (k > TK_LANES) fetch(0);
+    for (int e0 = 0; e0 < E; e0 += TK_LANES) {
+        const int e = e0 + ln;
+        float ds = 0.f;   // dscore of expert e
+        for (int j = 0; j < k; ++j) {
+            if (j > 0 && j % TK_LANES == 0) fetch(j);
+            const float d = __shfl(my_dw, j % TK_LANES, TK_LANES);
+            if (__shfl(my_e, j % TK_LANES, TK_LANES) == e) ds = renorm ? (d - dot) / S : d;
+        }
+        if (k > TK_LANES) fetch(0);
+        if (e < E) dl[e] = s[e] * (ds - sdot);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -297,6 +421,27 @@ __global__ void __launch_bounds__(SORT_THREADS) sort_scan_kernel(int32_t* __rest
     else for (int i = threadIdx.x; i < nblk * E; i += SORT_THREADS) block_hist[i] += sh[i % E];
 }
 
+// Stores one group of 64 entries (flat positions p of consecutive lanes, expert e, -1: none) at its expert's cursor:
+// entries of one expert keep their order (stability).  A lane's rank among the earlier lanes of its expert comes from 64
+// scalar broadcasts and compares, whatever the number of experts (one ballot round per distinct expert of the group, with
+// a round trip to the cursor in each, took 2-4 times as long from 16 experts up).
+__device__ __forceinline__ void scatter_group(int e, int64_t p, int lane, int32_t* cursor, void* __restrict__ sorted_expert,
+                                              void* __restrict__ sorted_pos, int out64, int32_t* __restrict__ inv)
+{
+    int rank = 0;
+#pragma unroll
+    for (int j = 0; j < 63; ++j) rank += (__builtin_amdgcn_readlane(e, j) == e && j < lane) ? 1 : 0;
+    if (e >= 0) {
+        const int32_t dst = *(volatile int32_t*)(cursor + e) + rank;
+        store_idx(sorted_expert, dst, e, out64);
+        store_idx(sorted_pos, dst, p, out64);
+        if (inv) inv[p] = dst;
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (e >= 0) atomicAdd(&cursor[e], 1);   // (after every lane of the wave has read its cursor)
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Each workgroup re-reads its chunk; wave w owns a contiguous slice of it and walks it 64 entries at a time so
 // that destinations within one expert ascend with the flat position (stability).
 __global__ void __launch_bounds__(SORT_THREADS) sort_scatter_kernel(const void* __restrict__ expert_idx, int in64,
@@ -329,62 +474,52 @@ __global__ void __launch_bounds__(SORT_THREADS) sort_scatter_kernel(const void* 
     }
     __syncthreads();
     // pass 2: ranked scatter
-    volatile int32_t* cursor = sh + w * E;
     for (int i0 = 0; i0 < PER_WAVE; i0 += 64) {
         const int64_t p = wbase + i0 + lane;
         int e = -1;
         if (p < R) { const int64_t ee = load_idx(expert_idx, p, in64); e = (ee >= 0 && ee < E) ? (int)ee : -1; }
-        uint64_t rem = __ballot(e >= 0);
-        while (rem) {
-            const int leader = __ffsll((unsigned long long)rem) - 1;
-            const int e0 = __shfl(e, leader, 64);
-            const uint64_t m = __ballot(e == e0);
-            if (e == e0) {
-                const int rank = __popcll(m & ((1ull << lane) - 1ull));
-                const int32_t dst = cursor[e0] + rank;
-                store_idx(sorted_expert, dst, e0, out64);
-                store_idx(sorted_pos, dst, p, out64);
-                if (inv) inv[p] = dst;
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (lane == leader) cursor[e0] += __popcll(m);
-            __builtin_amdgcn_wave_barrier();
-            rem &= ~m;
-        }
+        scatter_group(e, p, lane, sh + w * E, sorted_expert, sorted_pos, out64, inv);
     }
 }
 
 // The whole sort in one launch, for batches small enough that every workgroup can afford to read ALL assignment ids
-// itself: a workgroup counts, per expert, the entries before its own chunk and the entries altogether (LDS atomics, each
-// wave into its own rows), which gives it its chunk's destination bases without a histogram
-// launch and a scan launch before it; then it scatters its chunk exactly as sort_scatter_kernel does.  Workgroup 0 also
-// writes the per-expert counts, the inclusive offsets and the block table.  Same results as the three-launch path.
-constexpr int64_t SORT_ONE_LAUNCH_MAX_ROWS = 16384;
+// itself: a workgroup counts, per expert, the entries before its own chunk and the others (LDS atomics), which gives it
+// its chunk's destination bases without a histogram launch and a scan launch before it; then it scatters its chunk, one
+// wave per 64 entries.  Workgroup 0 also writes the per-expert counts, the inclusive offsets and the block table.  Same
+// results as the three-launch path.  Latency bound, so every step is parallel: ids are requested in batches, the scan over
+// the experts runs as prefix sums of one wave (a single thread walking 64 experts took longer than all the rest).
+constexpr int64_t SORT_ONE_LAUNCH_MAX_ROWS = 65536;
 constexpr int SORT_ONE_LAUNCH_MAX_EXPERTS = 256;
+constexpr int SORT1_THREADS = SORT_CHUNK;   // one thread per entry of the chunk
 static_assert(SORT_CHUNK % 64 == 0, "a 64-entry group of the counting pass lies wholly before a chunk or not at all");
-__global__ void __launch_bounds__(SORT_THREADS) sort_one_launch_kernel(const void* __restrict__ expert_idx, int in64,
-                                                                       int64_t R, int E, int block_m,
-                                                                       void* __restrict__ sorted_expert,
-                                                                       void* __restrict__ sorted_pos, int out64,
-                                                                       void* __restrict__ counts, void* __restrict__ offsets,
-                                                                       void* __restrict__ padded_blocks, int64_t padded_cap,
-                                                                       int32_t* __restrict__ num_padded, int32_t* __restrict__ inv)
+__global__ void __launch_bounds__(SORT1_THREADS) sort_one_launch_kernel(const void* __restrict__ expert_idx, int in64,
+                                                                        int64_t R, int E, int block_m,
+                                                                        void* __restrict__ sorted_expert,
+                                                                        void* __restrict__ sorted_pos, int out64,
+                                                                        void* __restrict__ counts, void* __restrict__ offsets,
+                                                                        void* __restrict__ padded_blocks, int64_t padded_cap,
+                                                                        int32_t* __restrict__ num_padded, int32_t* __restrict__ inv)
 {
-    extern __shared__ int32_t sh[];  // before[NW][E], total[NW][E], then cursor[NW][E]
-    constexpr int NW = SORT_THREADS / 64;
-    constexpr int PER_WAVE = SORT_CHUNK / NW;
+    constexpr int NW = SORT1_THREADS / 64;
+    constexpr int COPIES = 4;        // count rows: a wave adds into row (wave % COPIES), which thins out same-address atomics
+    extern __shared__ int32_t sh[];  // before[COPIES][E], rest[COPIES][E], cursor[NW][E]
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     int32_t* before = sh;
-    int32_t* total = sh + NW * E;
-    int32_t* cur = sh + 2 * NW * E;
-    for (int i = threadIdx.x; i < 3 * NW * E; i += SORT_THREADS) sh[i] = 0;
+    int32_t* rest = sh + COPIES * E;
+    int32_t* cur = sh + 2 * COPIES * E;
+    for (int i = threadIdx.x; i < (2 * COPIES + NW) * E; i += SORT1_THREADS) sh[i] = 0;
     __syncthreads();
     const int64_t chunk_base = (int64_t)blockIdx.x * SORT_CHUNK;
-    // counts over the whole array: wave w walks entries [64 (w + NW j), +64), sixteen groups' ids requested together;
-    // LDS atomics into the wave's own rows (integer counts: the order of the additions does not matter)
+    // the own chunk's entry, and its per-wave histogram
+    const int64_t pown = chunk_base + threadIdx.x;
+    int eown = -1;
+    if (pown < R) { const int64_t ee = load_idx(expert_idx, pown, in64); eown = (ee >= 0 && ee < E) ? (int)ee : -1; }
+    // counts over the whole array: wave w walks entries [64 (w + NW j), +64), sixteen groups' ids requested together
+    // (integer counts: the order of the additions does not matter)
     constexpr int SB = 16;
+    int32_t* my_before = before + (w % COPIES) * E;
+    int32_t* my_rest = rest + (w % COPIES) * E;
     for (int64_t p0 = (int64_t)w * 64; p0 < R; p0 += (int64_t)NW * 64 * SB) {
-        int ev[SB];
         int64_t raw[SB];
         // (one branch on the index width around all the loads, so that they are in flight together; entries past the
         // end re-read the last one and are dropped below)
@@ -398,41 +533,44 @@ __global__ void __launch_bounds__(SORT_THREADS) sort_one_launch_kernel(const voi
 #pragma unroll
         for (int j = 0; j < SB; ++j) {
             const int64_t p = p0 + (int64_t)j * NW * 64 + lane;
-            ev[j] = (p < R && raw[j] >= 0 && raw[j] < E) ? (int)raw[j] : -1;
+            // a 64-entry group lies wholly before the chunk or not at all (chunks are multiples of 64 entries)
+            if (p < R && raw[j] >= 0 && raw[j] < E) atomicAdd(&(p0 + (int64_t)j * NW * 64 < chunk_base ? my_before : my_rest)[raw[j]], 1);
         }
+    }
+    if (eown >= 0) atomicAdd(&cur[w * E + eown], 1);
+    __syncthreads();
+    // wave 0: lane l owns experts [l * per, +per); totals, then their running sums over the lanes
+    const int per = (E + 63) / 64;
+    if (w == 0) {
+        int32_t sum = 0;
+        int64_t nblk = 0;
+        for (int q = 0; q < per; ++q) {
+            const int e = lane * per + q;
+            int32_t b = 0, t = 0;
+            if (e < E) {
 #pragma unroll
-        for (int j = 0; j < SB; ++j) {
-            if (ev[j] >= 0) {
-                atomicAdd(&total[w * E + ev[j]], 1);
-                // a 64-entry group lies wholly before the chunk or not at all (chunks are multiples of 64 entries)
-                if (p0 + (int64_t)j * NW * 64 < chunk_base) atomicAdd(&before[w * E + ev[j]], 1);
+                for (int c = 0; c < COPIES; ++c) { b += before[c * E + e]; t += rest[c * E + e]; }
+                before[e] = b;
+                rest[e] = b + t;
+                sum += b + t;
+                nblk += (b + t + block_m - 1) / block_m;
             }
         }
-    }
-    // per-wave histogram of the own chunk (as in sort_scatter_kernel)
-    const int64_t wbase = chunk_base + (int64_t)w * PER_WAVE;
-    for (int i = lane; i < PER_WAVE; i += 64) {
-        const int64_t p = wbase + i;
-        if (p < R) {
-            const int64_t e = load_idx(expert_idx, p, in64);
-            if (e >= 0 && e < E) atomicAdd(&cur[w * E + (int)e], 1);
+        int32_t incl = sum;
+        int64_t binc = nblk;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int32_t t = __shfl_up(incl, d);
+            const int64_t u = __shfl_up(binc, d);
+            if (lane >= d) { incl += t; binc += u; }
         }
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < E; e += SORT_THREADS) {
-        int32_t b = 0, t = 0;
-        for (int ww = 0; ww < NW; ++ww) { b += before[ww * E + e]; t += total[ww * E + e]; }
-        before[e] = b;
-        total[e] = t;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        // exclusive scan over the experts; workgroup 0 publishes counts, offsets and the block table
         const bool pub = blockIdx.x == 0;
-        int64_t run = 0, nb = 0;
-        for (int e = 0; e < E; ++e) {
-            const int64_t c = total[e];
-            const int64_t start = run;
+        int32_t run = incl - sum;
+        int64_t nb = binc - nblk;
+        for (int q = 0; q < per; ++q) {
+            const int e = lane * per + q;
+            if (e >= E) break;
+            const int32_t c = rest[e], start = run;
             run += c;
             if (pub) {
                 if (counts) store_idx(counts, e, c, out64);
@@ -440,40 +578,19 @@ __global__ void __launch_bounds__(SORT_THREADS) sort_one_launch_kernel(const voi
                 if (padded_blocks)
                     for (int64_t s_ = start; s_ < run; s_ += block_m) { if (nb < padded_cap) store_idx(padded_blocks, nb, s_, out64); ++nb; }
             }
-            total[e] = (int32_t)start;
+            rest[e] = start + before[e];   // this chunk's first destination of the expert
         }
-        if (pub && num_padded) *num_padded = (int32_t)nb;
+        if (pub && num_padded && lane == 63) *num_padded = (int32_t)binc;
     }
     __syncthreads();
-    // exclusive prefix over waves, seeded with this chunk's base = the expert's start + its entries before the chunk
-    for (int e = threadIdx.x; e < E; e += SORT_THREADS) {
-        int32_t run = total[e] + before[e];
+    // exclusive prefix over waves, seeded with the chunk's base
+    for (int e = threadIdx.x; e < E; e += SORT1_THREADS) {
+        int32_t run = rest[e];
+#pragma unroll
         for (int ww = 0; ww < NW; ++ww) { const int32_t c = cur[ww * E + e]; cur[ww * E + e] = run; run += c; }
     }
     __syncthreads();
-    volatile int32_t* cursor = cur + w * E;
-    for (int i0 = 0; i0 < PER_WAVE; i0 += 64) {
-        const int64_t p = wbase + i0 + lane;
-        int e = -1;
-        if (p < R) { const int64_t ee = load_idx(expert_idx, p, in64); e = (ee >= 0 && ee < E) ? (int)ee : -1; }
-        uint64_t rem = __ballot(e >= 0);
-        while (rem) {
-            const int leader = __ffsll((unsigned long long)rem) - 1;
-            const int e0 = __shfl(e, leader, 64);
-            const uint64_t m = __ballot(e == e0);
-            if (e == e0) {
-                const int rank = __popcll(m & ((1ull << lane) - 1ull));
-                const int32_t dst = cursor[e0] + rank;
-                store_idx(sorted_expert, dst, e0, out64);
-                store_idx(sorted_pos, dst, p, out64);
-                if (inv) inv[p] = dst;
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (lane == leader) cursor[e0] += __popcll(m);
-            __builtin_amdgcn_wave_barrier();
-            rem &= ~m;
-        }
-    }
+    scatter_group(eown, pown, lane, cur + w * E, sorted_expert, sorted_pos, out64, inv);
 }
 
 // offsets[e] = number of entries of the non-decreasing array sorted_expert that are <= e  (inclusive running count)
@@ -510,12 +627,19 @@ int moe_launch_router_logits(const void* x, int64_t ldx, const void* wg, int64_t
                              int64_t ntok, int64_t d, int E, hipStream_t stream)
 {
     if (ntok == 0) return MOE_OK;
-    const int64_t waves = (ntok + ROUTER_TOKENS_PER_WAVE - 1) / ROUTER_TOKENS_PER_WAVE;
-    const unsigned grid = (unsigned)((waves + 3) / 4);
+    const int groups = (E + ROUTER_EXPERT_GROUP - 1) / ROUTER_EXPERT_GROUP;
+    // 4 tokens per wave share each weight fetch, as soon as that still leaves a wave for every SIMD; 2 for fewer tokens
+    const int tokens = ((ntok + 3) / 4) * groups >= 4 * (int64_t)moe_device_cus() ? 4 : 2;
+    const int64_t waves = (ntok + tokens - 1) / tokens;
+    const dim3 grid((unsigned)((waves + 3) / 4), (unsigned)groups);
     const int64_t per16 = dtype == MOE_F32 ? 4 : 8;
     const bool vec_ok = ((uintptr_t)x % 16 == 0) && ((uintptr_t)wg % 16 == 0) && ldx % per16 == 0 && ldw % per16 == 0;
-    MOE_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((router_logits_kernel<T>), dim3(grid), dim3(256), 0, stream,
-                                                 (const T*)x, ldx, (const T*)wg, ldw, logits, ntok, d, E, vec_ok));
+    if (tokens == 4)
+        MOE_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((router_logits_kernel<T, 4>), grid, dim3(256), 0, stream, (const T*)x, ldx,
+                                                     (const T*)wg, ldw, logits, ntok, d, E, vec_ok));
+    else
+        MOE_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((router_logits_kernel<T, 2>), grid, dim3(256), 0, stream, (const T*)x, ldx,
+                                                     (const T*)wg, ldw, logits, ntok, d, E, vec_ok));
     return moe_launch_status();
 }
 
@@ -545,8 +669,17 @@ int moe_launch_router_topk(const float* logits, float* scores, float* topw, int3
                            int renorm, hipStream_t stream)
 {
     if (ntok == 0) return MOE_OK;
-    hipLaunchKernelGGL(router_topk_kernel, dim3((unsigned)((ntok + 255) / 256)), dim3(256), 0, stream, logits, scores,
-                       topw, topi, ntok, E, k, renorm);
+    const dim3 grid((unsigned)((ntok * TK_LANES + 255) / 256));
+#define TOPK(n) hipLaunchKernelGGL(router_topk_kernel<n>, grid, dim3(256), 0, stream, logits, scores, topw, topi, ntok, E, k, renorm)
+    if (E <= TK_LANES) TOPK(1);
+    else if (E <= 2 * TK_LANES) TOPK(2);
+    else if (E <= 4 * TK_LANES) TOPK(4);
+    else if (E <= 8 * TK_LANES) TOPK(8);
+    else if (E <= TK_LANES * TK_MAX_PER_LANE) TOPK(TK_MAX_PER_LANE);
+    else
+        hipLaunchKernelGGL(router_topk_wide_kernel, dim3((unsigned)((ntok + 255) / 256)), dim3(256), 0, stream, logits, scores,
+                           topw, topi, ntok, E, k, renorm);
+#undef TOPK
     return moe_launch_status();
 }
 
@@ -554,7 +687,7 @@ int moe_launch_router_bwd(const float* dw, const float* w, const int32_t* topi, 
                           int64_t ntok, int E, int k, int renorm, hipStream_t stream)
 {
     if (ntok == 0) return MOE_OK;
-    hipLaunchKernelGGL(router_bwd_kernel, dim3((unsigned)((ntok + 255) / 256)), dim3(256), 0, stream, dw, w, topi,
+    hipLaunchKernelGGL(router_bwd_kernel, dim3((unsigned)((ntok * TK_LANES + 255) / 256)), dim3(256), 0, stream, dw, w, topi,
                        scores, dlogits, ntok, E, k, renorm);
     return moe_launch_status();
 }
@@ -573,7 +706,7 @@ int moe_launch_sort(const void* expert_idx, int in64, int64_t R, int E, int bloc
     if (workspace_bytes < moe_sort_ws_bytes(R, E)) return MOE_ERR_WORKSPACE;
     const int nblk = (int)((R + SORT_CHUNK - 1) / SORT_CHUNK);
     if (nblk > 0 && R <= SORT_ONE_LAUNCH_MAX_ROWS && E <= SORT_ONE_LAUNCH_MAX_EXPERTS) {
-        hipLaunchKernelGGL(sort_one_launch_kernel, dim3(nblk), dim3(SORT_THREADS), 3 * (SORT_THREADS / 64) * E * sizeof(int32_t), stream,
+        hipLaunchKernelGGL(sort_one_launch_kernel, dim3(nblk), dim3(SORT1_THREADS), (8 + SORT1_THREADS / 64) * E * sizeof(int32_t), stream,
                            expert_idx, in64, R, E, block_m, sorted_expert, sorted_pos, out64, counts, offsets, padded_blocks,
                            padded_cap, num_padded, inv);
         return moe_launch_status();

@@ -287,3 +287,40 @@ def test_forward_router_switches(dev, oracle, case):
     assert rel(xd.grad, xo.grad) < 1e-2 and rel(wd.grad, wo.grad) < 1e-2
     if bias is not None:
         assert rel(bd.grad, bo.grad) < 1e-2
+
+
+@pytest.mark.parametrize("T,E,k", [(33, 9, 1), (50, 16, 16), (50, 17, 17), (40, 33, 2), (257, 64, 8), (30, 65, 20), (20, 128, 4),
+                                   (9, 129, 9), (70, 256, 3), (5, 257, 3)])
+@pytest.mark.parametrize("renorm", [True, False])
+def test_topk_and_its_backward_at_the_expert_counts_where_the_kernel_changes(dev, oracle, T, E, k, renorm):
+    """16 lanes share a token, 1 to 16 experts per lane, one thread per token above 256 experts; more selections than lanes."""
+    _, router, _ = _mods()
+    torch.manual_seed(T * E)
+    logits = torch.randn(T, E, requires_grad=True)
+    so, wo, io = oracle.router_from_logits(logits, k, renorm)
+    s, w, i = router.router_topk(logits.detach().to(dev), k, renorm)
+    assert torch.equal(i.cpu().long(), io)
+    assert torch.allclose(s.cpu(), so, atol=2e-7) and torch.allclose(w.cpu(), wo, atol=5e-7)
+    dw = torch.randn(T, k)
+    wo.backward(dw)
+    dl = router.router_topk_bwd(dw.to(dev), w, i, s, renorm)
+    # fp32 sums of at most k + 1 terms of size |dw| <= 5
+    assert torch.allclose(dl.cpu(), logits.grad, atol=(k + 1) * 5 * 2.0 ** -23 * 4)
+
+
+def test_topk_of_nan_rows_takes_experts_in_order(dev):
+    _, router, _ = _mods()
+    logits = torch.randn(3, 20)
+    logits[1] = float("nan")
+    _, w, i = router.router_topk(logits.to(dev), 4)
+    assert i[1].tolist() == [0, 1, 2, 3] and bool(torch.isnan(w[1]).all()) and not bool(torch.isnan(w[0]).any())
+
+
+@pytest.mark.parametrize("R,E", [(512, 256), (513, 256), (511, 64), (65536, 8), (65536, 256), (65537, 64), (2000, 257)])
+def test_sort_at_the_limits_of_the_one_launch_kernel(dev, oracle, R, E):
+    _, router, ops = _mods()
+    idx = np.random.default_rng(R).integers(0, E, size=R)
+    exp = oracle.sort_by_expert_c(idx, E)
+    sei, ssi, counts, offs, inv = router.sort_assignments(torch.from_numpy(idx).int().to(dev), E)
+    for got, name in ((sei, "sorted_expert"), (ssi, "sorted_pos"), (counts, "counts"), (offs, "offsets"), (inv, "inv")):
+        assert np.array_equal(got.cpu().numpy(), exp[name]), name
