@@ -95,9 +95,24 @@ struct WorkItem {
     int split_item;            // exchange slot of this part (the slots of a tile are consecutive, in part order)
     int split_tile;            // counter of the split tile
     int mtile;                 // number of the row tile among all row tiles (experts in order, BM rows each)
-    int mt_in_group;           // number of the row tile within its expert's group (0: the group's first tile)
 };
 
+// Rows of row tile mt of a group's mte tiles: the group's 16-row blocks are dealt evenly to its tiles (mte = the number of
+// 256-row tiles the group needs).  Measured per round of tiles at K=4096: 99 us with 16 row blocks, 87 with 13, and a tail
+// of 1-3 blocks behind full tiles about as much as a full one (its waves wait for the same weight tiles), so 1060 rows run
+// as five tiles of 13-14 blocks instead of four of 16 and one of 3.  8192 rows over 8 experts: gate/up launch 1630 -> 1556 us,
+// the layer's forward and backward 5029 -> 4950 us.
+__device__ __forceinline__ void even_rows(int64_t start, int64_t end, int64_t mt, int64_t mte, int64_t* row0, int64_t* row1)
+{
+    const int64_t blocks = (end - start + 15) / 16, per = blocks / mte, more = blocks % mte;
+    const int64_t b0 = mt * per + (mt < more ? mt : more);
+    *row0 = start + b0 * 16;
+    const int64_t r1 = *row0 + (per + (mt < more ? 1 : 0)) * 16;
+    *row1 = r1 < end ? r1 : end;
+}
+
+// EVEN: rows as the GEMM deals them to the tiles of a group (even_rows); otherwise those of the tile's 256-row slot
+template <bool EVEN>
 __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int off64, int E, int ntiles_n, int ktiles,
                                                      int max_split, int ncu)
 {
@@ -162,15 +177,14 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
         const int64_t local = t - before * ntiles_n;
         const int nt = (int)(local / mte);
         const int64_t mt = local % mte;
-        const int64_t row0 = start + mt * BM;
-        const int64_t row1 = (row0 + BM < end) ? row0 + BM : end;
+        int64_t row0 = start + mt * BM, row1 = (row0 + BM < end) ? row0 + BM : end;
+        if (EVEN) even_rows(start, end, mt, mte, &row0, &row1);
         // the shuffles return per-lane values; everything derived from the item is uniform and belongs in scalar registers
         w.expert = __builtin_amdgcn_readfirstlane(expert);
         w.nt = __builtin_amdgcn_readfirstlane(nt);
         w.row0 = uniform_i64(row0);
         w.row1 = uniform_i64(row1);
         w.mtile = __builtin_amdgcn_readfirstlane((int)(before + mt));
-        w.mt_in_group = __builtin_amdgcn_readfirstlane((int)mt);
         w.valid = true;
     } else {
         int64_t mtiles_before = 0;   // row tiles of the experts before `base`
@@ -188,8 +202,8 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
             w.nt = (int)(local / mte);
             w.row0 = start + mt * BM;
             w.row1 = (w.row0 + BM < end) ? w.row0 + BM : end;
+            if (EVEN) even_rows(start, end, mt, mte, &w.row0, &w.row1);
             w.mtile = (int)(mtiles_before + before + mt);
-            w.mt_in_group = (int)mt;
             w.valid = true;
             break;
         }
@@ -205,7 +219,7 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
 // (valid, expert, n tile, first row, one-past-last row, part, parts, exchange slot), the split tile's counter in the 9th.
 __global__ void gemm_plan_kernel(const void* offsets, int off64, int E, int ntiles_n, int ktiles, int max_split, int ncu, int* out)
 {
-    const WorkItem w = decode_work_item(offsets, off64, E, ntiles_n, ktiles, max_split, ncu);
+    const WorkItem w = decode_work_item<false>(offsets, off64, E, ntiles_n, ktiles, max_split, ncu);
     if (threadIdx.x == 0) {
         int* o = out + (int64_t)blockIdx.x * 9;
         o[0] = w.valid; o[1] = w.expert; o[2] = w.nt; o[3] = (int)w.row0; o[4] = (int)w.row1;
@@ -231,11 +245,14 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     const int ntiles_n = (EPI_IS_PAIR(EPI)) ? (int)((p.N + BN / 2 - 1) / (BN / 2)) : (int)((p.N + BN - 1) / BN);
     const int ktiles_seg = KTAIL ? (int)((p.K + BK - 1) / BK) : (int)(p.K / BK);
     const int ktiles = ktiles_seg * p.nseg;
-    const WorkItem item = decode_work_item(p.offsets, p.off64, p.E, ntiles_n, ktiles, p.max_split, p.num_cus);
+    const WorkItem item = decode_work_item<true>(p.offsets, p.off64, p.E, ntiles_n, ktiles, p.max_split, p.num_cus);
     if (!item.valid) return;
     const int expert = item.expert, nt = item.nt, part = item.part, nparts = item.nparts, split_item = item.split_item;
     const int64_t row0 = item.row0, row1 = item.row1;
     const int nrows = (int)(row1 - row0);
+    // the two rows of waves share the tile's 16-row blocks: wave rows [wrow0, wrow0 + wrows) of the tile
+    const int nblocks = (nrows + 15) / 16, wrow0 = __builtin_amdgcn_readfirstlane(wm * ((nblocks + 1) / 2) * 16);
+    const int wrows = __builtin_amdgcn_readfirstlane(wm == 0 ? (nrows < ((nblocks + 1) / 2) * 16 ? nrows : ((nblocks + 1) / 2) * 16) : (nrows > wrow0 ? nrows - wrow0 : 0));
     const int64_t n0 = (int64_t)nt * ((EPI_IS_PAIR(EPI)) ? BN / 2 : BN);
 
     // ---- row tables
@@ -330,7 +347,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     int a_frag_off[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
-        a_frag_off[ks] = (wm * WTM + (lane & 15)) * 128 + (((ks * 4 + (lane >> 4)) ^ ((lane >> 1) & 7)) << 4);
+        a_frag_off[ks] = (wrow0 + (lane & 15)) * 128 + (((ks * 4 + (lane >> 4)) ^ ((lane >> 1) & 7)) << 4);
     int b_frag_off[NN ? NB : 2];
     if (!NN) {
 #pragma unroll
@@ -358,13 +375,11 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[mb][nb][r] = 0.f;
 
-    // number of 16-row MFMA blocks of this wave that hold at least one real row
-    int mb_cnt = (nrows - wm * WTM + 15) / 16;
-    mb_cnt = mb_cnt < 0 ? 0 : (mb_cnt > MB ? MB : mb_cnt);
-    // the same in every lane: as a scalar it selects the wave's copy of the K loop with one branch, and the checks in
-    // the slab step are scalar branches (under a vector condition the compiler masks single MFMAs instead of branching
-    // around them, and the matrix cores ignore the mask)
-    mb_cnt = __builtin_amdgcn_readfirstlane(mb_cnt);
+    // number of 16-row MFMA blocks of this wave that hold at least one real row.  The same in every lane: as a scalar it
+    // selects the wave's copy of the K loop with one branch, and the checks in the slab step and the epilogue are scalar
+    // branches (under a vector condition the compiler masks single MFMAs instead of branching around them, and the matrix
+    // cores ignore the mask)
+    const int mb_cnt = __builtin_amdgcn_readfirstlane((wrows + 15) / 16);
 
     const int kb = ktiles * part / nparts;
     const int ke = ktiles * (part + 1) / nparts;
@@ -461,12 +476,13 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     // stage just freed), the two after that weight tile kt+3 (into the B stage just freed).  The next barrier then only
     // has to see the activation loads -- requested first, mostly cache hits -- and the weight tile requested a whole
     // tile earlier: the youngest LPT loads, weight loads that may well be waiting for HBM, stay in flight across it.
-    // NBLK: how many of the wave's MB 16-row blocks take part -- MB for every wave of a full tile; in a ragged tile each
-    // wave runs the copy of the loop that fits its own rows, the count of its live blocks rounded up to 0, 1, 2, MBH or MB
+    // NBLK: how many of the wave's MB 16-row blocks take part; each wave runs the copy of the loop that fits its own rows
     // (0: no MFMAs, no fragment reads, the wave only issues its loads and meets the barriers).  A compile-time count, not a
-    // check per block: a check is a scalar branch per MFMA, and a tail tile of a few rows spent more time on those branches
-    // than on its MFMAs.  Blocks inside the count that lie past the group work on whatever their LDS rows hold (rows past
-    // the last 32-row block are never loaded); every consumer of the accumulators masks rows past the group.
+    // check per block: a check is a scalar branch per MFMA, and a tile of a few rows spent more time on those branches
+    // than on its MFMAs.  Blocks inside the count that lie past the group work on whatever their LDS rows hold; every
+    // consumer of the accumulators masks rows past the group.  FULL: all activation loads are issued, those of rows past
+    // the tile re-read its last row (branches around loads split the loop body, which costs a tile of many blocks more
+    // than the loads do); without it, for tiles of at most half the blocks, loads of dead rows are dropped.
     auto mainloop = [&](auto nblk_tag, auto full_tag) {
         constexpr int NBLK = decltype(nblk_tag)::value;
         constexpr bool FULL = decltype(full_tag)::value;
@@ -491,20 +507,6 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
 #pragma unroll
         for (int mb = 0; mb < MBH; ++mb) read_a1(smem, 0, 0, mb, af[0]);
         int bs = 0;   // B stage of tile kt
-        // A tail tile of at most two row blocks has next to no MFMA work and would run through K several times faster than
-        // the full row tiles that share its weight tiles: the weight tiles it fetches are then gone from L2 again before
-        // those arrive (measured on the gate/up launch: 0.8 GB more fetched from memory with three such tails), and its
-        // requests compete with theirs.  The waves of such a tile therefore take at least PACE_CYCLES per K tile (a full tile
-        // cannot take less: 2048 cycles are its MFMAs alone), which keeps it just ahead of them -- close enough to act as their
-        // prefetcher.  Measured over eight routing draws of 8192 rows: the launches of few rounds 1-2 % faster; the gate/up
-        // launch, whose sixteen rounds are bound by the sum of the tiles' times, 2 % slower than with unpaced tails --
-        // the price of not fetching those weight tiles twice.  The copy of the loop is chosen per wave (its live blocks);
-        // whether it paces is decided per tile: only a tail that follows full row tiles of its group shares weight tiles
-        // with anybody -- a group's first tile (small batches, many experts with a few rows each) runs unpaced.
-        constexpr bool PACED = !FULL && NBLK <= 2;
-        const bool pace = PACED && item.mt_in_group > 0;
-        constexpr int64_t PACE_CYCLES = 2048;
-        int64_t pace_t0 = pace ? (int64_t)__builtin_readcyclecounter() : 0;
         // one K tile; SLAB: the activation loads it requests (for tile kt+2) fetch the slab image instead
         auto tile = [&](int kt, auto slab_tag) {
             constexpr bool SLAB = decltype(slab_tag)::value;
@@ -520,10 +522,6 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
                 // ra / rb: where the fragments of the next half step come from; for the last one of a tile, the first of
                 // the next tile.  (After the last tile this fetches fragments nobody uses.)
                 if (hs == 3) {
-                    if (pace) {   // (see PACE_CYCLES; a sleep is 128 cycles, so the count bounds the wait whatever the counter's rate)
-                        for (int n = 0; n < 24 && (int64_t)__builtin_readcyclecounter() - pace_t0 < PACE_CYCLES; ++n) __builtin_amdgcn_s_sleep(2);
-                        pace_t0 = (int64_t)__builtin_readcyclecounter();
-                    }
                     __builtin_amdgcn_s_waitcnt(0x0F70 | LPT);   // all but the youngest LPT loads: tile kt+1 has landed
                     __syncthreads();                            // for every wave; and every wave is done reading tile kt
                 }
@@ -584,11 +582,14 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
         __builtin_amdgcn_s_waitcnt(0x0F70);   // loads past the last tile must not land in the epilogue's staging
         __syncthreads();   // operand buffers are free for the epilogue staging
     };
-    // full tiles run a loop body without any checks; in a ragged tile the activation loads of dead row blocks are dropped
-    // and every wave takes the loop for the number of its live blocks (a scalar: the same in all lanes of the wave)
-    if (live_rows == BM) mainloop(std::integral_constant<int, MB>{}, std::true_type{});
-    else if (mb_cnt > MBH) mainloop(std::integral_constant<int, MB>{}, std::false_type{});
-    else if (mb_cnt > 2) mainloop(std::integral_constant<int, MBH>{}, std::false_type{});
+    // (one scalar compare chain per wave; the counts of a tile's two rows of waves differ by at most one)
+    if (nblocks > MB) {
+        if (mb_cnt == MB) mainloop(std::integral_constant<int, MB>{}, std::true_type{});
+        else if (mb_cnt == 7) mainloop(std::integral_constant<int, 7>{}, std::true_type{});
+        else if (mb_cnt == 6) mainloop(std::integral_constant<int, 6>{}, std::true_type{});
+        else if (mb_cnt == 5) mainloop(std::integral_constant<int, 5>{}, std::true_type{});
+        else mainloop(std::integral_constant<int, MBH>{}, std::true_type{});
+    } else if (mb_cnt > 2) mainloop(std::integral_constant<int, MBH>{}, std::false_type{});
     else if (mb_cnt == 2) mainloop(std::integral_constant<int, 2>{}, std::false_type{});
     else if (mb_cnt == 1) mainloop(std::integral_constant<int, 1>{}, std::false_type{});
     else mainloop(std::integral_constant<int, 0>{}, std::false_type{});
@@ -611,6 +612,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
         const uint32_t slot_bytes = (uint32_t)split_item * (uint32_t)(BM * BN * sizeof(float));
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
+            if (mb < mb_cnt)
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 u32x4_t v;
@@ -629,6 +631,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
         const uint32_t first_bytes = (uint32_t)(split_item - part) * (uint32_t)(BM * BN * sizeof(float));
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
+            if (mb < mb_cnt)
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 const uint32_t o = first_bytes + (uint32_t)(((mb * NB + nb) * NTHREADS + tid) * 16);
@@ -684,7 +687,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
                     }
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb) {
-                        int r = wm * WTM + mb * 16 + (lane & 15);
+                        int r = wrow0 + mb * 16 + (lane & 15);
                         if (r >= nrows) r = nrows - 1;
                         bf16x8_t v = {};
                         if (live) v = *(const bf16x8_t*)(Q + (row0 + r) * 16 + 8 * kc);
@@ -731,7 +734,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb) {
                         bf16x8_t v = {};
-                        if (live) v = *(const bf16x8_t*)(img + (wm * WTM + mb * 16 + (lane & 15)) * 32);
+                        if (live) v = *(const bf16x8_t*)(img + (wrow0 + mb * 16 + (lane & 15)) * 32);
                         sa[s][mb] = v;
                     }
                     continue;
@@ -748,7 +751,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
                 }
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) {
-                    int r = wm * WTM + mb * 16 + (lane & 15);
+                    int r = wrow0 + mb * 16 + (lane & 15);
                     if (r >= nrows) r = nrows - 1;
                     bf16x8_t v = {};
                     if (live) v = *(const bf16x8_t*)(Q + (row0 + r) * 16 + 8 * kc);
@@ -783,7 +786,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     float rs[MB];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
-        const int rl = wm * WTM + mb * 16 + mrow;
+        const int rl = wrow0 + mb * 16 + mrow;
         rs[mb] = (p.row_scale && rl < nrows) ? p.row_scale[row0 + rl] : 1.f;
     }
     auto pack4 = [](float a, float b, float c, float d) {
@@ -815,19 +818,19 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
             for (int it = 0; it < iters; ++it) {
                 const int m = it * rows_per_it + lane / lpr;
                 const u32x4_t v = *(const u32x4_t*)(stg + m * (sw * 2) + slot * 16);
-                const int rl = wm * WTM + m;
+                const int rl = wrow0 + m;
                 const int64_t n = ncol0 + swz(sw, m, slot) * 8;
-                if (rl < nrows && n < p.N) *(u32x4_t*)(Y + s_outrow[rl] * ld + n) = v;
+                if (m < wrows && n < p.N) *(u32x4_t*)(Y + s_outrow[rl] * ld + n) = v;
             }
         } else {
 #pragma unroll 8
             for (int it = 0; it < iters; ++it) {
                 const int m = it * rows_per_it + lane / lpr;
                 const u32x4_t v = *(const u32x4_t*)(stg + m * (sw * 2) + slot * 16);
-                const int rl = wm * WTM + m;
+                const int rl = wrow0 + m;
                 const int64_t n = ncol0 + swz(sw, m, slot) * 8;
                 const uint32_t orow = scattered ? (uint32_t)s_outrow[rl] : (uint32_t)rl;
-                const uint32_t off = (rl < nrows && n < p.N) ? orow * ld2 + (uint32_t)n * 2 : 0xFFFFFFF0u;
+                const uint32_t off = (m < wrows && n < p.N) ? orow * ld2 + (uint32_t)n * 2 : 0xFFFFFFF0u;
                 __builtin_amdgcn_raw_buffer_store_b128(v, ybuf, off, 0, 0);
             }
         }
@@ -912,11 +915,11 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
 #pragma unroll
                     for (int reg = 0; reg < 4; ++reg) sum[reg] += v[reg];
                 }
-                const int rl0 = wm * WTM + mb * 16 + 4 * tg;
-                float* dst = p.CCP[0] + ((int64_t)nt * p.cc_rows + row0 + rl0) * 16 + ti;
+                const int rl0 = mb * 16 + 4 * tg;   // row of this wave's rows
+                float* dst = p.CCP[0] + ((int64_t)nt * p.cc_rows + row0 + wrow0 + rl0) * 16 + ti;
 #pragma unroll
                 for (int reg = 0; reg < 4; ++reg)
-                    if (rl0 + reg < nrows) dst[reg * 16] = sum[reg];
+                    if (rl0 + reg < wrows) dst[reg * 16] = sum[reg];
             }
         }
     } else {  // MOE_EPI_SWIGLU_BWD: acc = dh; dgate = dh * up * sig(g) * (1 + g (1 - sig(g))), dup = dh * silu(g)
@@ -940,9 +943,9 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
         u32x4_t g8[PD], u8[PD];
         auto seg_addr = [&](int it, uint32_t& hoff, uint32_t& yoff) {
             const int m = it * ROWS_PER_IT + lane / LPR;
-            const int rl = wm * WTM + m;
+            const int rl = wrow0 + m;
             const int64_t n = n0 + wn * WTN + swz(WTN, m, slot) * 8;
-            const bool valid = rl < nrows && n < p.N;
+            const bool valid = m < wrows && n < p.N;
             const uint32_t row = (uint32_t)rl;
             hoff = valid ? row * ldh2 + (uint32_t)n * 2 : 0xFFFFFFF0u;   // out of range: reads zeros, writes nothing
             yoff = valid ? row * ldy2 + (uint32_t)n * 2 : 0xFFFFFFF0u;
@@ -1054,7 +1057,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
                     // their dh need not be finite: the accumulators of row blocks without real rows can hold anything (an
                     // MFMA that the compiler left under an execution mask instead of a branch runs all the same -- the
                     // matrix cores ignore the mask -- on fragments of rows that were never loaded), and 0 * inf is not 0.
-                    if (FUSED && wm * WTM + m >= nrows) og8[q][w2] = ou8[q][w2] = 0u;
+                    if (FUSED && m >= wrows) og8[q][w2] = ou8[q][w2] = 0u;
                 }
                 if (it + PD < NIT) fetch(it + PD, it % PD);
                 __builtin_amdgcn_raw_buffer_store_b128(og8[q], dgbuf, yoff, 0, STREAMING);
@@ -1080,7 +1083,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
                         *(u32x4_t*)(stg + m * (WTN * 2) + slot * 16) = mat == 0 ? og8[q] : (mat == 1 ? ou8[q] : hh8[q]);
                     }
                     asm volatile("" ::: "memory");   // the reads below follow the writes above in program order
-                    const uint8_t* pim = rc_img + mat * RC_IMG_BYTES + (wm * WTM + blk * 32 + trow) * 32 + (ti & 3) * 8;
+                    const uint8_t* pim = rc_img + mat * RC_IMG_BYTES + (wrow0 + blk * 32 + trow) * 32 + (ti & 3) * 8;
                     pf[gen] = tr_read(pim, pim + 4 * 32);
 #pragma unroll
                     for (int ib = 0; ib < IBLK; ++ib) {
@@ -1145,11 +1148,11 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
 #pragma unroll
                         for (int reg = 0; reg < 4; ++reg) sum[reg] += v[reg];
                     }
-                    const int rl0 = wm * WTM + wn * 32 + rb * 16 + 4 * tg;
-                    float* dst = p.CCP[mat] + ((int64_t)nt * p.cc_rows + row0 + rl0) * 16 + ti;
+                    const int rl0 = wn * 32 + rb * 16 + 4 * tg;   // row of this wave's rows
+                    float* dst = p.CCP[mat] + ((int64_t)nt * p.cc_rows + row0 + wrow0 + rl0) * 16 + ti;
 #pragma unroll
                     for (int reg = 0; reg < 4; ++reg)
-                        if (rl0 + reg < nrows) dst[reg * 16] = sum[reg];
+                        if (rl0 + reg < wrows) dst[reg * 16] = sum[reg];
                 }
             __builtin_amdgcn_s_waitcnt(0xC07F);
             __syncthreads();   // the slices are free again for the exchange below

@@ -443,3 +443,21 @@ def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case):
 def max_split_ok(pair):
     return not pair
 
+
+
+@pytest.mark.parametrize("counts", [[257, 272, 273, 1], [511, 512, 513, 15], [769, 16, 1025, 0], [144, 145, 287, 31]])
+@pytest.mark.parametrize("layout", ["k_contiguous", "n_contiguous"])
+def test_grouped_gemm_rows_dealt_evenly_to_tiles(dev, oracle, counts, layout):
+    """Groups of one block more or less than a whole number of tiles: every row exactly once, whatever tile it falls into."""
+    ops = _ops()
+    torch.manual_seed(21)
+    E, K, N = len(counts), 512, 320
+    R = sum(counts)
+    sei = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ssi = torch.randperm(R, generator=torch.Generator().manual_seed(2))
+    X, W = torch.randn(R, K).bfloat16(), (torch.randn(E, K, N) * 0.05).bfloat16()
+    Wd = W.permute(0, 2, 1).contiguous().to(dev).permute(0, 2, 1) if layout == "k_contiguous" else W.to(dev)
+    y = ops.scatter2scatter(X.to(dev), Wd, sei.to(dev), ssi.to(dev), 1)
+    ref = oracle.scatter2scatter_lora(X, W, None, None, 0, sei, ssi, 1)
+    # one bf16 rounding of fp32 sums: half an ulp, 2^-9 of the value, and the sum's own error far below it
+    assert float((y.float().cpu() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
