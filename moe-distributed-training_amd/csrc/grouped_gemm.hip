@@ -76,8 +76,13 @@ __device__ __forceinline__ i32x4_t make_buffer(const void* base, uint32_t num_re
     r.w = 0x00020000;                                                 // 32-bit data format
     return r;
 }
+// NT: non-temporal, for data that nobody else will read again.
+template <bool NT = false>
 __device__ __forceinline__ void load_to_lds_16(i32x4_t rsrc, uint32_t lane_off, uint32_t uniform_off, uint32_t lds_addr)
 {
+    if constexpr (NT)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(lane_off), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(uniform_off)) : "memory", "m0");
+    else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(lane_off), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(uniform_off)) : "memory", "m0");
 }
 
@@ -94,6 +99,7 @@ struct WorkItem {
     int part, nparts;          // K part of a split tile (0 of 1: whole tile)
     int split_item;            // exchange slot of this part (the slots of a tile are consecutive, in part order)
     int split_tile;            // counter of the split tile
+    bool only_tile;            // the group fits in this one row tile
     int mtile;                 // number of the row tile among all row tiles (experts in order, BM rows each)
 };
 
@@ -185,6 +191,7 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
         w.row0 = uniform_i64(row0);
         w.row1 = uniform_i64(row1);
         w.mtile = __builtin_amdgcn_readfirstlane((int)(before + mt));
+        w.only_tile = __builtin_amdgcn_readfirstlane((int)(mte == 1)) != 0;
         w.valid = true;
     } else {
         int64_t mtiles_before = 0;   // row tiles of the experts before `base`
@@ -204,6 +211,7 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
             w.row1 = (w.row0 + BM < end) ? w.row0 + BM : end;
             if (EVEN) even_rows(start, end, mt, mte, &w.row0, &w.row1);
             w.mtile = (int)(mtiles_before + before + mt);
+            w.only_tile = mte == 1;
             w.valid = true;
             break;
         }
@@ -244,7 +252,8 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     // ---- work item -> (expert, n tile, m tile, K part)
     const int ntiles_n = (EPI_IS_PAIR(EPI)) ? (int)((p.N + BN / 2 - 1) / (BN / 2)) : (int)((p.N + BN - 1) / BN);
     const int ktiles_seg = KTAIL ? (int)((p.K + BK - 1) / BK) : (int)(p.K / BK);
-    const int ktiles = ktiles_seg * p.nseg;
+    constexpr bool TWO_SEG = EPI == MOE_EPI_STORE;   // (the only epilogue that launches with two K segments)
+    const int ktiles = TWO_SEG ? ktiles_seg * p.nseg : ktiles_seg;
     const WorkItem item = decode_work_item<true>(p.offsets, p.off64, p.E, ntiles_n, ktiles, p.max_split, p.num_cus);
     if (!item.valid) return;
     const int expert = item.expert, nt = item.nt, part = item.part, nparts = item.nparts, split_item = item.split_item;
@@ -286,12 +295,12 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     // (KTAIL: the masked loads of a partial K tile use the offset OUT_OF_RANGE, which must lie at or above the descriptors'
     // range -- with the full 32-bit range it would be a valid offset and the load would touch memory 4 GiB past the base)
     constexpr uint32_t LOAD_RANGE = KTAIL ? 0x80000000u : 0xFFFFFFFFu;
-    const i32x4_t a_buf0 = make_buffer(p.X[0] + a_row_base * p.ldx, LOAD_RANGE), a_buf1 = make_buffer((p.X[1] ? p.X[1] : p.X[0]) + a_row_base * p.ldx, LOAD_RANGE);
+    const i32x4_t a_buf0 = make_buffer(p.X[0] + a_row_base * p.ldx, LOAD_RANGE), a_buf1 = make_buffer((TWO_SEG && p.X[1] ? p.X[1] : p.X[0]) + a_row_base * p.ldx, LOAD_RANGE);
     // B: offsets within this expert's matrix.  For the SwiGLU pair image rows [0,128) come from W[0] and [128,256)
     // from W[1], which are whole load instructions (the first and second half of a wave's LPT); otherwise W[0] / W[1]
     // are the two K segments.
     uint32_t b_off[LPT];
-    const i32x4_t b_buf0 = make_buffer(p.W[0] + (int64_t)expert * p.swe, LOAD_RANGE), b_buf1 = make_buffer((p.W[1] ? p.W[1] : p.W[0]) + (int64_t)expert * p.swe, LOAD_RANGE);
+    const i32x4_t b_buf0 = make_buffer(p.W[0] + (int64_t)expert * p.swe, LOAD_RANGE), b_buf1 = make_buffer(((TWO_SEG || EPI_IS_PAIR(EPI)) && p.W[1] ? p.W[1] : p.W[0]) + (int64_t)expert * p.swe, LOAD_RANGE);
     if (!NN) {
         // B image as A: row = n (BN rows of 64 k)
 #pragma unroll
@@ -400,9 +409,19 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     // load instructions (their rows differ by multiples of 64).
     constexpr uint32_t OUT_OF_RANGE = 0xFFFFFFF0u;
     const uint32_t ktail_kq = (uint32_t)(((lane & 7) ^ (((lane >> 4) + 4 * (wave & 1)) & 7)) * 8);
-    auto issue_a = [&](int kt, int jj, int stage, bool ragged) {
+    // Only tile of its group: the K tiles are walked from a start that differs from one output tile to the next (and wraps
+    // round).  With K-contiguous weights of a power-of-two pitch the 128-byte pieces that all workgroups want at one time
+    // would otherwise lie on a few memory channels (8 experts x 6 rows, K=4096, N=14336: 4.8 TB/s of weights, rotated 6.4; with
+    // several row tiles per group, rotating by XCD measured no faster).
+    const int krot = __builtin_amdgcn_readfirstlane((int)((uint32_t)(nt + expert * 8) % (uint32_t)(ke - kb)));
+    auto rotated = [&](int kt) {
+        kt += krot;
+        return kt >= ke ? kt - (ke - kb) : kt;
+    };
+    auto issue_a = [&](int kt, int jj, int stage, bool ragged, auto once) {
         kt = __builtin_amdgcn_readfirstlane(kt < ke ? kt : ke - 1);
-        const int seg = (kt >= ktiles_seg) ? 1 : 0;
+        if constexpr (decltype(once)::value) kt = rotated(kt);
+        const int seg = (TWO_SEG && kt >= ktiles_seg) ? 1 : 0;
         const uint32_t k0 = (uint32_t)(kt - seg * ktiles_seg) * BK;
         if constexpr (KTAIL) {
             uint32_t voff = a_off[jj], soff = k0 * 2;
@@ -420,9 +439,11 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
         const i32x4_t d = jj == 0 ? q_buf0 : (jj == 1 ? q_buf1 : (jj == 2 ? l_buf0 : l_buf1));
         load_to_lds_16(d, jj < 2 ? slab_off_q : slab_off_l, (uint32_t)(jj < 2 ? row0 : n0) * 32u, dst);
     };
-    auto issue_b = [&](int kt, int idx, int stage) {
+    auto issue_b = [&](int kt, int idx, int stage, auto nt_tag) {
+        constexpr bool NT = decltype(nt_tag)::value;
         kt = __builtin_amdgcn_readfirstlane(kt < ke ? kt : ke - 1);
-        const int seg = (kt >= ktiles_seg) ? 1 : 0;
+        if constexpr (NT) kt = rotated(kt);
+        const int seg = (TWO_SEG && kt >= ktiles_seg) ? 1 : 0;
         const uint32_t k0 = (uint32_t)(kt - seg * ktiles_seg) * BK;
         const bool second = (EPI_IS_PAIR(EPI)) ? (idx >= LPT / 2) : (seg != 0);
         if constexpr (KTAIL) {
@@ -433,9 +454,9 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
                 voff = in ? voff + soff : OUT_OF_RANGE;
                 soff = 0;
             }
-            load_to_lds_16(second ? b_buf1 : b_buf0, voff, soff, smem_u + B_REGION + stage * B_STAGE_BYTES + idx * (NWAVES * 1024));
+            load_to_lds_16<NT>(second ? b_buf1 : b_buf0, voff, soff, smem_u + B_REGION + stage * B_STAGE_BYTES + idx * (NWAVES * 1024));
         } else {
-        load_to_lds_16(second ? b_buf1 : b_buf0, b_off[idx], NN ? k0 * (uint32_t)p.ldw * 2 : k0 * 2, smem_u + B_REGION + stage * B_STAGE_BYTES + idx * (NWAVES * 1024));
+        load_to_lds_16<NT>(second ? b_buf1 : b_buf0, b_off[idx], NN ? k0 * (uint32_t)p.ldw * 2 : k0 * 2, smem_u + B_REGION + stage * B_STAGE_BYTES + idx * (NWAVES * 1024));
         }
     };
 
@@ -483,22 +504,22 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     // consumer of the accumulators masks rows past the group.  FULL: all activation loads are issued, those of rows past
     // the tile re-read its last row (branches around loads split the loop body, which costs a tile of many blocks more
     // than the loads do); without it, for tiles of at most half the blocks, loads of dead rows are dropped.
-    auto mainloop = [&](auto nblk_tag, auto full_tag) {
+    auto mainloop = [&](auto nblk_tag, auto full_tag, auto once) {
         constexpr int NBLK = decltype(nblk_tag)::value;
         constexpr bool FULL = decltype(full_tag)::value;
 #pragma unroll
-        for (int i = 0; i < LPT; ++i) issue_a(kb, i, 0, !FULL);
+        for (int i = 0; i < LPT; ++i) issue_a(kb, i, 0, !FULL, once);
 #pragma unroll
-        for (int i = 0; i < LPT; ++i) issue_b(kb, i, 0);
+        for (int i = 0; i < LPT; ++i) issue_b(kb, i, 0, once);
         if (lds_slabs && kb + 1 == ke) {
 #pragma unroll
             for (int i = 0; i < LPT; ++i) issue_slab(i, 1);
         } else {
 #pragma unroll
-            for (int i = 0; i < LPT; ++i) issue_a(kb + 1, i, 1, !FULL);
+            for (int i = 0; i < LPT; ++i) issue_a(kb + 1, i, 1, !FULL, once);
         }
 #pragma unroll
-        for (int i = 0; i < LPT; ++i) issue_b(kb + 1, i, 1);
+        for (int i = 0; i < LPT; ++i) issue_b(kb + 1, i, 1, once);
         __builtin_amdgcn_s_waitcnt(0x0F70 | LPT);   // everything but weight tile kb+1 has landed
         __syncthreads();                            // (also: every wave has read the row tables that share B stage 2)
         bf16x8_t af[2][MBH], bf[2][NB];
@@ -556,12 +577,12 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
                         else if (q - nbr < MBH) { if ((nhs & 1) * MBH + (q - nbr) < NBLK) read_a1(ra, nhs >> 1, nhs & 1, q - nbr, af[cur_a ^ 1]); __builtin_amdgcn_sched_barrier(0); }
                     }
                     if (hs == 3 && m % A_LOAD_GAP == 0 && m / A_LOAD_GAP < LPT) {
-                        if (SLAB) issue_slab(m / A_LOAD_GAP, as); else issue_a(kt + 2, m / A_LOAD_GAP, as, !FULL);
+                        if (SLAB) issue_slab(m / A_LOAD_GAP, as); else issue_a(kt + 2, m / A_LOAD_GAP, as, !FULL, once);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     const int gb = hs * MFMAS_PER_STEP + m;   // MFMAs since the tile's first
                     if (hs < 3 && gb % B_LOAD_GAP == 0 && gb / B_LOAD_GAP < LPT) {
-                        issue_b(kt + 2, gb / B_LOAD_GAP, bs2);
+                        issue_b(kt + 2, gb / B_LOAD_GAP, bs2, once);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     if (mh * MBH + mb < NBLK)
@@ -583,16 +604,24 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
         __syncthreads();   // operand buffers are free for the epilogue staging
     };
     // (one scalar compare chain per wave; the counts of a tile's two rows of waves differ by at most one)
+    // The only tile of its group is also the only reader of its weight tiles: their loads are non-temporal (a streaming read
+    // reaches 7.0 TB/s that way, 6.1 without; 24 tokens over 8 experts: 589 -> 539 us forward.  Where several row tiles share the
+    // weight tiles the hint costs 2 %: it works against the sharing in L2).
+    using T_ = std::true_type;
+    using F_ = std::false_type;
     if (nblocks > MB) {
-        if (mb_cnt == MB) mainloop(std::integral_constant<int, MB>{}, std::true_type{});
-        else if (mb_cnt == 7) mainloop(std::integral_constant<int, 7>{}, std::true_type{});
-        else if (mb_cnt == 6) mainloop(std::integral_constant<int, 6>{}, std::true_type{});
-        else if (mb_cnt == 5) mainloop(std::integral_constant<int, 5>{}, std::true_type{});
-        else mainloop(std::integral_constant<int, MBH>{}, std::true_type{});
-    } else if (mb_cnt > 2) mainloop(std::integral_constant<int, MBH>{}, std::false_type{});
-    else if (mb_cnt == 2) mainloop(std::integral_constant<int, 2>{}, std::false_type{});
-    else if (mb_cnt == 1) mainloop(std::integral_constant<int, 1>{}, std::false_type{});
-    else mainloop(std::integral_constant<int, 0>{}, std::false_type{});
+        if (item.only_tile) {
+            if (mb_cnt > 6) mainloop(std::integral_constant<int, MB>{}, T_{}, T_{});
+            else mainloop(std::integral_constant<int, 6>{}, T_{}, T_{});
+        } else if (mb_cnt == MB) mainloop(std::integral_constant<int, MB>{}, T_{}, F_{});
+        else if (mb_cnt == 7) mainloop(std::integral_constant<int, 7>{}, T_{}, F_{});
+        else if (mb_cnt == 6) mainloop(std::integral_constant<int, 6>{}, T_{}, F_{});
+        else if (mb_cnt == 5) mainloop(std::integral_constant<int, 5>{}, T_{}, F_{});
+        else mainloop(std::integral_constant<int, MBH>{}, T_{}, F_{});
+    } else if (mb_cnt > 2) mainloop(std::integral_constant<int, MBH>{}, F_{}, T_{});
+    else if (mb_cnt == 2) mainloop(std::integral_constant<int, 2>{}, F_{}, T_{});
+    else if (mb_cnt == 1) mainloop(std::integral_constant<int, 1>{}, F_{}, T_{});
+    else mainloop(std::integral_constant<int, 0>{}, F_{}, T_{});
     if (!p.y_grouped) {   // the output row table again: weight tiles have passed through its place
         for (int r = tid; r < BM; r += NTHREADS) s_outrow[r] = load_idx(p.pos, row0 + ((r < nrows) ? r : nrows - 1), p.pos64);
         __syncthreads();
@@ -1279,7 +1308,7 @@ bool moe_gemm_mfma_supported(const MoeGemmParams& p, int64_t R)
     if (!al16(p.X[0]) || !al16(p.X[1]) || !al16(p.W[0]) || !al16(p.W[1])) return false;
     for (int i = 0; i < MOE_MAX_SLABS; ++i)
         if (!al16(p.Q[i]) || !al16(p.LB[i])) return false;   // (slabs beyond these: multiples of 16 bytes from Q[0] / LB[0], checked below)
-    if (p.nseg < 1 || p.nseg > 2 || p.nslab < 0 || (p.slab_mode == 1 && p.nslab % 2 != 0)) return false;
+    if (p.nseg < 1 || p.nseg > 2 || (p.nseg == 2 && p.epi != MOE_EPI_STORE) || p.nslab < 0 || (p.slab_mode == 1 && p.nslab % 2 != 0)) return false;
     if (p.K % BK != 0 && p.epi != MOE_EPI_STORE) return false;   // a partial last K tile: the plain epilogue only
     if (p.nslab > MOE_MAX_SLABS) {
         const bool epi_ok = p.epi == MOE_EPI_STORE || (!p.nn && (p.epi == MOE_EPI_SWIGLU || p.epi == MOE_EPI_SWIGLU_BWD));

@@ -461,3 +461,21 @@ def test_grouped_gemm_rows_dealt_evenly_to_tiles(dev, oracle, counts, layout):
     ref = oracle.scatter2scatter_lora(X, W, None, None, 0, sei, ssi, 1)
     # one bf16 rounding of fp32 sums: half an ulp, 2^-9 of the value, and the sum's own error far below it
     assert float((y.float().cpu() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("rows", [1, 33, 128, 129, 176, 255, 256])
+@pytest.mark.parametrize("layout,K,N", [("k_contiguous", 1024, 1280), ("n_contiguous", 1024, 1280), ("k_contiguous", 64, 8), ("k_contiguous", 1000, 264)])
+def test_grouped_gemm_single_tile_groups(dev, oracle, rows, layout, K, N):
+    """Groups of one row tile walk the K tiles from a start of their own: every start, one K tile in all, a partial last one."""
+    ops = _ops()
+    torch.manual_seed(22)
+    E = 4
+    counts = [rows, 0, 1, rows]
+    sei = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ssi = torch.randperm(sum(counts), generator=torch.Generator().manual_seed(3))
+    X, W = torch.randn(sum(counts), K).bfloat16(), (torch.randn(E, K, N) * 0.05).bfloat16()
+    Wd = W.permute(0, 2, 1).contiguous().to(dev).permute(0, 2, 1) if layout == "k_contiguous" else W.to(dev)
+    y = ops.scatter2scatter(X.to(dev), Wd, sei.to(dev), ssi.to(dev), 1)
+    ref = oracle.scatter2scatter_lora(X, W, None, None, 0, sei, ssi, 1)
+    # one bf16 rounding of fp32 sums: half an ulp, 2^-9 of the value, and the sum's own error far below it
+    assert float((y.float().cpu() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
