@@ -1,4 +1,5 @@
-"""ctypes binding of libmoe_hip.so (C ABI declared in include/moe_hip.h).  No compute happens here."""
+"""ctypes binding of libmoe_hip.so (C ABI declared in include/moe_hip.h), and the torch extension module over the same
+library (csrc/torch_layer.cpp: the autograd functions).  No compute happens here."""
 from __future__ import annotations
 
 import ctypes
@@ -75,6 +76,11 @@ def _load() -> ctypes.CDLL:
 
 
 lib = _load()
+try:
+    from . import _native as native   # noqa: E402  (resolves libmoe_hip.so to the library loaded above)
+except ImportError as e:
+    raise ImportError(f"{os.path.join(_HERE, '_native.so')} is missing or does not fit: build it with "
+                      f"python -c 'import __graft_entry__ as g; g.build()' ({e})") from e
 
 
 def check(status: int, what: str) -> None:

@@ -1,0 +1,702 @@
+// The autograd side of the package in C++: the layer, the expert MLP, a single grouped projection and the router as
+// torch::autograd functions over the C ABI of libmoe_hip.so (include/moe_hip.h).  No device code and no arithmetic here:
+// shape checks, allocation of outputs and interims, and the order of the library calls, all on the current stream.
+//
+// Why native: a small layer step enqueues some twenty kernels of a few microseconds each; with the same sequence in Python
+// the host spent about 10 us per library call (argument conversion, allocation, stream lookup, the interpreter lock of the
+// backward thread) and the GPU waited for it.
+#include <torch/extension.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include "../../include/moe_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+using OptTensor = std::optional<Tensor>;
+
+// Python's assert statements of the reference's entry points: an AssertionError there, and here
+struct AssertionFailure : std::runtime_error { using std::runtime_error::runtime_error; };
+#define MOE_ASSERT(cond, msg) do { if (!(cond)) throw AssertionFailure(msg); } while (0)
+
+inline void check(int status, const char* what)
+{
+    TORCH_CHECK(status == MOE_OK, what, " failed: ", moe_hip_strerror(status), " (status ", status, ")");
+}
+
+inline int dtype_code(const Tensor& t)
+{
+    switch (t.scalar_type()) {
+    case at::kBFloat16: return MOE_BF16;
+    case at::kHalf: return MOE_F16;
+    case at::kFloat: return MOE_F32;
+    default: TORCH_CHECK_TYPE(false, "unsupported dtype ", t.scalar_type(), ": the HIP kernels take bfloat16, float16 or float32");
+    }
+}
+
+inline int is64(const Tensor& t)
+{
+    if (t.scalar_type() == at::kLong) return 1;
+    TORCH_CHECK_TYPE(t.scalar_type() == at::kInt, "index tensors must be int32 or int64, got ", t.scalar_type());
+    return 0;
+}
+
+inline void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+inline void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+inline void require_gpu(std::initializer_list<const Tensor*> ts)
+{
+    const Tensor* first = nullptr;
+    for (const Tensor* t : ts) {
+        if (!t->defined()) continue;
+        TORCH_CHECK(t->is_cuda(), "moe_distributed_training_amd runs on the GPU only (got a CPU tensor); there is no host fallback");
+        if (!first) first = t;
+        TORCH_CHECK(t->device() == first->device(), "all tensors must live on the same device");
+    }
+}
+
+inline Tensor bytes_on(const Tensor& like, size_t n)
+{
+    return at::empty({(int64_t)(n < 256 ? 256 : n)}, like.options().dtype(at::kByte));
+}
+
+inline Tensor unit_inner(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
+
+inline bool wants_grad(std::initializer_list<const Tensor*> ts)
+{
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor* t : ts)
+        if (t->defined() && t->requires_grad()) return true;
+    return false;
+}
+
+inline Tensor val(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+// (an autograd function takes an absent tensor as an empty optional, not as an undefined tensor)
+inline OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); }
+
+// ---------------------------------------------------------------------------------------------------------------
+// library calls with their allocations
+// ---------------------------------------------------------------------------------------------------------------
+Tensor combine(const Tensor& y, const Tensor& gates, const int32_t* inv, int64_t k, int64_t T, const float* extra_coef = nullptr,
+               const Tensor& extra_rows = Tensor(), int64_t n_extra = 0)
+{
+    Tensor out = at::empty({T, y.size(1)}, y.options());
+    check(moe_combine(ptr(y), y.stride(0), ptr(out), out.stride(0), ptr(gates), gates.defined() ? dtype_code(gates) : 0, inv, (int)k, T, y.size(1),
+                      dtype_code(y), extra_coef, ptr(extra_rows), extra_rows.defined() ? extra_rows.stride(0) : 0, (int)n_extra, stream_of(y)),
+          "moe_combine");
+    return out;
+}
+
+Tensor combine_dgates(const Tensor& y, const Tensor& dout, int64_t k, at::ScalarType dt, const int32_t* inv)
+{
+    Tensor dg = at::empty({dout.size(0), k}, y.options().dtype(dt));
+    check(moe_combine_dgates(ptr(y), y.stride(0), ptr(dout), dout.stride(0), ptr(dg), dtype_code(dg), inv, (int)k, dout.size(0), y.size(1),
+                             dtype_code(y), stream_of(y)), "moe_combine_dgates");
+    return dg;
+}
+
+Tensor group_rows(const Tensor& src, const void* pos, int pos64, int64_t n, int64_t fan_out, const Tensor& coeff = Tensor())
+{
+    Tensor out = at::empty({n, src.size(1)}, src.options());
+    check(moe_group_rows(ptr(src), src.stride(0), ptr(out), out.stride(0), pos, pos64, (int)fan_out, ptr(coeff),
+                         coeff.defined() ? dtype_code(coeff) : 0, n, src.size(1), dtype_code(src), stream_of(src)), "moe_group_rows");
+    return out;
+}
+
+Tensor group_bwd_w(const Tensor& dy, const Tensor& x, const void* offsets, int off64, int64_t E)
+{
+    Tensor dw = at::empty({E, x.size(1), dy.size(1)}, dy.options());
+    check(moe_group_bwd_w(ptr(dy), dy.stride(0), dy.stride(1), ptr(x), x.stride(0), x.stride(1), ptr(dw), dw.stride(0), dw.stride(1), dw.stride(2),
+                          offsets, off64, (int)E, x.size(0), x.size(1), dy.size(1), dtype_code(dy), stream_of(dy)), "moe_group_bwd_w");
+    return dw;
+}
+
+Tensor scatter2scatter(const Tensor& X, const Tensor& W, const Tensor& A, const Tensor& B, double scaling, const Tensor& ssi, const Tensor& eo,
+                       int64_t k, bool x_grouped, bool y_grouped)
+{
+    const int64_t L = ssi.size(0), E = W.size(0), K = W.size(1), N = W.size(2);
+    const int rank = A.defined() ? (int)A.size(2) : 0;
+    Tensor out = at::empty({L, N}, X.options());
+    if (L == 0) return out;
+    Tensor ws = bytes_on(X, moe_scatter2scatter_workspace_bytes(L, (int)E, K, N, rank));
+    auto st = [](const Tensor& t, int i) { return t.defined() ? t.stride(i) : (int64_t)0; };
+    check(moe_scatter2scatter(ptr(X), X.stride(0), X.stride(1), ptr(W), W.stride(0), W.stride(1), W.stride(2), ptr(A), st(A, 0), st(A, 1), st(A, 2),
+                              ptr(B), st(B, 0), st(B, 1), st(B, 2), rank, (float)scaling, ptr(out), out.stride(0), out.stride(1), ptr(ssi), is64(ssi),
+                              ptr(eo), is64(eo), (int)E, L, K, N, (int)k, x_grouped, y_grouped, dtype_code(X), ptr(ws), (size_t)ws.numel(), stream_of(X)),
+          "moe_scatter2scatter");
+    return out;
+}
+
+Tensor offsets_from_sorted(const Tensor& sei, int64_t E)
+{
+    Tensor s = sei.contiguous(), out = at::empty({E}, s.options());
+    check(moe_expert_offsets(ptr(s), is64(s), s.numel(), (int)E, ptr(out), is64(out), stream_of(s)), "moe_expert_offsets");
+    return out;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// adapters: the six factors as views (E, K, r) / (E, r, N), or in the storage of the block module --
+// A.weight (E*hidden, r) and B.weight (E*ffn, r) per projection, w2's factors swapped (megablocks_utils/peft_utils.py:37-38,68-70)
+// ---------------------------------------------------------------------------------------------------------------
+struct Lora {
+    const void* p[6] = {};
+    int64_t s[18] = {};
+    int rank = 0;
+    const void* const* ptrs() const { return rank ? p : nullptr; }
+    const int64_t* strides() const { return rank ? s : nullptr; }
+};
+
+// order a1, b1, a3, b3, a2, b2
+Lora describe_lora(const Tensor* t, bool storage, int64_t d, int64_t f)
+{
+    Lora l;
+    if (!t[0].defined()) return l;
+    l.rank = (int)(storage ? t[0].size(1) : t[0].size(2));
+    const int64_t r = l.rank;
+    for (int i = 0; i < 6; ++i) {
+        int64_t* s = l.s + 3 * i;
+        l.p[i] = t[i].data_ptr();
+        if (!storage) { for (int j = 0; j < 3; ++j) s[j] = t[i].stride(j); continue; }
+        const bool on_ffn = i == 1 || i == 3 || i == 4;        // b1, b3 and a2 live in (E*ffn, r) storage
+        s[0] = (on_ffn ? f : d) * r;
+        const bool a_like = i % 2 == 0;                        // (E, K, r): k stride r, rank stride 1; else (E, r, N)
+        s[1] = a_like ? r : 1;
+        s[2] = a_like ? 1 : r;
+    }
+    return l;
+}
+
+// what the fused launches take (the same limits the library checks before it enqueues anything)
+bool fast_path_ok(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor* lora, bool storage, int64_t E, int64_t d,
+                  int64_t f)
+{
+    (void)E;
+    if (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf) return false;
+    if (w1.scalar_type() != x.scalar_type()) return false;
+    const bool has = lora[0].defined();
+    for (int i = 0; i < 6 && has; ++i)
+        if (lora[i].scalar_type() != x.scalar_type() || (storage && !lora[i].is_contiguous())) return false;
+    if (d % 64 || f % 64 || x.stride(-1) != 1 || x.stride(0) % 8) return false;
+    if (!w1.is_contiguous() || !w2.is_contiguous() || !w3.is_contiguous()) return false;
+    if (has && (storage ? lora[0].size(1) : lora[0].size(2)) > 128) return false;   // up to eight 16-wide rank chunks
+    // gathered activation rows and one expert's matrix are addressed with 32-bit byte offsets
+    return (x.size(0) * x.stride(0) + d) * 2 < ((int64_t)1 << 32) && (f * d + d) * 2 < ((int64_t)1 << 32);
+}
+
+struct MlpShape { int64_t E, d, f, R; int fan_out; double scaling; };
+
+struct MlpOut { Tensor gate, up, h, y, saved; };
+
+// save: keep gate, up (only the backward pass reads them)
+MlpOut mlp_forward(const Tensor& x, const Tensor& w1, const Tensor& w3, const Tensor& w2, const Lora& lora, const MlpShape& s, const void* ssi,
+                   int ssi64, const void* offsets, int off64, bool y_grouped, bool save)
+{
+    MlpOut o;
+    if (save) {
+        o.gate = at::empty({s.R, s.f}, x.options());
+        o.up = at::empty({s.R, s.f}, x.options());
+    }
+    o.h = at::empty({s.R, s.f}, x.options());
+    o.y = at::empty({s.R, s.d}, x.options());
+    o.saved = bytes_on(x, moe_mlp_saved_bytes(s.R, lora.rank));
+    Tensor ws = bytes_on(x, moe_mlp_workspace_bytes(s.R, (int)s.E, s.d, s.f, lora.rank));
+    check(moe_mlp_fwd(ptr(x), x.stride(0), ptr(w1), ptr(w3), ptr(w2), lora.ptrs(), lora.strides(), lora.rank, (float)s.scaling, ptr(o.gate), ptr(o.up),
+                      ptr(o.h), ptr(o.y), o.y.stride(0), ssi, ssi64, offsets, off64, (int)s.E, s.R, s.d, s.f, s.fan_out, y_grouped, dtype_code(x),
+                      ptr(o.saved), ptr(ws), (size_t)ws.numel(), stream_of(x)), "moe_mlp_fwd");
+    return o;
+}
+
+struct MlpGrads { Tensor dx_rows, dgate, dup, lora[6]; };
+
+MlpGrads mlp_backward(const Tensor& dy, bool dy_grouped, int64_t dy_fan_out, const float* row_scale, const Tensor& x, const Tensor& w1, const Tensor& w3,
+                      const Tensor& w2, const Tensor* lora_t, const Lora& lora, const MlpShape& s, const Tensor& gate, const Tensor& up, const Tensor& h,
+                      const Tensor& saved, const void* ssi, int ssi64, const void* offsets, int off64)
+{
+    MlpGrads g;
+    g.dgate = at::empty({s.R, s.f}, x.options());
+    g.dup = at::empty({s.R, s.f}, x.options());
+    g.dx_rows = at::empty({s.R, s.d}, x.options());
+    Tensor ws = bytes_on(x, moe_mlp_workspace_bytes(s.R, (int)s.E, s.d, s.f, lora.rank));
+    void* gp[6] = {};
+    int64_t gs[18] = {};
+    if (lora.rank)
+        for (int i = 0; i < 6; ++i) {
+            g.lora[i] = at::empty_like(lora_t[i]);   // storage and, for views, strides of the factor
+            gp[i] = g.lora[i].data_ptr();
+            for (int j = 0; j < 3; ++j) gs[3 * i + j] = g.lora[i].dim() == 3 ? g.lora[i].stride(j) : lora.s[3 * i + j];
+        }
+    check(moe_mlp_bwd(ptr(dy), dy.stride(0), dy_grouped, (int)dy_fan_out, row_scale, ptr(x), x.stride(0), ptr(w1), ptr(w3), ptr(w2), lora.ptrs(),
+                      lora.strides(), lora.rank ? gp : nullptr, lora.rank ? gs : nullptr, lora.rank, (float)s.scaling, ptr(gate), ptr(up), ptr(h),
+                      ptr(g.dgate), ptr(g.dup), ptr(g.dx_rows), g.dx_rows.stride(0), 0, ssi, ssi64, offsets, off64, (int)s.E, s.R, s.d, s.f, s.fan_out,
+                      dtype_code(x), ptr(saved), ptr(ws), (size_t)ws.numel(), stream_of(x)), "moe_mlp_bwd");
+    return g;
+}
+
+// Gradients of the stored (E, f, d) expert weights (full fine-tuning; the reference gets them from scattermoe's group_bwd_W):
+// dW2[e] = h_e^T dy_e, dW1[e] = dgate_e^T x_e, dW3[e] = dup_e^T x_e over each expert's rows -- already in the storage
+// orientation.  coeff: the per-assignment gate weights folded into dy (or undefined).
+void base_weight_grads(const bool* needs /* w1, w3, w2 */, const Tensor& x, const Tensor& dy, bool dy_grouped, int64_t dy_fan_out, const Tensor& coeff,
+                       const MlpGrads& g, const Tensor& h, const void* ssi, int ssi64, const void* offsets, int off64, const MlpShape& s, Tensor* dw)
+{
+    if (needs[0] || needs[1]) {
+        Tensor x_g = group_rows(x, ssi, ssi64, s.R, s.fan_out);
+        if (needs[0]) dw[0] = group_bwd_w(x_g, g.dgate, offsets, off64, s.E);
+        if (needs[1]) dw[1] = group_bwd_w(x_g, g.dup, offsets, off64, s.E);
+    }
+    if (needs[2]) dw[2] = group_bwd_w(dy_grouped ? dy : group_rows(dy, ssi, ssi64, s.R, dy_fan_out, coeff), h, offsets, off64, s.E);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// router
+// ---------------------------------------------------------------------------------------------------------------
+Tensor router_input_grad(const Tensor& dlogits, const Tensor& weight, at::ScalarType dt)
+{
+    Tensor w = unit_inner(weight.scalar_type() == dt ? weight : weight.to(dt));
+    const int64_t T = dlogits.size(0);
+    Tensor out = at::empty({T, w.size(1)}, w.options());
+    check(moe_combine(nullptr, 0, ptr(out), out.stride(0), nullptr, 0, nullptr, 0, T, w.size(1), dtype_code(out), (const float*)ptr(dlogits), ptr(w),
+                      w.stride(0), (int)dlogits.size(1), stream_of(w)), "moe_combine (router input gradient)");
+    return out;
+}
+
+Tensor router_weight_grad(const Tensor& x, const Tensor& dlogits)
+{
+    const int64_t T = x.size(0), d = x.size(1), E = dlogits.size(1);
+    Tensor out = at::empty({E, d}, x.options());
+    Tensor ws = bytes_on(x, moe_router_weight_grad_workspace_bytes(T, d, (int)E));
+    check(moe_router_weight_grad(ptr(x), x.stride(0), (const float*)ptr(dlogits), ptr(out), out.stride(0), T, d, (int)E, dtype_code(x), ptr(ws),
+                                 (size_t)ws.numel(), stream_of(x)), "moe_router_weight_grad");
+    return out;
+}
+
+struct RouterOut { Tensor scores, weights, indices; };
+
+RouterOut router_forward(const Tensor& x, const Tensor& wg, int64_t k, bool normalize)
+{
+    const int64_t T = x.size(0), d = x.size(1), E = wg.size(0);
+    MOE_ASSERT(wg.scalar_type() == x.scalar_type() && wg.size(1) == d, "router weight and input do not fit");
+    MOE_ASSERT(k >= 1 && k <= E, "top_k must be between 1 and the number of experts");
+    const auto f32 = x.options().dtype(at::kFloat);
+    Tensor logits = at::empty({T, E}, f32);
+    RouterOut o{at::empty({T, E}, f32), at::empty({T, k}, f32), at::empty({T, k}, x.options().dtype(at::kInt))};
+    check(moe_router_forward(ptr(x), x.stride(0), ptr(wg), wg.stride(0), dtype_code(x), (float*)ptr(logits), (float*)ptr(o.scores), (float*)ptr(o.weights),
+                             (int32_t*)ptr(o.indices), T, d, (int)E, (int)k, normalize, stream_of(x)), "moe_router_forward");
+    return o;
+}
+
+Tensor router_topk_bwd(const Tensor& dw, const Tensor& weights, const Tensor& indices, const Tensor& scores, bool normalize)
+{
+    Tensor d = dw.contiguous().to(at::kFloat), dl = at::empty_like(scores);
+    check(moe_router_topk_bwd((const float*)ptr(d), (const float*)ptr(weights), (const int32_t*)ptr(indices), (const float*)ptr(scores), (float*)ptr(dl),
+                              scores.size(0), (int)scores.size(1), (int)weights.size(1), normalize, stream_of(scores)), "moe_router_topk_bwd");
+    return dl;
+}
+
+struct RouterFn : Function<RouterFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& wg, int64_t k, bool normalize)
+    {
+        RouterOut o = router_forward(x, wg, k, normalize);
+        ctx->save_for_backward({x, wg, o.scores, o.weights, o.indices});
+        ctx->saved_data["normalize"] = normalize;
+        ctx->mark_non_differentiable({o.indices});
+        ctx->set_materialize_grads(false);
+        return {o.scores, o.weights, o.indices};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &x = sv[0], &wg = sv[1], &scores = sv[2], &w = sv[3], &idx = sv[4];
+        const c10::DeviceGuard guard(x.device());
+        Tensor dl = router_topk_bwd(g[1].defined() ? g[1] : at::zeros_like(w), w, idx, scores, ctx->saved_data["normalize"].toBool());
+        if (g[0].defined()) {
+            // softmax backward for a gradient that reaches the full score matrix (e.g. an auxiliary loss)
+            Tensor ds = g[0].to(at::kFloat);
+            dl = dl + scores * (ds - (ds * scores).sum(-1, true));
+        }
+        return {ctx->needs_input_grad(0) ? router_input_grad(dl, wg, x.scalar_type()) : Tensor(),
+                ctx->needs_input_grad(1) ? router_weight_grad(x, dl) : Tensor(), Tensor(), Tensor()};
+    }
+};
+
+variable_list router(const Tensor& x_, const Tensor& wg_, int64_t k, bool normalize)
+{
+    require_gpu({&x_, &wg_});
+    const c10::DeviceGuard guard(x_.device());
+    Tensor x = unit_inner(x_), wg = unit_inner(wg_);
+    if (wants_grad({&x, &wg})) return RouterFn::apply(x, wg, k, normalize);
+    RouterOut o = router_forward(x, wg, k, normalize);
+    return {o.scores, o.weights, o.indices};
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// one grouped projection, with or without adapters: scattermoe_utils/parallel_linear_lora.py:11-149 of the reference
+// ---------------------------------------------------------------------------------------------------------------
+struct LinearCfg { double scaling, scaling_ab; int64_t k; bool grouped_in, grouped_out; };   // scaling_ab: of the adapters' gradients
+
+Tensor linear_rows(const Tensor& x, const Tensor& W, const Tensor& A, const Tensor& B, const Tensor& ssi, const Tensor& eo, const LinearCfg& c)
+{
+    return scatter2scatter(x, W, A, B, c.scaling, ssi, eo, c.k, c.grouped_in, c.grouped_out);
+}
+
+struct LinearFn : Function<LinearFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& W, const OptTensor& A_, const OptTensor& B_, const OptTensor& gates_,
+                          const Tensor& ssi, const Tensor& eo, const LinearCfg& c)
+    {
+        const Tensor A = val(A_), B = val(B_), gates = val(gates_);
+        Tensor y = linear_rows(x, W, A, B, ssi, eo, c), y_rows;
+        if (gates.defined()) {   // rows of y are token-major (t*k+j): weighted sum of each token's k rows (reference :30-35)
+            y_rows = y;
+            y = combine(y_rows, gates, nullptr, gates.size(1), gates.size(0));
+        }
+        ctx->save_for_backward({x, W, A, B, gates, ssi, eo, y_rows});
+        ctx->saved_data["scaling"] = c.scaling;
+        ctx->saved_data["scaling_ab"] = c.scaling_ab;
+        ctx->saved_data["k"] = c.k;
+        ctx->saved_data["flags"] = (int64_t)(c.grouped_in | (c.grouped_out << 1));
+        return y;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &x = sv[0], &W = sv[1], &A = sv[2], &B = sv[3], &gates = sv[4], &ssi = sv[5], &eo = sv[6], &y_rows = sv[7];
+        const c10::DeviceGuard guard(x.device());
+        const double scaling = ctx->saved_data["scaling"].toDouble();
+        const int64_t k = ctx->saved_data["k"].toInt(), flags = ctx->saved_data["flags"].toInt(), E = W.size(0), L = ssi.size(0);
+        const bool grouped_in = flags & 1, grouped_out = flags & 2;
+        Tensor dout = g[0].contiguous(), d_gates, coeff, dA, dB, dW;
+        int64_t gate_fan = 1;
+        if (gates.defined()) {
+            d_gates = combine_dgates(y_rows, dout, gates.size(1), gates.scalar_type(), nullptr);   // reference :70-72
+            coeff = gates.reshape({-1});
+            gate_fan = gates.size(1);
+        }
+        // gradients of adapters and weights need dY and X in expert-grouped order (reference :83-99)
+        Tensor dy_g = grouped_out ? dout : group_rows(dout, ptr(ssi), is64(ssi), L, gate_fan, coeff);
+        Tensor x_g = grouped_in ? x : group_rows(x, ptr(ssi), is64(ssi), L, k);
+        if (A.defined()) {
+            const int64_t K = x_g.size(1), N = dy_g.size(1), r = A.size(2);
+            dA = at::empty({E, K, r}, dy_g.options());
+            dB = at::empty({E, r, N}, dy_g.options());
+            const int dt = dtype_code(dy_g);
+            Tensor ws = bytes_on(x, moe_group_bwd_ab_workspace_bytes(L, (int)E, K, N, (int)r, dt));
+            check(moe_group_bwd_ab(ptr(dy_g), dy_g.stride(0), dy_g.stride(1), ptr(x_g), x_g.stride(0), x_g.stride(1), ptr(A), A.stride(0), A.stride(1),
+                                   A.stride(2), ptr(B), B.stride(0), B.stride(1), B.stride(2), (int)r,
+                                   (float)ctx->saved_data["scaling_ab"].toDouble(), ptr(dA), dA.stride(0), dA.stride(1),
+                                   dA.stride(2), ptr(dB), dB.stride(0), dB.stride(1), dB.stride(2), ptr(eo), is64(eo), (int)E, L, K, N, dt, ptr(ws),
+                                   (size_t)ws.numel(), stream_of(x)), "moe_group_bwd_ab");
+        } else if (ctx->needs_input_grad(1)) {
+            dW = group_bwd_w(dy_g, x_g, ptr(eo), is64(eo), E);
+        }
+        // dX = dY W^T + s (dY B^T) A^T: the same grouped GEMM on transposed views (reference :116-128), then the fan-out sum (:134)
+        Tensor dx = scatter2scatter(dy_g, W.transpose(1, 2), A.defined() ? B.transpose(1, 2) : Tensor(), A.defined() ? A.transpose(1, 2) : Tensor(), scaling,
+                                    ssi, eo, 1, true, grouped_in);
+        if (k != 1) dx = combine(dx, Tensor(), nullptr, k, dx.size(0) / k);
+        return {dx, dW, dA, dB, d_gates, Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor linear_checked(const Tensor& x_, const Tensor& W, const Tensor& A, const Tensor& B, double scaling, double scaling_ab, int64_t k, const Tensor& sei, const Tensor& ssi_,
+                      const Tensor& eo_, const Tensor& gates_, bool grouped_in, bool grouped_out)
+{
+    require_gpu({&x_, &W, &A, &B, &sei, &ssi_, &eo_, &gates_});
+    const c10::DeviceGuard guard(x_.device());
+    MOE_ASSERT(ssi_.size(0) == sei.size(0), "sorted_scattered_idxs and sorted_expert_idxs differ in length");
+    MOE_ASSERT(ssi_.size(0) == x_.size(0) * k, "the number of assignments is not rows of X times k");
+    MOE_ASSERT(x_.dim() == 2 && W.dim() == 3 && x_.size(1) == W.size(1), "X and W have inconsistent inner dims.");
+    MOE_ASSERT(W.scalar_type() == x_.scalar_type(), "X and W must share a dtype");
+    if (A.defined()) {
+        MOE_ASSERT(W.size(1) == A.size(1), "A has incorrect input size.");
+        MOE_ASSERT(W.size(2) == B.size(2), "B has incorrect output size.");
+        MOE_ASSERT(A.size(2) == B.size(1), "A and B have inconsistent inner dims.");
+        MOE_ASSERT(A.scalar_type() == x_.scalar_type() && B.scalar_type() == x_.scalar_type(), "A, B and X must share a dtype");
+    }
+    Tensor x = unit_inner(x_), ssi = ssi_.contiguous(), eo = eo_.defined() ? eo_.contiguous() : offsets_from_sorted(sei, W.size(0));
+    Tensor gates = gates_.defined() ? gates_.contiguous() : Tensor();
+    const LinearCfg c{scaling, scaling_ab, k, grouped_in, grouped_out};
+    if (wants_grad({&x, &W, &A, &B, &gates})) return LinearFn::apply(x, W, opt(A), opt(B), opt(gates), ssi, eo, c);
+    Tensor y = linear_rows(x, W, A, B, ssi, eo, c);
+    return gates.defined() ? combine(y, gates, nullptr, gates.size(1), gates.size(0)) : y;
+}
+
+// lora_r: the rank the caller names (it scales the adapters' gradients, reference :102); the forward product is scaled by the factors' own
+Tensor linear(const Tensor& x, const Tensor& W, const OptTensor& A, const OptTensor& B, double lora_r, double lora_alpha, int64_t k, const Tensor& sei,
+              const Tensor& ssi, const OptTensor& eo, const OptTensor& gates, bool grouped_in, bool grouped_out)
+{
+    const Tensor a = val(A);
+    return linear_checked(x, W, a, val(B), a.defined() ? lora_alpha / (double)a.size(2) : 0.0, a.defined() ? lora_alpha / lora_r : 0.0, k, sei, ssi, val(eo),
+                          val(gates), grouped_in, grouped_out);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// pieces of the unfused route
+// ---------------------------------------------------------------------------------------------------------------
+Tensor swiglu_forward(const Tensor& gate, const Tensor& up)
+{
+    Tensor h = at::empty_like(gate);
+    check(moe_swiglu(ptr(gate), ptr(up), ptr(h), gate.numel(), dtype_code(gate), stream_of(gate)), "moe_swiglu");
+    return h;
+}
+
+struct SwigluFn : Function<SwigluFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& gate, const Tensor& up)
+    {
+        ctx->save_for_backward({gate, up});
+        return swiglu_forward(gate, up);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto sv = ctx->get_saved_variables();
+        const c10::DeviceGuard guard(sv[0].device());
+        Tensor dh = g[0].contiguous(), dg = at::empty_like(sv[0]), du = at::empty_like(sv[1]);
+        check(moe_swiglu_bwd(ptr(sv[0]), ptr(sv[1]), ptr(dh), ptr(dg), ptr(du), dh.numel(), dtype_code(dh), stream_of(dh)), "moe_swiglu_bwd");
+        return {dg, du};
+    }
+};
+
+Tensor swiglu(const Tensor& gate_, const Tensor& up_)
+{
+    require_gpu({&gate_, &up_});
+    const c10::DeviceGuard guard(gate_.device());
+    Tensor gate = gate_.contiguous(), up = up_.contiguous();
+    return wants_grad({&gate, &up}) ? SwigluFn::apply(gate, up) : swiglu_forward(gate, up);
+}
+
+// out[t] = sum_j w[t,j] * y_grouped[inv[t*k+j]]  (megablocks ops.scatter, config_utils.py:251)
+struct GatherCombineFn : Function<GatherCombineFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& y, const Tensor& w, const Tensor& inv, const Tensor& ssi)
+    {
+        ctx->save_for_backward({y, w, inv, ssi});
+        return combine(y, w, (const int32_t*)ptr(inv), w.size(1), w.size(0));
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &y = sv[0], &w = sv[1], &inv = sv[2], &ssi = sv[3];
+        const c10::DeviceGuard guard(y.device());
+        Tensor dout = g[0].contiguous();
+        Tensor d_w = combine_dgates(y, dout, w.size(1), w.scalar_type(), (const int32_t*)ptr(inv));
+        // dy_grouped[i] = w[pos_i] * dout[pos_i // k]; pos, the inverse of inv, is the sort's own sorted_scattered_idxs
+        Tensor d_y = group_rows(dout, ptr(ssi), is64(ssi), ssi.numel(), w.size(1), w.reshape({-1}));
+        return {d_y, d_w, Tensor(), Tensor()};
+    }
+};
+
+// int32, one buffer: sorted expert ids, sorted positions, inverse permutation (R each), inclusive offsets (E)
+struct Sorted {
+    Tensor ints;
+    int64_t R = 0, E = 0;
+    int32_t* at(int64_t i) const { return (int32_t*)ints.data_ptr() + i; }
+    int32_t* sei() const { return at(0); }
+    int32_t* ssi() const { return at(R); }
+    int32_t* inv() const { return at(2 * R); }
+    int32_t* offsets() const { return at(3 * R); }
+};
+
+Sorted sort_assignments(const Tensor& indices, int64_t E)
+{
+    const int64_t R = indices.numel();
+    Sorted s{at::empty({3 * R + E}, indices.options()), R, E};
+    Tensor ws = bytes_on(indices, moe_sort_workspace_bytes(R, (int)E));
+    check(moe_sort_by_expert(ptr(indices), 0, R, (int)E, 128, s.sei(), s.ssi(), 0, nullptr, s.offsets(), nullptr, 0, nullptr, s.inv(), ptr(ws), (size_t)ws.numel(), stream_of(indices)), "moe_sort_by_expert");
+    return s;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// expert MLP on expert-grouped assignments (the reference's scattermoe_permute_and_compute, config_utils.py:99-185)
+// ---------------------------------------------------------------------------------------------------------------
+struct MlpCfg { double scaling; int64_t fan_out; bool y_grouped; };
+
+struct ExpertMlpFn : Function<ExpertMlpFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const Tensor& w3, const Tensor& w2, const OptTensor& a1, const OptTensor& b1,
+                          const OptTensor& a3, const OptTensor& b3, const OptTensor& a2, const OptTensor& b2, const OptTensor& gates_,
+                          const Tensor& ssi, const Tensor& offsets, const MlpCfg& c)
+    {
+        const Tensor lt[6] = {val(a1), val(b1), val(a3), val(b3), val(a2), val(b2)}, gates = val(gates_);
+        const Lora lora = describe_lora(lt, false, w1.size(2), w1.size(1));
+        const MlpShape s{w1.size(0), w1.size(2), w1.size(1), ssi.numel(), (int)c.fan_out, c.scaling};
+        MlpOut o = mlp_forward(x, w1, w3, w2, lora, s, ptr(ssi), is64(ssi), ptr(offsets), is64(offsets), c.y_grouped, true);
+        Tensor out = gates.defined() ? combine(o.y, gates, nullptr, gates.size(1), gates.size(0)) : o.y;
+        ctx->save_for_backward({x, w1, w3, w2, lt[0], lt[1], lt[2], lt[3], lt[4], lt[5], gates, ssi, offsets, o.gate, o.up, o.h, o.saved, gates.defined() ? o.y : Tensor()});
+        ctx->saved_data["scaling"] = c.scaling;
+        ctx->saved_data["fan_out"] = c.fan_out;
+        ctx->saved_data["y_grouped"] = c.y_grouped;
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g_)
+    {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &x = sv[0], &w1 = sv[1], &w3 = sv[2], &w2 = sv[3], &gates = sv[10], &ssi = sv[11], &offsets = sv[12];
+        const c10::DeviceGuard guard(x.device());
+        const Lora lora = describe_lora(&sv[4], false, w1.size(2), w1.size(1));
+        const MlpShape s{w1.size(0), w1.size(2), w1.size(1), ssi.numel(), (int)ctx->saved_data["fan_out"].toInt(), ctx->saved_data["scaling"].toDouble()};
+        Tensor dout = g_[0].contiguous(), d_gates, row_scale;
+        bool dy_grouped = ctx->saved_data["y_grouped"].toBool();
+        int64_t dy_fan = 1;
+        if (gates.defined()) {
+            dy_fan = gates.size(1);
+            dy_grouped = false;
+            d_gates = combine_dgates(sv[17], dout, dy_fan, gates.scalar_type(), nullptr);
+            row_scale = group_rows(gates.reshape({-1, 1}).to(at::kFloat), ptr(ssi), is64(ssi), s.R, 1);   // gate of each sorted position
+        }
+        MlpGrads g = mlp_backward(dout, dy_grouped, dy_fan, (const float*)ptr(row_scale), x, w1, w3, w2, &sv[4], lora, s, sv[13], sv[14], sv[15], sv[16],
+                                  ptr(ssi), is64(ssi), ptr(offsets), is64(offsets));
+        Tensor d_x = s.fan_out == 1 ? g.dx_rows : combine(g.dx_rows, Tensor(), nullptr, s.fan_out, s.R / s.fan_out);
+        Tensor dw[3];
+        const bool needs[3] = {ctx->needs_input_grad(1), ctx->needs_input_grad(2), ctx->needs_input_grad(3)};
+        if (needs[0] || needs[1] || needs[2])
+            base_weight_grads(needs, x, dout, dy_grouped, dy_fan, gates.defined() ? gates.reshape({-1}) : Tensor(), g, sv[15], ptr(ssi), is64(ssi),
+                              ptr(offsets), is64(offsets), s, dw);
+        return {d_x, dw[0], dw[1], dw[2], g.lora[0], g.lora[1], g.lora[2], g.lora[3], g.lora[4], g.lora[5], d_gates, Tensor(), Tensor(), Tensor()};
+    }
+};
+
+bool mlp_fast_path(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& w3, const std::vector<Tensor>& lora)
+{
+    Tensor lt[6];
+    for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
+    return fast_path_ok(x, w1, w2, w3, lt, false, w1.size(0), w1.size(2), w1.size(1));
+}
+
+// lora: empty, or the six factor views a1, b1, a3, b3, a2, b2
+Tensor expert_mlp(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& w3, int64_t fan_out, const Tensor& ssi_, const Tensor& offsets_,
+                  const std::vector<Tensor>& lora, double lora_alpha, const OptTensor& gates_, bool grouped_out)
+{
+    require_gpu({&x, &w1, &w2, &w3, &ssi_, &offsets_});
+    const c10::DeviceGuard guard(x.device());
+    Tensor lt[6];
+    for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
+    TORCH_CHECK(fast_path_ok(x, w1, w2, w3, lt, false, w1.size(0), w1.size(2), w1.size(1)),
+                "fused_expert_mlp needs bf16, contiguous (E,f,d) weights, d and f multiples of 64 and rank <= 128; use scattermoe_permute_and_compute for "
+                "other cases");
+    Tensor ssi = ssi_.contiguous(), offsets = offsets_.contiguous(), gates = gates_.has_value() ? gates_->contiguous() : Tensor();
+    const MlpCfg c{lt[0].defined() ? lora_alpha / (double)lt[0].size(2) : 0.0, fan_out, grouped_out && !gates.defined()};
+    if (wants_grad({&x, &w1, &w2, &w3, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5], &gates}))
+        return ExpertMlpFn::apply(x, w1, w3, w2, opt(lt[0]), opt(lt[1]), opt(lt[2]), opt(lt[3]), opt(lt[4]), opt(lt[5]), opt(gates), ssi, offsets, c);
+    const MlpShape s{w1.size(0), w1.size(2), w1.size(1), ssi.numel(), (int)fan_out, c.scaling};
+    MlpOut o = mlp_forward(x, w1, w3, w2, describe_lora(lt, false, s.d, s.f), s, ptr(ssi), is64(ssi), ptr(offsets), is64(offsets), c.y_grouped, false);
+    return gates.defined() ? combine(o.y, gates, nullptr, gates.size(1), gates.size(0)) : o.y;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// whole layer: router -> sort -> expert MLP -> weighted combine, one autograd node
+// ---------------------------------------------------------------------------------------------------------------
+struct LayerCfg { double scaling; int64_t E, d, f, k; bool normalize, storage; };
+
+struct LayerOut { RouterOut rt; Sorted so; MlpOut mlp; Tensor out; };
+
+LayerOut layer_forward(const Tensor& x, const Tensor& wg, const Tensor& w1, const Tensor& w3, const Tensor& w2, const Tensor* lt, const LayerCfg& c, bool save)
+{
+    LayerOut o;
+    o.rt = router_forward(x, unit_inner(wg), c.k, c.normalize);
+    o.so = sort_assignments(o.rt.indices, c.E);
+    const MlpShape s{c.E, c.d, c.f, x.size(0) * c.k, (int)c.k, c.scaling};
+    o.mlp = mlp_forward(x, w1, w3, w2, describe_lora(lt, c.storage, c.d, c.f), s, o.so.ssi(), 0, o.so.offsets(), 0, false, save);
+    o.out = combine(o.mlp.y, o.rt.weights, nullptr, c.k, x.size(0));
+    return o;
+}
+
+struct LayerFn : Function<LayerFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& wg, const Tensor& w1, const Tensor& w3, const Tensor& w2,
+                                 const OptTensor& a1, const OptTensor& b1, const OptTensor& a3, const OptTensor& b3, const OptTensor& a2,
+                                 const OptTensor& b2, const LayerCfg& c)
+    {
+        const Tensor lt[6] = {val(a1), val(b1), val(a3), val(b3), val(a2), val(b2)};
+        LayerOut o = layer_forward(x, wg, w1, w3, w2, lt, c, true);
+        ctx->save_for_backward({x, wg, w1, w3, w2, lt[0], lt[1], lt[2], lt[3], lt[4], lt[5], o.rt.scores, o.rt.weights, o.rt.indices, o.so.ints, o.mlp.gate, o.mlp.up,
+                                o.mlp.h, o.mlp.y, o.mlp.saved});
+        ctx->saved_data["scaling"] = c.scaling;
+        ctx->saved_data["sizes"] = std::vector<int64_t>{c.E, c.d, c.f, c.k, c.normalize, c.storage};
+        ctx->mark_non_differentiable({o.rt.indices});
+        ctx->set_materialize_grads(false);   // an unused expert_weights output must not cost a zero-fill per step
+        return {o.out, o.rt.weights, o.rt.indices};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g_)
+    {
+        const auto sv = ctx->get_saved_variables();
+        const Tensor &x = sv[0], &wg = sv[1], &w1 = sv[2], &w3 = sv[3], &w2 = sv[4], &scores = sv[11], &weights = sv[12], &indices = sv[13], &y = sv[18];
+        const c10::DeviceGuard guard(x.device());
+        const auto sz = ctx->saved_data["sizes"].toIntVector();
+        const int64_t k = sz[3], T = x.size(0);
+        const Sorted so{sv[14], T * k, sz[0]};
+        const bool normalize = sz[4] != 0, storage = sz[5] != 0;
+        const MlpShape s{sz[0], sz[1], sz[2], T * k, (int)k, ctx->saved_data["scaling"].toDouble()};
+        const Lora lora = describe_lora(&sv[5], storage, s.d, s.f);
+        Tensor dout = g_[0].defined() ? g_[0].contiguous() : at::zeros_like(x);
+        Tensor d_gates = combine_dgates(y, dout, k, at::kFloat, nullptr);
+        if (g_[1].defined()) d_gates = d_gates + g_[1].to(at::kFloat);   // the caller also used the returned expert weights (e.g. in an auxiliary loss)
+        Tensor dlogits = router_topk_bwd(d_gates, weights, indices, scores, normalize);
+        Tensor row_scale = group_rows(weights.view({-1, 1}), so.ssi(), 0, s.R, 1);
+        MlpGrads g = mlp_backward(dout, false, k, (const float*)ptr(row_scale), x, w1, w3, w2, &sv[5], lora, s, sv[15], sv[16], sv[17], sv[19], so.ssi(), 0,
+                                  so.offsets(), 0);
+        Tensor dw[3];
+        const bool needs[3] = {ctx->needs_input_grad(2), ctx->needs_input_grad(3), ctx->needs_input_grad(4)};
+        if (needs[0] || needs[1] || needs[2]) {
+            base_weight_grads(needs, x, dout, false, k, weights.view({-1}), g, sv[17], so.ssi(), 0, so.offsets(), 0, s, dw);
+            const Tensor* w[3] = {&w1, &w3, &w2};
+            for (int i = 0; i < 3; ++i)
+                if (dw[i].defined()) dw[i] = dw[i].view(w[i]->sizes());
+        }
+        // fan-out sum of the k expert rows of each token plus the router's contribution dlogits @ wg, one pass
+        Tensor d_x = combine(g.dx_rows, Tensor(), nullptr, k, T, (const float*)ptr(dlogits), unit_inner(wg), s.E);
+        Tensor d_wg = ctx->needs_input_grad(1) ? router_weight_grad(x, dlogits) : Tensor();
+        return {d_x, d_wg, dw[0], dw[1], dw[2], g.lora[0], g.lora[1], g.lora[2], g.lora[3], g.lora[4], g.lora[5], Tensor()};
+    }
+};
+
+// x (T, d); wg (E, d); expert weights (E, f, d), or (E*f, d) with `storage`; lora: empty, or six factors -- views, or with
+// `storage` the block's A.weight / B.weight as a1, b1, a3, b3, a2 (= B of w2), b2 (= A of w2).
+// -> out (T, d), expert weights (T, k) fp32, expert indices (T, k) int32
+variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1, const Tensor& w2, const Tensor& w3, int64_t E, int64_t f, int64_t k,
+                    const std::vector<Tensor>& lora, double lora_alpha, bool normalize, bool storage)
+{
+    require_gpu({&x, &wg, &w1, &w2, &w3});
+    const c10::DeviceGuard guard(x.device());
+    const int64_t d = x.size(1);
+    Tensor lt[6];
+    for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
+    const int64_t rank = lt[0].defined() ? lt[0].size(storage ? 1 : 2) : 0;
+    const double scaling = rank ? lora_alpha / (double)rank : 0.0;
+    if (fast_path_ok(x, w1, w2, w3, lt, storage, E, d, f)) {
+        const LayerCfg c{scaling, E, d, f, k, normalize, storage};
+        if (wants_grad({&x, &wg, &w1, &w2, &w3, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]}))
+            return LayerFn::apply(x, wg, w1, w3, w2, opt(lt[0]), opt(lt[1]), opt(lt[2]), opt(lt[3]), opt(lt[4]), opt(lt[5]), c);
+        LayerOut o = layer_forward(x, wg, w1, w3, w2, lt, c, false);
+        return {o.out, o.rt.weights, o.rt.indices};
+    }
+    // unfused route: the reference's three projections (config_utils.py:127-166), the combine of ops.scatter (:251)
+    const variable_list rt = router(x, wg, k, normalize);
+    const Sorted so = sort_assignments(rt[2], E);
+    const Tensor sei = so.ints.narrow(0, 0, so.R), ssi = so.ints.narrow(0, so.R, so.R), inv = so.ints.narrow(0, 2 * so.R, so.R),
+                 offsets = so.ints.narrow(0, 3 * so.R, E);
+    if (storage && rank) {
+        for (int i = 0; i < 6; ++i) {
+            const bool on_ffn = i == 1 || i == 3 || i == 4;
+            Tensor v = lt[i].view({E, on_ffn ? f : d, rank});
+            lt[i] = i % 2 == 0 ? v : v.transpose(1, 2);
+        }
+    }
+    auto proj = [&](const Tensor& in, const Tensor& w, bool n_contiguous, int ia, int64_t fan, bool gin) {
+        Tensor W = w.view({E, f, d});
+        return linear_checked(in, n_contiguous ? W : W.transpose(1, 2), lt[ia], lt[ia + 1], scaling, scaling, fan, sei, ssi, offsets, Tensor(), gin, true);
+    };
+    Tensor h = swiglu(proj(x, w1, false, 0, k, false), proj(x, w3, false, 2, k, false));
+    Tensor y = proj(h, w2, true, 4, 1, true);
+    Tensor out = wants_grad({&y, &rt[1]}) ? GatherCombineFn::apply(y, rt[1], inv, ssi) : combine(y, rt[1], so.inv(), k, x.size(0));
+    return {out, rt[1], rt[2]};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
+{
+    py::register_exception<AssertionFailure>(m, "ShapeError", PyExc_AssertionError);
+    m.def("router", &router, py::call_guard<py::gil_scoped_release>());
+    m.def("linear", &linear, py::call_guard<py::gil_scoped_release>());
+    m.def("swiglu", &swiglu, py::call_guard<py::gil_scoped_release>());
+    m.def("mlp_fast_path", &mlp_fast_path);
+    m.def("expert_mlp", &expert_mlp, py::call_guard<py::gil_scoped_release>());
+    m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
+}

@@ -4,21 +4,20 @@ Follows ``scattermoe_permute_and_compute`` of the reference (megablocks_utils/co
 views it builds (``get_mlp_weights`` :28-35, ``get_mlp_weights_lora`` :37-61).  For bf16 tensors of Mixtral-like
 shape the three projections run as two fused launches (dual-weight GEMM with SwiGLU epilogue, then w2) through
 ``moe_mlp_fwd`` / ``moe_mlp_bwd`` of libmoe_hip.so; everything else goes through the same three
-``parallel_linear(_lora)`` calls the reference makes, which use the generic HIP kernels.
+``parallel_linear(_lora)`` calls the reference makes, which use the generic HIP kernels.  The sequences of library calls
+and their autograd nodes are in csrc/torch_layer.cpp.
 """
 from __future__ import annotations
 
-import ctypes
 from typing import NamedTuple, Optional, Tuple
 
 import torch
 import torch.nn as nn
 
-from .._lib import lib, check, dtype_code, is64, ptr, require_gpu, stream_ptr, workspace
+from .._lib import native, require_gpu
 from ..scattermoe_utils.kernels import ops
 from ..scattermoe_utils.parallel_experts import parallel_linear
 from ..scattermoe_utils.parallel_linear_lora import parallel_linear_lora
-from . import router as _router
 
 
 # ---------------------------------------------------------------------------------------------------------------
@@ -58,157 +57,14 @@ class LoraViews(NamedTuple):
     b2: torch.Tensor
 
 
-def _fast_path_ok(x, w1, w2, w3, lora: Optional[LoraViews]) -> bool:
-    if x.dtype not in (torch.bfloat16, torch.float16) or w1.dtype != x.dtype:
-        return False
-    if lora is not None and any(t.dtype != x.dtype for t in lora):
-        return False
-    E, f, d = w1.shape
-    if d % 64 or f % 64 or x.stride(-1) != 1 or x.stride(0) % 8:
-        return False
-    if not (w1.is_contiguous() and w2.is_contiguous() and w3.is_contiguous()):
-        return False
-    if lora is not None and lora.a1.size(2) > 128:   # the fused launches take an adapter as up to eight 16-wide rank chunks
-        return False
-    # gathered activation rows and one expert's matrix are addressed with 32-bit byte offsets (the same check the library
-    # makes before it enqueues anything); the number of rows is otherwise not limited
-    if (x.size(0) * x.stride(0) + d) * 2 >= 1 << 32 or (f * d + d) * 2 >= 1 << 32:
-        return False
-    return True
-
-
-def _lora_arrays(tensors):
-    ptrs = (ctypes.c_void_p * 6)(*[t.data_ptr() for t in tensors])
-    strides = (ctypes.c_int64 * 18)(*[s for t in tensors for s in t.stride()])
-    return ptrs, strides
-
-
-class _SwiGLU(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, gate, up):
-        ctx.save_for_backward(gate, up)
-        return ops.swiglu(gate, up)
-
-    @staticmethod
-    def backward(ctx, dh):
-        gate, up = ctx.saved_tensors
-        return ops.swiglu_bwd(gate, up, dh)
-
-
-def _mlp_fwd(x, w1, w3, w2, lora, scaling, ssi, offsets, fan_out, y_grouped, save_gate_up=True):
-    dev = x.device
-    E, f, d = w1.shape
-    R = ssi.numel()
-    rank = 0 if lora is None else lora.a1.size(2)
-    gate = torch.empty((R, f), dtype=x.dtype, device=dev) if save_gate_up else None
-    up = torch.empty((R, f), dtype=x.dtype, device=dev) if save_gate_up else None
-    h = torch.empty((R, f), dtype=x.dtype, device=dev)
-    y = torch.empty((R, d), dtype=x.dtype, device=dev)
-    saved = workspace(lib.moe_mlp_saved_bytes(R, rank), dev)
-    ws = workspace(lib.moe_mlp_workspace_bytes(R, E, d, f, rank), dev)
-    lp, ls = (None, None) if lora is None else _lora_arrays(lora)
-    check(lib.moe_mlp_fwd(ptr(x), x.stride(0), ptr(w1), ptr(w3), ptr(w2), lp, ls, rank, scaling, ptr(gate), ptr(up),
-                          ptr(h), ptr(y), y.stride(0), ptr(ssi), is64(ssi), ptr(offsets), is64(offsets), E, R, d, f,
-                          fan_out, int(y_grouped), dtype_code(x), ptr(saved), ptr(ws), ws.numel(), stream_ptr(dev)), "moe_mlp_fwd")
-    return gate, up, h, y, saved
-
-
-def _mlp_bwd(dy, dy_grouped, dy_fan_out, row_scale, x, w1, w3, w2, lora, scaling, gate, up, h, saved, ssi, offsets,
-             fan_out, dx_grouped):
-    dev = x.device
-    E, f, d = w1.shape
-    R = ssi.numel()
-    rank = 0 if lora is None else lora.a1.size(2)
-    dgate = torch.empty_like(gate)
-    dup = torch.empty_like(up)
-    dx_rows = torch.empty((R, d), dtype=x.dtype, device=dev)
-    ws = workspace(lib.moe_mlp_workspace_bytes(R, E, d, f, rank), dev)
-    grads = None
-    lp = ls = gp = gs = None
-    if lora is not None:
-        grads = tuple(torch.empty_like(t) for t in lora)
-        lp, ls = _lora_arrays(lora)
-        gp, gs = _lora_arrays(grads)
-    check(lib.moe_mlp_bwd(ptr(dy), dy.stride(0), int(dy_grouped), dy_fan_out, ptr(row_scale), ptr(x), x.stride(0),
-                          ptr(w1), ptr(w3), ptr(w2), lp, ls, gp, gs, rank, scaling, ptr(gate), ptr(up), ptr(h),
-                          ptr(dgate), ptr(dup), ptr(dx_rows), dx_rows.stride(0), int(dx_grouped), ptr(ssi), is64(ssi),
-                          ptr(offsets), is64(offsets), E, R, d, f, fan_out, dtype_code(x), ptr(saved), ptr(ws), ws.numel(),
-                          stream_ptr(dev)), "moe_mlp_bwd")
-    return dx_rows, grads, dgate, dup
-
-
-def _base_weight_grads(needs, x, dy, dy_grouped, dy_fan_out, coeff, dgate, dup, h, ssi, offsets, fan_out, E):
-    """Gradients of the stored (E, f, d) expert weights (full fine-tuning; the reference gets them from
-    scattermoe's group_bwd_W in ParallelLinear.backward): dW2[e] = h_e^T dy_e, dW1[e] = dgate_e^T x_e,
-    dW3[e] = dup_e^T x_e over each expert's grouped rows -- already in the storage orientation, no transposes.
-    `needs` = (w1, w3, w2) flags; `coeff` the per-assignment gate weights folded into dy (or None)."""
-    d_w1 = d_w3 = d_w2 = None
-    if needs[0] or needs[1]:
-        x_g = ops.group(x, ssi, fan_out=fan_out)
-        if needs[0]:
-            d_w1 = ops.group_bwd_W(x_g, dgate, offsets, E)
-        if needs[1]:
-            d_w3 = ops.group_bwd_W(x_g, dup, offsets, E)
-    if needs[2]:
-        dy_g = dy if dy_grouped else ops.group(dy, ssi, coeff=coeff, fan_out=dy_fan_out)
-        d_w2 = ops.group_bwd_W(dy_g, h, offsets, E)
-    return d_w1, d_w3, d_w2
-
-
-class FusedExpertMLP(torch.autograd.Function):
-    """silu(x W1^T) * (x W3^T) -> W2 over ragged expert groups, with adapters, optional gate-weighted combine."""
-
-    @staticmethod
-    def forward(ctx, x, w1, w3, w2, a1, b1, a3, b3, a2, b2, lora_alpha, gates, ssi, offsets, fan_out, grouped_out):
-        lora = None if a1 is None else LoraViews(a1, b1, a3, b3, a2, b2)
-        scaling = 0.0 if lora is None else float(lora_alpha) / a1.size(2)
-        y_grouped = bool(grouped_out) and gates is None
-        gate, up, h, y, saved = _mlp_fwd(x, w1, w3, w2, lora, scaling, ssi, offsets, fan_out, y_grouped)
-        out = y if gates is None else ops.combine(y, gates)
-        ctx.save_for_backward(x, w1, w3, w2, a1, b1, a3, b3, a2, b2, gates, ssi, offsets, gate, up, h, saved,
-                              y if gates is not None else None)
-        ctx.cfg = (scaling, fan_out, y_grouped)
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        (x, w1, w3, w2, a1, b1, a3, b3, a2, b2, gates, ssi, offsets, gate, up, h, saved, y) = ctx.saved_tensors
-        scaling, fan_out, y_grouped = ctx.cfg
-        lora = None if a1 is None else LoraViews(a1, b1, a3, b3, a2, b2)
-        dout = dout.contiguous()
-        d_gates = row_scale = None
-        if gates is not None:
-            k = gates.size(1)
-            d_gates = ops.combine_dgates(y, dout, k, gates.dtype)
-            row_scale = ops.group(gates.reshape(-1, 1).float(), ssi)          # gate of each sorted position
-            dy_grouped, dy_fan = False, k
-        else:
-            dy_grouped, dy_fan = y_grouped, 1
-        dx_rows, grads, dgate, dup = _mlp_bwd(dout, dy_grouped, dy_fan, row_scale, x, w1, w3, w2, lora, scaling, gate, up,
-                                              h, saved, ssi, offsets, fan_out, False)
-        d_x = dx_rows if fan_out == 1 else ops.combine(dx_rows, None, k=fan_out)
-        g = grads if grads is not None else (None,) * 6
-        d_w = (None, None, None)
-        if any(ctx.needs_input_grad[1:4]):
-            d_w = _base_weight_grads(ctx.needs_input_grad[1:4], x, dout, dy_grouped, dy_fan,
-                                     None if gates is None else gates.reshape(-1), dgate, dup, h, ssi, offsets, fan_out,
-                                     w1.size(0))
-        return (d_x,) + tuple(d_w) + tuple(g) + (None, d_gates, None, None, None, None)
-
-
 def fused_expert_mlp(x, w1, w2, w3, k, sorted_scattered_idxs, expert_offsets, lora: Optional[LoraViews] = None,
                      lora_alpha: float = 1.0, gates: Optional[torch.Tensor] = None, grouped_out: bool = False):
     """Expert MLP on expert-grouped assignments.  x (rows, d); w1, w2, w3 (E, f, d) in the reference's storage
     layout; ``k`` = fan-out of x rows (top_k, or 1 for pre-dispatched rows).  With ``gates`` (T, k) the k expert
     rows of each token are combined and (T, d) is returned; otherwise one row per assignment, in grouped order
     when ``grouped_out`` else at its flat position."""
-    require_gpu(x, w1, w2, w3, sorted_scattered_idxs, expert_offsets)
-    lt = (None,) * 6 if lora is None else tuple(lora)
-    if not _fast_path_ok(x, w1, w2, w3, lora):
-        raise RuntimeError("fused_expert_mlp needs bf16, contiguous (E,f,d) weights, d and f multiples of 64 and rank <= 128; "
-                           "use scattermoe_permute_and_compute for other cases")
-    return FusedExpertMLP.apply(x, w1, w3, w2, *lt, lora_alpha, gates, sorted_scattered_idxs.contiguous(),
-                                expert_offsets.contiguous(), k, grouped_out)
+    return native.expert_mlp(x, w1, w2, w3, k, sorted_scattered_idxs, expert_offsets, [] if lora is None else list(lora),
+                             lora_alpha, gates, grouped_out)
 
 
 def scattermoe_permute_and_compute(x, w1, w2, w3, ffn_hidden_size, hidden_size, top_k, bin_ids, indices, num_experts,
@@ -237,7 +93,7 @@ def scattermoe_permute_and_compute(x, w1, w2, w3, ffn_hidden_size, hidden_size, 
         lora = LoraViews(v["a1"], v["b1"], v["a3"], v["b3"], v["a2"], v["b2"])
     elif lora_views is not None:
         lora, alpha = lora_views, lora_alpha
-    if _fast_path_ok(x, W["w1"], W["w2"], W["w3"], lora):
+    if native.mlp_fast_path(x, W["w1"], W["w2"], W["w3"], [] if lora is None else list(lora)):
         return fused_expert_mlp(x, W["w1"], W["w2"], W["w3"], fan, indices, expert_offsets, lora, alpha, None, grouped_out)
     # generic route: the reference's three calls (:127-166)
     def proj(inp, name, kk, gin, gout):
@@ -249,92 +105,26 @@ def scattermoe_permute_and_compute(x, w1, w2, w3, ffn_hidden_size, hidden_size, 
                                     gin, gout)
     h1 = proj(x, "w1", fan, False, True)
     h3 = proj(x, "w3", fan, False, True)
-    h = _SwiGLU.apply(h1, h3)
+    h = native.swiglu(h1, h3)
     return proj(h, "w2", 1, True, grouped_out)
 
 
 # ---------------------------------------------------------------------------------------------------------------
 # whole layer: router -> sort -> expert MLP -> weighted combine, one autograd node
 # ---------------------------------------------------------------------------------------------------------------
-class MoELayerFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, wg, w1, w3, w2, a1, b1, a3, b3, a2, b2, lora_alpha, top_k, normalize):
-        lora = None if a1 is None else LoraViews(a1, b1, a3, b3, a2, b2)
-        scaling = 0.0 if lora is None else float(lora_alpha) / a1.size(2)
-        rt = _router.route_and_sort(x, wg, top_k, normalize)
-        gate, up, h, y, saved = _mlp_fwd(x, w1, w3, w2, lora, scaling, rt.sorted_scattered_idxs, rt.expert_offsets,
-                                         top_k, False)
-        out = ops.combine(y, rt.weights)
-        ctx.save_for_backward(x, wg, w1, w3, w2, a1, b1, a3, b3, a2, b2, rt.scores, rt.weights, rt.indices,
-                              rt.sorted_scattered_idxs, rt.expert_offsets, gate, up, h, y, saved)
-        ctx.cfg = (scaling, top_k, normalize)
-        ctx.mark_non_differentiable(rt.indices)
-        ctx.set_materialize_grads(False)   # an unused expert_weights output must not cost a zero-fill per step
-        return out, rt.weights, rt.indices
-
-    @staticmethod
-    def backward(ctx, dout, _dw, _di):
-        (x, wg, w1, w3, w2, a1, b1, a3, b3, a2, b2, scores, weights, indices, ssi, offsets, gate, up, h, y,
-         saved) = ctx.saved_tensors
-        scaling, k, normalize = ctx.cfg
-        lora = None if a1 is None else LoraViews(a1, b1, a3, b3, a2, b2)
-        dout = torch.zeros_like(x) if dout is None else dout.contiguous()
-        d_gates = ops.combine_dgates(y, dout, k, torch.float32)
-        if _dw is not None:   # the caller also used the returned expert weights (e.g. in an auxiliary loss)
-            d_gates = d_gates + _dw.to(d_gates.dtype)
-        dlogits = _router.router_topk_bwd(d_gates, weights, indices, scores, normalize)
-        row_scale = ops.group(weights.reshape(-1, 1), ssi)
-        dx_rows, grads, dgate, dup = _mlp_bwd(dout, False, k, row_scale, x, w1, w3, w2, lora, scaling, gate, up, h, saved,
-                                              ssi, offsets, k, False)
-        d_w = (None, None, None)
-        if any(ctx.needs_input_grad[2:5]):
-            d_w = _base_weight_grads(ctx.needs_input_grad[2:5], x, dout, False, k, weights.reshape(-1), dgate, dup, h, ssi,
-                                     offsets, k, w1.size(0))
-        # fan-out sum of the k expert rows of each token plus the router's contribution dlogits @ wg, one pass
-        d_x = ops.combine(dx_rows, None, k=k, extra_coef=dlogits, extra_rows=wg if wg.stride(-1) == 1 else wg.contiguous())
-        d_wg = _router.router_weight_grad(x, dlogits) if ctx.needs_input_grad[1] else None
-        g = grads if grads is not None else (None,) * 6
-        return (d_x, d_wg) + tuple(d_w) + tuple(g) + (None, None, None)
-
-
 def moe_layer_forward(x, wg, w1, w2, w3, top_k=2, lora: Optional[LoraViews] = None, lora_alpha: float = 1.0,
                       normalize: bool = True):
     """x (T, d) bf16 -> (out (T, d), expert_weights (T, k) fp32, expert_indices (T, k) int32).
     wg (E, d) router weight; w1, w2, w3 (E, f, d) expert weights in the reference's storage layout."""
-    require_gpu(x, wg, w1, w2, w3)
+    return _layer(x, wg, w1, w2, w3, w1.size(0), w1.size(1), top_k, [] if lora is None else list(lora), lora_alpha, normalize, False)
+
+
+def _layer(x, wg, w1, w2, w3, E, f, top_k, lora, lora_alpha, normalize, storage):
     if x.size(0) == 0:   # an empty batch routes nothing: empty outputs, and backward leaves every parameter's grad unset
+        require_gpu(x, wg, w1, w2, w3)
         return (x.clone(), torch.zeros((0, top_k), dtype=torch.float32, device=x.device),
                 torch.zeros((0, top_k), dtype=torch.int32, device=x.device))
-    if not _fast_path_ok(x, w1, w2, w3, lora):
-        scores, ew, ei = _router.forward_router(x, wg, top_k, normalize)
-        sei, ssi, counts, offsets, inv = _router.sort_assignments(ei.int(), w1.size(0))
-        E, f, d = w1.shape
-        y = scattermoe_permute_and_compute(x, w1.reshape(E * f, d), w2.reshape(E * f, d), w3.reshape(E * f, d), f, d,
-                                           top_k, sei, ssi, E, None, moe_expert_model_parallelism=False,
-                                           expert_offsets=offsets, lora_views=lora, lora_alpha=lora_alpha)
-        out = _GatherCombine.apply(y, ew, inv, ssi)
-        return out, ew, ei.int()
-    lt = (None,) * 6 if lora is None else tuple(lora)
-    return MoELayerFn.apply(x, wg, w1, w3, w2, *lt, lora_alpha, top_k, normalize)
-
-
-class _GatherCombine(torch.autograd.Function):
-    """out[t] = sum_j w[t,j] * y_grouped[inv[t*k+j]]  (megablocks ops.scatter, config_utils.py:251)."""
-
-    @staticmethod
-    def forward(ctx, y, w, inv, ssi):
-        ctx.save_for_backward(y, w, inv, ssi)
-        return ops.combine(y, w, inv=inv)
-
-    @staticmethod
-    def backward(ctx, dout):
-        y, w, inv, ssi = ctx.saved_tensors
-        dout = dout.contiguous()
-        k = w.size(1)
-        d_w = ops.combine_dgates(y, dout, k, w.dtype, inv=inv)
-        # dy_grouped[i] = w[pos_i] * dout[pos_i // k]; pos, the inverse of inv, is the sort's own sorted_scattered_idxs
-        d_y = ops.group(dout, ssi, coeff=w.reshape(-1), fan_out=k)
-        return d_y, d_w, None, None
+    return native.layer(x, wg, w1, w2, w3, E, f, top_k, lora, lora_alpha, bool(normalize), storage)
 
 
 class ScatterMoEBlock(nn.Module):
@@ -382,9 +172,12 @@ class ScatterMoEBlock(nn.Module):
     def forward(self, hidden_states: torch.Tensor):
         shape = hidden_states.shape
         x = hidden_states.reshape(-1, shape[-1])
-        E, f, d = self.num_experts, self.ffn_hidden_size, self.hidden_size
-        out, _, _ = moe_layer_forward(x, self.router, self.w1.view(E, f, d), self.w2.view(E, f, d),
-                                      self.w3.view(E, f, d), self.top_k, self.lora_views(), self.lora_alpha)
+        E, f = self.num_experts, self.ffn_hidden_size
+        lora = []
+        if self.lora_r > 0:   # the factors in their storage, in the order a1, b1, a3, b3, a2, b2 (w2's are swapped, see lora_views)
+            lora = [resolve_dtensor(t) for t in (self.lora_A_w1, self.lora_B_w1, self.lora_A_w3, self.lora_B_w3, self.lora_B_w2, self.lora_A_w2)]
+        out = _layer(x, resolve_dtensor(self.router), resolve_dtensor(self.w1), resolve_dtensor(self.w2), resolve_dtensor(self.w3), E, f,
+                     self.top_k, lora, self.lora_alpha, True, True)[0]
         out = out.view(shape)
         if self.bias is not None:
             if self.return_bias:

@@ -8,7 +8,7 @@ from typing import NamedTuple, Optional
 
 import torch
 
-from .._lib import lib, check, dtype_code, ptr, require_gpu, stream_ptr, workspace
+from .._lib import lib, check, dtype_code, native, ptr, require_gpu, stream_ptr, workspace
 from ..scattermoe_utils.kernels import ops
 
 
@@ -115,28 +115,6 @@ def router_weight_grad(x2: torch.Tensor, dlogits: torch.Tensor) -> torch.Tensor:
     return out
 
 
-class _RouterFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x2, weight, top_k, normalize):
-        _, scores, w, idx = router_forward(x2, weight, top_k, normalize)
-        ctx.save_for_backward(x2, weight, scores, w, idx)
-        ctx.normalize = normalize
-        ctx.mark_non_differentiable(idx)
-        return scores, w, idx
-
-    @staticmethod
-    def backward(ctx, d_scores, d_w, _d_idx):
-        x2, weight, scores, w, idx = ctx.saved_tensors
-        dl = router_topk_bwd(d_w, w, idx, scores, ctx.normalize)
-        if d_scores is not None:
-            # softmax backward for a gradient that reaches the full score matrix (e.g. an auxiliary loss)
-            ds = d_scores.float()
-            dl = dl + scores * (ds - (ds * scores).sum(-1, keepdim=True))
-        dx = router_input_grad(dl, weight, x2.dtype) if ctx.needs_input_grad[0] else None
-        dwg = router_weight_grad(x2, dl) if ctx.needs_input_grad[1] else None
-        return dx, dwg, None, None
-
-
 class _LogitsFn(torch.autograd.Function):
     """fp32 router logits with autograd, for the router variants that put something between the linear layer and the
     softmax."""
@@ -192,7 +170,7 @@ def forward_router(x: torch.Tensor, weight: torch.Tensor, top_k: int, moe_normal
     p = moe_normalize_expert_weights
     p = None if p in (None, False, 0) else (1 if p is True else p)
     if bias is None and p in (None, 1):
-        scores, w, idx = _RouterFn.apply(x2, weight, top_k, p == 1)
+        scores, w, idx = native.router(x2, weight, top_k, p == 1)
     else:
         logits = _LogitsFn.apply(x2, weight)
         if bias is not None:

@@ -6,46 +6,17 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from .kernels import ops
+from .._lib import native
 
 
-class ParallelLinear(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, expert_weights, k, sorted_expert_idxs, sorted_scattered_idxs, padded_block_idxs,
-                expert_offsets, gates=None, grouped_in=False, grouped_out=False):
-        x = x.contiguous() if x.stride(-1) != 1 else x
-        y = ops._scatter2scatter(x, expert_weights, None, None, 0.0, sorted_expert_idxs, sorted_scattered_idxs, k,
-                                 grouped_in, grouped_out, None, expert_offsets)
-        if gates is not None:
-            y_rows = y
-            y = ops.combine(y_rows, gates)
-        else:
-            y_rows = None
-        ctx.save_for_backward(x, expert_weights, sorted_expert_idxs, sorted_scattered_idxs, padded_block_idxs,
-                              expert_offsets, gates, y_rows)
-        ctx.flags = (grouped_in, grouped_out, k)
-        return y
+class ParallelLinear:
+    """One autograd node (C++); its backward returns the gradients of ``x``, ``expert_weights`` and ``gates``."""
 
     @staticmethod
-    def backward(ctx, grad_out):
-        (x, W, sei, ssi, pbi, eo, gates, y_rows) = ctx.saved_tensors
-        grouped_in, grouped_out, k = ctx.flags
-        grad_out = grad_out.contiguous()
-        d_gates = None
-        coeff, gate_fan, dy_buf = None, 1, None
-        if gates is not None:
-            d_gates = ops.combine_dgates(y_rows, grad_out, gates.size(1), gates.dtype)
-            coeff, gate_fan = gates.reshape(-1), gates.size(1)
-            dy_buf = y_rows
-        dy_g = grad_out if grouped_out else ops.group(grad_out, ssi, fan_out=gate_fan, coeff=coeff, out=dy_buf)
-        x_g = x if grouped_in else ops.group(x, ssi, fan_out=k)
-        d_w = None
-        if ctx.needs_input_grad[1]:
-            d_w = ops.group_bwd_W(dy_g, x_g, eo, W.size(0))
-        dx_rows = ops._scatter2scatter(dy_g, W.permute(0, 2, 1), None, None, 0.0, sei, ssi, 1, True, grouped_in,
-                                       None if grouped_in else x_g, eo)
-        d_x = dx_rows if k == 1 else ops.combine(dx_rows, None, k=k)
-        return (d_x, d_w, None, None, None, None, None, d_gates, None, None)
+    def apply(x, expert_weights, k, sorted_expert_idxs, sorted_scattered_idxs, padded_block_idxs, expert_offsets,
+              gates=None, grouped_in=False, grouped_out=False):
+        return native.linear(x, expert_weights, None, None, 1, 0, k, sorted_expert_idxs, sorted_scattered_idxs,
+                             expert_offsets, gates, grouped_in, grouped_out)
 
 
 def parallel_linear(inputs, expert_weights, k, sorted_expert_idxs, sorted_scattered_idxs, padded_block_idxs,

@@ -9,53 +9,18 @@ point ``parallel_linear_lora`` (:151-187), same positional arguments.  Differenc
 """
 from __future__ import annotations
 
-import torch
-
-from .kernels import ops
+from .._lib import native
 
 
-class ParallelLinearLora(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, expert_weights, expert_lora_A, expert_lora_B, lora_r, lora_alp, k,
-                sorted_expert_idxs, sorted_scattered_idxs, padded_block_idxs, expert_offsets,
-                gates=None, grouped_in=False, grouped_out=False):
-        x = x.contiguous() if x.stride(-1) != 1 else x
-        y = ops._scatter2scatter(x, expert_weights, expert_lora_A, expert_lora_B, lora_alp, sorted_expert_idxs,
-                                 sorted_scattered_idxs, k, grouped_in, grouped_out, None, expert_offsets)
-        if gates is not None:
-            # rows of y are token-major (t*k+j): weighted sum of each token's k rows (reference :30-35)
-            y_rows = y
-            y = ops.combine(y_rows, gates)
-        else:
-            y_rows = None
-        ctx.save_for_backward(x, expert_weights, expert_lora_A, expert_lora_B, sorted_expert_idxs,
-                              sorted_scattered_idxs, padded_block_idxs, expert_offsets, gates, y_rows)
-        ctx.flags = (grouped_in, grouped_out, k, lora_r, lora_alp)
-        return y
+class ParallelLinearLora:
+    """``apply`` with the reference's 14 positional inputs; one autograd node (C++) whose backward returns the gradients of
+    ``x``, both adapter factors and ``gates``."""
 
     @staticmethod
-    def backward(ctx, grad_out):
-        (x, W, A, B, sei, ssi, pbi, eo, gates, y_rows) = ctx.saved_tensors
-        grouped_in, grouped_out, k, lora_r, lora_alp = ctx.flags
-        grad_out = grad_out.contiguous()
-        d_gates = None
-        coeff, gate_fan, dy_buf = None, 1, None
-        if gates is not None:
-            d_gates = ops.combine_dgates(y_rows, grad_out, gates.size(1), gates.dtype)   # reference :70-72
-            coeff, gate_fan = gates.reshape(-1), gates.size(1)
-            dy_buf = y_rows                                                              # reuse the expanded buffer
-        # gradients of the adapters need dY and X in expert-grouped order (reference :83-99)
-        dy_g = grad_out if grouped_out else ops.group(grad_out, ssi, fan_out=gate_fan, coeff=coeff, out=dy_buf)
-        x_g = x if grouped_in else ops.group(x, ssi, fan_out=k)
-        dA, dB = ops.group_bwd_AB(dy_g, x_g, A, B, lora_alp / lora_r, eo, W.size(0))      # reference :102-108
-        # dX = dY W^T + s (dY B^T) A^T: the same grouped GEMM on transposed views (reference :116-128)
-        dx_rows = ops._scatter2scatter(dy_g, W.permute(0, 2, 1), B.permute(0, 2, 1), A.permute(0, 2, 1), lora_alp,
-                                       sei, ssi, 1, True, grouped_in, None if grouped_in else x_g, eo)
-        if k == 1:
-            d_x = dx_rows
-        else:
-            d_x = ops.combine(dx_rows, None, k=k)                                        # fan-out sum, reference :134
-        return (d_x, None, dA, dB, None, None, None, None, None, None, None, d_gates, None, None)
+    def apply(x, expert_weights, expert_lora_A, expert_lora_B, lora_r, lora_alp, k, sorted_expert_idxs,
+              sorted_scattered_idxs, padded_block_idxs, expert_offsets, gates=None, grouped_in=False, grouped_out=False):
+        return native.linear(x, expert_weights, expert_lora_A, expert_lora_B, lora_r, lora_alp, k, sorted_expert_idxs,
+                             sorted_scattered_idxs, expert_offsets, gates, grouped_in, grouped_out)
 
 
 def parallel_linear_lora(inputs, expert_weights, expert_lora_A, expert_lora_B, lora_r, lora_alp, k,
