@@ -83,6 +83,11 @@ except ImportError as e:
                       f"python -c 'import __graft_entry__ as g; g.build()' ({e})") from e
 
 
+def entry(name: str):
+    """The native function, or inside torch.jit.trace the same function as an operator, which a trace can record."""
+    return getattr(torch.ops.moe_hip if torch.jit.is_tracing() else native, name)
+
+
 def check(status: int, what: str) -> None:
     if status != 0:
         raise RuntimeError(f"{what} failed: {lib.moe_hip_strerror(status).decode()} (status {status})")

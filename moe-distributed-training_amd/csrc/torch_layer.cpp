@@ -6,6 +6,9 @@
 // the host spent about 10 us per library call (argument conversion, allocation, stream lookup, the interpreter lock of the
 // backward thread) and the GPU waited for it.
 #include <torch/extension.h>
+#include <torch/library.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/utils/pybind.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include "../../include/moe_hip.h"
@@ -19,7 +22,10 @@ using torch::autograd::variable_list;
 using OptTensor = std::optional<Tensor>;
 
 // Python's assert statements of the reference's entry points: an AssertionError there, and here
-struct AssertionFailure : std::runtime_error { using std::runtime_error::runtime_error; };
+struct AssertionFailure : torch::PyTorchError {
+    explicit AssertionFailure(const std::string& m) : PyTorchError(m) {}
+    PyObject* python_type() override { return PyExc_AssertionError; }
+};
 #define MOE_ASSERT(cond, msg) do { if (!(cond)) throw AssertionFailure(msg); } while (0)
 
 inline void check(int status, const char* what)
@@ -65,11 +71,13 @@ inline Tensor bytes_on(const Tensor& like, size_t n)
 
 inline Tensor unit_inner(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
 
-inline bool wants_grad(std::initializer_list<const Tensor*> ts)
+// Whether the call has to go through its autograd node: a gradient is recorded, or an input carries a forward-mode tangent
+// (which the node refuses; the plain sequence of library calls would drop it).
+inline bool needs_node(std::initializer_list<const Tensor*> ts)
 {
-    if (!at::GradMode::is_enabled()) return false;
+    const bool grad = at::GradMode::is_enabled();
     for (const Tensor* t : ts)
-        if (t->defined() && t->requires_grad()) return true;
+        if (t->defined() && ((grad && t->requires_grad()) || t->_fw_grad(0).defined())) return true;
     return false;
 }
 
@@ -326,7 +334,7 @@ variable_list router(const Tensor& x_, const Tensor& wg_, int64_t k, bool normal
     require_gpu({&x_, &wg_});
     const c10::DeviceGuard guard(x_.device());
     Tensor x = unit_inner(x_), wg = unit_inner(wg_);
-    if (wants_grad({&x, &wg})) return RouterFn::apply(x, wg, k, normalize);
+    if (needs_node({&x, &wg})) return RouterFn::apply(x, wg, k, normalize);
     RouterOut o = router_forward(x, wg, k, normalize);
     return {o.scores, o.weights, o.indices};
 }
@@ -416,7 +424,7 @@ Tensor linear_checked(const Tensor& x_, const Tensor& W, const Tensor& A, const 
     Tensor x = unit_inner(x_), ssi = ssi_.contiguous(), eo = eo_.defined() ? eo_.contiguous() : offsets_from_sorted(sei, W.size(0));
     Tensor gates = gates_.defined() ? gates_.contiguous() : Tensor();
     const LinearCfg c{scaling, scaling_ab, k, grouped_in, grouped_out};
-    if (wants_grad({&x, &W, &A, &B, &gates})) return LinearFn::apply(x, W, opt(A), opt(B), opt(gates), ssi, eo, c);
+    if (needs_node({&x, &W, &A, &B, &gates})) return LinearFn::apply(x, W, opt(A), opt(B), opt(gates), ssi, eo, c);
     Tensor y = linear_rows(x, W, A, B, ssi, eo, c);
     return gates.defined() ? combine(y, gates, nullptr, gates.size(1), gates.size(0)) : y;
 }
@@ -461,7 +469,7 @@ Tensor swiglu(const Tensor& gate_, const Tensor& up_)
     require_gpu({&gate_, &up_});
     const c10::DeviceGuard guard(gate_.device());
     Tensor gate = gate_.contiguous(), up = up_.contiguous();
-    return wants_grad({&gate, &up}) ? SwigluFn::apply(gate, up) : swiglu_forward(gate, up);
+    return needs_node({&gate, &up}) ? SwigluFn::apply(gate, up) : swiglu_forward(gate, up);
 }
 
 // out[t] = sum_j w[t,j] * y_grouped[inv[t*k+j]]  (megablocks ops.scatter, config_utils.py:251)
@@ -573,7 +581,7 @@ Tensor expert_mlp(const Tensor& x, const Tensor& w1, const Tensor& w2, const Ten
                 "other cases");
     Tensor ssi = ssi_.contiguous(), offsets = offsets_.contiguous(), gates = gates_.has_value() ? gates_->contiguous() : Tensor();
     const MlpCfg c{lt[0].defined() ? lora_alpha / (double)lt[0].size(2) : 0.0, fan_out, grouped_out && !gates.defined()};
-    if (wants_grad({&x, &w1, &w2, &w3, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5], &gates}))
+    if (needs_node({&x, &w1, &w2, &w3, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5], &gates}))
         return ExpertMlpFn::apply(x, w1, w3, w2, opt(lt[0]), opt(lt[1]), opt(lt[2]), opt(lt[3]), opt(lt[4]), opt(lt[5]), opt(gates), ssi, offsets, c);
     const MlpShape s{w1.size(0), w1.size(2), w1.size(1), ssi.numel(), (int)fan_out, c.scaling};
     MlpOut o = mlp_forward(x, w1, w3, w2, describe_lora(lt, false, s.d, s.f), s, ptr(ssi), is64(ssi), ptr(offsets), is64(offsets), c.y_grouped, false);
@@ -646,22 +654,52 @@ struct LayerFn : Function<LayerFn> {
     }
 };
 
+// The factors as views (E, K, r) / (E, r, N) of their storage
+void lora_storage_to_views(Tensor* lt, int64_t E, int64_t d, int64_t f, int64_t rank)
+{
+    for (int i = 0; i < 6; ++i) {
+        const bool on_ffn = i == 1 || i == 3 || i == 4;
+        Tensor v = lt[i].view({E, on_ffn ? f : d, rank});
+        lt[i] = i % 2 == 0 ? v : v.transpose(1, 2);
+    }
+}
+
 // x (T, d); wg (E, d); expert weights (E, f, d), or (E*f, d) with `storage`; lora: empty, or six factors -- views, or with
 // `storage` the block's A.weight / B.weight as a1, b1, a3, b3, a2 (= B of w2), b2 (= A of w2).
 // -> out (T, d), expert weights (T, k) fp32, expert indices (T, k) int32
-variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1, const Tensor& w2, const Tensor& w3, int64_t E, int64_t f, int64_t k,
+variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const Tensor& w2_, const Tensor& w3_, int64_t E, int64_t f, int64_t k,
                     const std::vector<Tensor>& lora, double lora_alpha, bool normalize, bool storage)
 {
-    require_gpu({&x, &wg, &w1, &w2, &w3});
+    require_gpu({&x, &wg, &w1_, &w2_, &w3_});
     const c10::DeviceGuard guard(x.device());
     const int64_t d = x.size(1);
+    // (the fused launches take sizes from E, f and the input's columns, so every weight is held against them here)
+    TORCH_CHECK(wg.dim() == 2 && wg.size(0) == E, "router weight of ", wg.sizes(), " does not fit ", E, " experts");
+    auto whole = [&](const Tensor& w) {   // storage order, as the launches address it
+        TORCH_CHECK(w.size(-1) == d && (storage ? w.numel() == E * f * d : w.numel() >= E * f * d), "expert weights of ", w.sizes(), " do not fit ", E, " experts of ", f, " x ", d);
+        return w.contiguous();
+    };
+    const Tensor w1 = whole(w1_), w2 = whole(w2_), w3 = whole(w3_);
     Tensor lt[6];
     for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
     const int64_t rank = lt[0].defined() ? lt[0].size(storage ? 1 : 2) : 0;
     const double scaling = rank ? lora_alpha / (double)rank : 0.0;
+    if (rank && storage) {
+        bool contiguous = true;
+        for (int i = 0; i < 6; ++i) {
+            const bool on_ffn = i == 1 || i == 3 || i == 4;
+            TORCH_CHECK(lt[i].numel() == E * (on_ffn ? f : d) * rank, "adapter factor of ", lt[i].sizes(), " does not fit ", E, " experts of ",
+                        on_ffn ? f : d, " rows and rank ", rank);
+            contiguous = contiguous && lt[i].is_contiguous();
+        }
+        if (!contiguous) {
+            lora_storage_to_views(lt, E, d, f, rank);
+            storage = false;
+        }
+    }
     if (fast_path_ok(x, w1, w2, w3, lt, storage, E, d, f)) {
         const LayerCfg c{scaling, E, d, f, k, normalize, storage};
-        if (wants_grad({&x, &wg, &w1, &w2, &w3, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]}))
+        if (needs_node({&x, &wg, &w1, &w2, &w3, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]}))
             return LayerFn::apply(x, wg, w1, w3, w2, opt(lt[0]), opt(lt[1]), opt(lt[2]), opt(lt[3]), opt(lt[4]), opt(lt[5]), c);
         LayerOut o = layer_forward(x, wg, w1, w3, w2, lt, c, false);
         return {o.out, o.rt.weights, o.rt.indices};
@@ -671,32 +709,47 @@ variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1, const T
     const Sorted so = sort_assignments(rt[2], E);
     const Tensor sei = so.ints.narrow(0, 0, so.R), ssi = so.ints.narrow(0, so.R, so.R), inv = so.ints.narrow(0, 2 * so.R, so.R),
                  offsets = so.ints.narrow(0, 3 * so.R, E);
-    if (storage && rank) {
-        for (int i = 0; i < 6; ++i) {
-            const bool on_ffn = i == 1 || i == 3 || i == 4;
-            Tensor v = lt[i].view({E, on_ffn ? f : d, rank});
-            lt[i] = i % 2 == 0 ? v : v.transpose(1, 2);
-        }
-    }
+    if (storage && rank) lora_storage_to_views(lt, E, d, f, rank);
     auto proj = [&](const Tensor& in, const Tensor& w, bool n_contiguous, int ia, int64_t fan, bool gin) {
         Tensor W = w.view({E, f, d});
         return linear_checked(in, n_contiguous ? W : W.transpose(1, 2), lt[ia], lt[ia + 1], scaling, scaling, fan, sei, ssi, offsets, Tensor(), gin, true);
     };
     Tensor h = swiglu(proj(x, w1, false, 0, k, false), proj(x, w3, false, 2, k, false));
     Tensor y = proj(h, w2, true, 4, 1, true);
-    Tensor out = wants_grad({&y, &rt[1]}) ? GatherCombineFn::apply(y, rt[1], inv, ssi) : combine(y, rt[1], so.inv(), k, x.size(0));
+    Tensor out = needs_node({&y, &rt[1]}) ? GatherCombineFn::apply(y, rt[1], inv, ssi) : combine(y, rt[1], so.inv(), k, x.size(0));
     return {out, rt[1], rt[2]};
 }
 
 }  // namespace
 
+// Called from Python without the interpreter lock.  The wrapper carries a Python exception that is raised below (a saved-tensor
+// hook's, such as the one that ends a recomputation of activation checkpointing early) through as itself.
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
-    py::register_exception<AssertionFailure>(m, "ShapeError", PyExc_AssertionError);
-    m.def("router", &router, py::call_guard<py::gil_scoped_release>());
-    m.def("linear", &linear, py::call_guard<py::gil_scoped_release>());
-    m.def("swiglu", &swiglu, py::call_guard<py::gil_scoped_release>());
-    m.def("mlp_fast_path", &mlp_fast_path);
-    m.def("expert_mlp", &expert_mlp, py::call_guard<py::gil_scoped_release>());
-    m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
+    m.def("router", torch::wrap_pybind_function_no_gil(router));
+    m.def("linear", torch::wrap_pybind_function_no_gil(linear));
+    m.def("swiglu", torch::wrap_pybind_function_no_gil(swiglu));
+    m.def("mlp_fast_path", torch::wrap_pybind_function(mlp_fast_path));
+    m.def("expert_mlp", torch::wrap_pybind_function_no_gil(expert_mlp));
+    m.def("layer", torch::wrap_pybind_function_no_gil(layer));
+}
+
+// The same functions as dispatcher operators, for torch.jit.trace: a trace records operators, and of the functions above it
+// would see their allocations only.  (Calls outside a trace take the functions above, which cost less to enter.)
+TORCH_LIBRARY(moe_hip, m)
+{
+    m.def("router", [](const Tensor& x, const Tensor& wg, int64_t k, bool normalize) { return router(x, wg, k, normalize); });
+    m.def("linear", [](const Tensor& x, const Tensor& W, const OptTensor& A, const OptTensor& B, double lora_r, double lora_alpha, int64_t k,
+                       const Tensor& sei, const Tensor& ssi, const OptTensor& eo, const OptTensor& gates, bool grouped_in, bool grouped_out) {
+        return linear(x, W, A, B, lora_r, lora_alpha, k, sei, ssi, eo, gates, grouped_in, grouped_out);
+    });
+    m.def("swiglu", [](const Tensor& gate, const Tensor& up) { return swiglu(gate, up); });
+    m.def("expert_mlp", [](const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& w3, int64_t fan_out, const Tensor& ssi,
+                           const Tensor& offsets, at::TensorList lora, double lora_alpha, const OptTensor& gates, bool grouped_out) {
+        return expert_mlp(x, w1, w2, w3, fan_out, ssi, offsets, lora.vec(), lora_alpha, gates, grouped_out);
+    });
+    m.def("layer", [](const Tensor& x, const Tensor& wg, const Tensor& w1, const Tensor& w2, const Tensor& w3, int64_t E, int64_t f, int64_t k,
+                      at::TensorList lora, double lora_alpha, bool normalize, bool storage) {
+        return layer(x, wg, w1, w2, w3, E, f, k, lora.vec(), lora_alpha, normalize, storage);
+    });
 }

@@ -14,7 +14,7 @@ from typing import NamedTuple, Optional, Tuple
 import torch
 import torch.nn as nn
 
-from .._lib import native, require_gpu
+from .._lib import entry, native, require_gpu
 from ..scattermoe_utils.kernels import ops
 from ..scattermoe_utils.parallel_experts import parallel_linear
 from ..scattermoe_utils.parallel_linear_lora import parallel_linear_lora
@@ -63,8 +63,8 @@ def fused_expert_mlp(x, w1, w2, w3, k, sorted_scattered_idxs, expert_offsets, lo
     layout; ``k`` = fan-out of x rows (top_k, or 1 for pre-dispatched rows).  With ``gates`` (T, k) the k expert
     rows of each token are combined and (T, d) is returned; otherwise one row per assignment, in grouped order
     when ``grouped_out`` else at its flat position."""
-    return native.expert_mlp(x, w1, w2, w3, k, sorted_scattered_idxs, expert_offsets, [] if lora is None else list(lora),
-                             lora_alpha, gates, grouped_out)
+    return entry("expert_mlp")(x, w1, w2, w3, k, sorted_scattered_idxs, expert_offsets, [] if lora is None else list(lora),
+                               lora_alpha, gates, grouped_out)
 
 
 def scattermoe_permute_and_compute(x, w1, w2, w3, ffn_hidden_size, hidden_size, top_k, bin_ids, indices, num_experts,
@@ -105,7 +105,7 @@ def scattermoe_permute_and_compute(x, w1, w2, w3, ffn_hidden_size, hidden_size, 
                                     gin, gout)
     h1 = proj(x, "w1", fan, False, True)
     h3 = proj(x, "w3", fan, False, True)
-    h = native.swiglu(h1, h3)
+    h = entry("swiglu")(h1, h3)
     return proj(h, "w2", 1, True, grouped_out)
 
 
@@ -124,7 +124,7 @@ def _layer(x, wg, w1, w2, w3, E, f, top_k, lora, lora_alpha, normalize, storage)
         require_gpu(x, wg, w1, w2, w3)
         return (x.clone(), torch.zeros((0, top_k), dtype=torch.float32, device=x.device),
                 torch.zeros((0, top_k), dtype=torch.int32, device=x.device))
-    return native.layer(x, wg, w1, w2, w3, E, f, top_k, lora, lora_alpha, bool(normalize), storage)
+    return entry("layer")(x, wg, w1, w2, w3, E, f, top_k, lora, lora_alpha, bool(normalize), storage)
 
 
 class ScatterMoEBlock(nn.Module):

@@ -8,7 +8,7 @@ from typing import NamedTuple, Optional
 
 import torch
 
-from .._lib import lib, check, dtype_code, native, ptr, require_gpu, stream_ptr, workspace
+from .._lib import lib, check, dtype_code, entry, ptr, require_gpu, stream_ptr, workspace
 from ..scattermoe_utils.kernels import ops
 
 
@@ -170,7 +170,7 @@ def forward_router(x: torch.Tensor, weight: torch.Tensor, top_k: int, moe_normal
     p = moe_normalize_expert_weights
     p = None if p in (None, False, 0) else (1 if p is True else p)
     if bias is None and p in (None, 1):
-        scores, w, idx = native.router(x2, weight, top_k, p == 1)
+        scores, w, idx = entry("router")(x2, weight, top_k, p == 1)
     else:
         logits = _LogitsFn.apply(x2, weight)
         if bias is not None:

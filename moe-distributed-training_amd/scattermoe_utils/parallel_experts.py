@@ -6,7 +6,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from .._lib import native
+from .._lib import entry
 
 
 class ParallelLinear:
@@ -15,8 +15,8 @@ class ParallelLinear:
     @staticmethod
     def apply(x, expert_weights, k, sorted_expert_idxs, sorted_scattered_idxs, padded_block_idxs, expert_offsets,
               gates=None, grouped_in=False, grouped_out=False):
-        return native.linear(x, expert_weights, None, None, 1, 0, k, sorted_expert_idxs, sorted_scattered_idxs,
-                             expert_offsets, gates, grouped_in, grouped_out)
+        return entry("linear")(x, expert_weights, None, None, 1, 0, k, sorted_expert_idxs, sorted_scattered_idxs,
+                               expert_offsets, gates, grouped_in, grouped_out)
 
 
 def parallel_linear(inputs, expert_weights, k, sorted_expert_idxs, sorted_scattered_idxs, padded_block_idxs,

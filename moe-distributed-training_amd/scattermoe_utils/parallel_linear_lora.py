@@ -9,7 +9,7 @@ point ``parallel_linear_lora`` (:151-187), same positional arguments.  Differenc
 """
 from __future__ import annotations
 
-from .._lib import native
+from .._lib import entry
 
 
 class ParallelLinearLora:
@@ -19,8 +19,8 @@ class ParallelLinearLora:
     @staticmethod
     def apply(x, expert_weights, expert_lora_A, expert_lora_B, lora_r, lora_alp, k, sorted_expert_idxs,
               sorted_scattered_idxs, padded_block_idxs, expert_offsets, gates=None, grouped_in=False, grouped_out=False):
-        return native.linear(x, expert_weights, expert_lora_A, expert_lora_B, lora_r, lora_alp, k, sorted_expert_idxs,
-                             sorted_scattered_idxs, expert_offsets, gates, grouped_in, grouped_out)
+        return entry("linear")(x, expert_weights, expert_lora_A, expert_lora_B, lora_r, lora_alp, k, sorted_expert_idxs,
+                               sorted_scattered_idxs, expert_offsets, gates, grouped_in, grouped_out)
 
 
 def parallel_linear_lora(inputs, expert_weights, expert_lora_A, expert_lora_B, lora_r, lora_alp, k,
