@@ -112,11 +112,13 @@ constexpr int MOE_PACK_MAX_JOBS = 12;
 struct MoePackJob { const uint16_t* src; int64_t se, sk, sr; uint16_t* dst; int64_t K; int transpose; int rank; };   // rank <= 16 columns, zero padded to 16
 struct MoePackBatch { MoePackJob job[MOE_PACK_MAX_JOBS]; int njobs; int E; int* zero_ptr; int zero_n; };   // zero_ptr[0..zero_n) is cleared by the launch
 int moe_launch_pack_lora_batch(const MoePackBatch& jobs, hipStream_t stream);
-int moe_launch_pack_lora(const void* src, int64_t se, int64_t sk, int64_t sr, void* dst, int E, int64_t K, int rank,
-                         int transpose, hipStream_t stream);
-int moe_launch_rows_lora(const void* X, int64_t ldx, const void* At, void* Q, void* Qt, int64_t ldqt, const void* pos,
-                         int pos64, const void* offsets, int off64, int E, int64_t R, int64_t K, int fan_out,
-                         int x_grouped, float scaling, const float* qt_row_scale, hipStream_t stream, int f16 = 0);
+// up to MOE_LORA_MAX_JOBS products in one launch over the same row order: Q = scaling * X . A in storage type, [R][16], its
+// transposed copy Qt (row pitch ldqt) and a copy of Q scaled like Qt (each optional)
+constexpr int MOE_LORA_MAX_JOBS = 4;
+struct MoeRowsLoraJob { const void* X; int64_t ldx, K; const void* At; void* Q; void* Qt; void* q_scaled; };
+int moe_launch_rows_lora_jobs(const MoeRowsLoraJob* jobs, int njobs, int64_t ldqt, const void* pos, int pos64, const void* offsets,
+                              int off64, int E, int64_t R, int fan_out, int x_grouped, float scaling, const float* qt_row_scale,
+                              hipStream_t stream, int f16);
 // two products over the same rows in one launch (X2 == nullptr: only the first)
 // q_scaled (optional): a third output of the first product, [R][16] like Q but multiplied by qt_row_scale like Qt
 int moe_launch_rows_lora2(const void* X, const void* X2, int64_t ldx, const void* At, const void* At2, void* Q, void* Q2,
@@ -139,10 +141,12 @@ int moe_launch_xtp2(const void* X, const void* X2, int64_t ldx, const void* pos,
                     const void* Pt2, int64_t ldpt, const float* p_row_scale, void* out, void* out2, const int64_t* so,
                     const int64_t* so2, int rank, int rank2, const void* offsets, int off64, int E, int64_t R, int64_t K,
                     float scale, void* workspace, size_t workspace_bytes, hipStream_t stream, int f16 = 0);
-int moe_launch_xtp(const void* X, int64_t ldx, const void* pos, int pos64, int fan_out, const void* Pt, int64_t ldpt,
-                   const float* p_row_scale, void* out, int64_t soe, int64_t sok, int64_t sor, int rank,
-                   const void* offsets, int off64, int E, int64_t R, int64_t K, float scale, void* workspace,
-                   size_t workspace_bytes, hipStream_t stream, int f16 = 0);
+// up to MOE_LORA_MAX_JOBS reductions over the same row order in one launch pair; needs njobs times moe_xtp_workspace_bytes of
+// the widest job
+struct MoeXtpJob { const void* X; int64_t ldx, K; const void* Pt; void* out; int64_t so[3]; int rank; };
+int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, const void* pos, int pos64, int fan_out, int64_t ldpt, const float* p_row_scale,
+                        const void* offsets, int off64, int E, int64_t R, float scale, void* workspace, size_t workspace_bytes,
+                        hipStream_t stream, int f16);
 
 // router + integer pipeline
 int moe_launch_router_logits(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits,

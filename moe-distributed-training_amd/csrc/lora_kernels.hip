@@ -25,25 +25,6 @@ __device__ __forceinline__ void unit_and_job(int njobs, int64_t* unit, int* job)
 }
 inline unsigned job_grid(int64_t units, int njobs) { return (unsigned)((units + JOB_GROUP - 1) / JOB_GROUP * JOB_GROUP * njobs); }
 
-// (fragment order covers K rounded up to whole 32-wide fragments; positions at or past K hold zeros, so a consumer may
-// feed them anything finite)
-__global__ void pack_lora_kernel(const uint16_t* __restrict__ src, int64_t se, int64_t sk, int64_t sr,
-                                 uint16_t* __restrict__ dst, int64_t K, int64_t Kimg, int rank, int transpose, int64_t total)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const int64_t e = i / (Kimg * 16), rem = i % (Kimg * 16);
-    int64_t k;
-    int r;
-    if (transpose) {   // fragment order: one 16x16x32 operand fragment is 1 KiB of consecutive memory
-        const int64_t kb = rem / 512;
-        const int lane = (int)(rem % 512) / 8, t = (int)(rem % 8);
-        r = lane & 15;
-        k = kb * 32 + 8 * (lane >> 4) + t;
-    } else { k = rem / 16; r = (int)(rem % 16); }           // dst[e][k][r]
-    dst[i] = (r < rank && k < K) ? src[e * se + k * sk + r * sr] : (uint16_t)0;
-}
-
 // several pack jobs in one launch (blockIdx.y selects the job): the six factors of an MLP block are a few MB in total,
 // so separate launches would cost more in launch latency than in data movement.  A thread produces 16 bytes: the 8
 // consecutive output elements of a chunk walk the source with one stride (rank stride in [K][16] order, k stride in
@@ -51,36 +32,44 @@ __global__ void pack_lora_kernel(const uint16_t* __restrict__ src, int64_t se, i
 // which saves that caller a launch of its own.
 __global__ void pack_lora_batch_kernel(const MoePackBatch jobs)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.y == 0)
-        for (int z = i; z < jobs.zero_n; z += gridDim.x * blockDim.x) jobs.zero_ptr[z] = 0;
+        for (int64_t z = i; z < jobs.zero_n; z += (int64_t)gridDim.x * blockDim.x) jobs.zero_ptr[z] = 0;
     const MoePackJob& j = jobs.job[blockIdx.y];
-    const int K = (int)j.K, rank = j.rank;
-    const int per_e = K * 2;                 // chunks per expert
+    const int64_t K = j.K;
+    const int rank = j.rank;
+    // chunks per expert; fragment order covers K rounded up to whole 32-wide fragments with zeros past K, so a consumer may
+    // feed those anything finite
+    const int64_t per_e = (j.transpose ? (K + 31) / 32 * 32 : K) * 2;
     if (i >= jobs.E * per_e) return;
-    const int e = i / per_e, rem = i % per_e;
-    int k, r;
+    int64_t e, rem;
+    if (jobs.E * per_e <= 0xffffffffll) { e = (uint32_t)i / (uint32_t)per_e; rem = (uint32_t)i % (uint32_t)per_e; }   // (a 64-bit division costs more than the copy)
+    else { e = i / per_e; rem = i % per_e; }
+    int64_t k;
+    int r;
     int64_t stride;
     if (j.transpose) {                        // chunk = (fragment kb, lane): r fixed, 8 consecutive k
-        const int kb = rem >> 6, lane = rem & 63;
+        const int64_t kb = rem >> 6;
+        const int lane = (int)(rem & 63);
         r = lane & 15;
         k = kb * 32 + 8 * (lane >> 4);
         stride = j.sk;
     } else {                                  // chunk = (k, half): k fixed, 8 consecutive r
         k = rem >> 1;
-        r = (rem & 1) * 8;
+        r = (int)(rem & 1) * 8;
         stride = j.sr;
     }
-    const uint16_t* sp = j.src + (int64_t)e * j.se + (int64_t)k * j.sk + (int64_t)r * j.sr;
+    const uint16_t* sp = j.src + e * j.se + k * j.sk + r * j.sr;
+    const int live = j.transpose ? (r < rank ? (k + 8 <= K ? 8 : (k < K ? (int)(K - k) : 0)) : 0) : (r + 8 <= rank ? 8 : rank - r);   // elements of the chunk that exist
     uint4 out;
-    if (j.transpose ? (r >= rank) : false) {
+    if (live <= 0) {
         out = make_uint4(0, 0, 0, 0);
-    } else if (stride == 1 && (((uintptr_t)sp) & 15) == 0 && (j.transpose || r + 8 <= rank)) {
+    } else if (stride == 1 && (((uintptr_t)sp) & 15) == 0 && live == 8) {
         out = *(const uint4*)sp;
     } else {
         uint16_t v[8];
 #pragma unroll
-        for (int t = 0; t < 8; ++t) v[t] = (j.transpose || r + t < rank) ? sp[t * stride] : (uint16_t)0;
+        for (int t = 0; t < 8; ++t) v[t] = t < live ? sp[t * stride] : (uint16_t)0;
         out.x = v[0] | ((uint32_t)v[1] << 16); out.y = v[2] | ((uint32_t)v[3] << 16);
         out.z = v[4] | ((uint32_t)v[5] << 16); out.w = v[6] | ((uint32_t)v[7] << 16);
     }
@@ -105,21 +94,23 @@ static_assert(RL_KSTEPS == RL_WAVES, "one K step per wave and stage");
 // values per lane) are then read from LDS.  Loading the fragments straight from global memory would make adjacent
 // lanes touch different rows, which the memory pipeline handles one lane at a time.  All global loads of the loop are
 // inline assembly with explicit s_waitcnt: compiler-managed loads would wait for the prefetches queued behind them.
-// one or two jobs per launch (see unit_and_job): same rows, shapes and scaling, different operand / output pointers
-struct RowsLoraJob { const uint16_t* X; const uint16_t* Af; uint16_t* Q; uint16_t* Qt; uint16_t* Qs; };   // Qs: optional row-major copy scaled like Qt
+// up to four jobs per launch (see unit_and_job): same row order and scaling, operands and outputs of their own
+struct RowsLoraJob { const uint16_t* X; const uint16_t* Af; uint16_t* Q; uint16_t* Qt; uint16_t* Qs; int64_t ldx, K; };   // Q, Qt, Qs: optional; Qs row-major like Q, scaled like Qt
+struct RowsLoraJobs { RowsLoraJob job[MOE_LORA_MAX_JOBS]; };
 // ROWS = 32 rows per workgroup, or 16 when a launch of 32-row tiles would leave most compute units with a single
 // workgroup (and so with too few loads in flight)
 template <int ROWS, typename Num>
-__global__ void __launch_bounds__(RL_THREADS) rows_lora_kernel(const RowsLoraJob job0, const RowsLoraJob job1, int64_t ldx,
+__global__ void __launch_bounds__(RL_THREADS) rows_lora_kernel(const RowsLoraJobs jobs,
                                                                int64_t ldqt, const void* __restrict__ pos, int pos64,
                                                                const void* __restrict__ offsets, int off64, int E,
-                                                               int64_t K, int fan_out, int x_grouped, float scaling,
+                                                               int fan_out, int x_grouped, float scaling,
                                                                const float* __restrict__ qt_row_scale, int njobs)
 {
     int64_t tile_id;
     int job_id;
     unit_and_job(njobs, &tile_id, &job_id);
-    const RowsLoraJob& job = job_id ? job1 : job0;
+    const RowsLoraJob& job = jobs.job[job_id];
+    const int64_t ldx = job.ldx, K = job.K;
     const uint16_t* __restrict__ X = job.X;
     const uint16_t* __restrict__ Af = job.Af;
     uint16_t* __restrict__ Q = job.Q;
@@ -206,7 +197,7 @@ __global__ void __launch_bounds__(RL_THREADS) rows_lora_kernel(const RowsLoraJob
 #pragma unroll
             for (int w = 0; w < RL_WAVES; ++w) v += red[w][row][col];
             v *= scaling;
-            Q[mo * 16 + col] = Num::from_f32(v);
+            if (Q) Q[mo * 16 + col] = Num::from_f32(v);
             const float vs = qt_row_scale ? v * qt_row_scale[mo] : v;
             if (Qt) Qt[(int64_t)col * ldqt + mo] = Num::from_f32(vs);
             if (job.Qs) job.Qs[mo * 16 + col] = Num::from_f32(vs);
@@ -225,25 +216,29 @@ constexpr int XTP_COLS = 4 * XTP_WCOLS;  // columns per workgroup
 // (8 x 16-byte loads) and transposes them in registers into 8 column fragments; the P fragment is one 16-byte
 // load from the transposed copy Pt.  Each wave owns 128 columns and walks the tile's rows 32 at a time with the
 // next block's loads in flight, so there is no cross-wave reduction.
-// one or two jobs per launch (see unit_and_job): same rows and shapes, different operands / outputs; job j's partials start
-// at partial + j * partial_stride
-struct XtpJob { const uint16_t* X; const uint16_t* Pt; uint16_t* out; int64_t soe, sok, sor; int rank; };   // rank: columns written (<= 16)
+// up to four jobs per launch (see unit_and_job): same row order, operands and outputs of their own; job j's partials start
+// at partial + j * partial_stride.  A single projection's adapter gradients are two jobs per 16 rank columns (X with P, dY
+// with Q), of 152 workgroups each at 3000 rows over 8 experts and 4096 columns: too few to fill the chip one at a time.
+struct XtpJob { const uint16_t* X; const uint16_t* Pt; uint16_t* out; int64_t soe, sok, sor; int rank; int64_t ldx, K; };   // rank: columns written (<= 16)
+struct XtpJobs { XtpJob job[MOE_LORA_MAX_JOBS]; };
 template <typename Num>
-__global__ void __launch_bounds__(XTP_THREADS) xtp_partial_kernel(const XtpJob job0, const XtpJob job1, int64_t ldx,
+__global__ void __launch_bounds__(XTP_THREADS) xtp_partial_kernel(const XtpJobs jobs,
                                                                   const void* __restrict__ pos, int pos64, int fan_out,
                                                                   int64_t ldpt,
                                                                   const float* __restrict__ p_row_scale,
                                                                   float* __restrict__ partial, int64_t partial_stride,
                                                                   const void* __restrict__ offsets, int off64, int E,
-                                                                  int64_t R, int64_t K, int njobs)
+                                                                  int64_t R, int njobs)
 {
     // unit = (row tile, column block), column block fastest
     int64_t unit;
     int job_id;
     unit_and_job(njobs, &unit, &job_id);
-    const int64_t kblocks = (K + XTP_COLS - 1) / XTP_COLS;
+    const XtpJob& job = jobs.job[job_id];
+    const int64_t ldx = job.ldx, K = job.K;
+    const int64_t kblocks = (K + XTP_COLS - 1) / XTP_COLS;   // (a job narrower than the launch's widest has units past its last row tile: they end below)
+    if (kblocks == 0) return;
     const int64_t tile_id = unit / kblocks, kblock = unit % kblocks;
-    const XtpJob& job = job_id ? job1 : job0;
     const uint16_t* __restrict__ X = job.X;
     const uint16_t* __restrict__ Pt = job.Pt;
     partial += (int64_t)job_id * partial_stride;
@@ -326,11 +321,11 @@ __global__ void __launch_bounds__(XTP_THREADS) xtp_partial_kernel(const XtpJob j
 // out[e][k][r] = scale * sum over the expert's partial tiles (ascending), zero for an empty expert.  A thread owns four
 // consecutive rank columns of one k (one 16-byte load per tile, several tiles in flight).
 template <typename Num>
-__global__ void xtp_reduce_kernel(const float* __restrict__ partial, int64_t partial_stride, const XtpJob job0,
-                                  const XtpJob job1, const void* __restrict__ offsets, int off64,
-                                  int E, int64_t K, float scale)
+__global__ void xtp_reduce_kernel(const float* __restrict__ partial, int64_t partial_stride, const XtpJobs jobs,
+                                  const void* __restrict__ offsets, int off64, int E, float scale)
 {
-    const XtpJob& job = blockIdx.z ? job1 : job0;
+    const XtpJob& job = jobs.job[blockIdx.z];
+    const int64_t K = job.K;
     uint16_t* __restrict__ out = job.out;
     const int64_t soe = job.soe, sok = job.sok, sor = job.sor;
     const int rank = job.rank;
@@ -416,45 +411,38 @@ int moe_launch_cc_reduce2(const float* partial, const float* partial2, int ntile
     return moe_launch_status();
 }
 
-int moe_launch_pack_lora(const void* src, int64_t se, int64_t sk, int64_t sr, void* dst, int E, int64_t K, int rank,
-                         int transpose, hipStream_t stream)
-{
-    if (rank < 1 || rank > 16) return MOE_ERR_UNSUPPORTED;
-    const int64_t Kimg = transpose ? (K + 31) / 32 * 32 : K;
-    const int64_t total = (int64_t)E * Kimg * 16;
-    if (total == 0) return MOE_OK;
-    hipLaunchKernelGGL(pack_lora_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream,
-                       (const uint16_t*)src, se, sk, sr, (uint16_t*)dst, K, Kimg, rank, transpose, total);
-    return moe_launch_status();
-}
-
 int moe_launch_pack_lora_batch(const MoePackBatch& jobs, hipStream_t stream)
 {
     if (jobs.njobs < 1 || jobs.njobs > MOE_PACK_MAX_JOBS) return MOE_ERR_UNSUPPORTED;
     for (int j = 0; j < jobs.njobs; ++j)
         if (jobs.job[j].rank < 1 || jobs.job[j].rank > 16) return MOE_ERR_UNSUPPORTED;
-    int64_t kmax = 0;
-    for (int j = 0; j < jobs.njobs; ++j) kmax = jobs.job[j].K > kmax ? jobs.job[j].K : kmax;
+    int64_t kmax = 0;   // rows of the largest image
+    for (int j = 0; j < jobs.njobs; ++j) {
+        const int64_t k = jobs.job[j].transpose ? (jobs.job[j].K + 31) / 32 * 32 : jobs.job[j].K;
+        kmax = k > kmax ? k : kmax;
+    }
     const int64_t total = (int64_t)jobs.E * kmax * 2;   // 16-byte chunks of the largest job
     if (total == 0 && jobs.zero_n == 0) return MOE_OK;
-    if (total > 0x7fffffff || jobs.zero_n < 0 || (jobs.zero_n > 0 && !jobs.zero_ptr)) return MOE_ERR_UNSUPPORTED;
+    if ((total + 255) / 256 > 0x7fffffff || jobs.zero_n < 0 || (jobs.zero_n > 0 && !jobs.zero_ptr)) return MOE_ERR_UNSUPPORTED;
     for (int j = 0; j < jobs.njobs; ++j)
-        if (((uintptr_t)jobs.job[j].dst % 16) != 0 || (jobs.job[j].transpose && jobs.job[j].K % 32 != 0)) return MOE_ERR_UNSUPPORTED;
+        if (((uintptr_t)jobs.job[j].dst % 16) != 0) return MOE_ERR_UNSUPPORTED;
     const unsigned gx = (unsigned)((total + 255) / 256);
     hipLaunchKernelGGL(pack_lora_batch_kernel, dim3(gx ? gx : 1u, (unsigned)jobs.njobs), dim3(256), 0, stream, jobs);
     return moe_launch_status();
 }
 
-int moe_launch_rows_lora2(const void* X, const void* X2, int64_t ldx, const void* At, const void* At2, void* Q, void* Q2,
-                          void* Qt, void* Qt2, int64_t ldqt, const void* pos, int pos64, const void* offsets, int off64,
-                          int E, int64_t R, int64_t K, int fan_out, int x_grouped, float scaling,
-                          const float* qt_row_scale, hipStream_t stream, void* q_scaled, int f16)
+int moe_launch_rows_lora_jobs(const MoeRowsLoraJob* jobs, int njobs, int64_t ldqt, const void* pos, int pos64, const void* offsets,
+                              int off64, int E, int64_t R, int fan_out, int x_grouped, float scaling, const float* qt_row_scale,
+                              hipStream_t stream, int f16)
 {
     if (R == 0) return MOE_OK;
-    const bool two = X2 != nullptr;
-    if (K % 8 != 0 || ldx % 8 != 0 || ((uintptr_t)X % 16) != 0 || ((uintptr_t)At % 16) != 0 ||
-        (two && (((uintptr_t)X2 % 16) != 0 || ((uintptr_t)At2 % 16) != 0)))
-        return MOE_ERR_UNSUPPORTED;
+    if (njobs < 1 || njobs > MOE_LORA_MAX_JOBS) return MOE_ERR_UNSUPPORTED;
+    RowsLoraJobs js = {};
+    for (int j = 0; j < njobs; ++j) {
+        const MoeRowsLoraJob& q = jobs[j];
+        if (q.K % 8 != 0 || q.ldx % 8 != 0 || ((uintptr_t)q.X % 16) != 0 || ((uintptr_t)q.At % 16) != 0) return MOE_ERR_UNSUPPORTED;
+        js.job[j] = {(const uint16_t*)q.X, (const uint16_t*)q.At, (uint16_t*)q.Q, (uint16_t*)q.Qt, (uint16_t*)q.q_scaled, q.ldx, q.K};
+    }
     static std::atomic<bool> attr_set[MOE_MAX_DEVICES];   // per device; forward and backward may call from different host threads
     const int dev = moe_current_device();
     if (!attr_set[dev]) {
@@ -465,29 +453,27 @@ int moe_launch_rows_lora2(const void* X, const void* X2, int64_t ldx, const void
             return MOE_ERR_LAUNCH;
         attr_set[dev] = true;
     }
-    const RowsLoraJob j0 = {(const uint16_t*)X, (const uint16_t*)At, (uint16_t*)Q, (uint16_t*)Qt, (uint16_t*)q_scaled};
-    const RowsLoraJob j1 = {(const uint16_t*)X2, (const uint16_t*)At2, (uint16_t*)Q2, (uint16_t*)Qt2, nullptr};
     // 32-row tiles halve the adapter traffic, but two workgroups fit a compute unit: use them when the launch has
     // about that many, otherwise 16-row tiles (three fit)
-    if ((R / 16 + E) * 2 + 16 >= ((int64_t)1 << 31)) return MOE_ERR_UNSUPPORTED;   // workgroups of the launch, as a 32-bit grid size
+    if ((R / 16 + E) * njobs + 8 * njobs >= ((int64_t)1 << 31)) return MOE_ERR_UNSUPPORTED;   // workgroups of the launch, as a 32-bit grid size
     const int cus = moe_device_cus();
-    const int64_t tiles32 = (R / 32 + E) * (two ? 2 : 1);
-    if (tiles32 >= 3 * (int64_t)cus / 2) {
-        hipLaunchKernelGGL((f16 ? rows_lora_kernel<32, NumF16> : rows_lora_kernel<32, NumBf16>), dim3(job_grid(R / 32 + E, two ? 2 : 1)), dim3(RL_THREADS), rl_lds(32), stream, j0, j1,
-                           ldx, ldqt, pos, pos64, offsets, off64, E, K, fan_out, x_grouped, scaling, qt_row_scale, two ? 2 : 1);
+    if ((R / 32 + E) * njobs >= 3 * (int64_t)cus / 2) {
+        hipLaunchKernelGGL((f16 ? rows_lora_kernel<32, NumF16> : rows_lora_kernel<32, NumBf16>), dim3(job_grid(R / 32 + E, njobs)), dim3(RL_THREADS), rl_lds(32), stream, js,
+                           ldqt, pos, pos64, offsets, off64, E, fan_out, x_grouped, scaling, qt_row_scale, njobs);
     } else {
-        hipLaunchKernelGGL((f16 ? rows_lora_kernel<16, NumF16> : rows_lora_kernel<16, NumBf16>), dim3(job_grid(R / 16 + E, two ? 2 : 1)), dim3(RL_THREADS), rl_lds(16), stream, j0, j1,
-                           ldx, ldqt, pos, pos64, offsets, off64, E, K, fan_out, x_grouped, scaling, qt_row_scale, two ? 2 : 1);
+        hipLaunchKernelGGL((f16 ? rows_lora_kernel<16, NumF16> : rows_lora_kernel<16, NumBf16>), dim3(job_grid(R / 16 + E, njobs)), dim3(RL_THREADS), rl_lds(16), stream, js,
+                           ldqt, pos, pos64, offsets, off64, E, fan_out, x_grouped, scaling, qt_row_scale, njobs);
     }
     return moe_launch_status();
 }
 
-int moe_launch_rows_lora(const void* X, int64_t ldx, const void* At, void* Q, void* Qt, int64_t ldqt, const void* pos,
-                         int pos64, const void* offsets, int off64, int E, int64_t R, int64_t K, int fan_out,
-                         int x_grouped, float scaling, const float* qt_row_scale, hipStream_t stream, int f16)
+int moe_launch_rows_lora2(const void* X, const void* X2, int64_t ldx, const void* At, const void* At2, void* Q, void* Q2,
+                          void* Qt, void* Qt2, int64_t ldqt, const void* pos, int pos64, const void* offsets, int off64,
+                          int E, int64_t R, int64_t K, int fan_out, int x_grouped, float scaling,
+                          const float* qt_row_scale, hipStream_t stream, void* q_scaled, int f16)
 {
-    return moe_launch_rows_lora2(X, nullptr, ldx, At, nullptr, Q, nullptr, Qt, nullptr, ldqt, pos, pos64, offsets, off64, E, R,
-                                 K, fan_out, x_grouped, scaling, qt_row_scale, stream, nullptr, f16);
+    const MoeRowsLoraJob jobs[2] = {{X, ldx, K, At, Q, Qt, q_scaled}, {X2, ldx, K, At2, Q2, Qt2, nullptr}};
+    return moe_launch_rows_lora_jobs(jobs, X2 ? 2 : 1, ldqt, pos, pos64, offsets, off64, E, R, fan_out, x_grouped, scaling, qt_row_scale, stream, f16);
 }
 
 size_t moe_xtp_workspace_bytes(int64_t R, int E, int64_t K)
@@ -495,33 +481,44 @@ size_t moe_xtp_workspace_bytes(int64_t R, int E, int64_t K)
     return (size_t)(R / XTP_RC + E) * (size_t)K * 16 * sizeof(float);
 }
 
+int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, const void* pos, int pos64, int fan_out, int64_t ldpt, const float* p_row_scale,
+                        const void* offsets, int off64, int E, int64_t R, float scale, void* workspace, size_t workspace_bytes,
+                        hipStream_t stream, int f16)
+{
+    if (njobs < 1 || njobs > MOE_LORA_MAX_JOBS) return MOE_ERR_UNSUPPORTED;
+    XtpJobs js = {};
+    int64_t kmax = 0;
+    for (int j = 0; j < njobs; ++j) {
+        const MoeXtpJob& q = jobs[j];
+        if (q.rank < 1 || q.rank > 16 || q.K % 8 != 0 || q.ldx % 8 != 0 || ((uintptr_t)q.X % 16) != 0 || ((uintptr_t)q.Pt % 16) != 0) return MOE_ERR_UNSUPPORTED;
+        js.job[j] = {(const uint16_t*)q.X, (const uint16_t*)q.Pt, (uint16_t*)q.out, q.so[0], q.so[1], q.so[2], q.rank, q.ldx, q.K};
+        kmax = q.K > kmax ? q.K : kmax;
+    }
+    if (E == 0 || kmax == 0) return MOE_OK;
+    if (ldpt % 16 != 0 || ldpt < (R + 31) / 32 * 32) return MOE_ERR_UNSUPPORTED;
+    const size_t one = moe_xtp_workspace_bytes(R, E, kmax);
+    if (workspace_bytes < one * njobs) return MOE_ERR_WORKSPACE;
+    const int64_t pstride = (int64_t)(one / sizeof(float));
+    if (R > 0) {
+        const int64_t units = ((kmax + XTP_COLS - 1) / XTP_COLS) * (R / XTP_RC + E);
+        if ((units + 8) * njobs >= ((int64_t)1 << 31)) return MOE_ERR_UNSUPPORTED;
+        hipLaunchKernelGGL(f16 ? xtp_partial_kernel<NumF16> : xtp_partial_kernel<NumBf16>, dim3(job_grid(units, njobs)), dim3(XTP_THREADS), 0, stream, js, pos, pos64, fan_out, ldpt,
+                           p_row_scale, (float*)workspace, pstride, offsets, off64, E, R, njobs);
+    }
+    dim3 rgrid((unsigned)((kmax * 4 + 255) / 256), (unsigned)E, (unsigned)njobs);
+    hipLaunchKernelGGL(f16 ? xtp_reduce_kernel<NumF16> : xtp_reduce_kernel<NumBf16>, rgrid, dim3(256), 0, stream, (const float*)workspace, pstride, js, offsets,
+                       off64, E, scale);
+    return moe_launch_status();
+}
+
 int moe_launch_xtp2(const void* X, const void* X2, int64_t ldx, const void* pos, int pos64, int fan_out, const void* Pt,
                     const void* Pt2, int64_t ldpt, const float* p_row_scale, void* out, void* out2, const int64_t* so,
                     const int64_t* so2, int rank, int rank2, const void* offsets, int off64, int E, int64_t R, int64_t K,
                     float scale, void* workspace, size_t workspace_bytes, hipStream_t stream, int f16)
 {
-    if (E == 0 || K == 0) return MOE_OK;
-    const bool two = X2 != nullptr;
-    if (rank < 1 || rank > 16 || (two && (rank2 < 1 || rank2 > 16))) return MOE_ERR_UNSUPPORTED;
-    if (K % 8 != 0 || ldx % 8 != 0 || ldpt % 16 != 0 || ldpt < (R + 31) / 32 * 32 || ((uintptr_t)X % 16) != 0 ||
-        ((uintptr_t)Pt % 16) != 0 || (two && (((uintptr_t)X2 % 16) != 0 || ((uintptr_t)Pt2 % 16) != 0)))
-        return MOE_ERR_UNSUPPORTED;
-    const size_t one = moe_xtp_workspace_bytes(R, E, K);
-    if (workspace_bytes < one * (two ? 2 : 1)) return MOE_ERR_WORKSPACE;
-    const int64_t tiles = R / XTP_RC + E;
-    const XtpJob j0 = {(const uint16_t*)X, (const uint16_t*)Pt, (uint16_t*)out, so[0], so[1], so[2], rank};
-    const XtpJob j1 = two ? XtpJob{(const uint16_t*)X2, (const uint16_t*)Pt2, (uint16_t*)out2, so2[0], so2[1], so2[2], rank2} : j0;
-    const int64_t pstride = (int64_t)(one / sizeof(float));
-    if (R > 0) {
-        const int64_t units = ((K + XTP_COLS - 1) / XTP_COLS) * tiles;
-        if (units * 2 + 16 >= ((int64_t)1 << 31)) return MOE_ERR_UNSUPPORTED;
-        hipLaunchKernelGGL(f16 ? xtp_partial_kernel<NumF16> : xtp_partial_kernel<NumBf16>, dim3(job_grid(units, two ? 2 : 1)), dim3(XTP_THREADS), 0, stream, j0, j1, ldx, pos, pos64, fan_out, ldpt,
-                           p_row_scale, (float*)workspace, pstride, offsets, off64, E, R, K, two ? 2 : 1);
-    }
-    dim3 rgrid((unsigned)((K * 4 + 255) / 256), (unsigned)E, two ? 2u : 1u);
-    hipLaunchKernelGGL(f16 ? xtp_reduce_kernel<NumF16> : xtp_reduce_kernel<NumBf16>, rgrid, dim3(256), 0, stream, (const float*)workspace, pstride, j0, j1, offsets,
-                       off64, E, K, scale);
-    return moe_launch_status();
+    MoeXtpJob jobs[2] = {{X, ldx, K, Pt, out, {so[0], so[1], so[2]}, rank}, {}};
+    if (X2) jobs[1] = {X2, ldx, K, Pt2, out2, {so2[0], so2[1], so2[2]}, rank2};
+    return moe_launch_xtp_jobs(jobs, X2 ? 2 : 1, pos, pos64, fan_out, ldpt, p_row_scale, offsets, off64, E, R, scale, workspace, workspace_bytes, stream, f16);
 }
 
 int moe_launch_xtp_reduce2(const float* partial, const float* partial2, void* out, void* out2, const int64_t* so,
@@ -531,20 +528,11 @@ int moe_launch_xtp_reduce2(const float* partial, const float* partial2, void* ou
     if (E == 0 || K == 0) return MOE_OK;
     const bool two = partial2 != nullptr;
     if (rank < 1 || rank > 16 || (two && (rank2 < 1 || rank2 > 16))) return MOE_ERR_UNSUPPORTED;
-    const XtpJob j0 = {nullptr, nullptr, (uint16_t*)out, so[0], so[1], so[2], rank};
-    const XtpJob j1 = two ? XtpJob{nullptr, nullptr, (uint16_t*)out2, so2[0], so2[1], so2[2], rank2} : j0;
+    XtpJobs js = {};
+    js.job[0] = {nullptr, nullptr, (uint16_t*)out, so[0], so[1], so[2], rank, 0, K};
+    if (two) js.job[1] = {nullptr, nullptr, (uint16_t*)out2, so2[0], so2[1], so2[2], rank2, 0, K};
     dim3 rgrid((unsigned)((K * 4 + 255) / 256), (unsigned)E, two ? 2u : 1u);
-    hipLaunchKernelGGL(f16 ? xtp_reduce_kernel<NumF16> : xtp_reduce_kernel<NumBf16>, rgrid, dim3(256), 0, stream, partial, two ? (int64_t)(partial2 - partial) : 0, j0, j1,
-                       offsets, off64, E, K, scale);
+    hipLaunchKernelGGL(f16 ? xtp_reduce_kernel<NumF16> : xtp_reduce_kernel<NumBf16>, rgrid, dim3(256), 0, stream, partial, two ? (int64_t)(partial2 - partial) : 0, js,
+                       offsets, off64, E, scale);
     return moe_launch_status();
-}
-
-int moe_launch_xtp(const void* X, int64_t ldx, const void* pos, int pos64, int fan_out, const void* Pt, int64_t ldpt,
-                   const float* p_row_scale, void* out, int64_t soe, int64_t sok, int64_t sor, int rank,
-                   const void* offsets, int off64, int E, int64_t R, int64_t K, float scale, void* workspace,
-                   size_t workspace_bytes, hipStream_t stream, int f16)
-{
-    const int64_t so[3] = {soe, sok, sor};
-    return moe_launch_xtp2(X, nullptr, ldx, pos, pos64, fan_out, Pt, nullptr, ldpt, p_row_scale, out, nullptr, so, nullptr, rank,
-                           0, offsets, off64, E, R, K, scale, workspace, workspace_bytes, stream, f16);
 }

@@ -263,19 +263,28 @@ int moe_scatter2scatter(const void* X, int64_t sxm, int64_t sxk, const void* W, 
                 // x A B = sum over 16-wide chunks c of x A[:, c] B[c, :]: a rank above 16 enters as several 16-wide K slabs
                 const int nh = (rank + 15) / 16;
                 void *At[MOE_MAX_STRIDED_SLABS] = {}, *LB[MOE_MAX_STRIDED_SLABS] = {}, *Q[MOE_MAX_STRIDED_SLABS] = {};
+                MoePackBatch pb = {};   // also clears the GEMM's K-split counters
+                pb.E = E; pb.zero_ptr = p.sk_counters; pb.zero_n = moe_gemm_num_counters();
+                p.counters_clean = 1;
                 for (int hf = 0; hf < nh; ++hf) {
                     At[hf] = ws.take(pack_bytes(E, K));
                     LB[hf] = ws.take(pack_bytes(E, N));
                     Q[hf] = ws.take(q_bytes(R));
                     const int r0 = 16 * hf, rk = (rank - r0 < 16) ? rank - r0 : 16;
-                    TRY(moe_launch_pack_lora((const uint16_t*)A + r0 * sar, sae, sak, sar, At[hf], E, K, rk, 1, S(stream)));
-                    TRY(moe_launch_pack_lora((const uint16_t*)B + r0 * sbr, sbe, sbn, sbr, LB[hf], E, N, rk, 0, S(stream)));
+                    pb.job[pb.njobs++] = {(const uint16_t*)A + r0 * sar, sae, sak, sar, (uint16_t*)At[hf], K, 1, rk};
+                    pb.job[pb.njobs++] = {(const uint16_t*)B + r0 * sbr, sbe, sbn, sbr, (uint16_t*)LB[hf], N, 0, rk};
+                    if (pb.njobs == MOE_PACK_MAX_JOBS || hf + 1 == nh) {
+                        TRY(moe_launch_pack_lora_batch(pb, S(stream)));
+                        pb.njobs = 0; pb.zero_n = 0;
+                    }
                     if (hf < MOE_MAX_SLABS) { p.Q[hf] = (const uint16_t*)Q[hf]; p.LB[hf] = (const uint16_t*)LB[hf]; }
                 }
-                for (int hf = 0; hf < nh; hf += 2)   // two products over the same rows per launch
-                    TRY(moe_launch_rows_lora2(X, hf + 1 < nh ? X : nullptr, sxm, At[hf], hf + 1 < nh ? At[hf + 1] : nullptr, Q[hf],
-                                              hf + 1 < nh ? Q[hf + 1] : nullptr, nullptr, nullptr, 0, pos, pos64, offsets, off64, E, R, K,
-                                              fan_out, x_grouped, scaling, nullptr, S(stream), nullptr, f16));
+                for (int hf = 0; hf < nh; hf += MOE_LORA_MAX_JOBS) {   // products over the same rows share a launch
+                    MoeRowsLoraJob jobs[MOE_LORA_MAX_JOBS];
+                    int n = 0;
+                    for (; n < MOE_LORA_MAX_JOBS && hf + n < nh; ++n) jobs[n] = {X, sxm, K, At[hf + n], Q[hf + n], nullptr, nullptr};
+                    TRY(moe_launch_rows_lora_jobs(jobs, n, 0, pos, pos64, offsets, off64, E, R, fan_out, x_grouped, scaling, nullptr, S(stream), f16));
+                }
                 p.nslab = nh; p.slab_mode = 0;
                 if (nh > 1) {   // the chunks' buffers were taken in turn: a fixed stride from one chunk to the next
                     p.q_slab_stride = (int64_t)((const uint16_t*)Q[1] - (const uint16_t*)Q[0]);
@@ -303,7 +312,7 @@ size_t moe_group_bwd_ab_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, 
     const size_t esz = dtype == MOE_F32 ? 4 : 2;
     const size_t generic = 2 * al((size_t)R * (size_t)(rank > 0 ? rank : 1) * esz) + 256;
     const int64_t mx = K > N ? K : N;
-    const size_t fast = pack_bytes(E, K) + pack_bytes(E, N) + 4 * q_bytes(R) + al(moe_xtp_workspace_bytes(R, E, mx)) + 256;
+    const size_t fast = (rank > 16 ? 2 : 1) * (pack_bytes(E, K) + pack_bytes(E, N) + 2 * q_bytes(R) + al(2 * moe_xtp_workspace_bytes(R, E, mx))) + 256;
     return generic > fast ? generic : fast;
 }
 
@@ -318,33 +327,42 @@ int moe_group_bwd_ab(const void* DY, int64_t sdm, int64_t sdn, const void* X, in
     Bump ws(workspace, workspace_bytes);
     if (bwd_ab_fast(K, N, rank, dtype, sdm, sdn, sxm, sxk, DY, X)) {
         const int64_t ldt = pad_rows(R);
-        void* At = ws.take(pack_bytes(E, K));   // [e][r][k] = A[e][k][r]
-        void* Bt = ws.take(pack_bytes(E, N));   // [e][r][n] = B[e][r][n]
-        void* Q = ws.take(q_bytes(R));
-        void* Qt = ws.take(q_bytes(R));
-        void* P = ws.take(q_bytes(R));
-        void* Pt = ws.take(q_bytes(R));
+        const int pairs = rank > 16 ? 2 : 1;
+        void *At[2], *Bt[2], *Qt[2], *Pt[2];   // packed [e][r][k] = A[e][k][r], [e][r][n] = B[e][r][n]; transposed interims (X A)^T, (DY B^T)^T
+        for (int c = 0; c < pairs; ++c) {
+            At[c] = ws.take(pack_bytes(E, K));
+            Bt[c] = ws.take(pack_bytes(E, N));
+            Qt[c] = ws.take(q_bytes(R));
+            Pt[c] = ws.take(q_bytes(R));
+        }
         const int64_t mx = K > N ? K : N;
-        const size_t xb = moe_xtp_workspace_bytes(R, E, mx);
+        const size_t xb = 2 * pairs * moe_xtp_workspace_bytes(R, E, mx);
         void* xw = ws.take(xb);
         if (!xw) return MOE_ERR_WORKSPACE;
         const int f16 = dtype == MOE_F16;
-        // column r of dA depends only on row r of B and row r of dB only on column r of A, so a rank above 16 is
-        // worked through in independent chunks of 16 rank columns
-        for (int r0 = 0; r0 < rank; r0 += 16) {
-            const int rk = (rank - r0 < 16) ? rank - r0 : 16;
-            const uint16_t* Ac = (const uint16_t*)A + r0 * sar;
-            const uint16_t* Bc = (const uint16_t*)B + r0 * sbr;
-            uint16_t* DAc = (uint16_t*)DA + r0 * sdar;
-            uint16_t* DBc = (uint16_t*)DB + r0 * sdbr;
-            TRY(moe_launch_pack_lora(Ac, sae, sak, sar, At, E, K, rk, 1, S(stream)));
-            TRY(moe_launch_pack_lora(Bc, sbe, sbn, sbr, Bt, E, N, rk, 1, S(stream)));
-            TRY(moe_launch_rows_lora(X, sxm, At, Q, Qt, ldt, nullptr, 0, offsets, off64, E, R, K, 1, 1, scaling, nullptr, S(stream), f16));
-            TRY(moe_launch_rows_lora(DY, sdm, Bt, P, Pt, ldt, nullptr, 0, offsets, off64, E, R, N, 1, 1, scaling, nullptr, S(stream), f16));
-            TRY(moe_launch_xtp(X, sxm, nullptr, 0, 1, Pt, ldt, nullptr, DAc, sdae, sdak, sdar, rk, offsets, off64, E, R, K,
-                               1.f, xw, xb, S(stream), f16));
-            TRY(moe_launch_xtp(DY, sdm, nullptr, 0, 1, Qt, ldt, nullptr, DBc, sdbe, sdbn, sdbr, rk, offsets, off64, E, R, N,
-                               1.f, xw, xb, S(stream), f16));
+        // Column r of dA depends only on row r of B and row r of dB only on column r of A, so a rank above 16 is worked
+        // through in independent chunks of 16 rank columns.  Two chunks, with both products of each, share every launch: the
+        // launches of one projection are small (1500 tokens, top-2, 8 experts, K = N = 4096: 152 to 200 workgroups per
+        // product).  Rank 32 there, forward and backward with this and the batched packing above: 419 -> 319 us.
+        for (int r0 = 0; r0 < rank; r0 += 32) {
+            MoePackBatch pb = {};
+            pb.E = E;
+            MoeRowsLoraJob rows[MOE_LORA_MAX_JOBS];
+            MoeXtpJob xtp[MOE_LORA_MAX_JOBS];
+            const int n = rank - r0 > 16 ? 2 : 1;
+            for (int c = 0; c < n; ++c) {   // jobs over X first, then those over DY: neighbours share their rows in L2
+                const int64_t rc = r0 + 16 * c;
+                const int rk = (rank - rc < 16) ? (int)(rank - rc) : 16;
+                pb.job[pb.njobs++] = {(const uint16_t*)A + rc * sar, sae, sak, sar, (uint16_t*)At[c], K, 1, rk};
+                pb.job[pb.njobs++] = {(const uint16_t*)B + rc * sbr, sbe, sbn, sbr, (uint16_t*)Bt[c], N, 1, rk};
+                rows[c] = {X, sxm, K, At[c], nullptr, Qt[c], nullptr};
+                rows[n + c] = {DY, sdm, N, Bt[c], nullptr, Pt[c], nullptr};
+                xtp[c] = {X, sxm, K, Pt[c], (uint16_t*)DA + rc * sdar, {sdae, sdak, sdar}, rk};
+                xtp[n + c] = {DY, sdm, N, Qt[c], (uint16_t*)DB + rc * sdbr, {sdbe, sdbn, sdbr}, rk};
+            }
+            TRY(moe_launch_pack_lora_batch(pb, S(stream)));
+            TRY(moe_launch_rows_lora_jobs(rows, 2 * n, ldt, nullptr, 0, offsets, off64, E, R, 1, 1, scaling, nullptr, S(stream), f16));
+            TRY(moe_launch_xtp_jobs(xtp, 2 * n, nullptr, 0, 1, ldt, nullptr, offsets, off64, E, R, 1.f, xw, xb, S(stream), f16));
         }
         return MOE_OK;
     }

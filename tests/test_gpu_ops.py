@@ -479,3 +479,34 @@ def test_grouped_gemm_single_tile_groups(dev, oracle, rows, layout, K, N):
     ref = oracle.scatter2scatter_lora(X, W, None, None, 0, sei, ssi, 1)
     # one bf16 rounding of fp32 sums: half an ulp, 2^-9 of the value, and the sum's own error far below it
     assert float((y.float().cpu() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("K,N", [(544, 2080), (1056, 96), (32, 544)])
+@pytest.mark.parametrize("r", [16, 17, 32, 33, 80])
+def test_group_bwd_ab_of_several_rank_chunks(dev, oracle, K, N, r):
+    """Up to two chunks of 16 rank columns, with both products of each, share a launch: partial chunks, an odd number of them, and
+    products of very different widths (one or several column blocks, K and N on either side)."""
+    ops = _ops()
+    torch.manual_seed(r)
+    counts = torch.tensor([257, 0, 31, 1])
+    eo, R, E = counts.cumsum(0), int(counts.sum()), len(counts)
+    X, DY = torch.randn(R, K).bfloat16(), torch.randn(R, N).bfloat16()
+    A, B = (torch.randn(E, K, r) * 0.1).bfloat16(), (torch.randn(E, r, N) * 0.1).bfloat16()
+    dA, dB = ops.group_bwd_AB(DY.to(dev), X.to(dev), A.to(dev), B.to(dev), 2.0, eo.to(dev), E)
+    dAo, dBo = oracle.group_bwd_AB(DY, X, A, B, 2.0, eo, E)
+    check_expert_grads(dA, dAo, TOL[torch.bfloat16] * 1.5, "dA"); check_expert_grads(dB, dBo, TOL[torch.bfloat16] * 1.5, "dB")
+
+
+@pytest.mark.parametrize("K,N,r", [(72, 64, 5), (1000, 264, 20), (200, 128, 100), (256, 320, 96)])
+def test_scatter2scatter_lora_packs_any_width_and_rank(dev, oracle, K, N, r):
+    """The pack launch takes up to six chunks of both factors: widths that are no whole fragment, ranks that need two launches."""
+    ops = _ops()
+    torch.manual_seed(r)
+    sei = torch.tensor([0] * 130 + [1] * 3 + [3] * 40)
+    ssi = torch.randperm(len(sei))
+    X, W = torch.randn(len(sei), K).bfloat16(), (torch.randn(4, K, N) * 0.05).bfloat16()
+    A, B = (torch.randn(4, K, r) * 0.1).bfloat16(), (torch.randn(4, r, N) * 0.1).bfloat16()
+    for Ad, Bd in ((A.to(dev), B.to(dev)), (A.permute(0, 2, 1).contiguous().to(dev).permute(0, 2, 1), B.permute(0, 2, 1).contiguous().to(dev).permute(0, 2, 1))):
+        y = ops.scatter2scatter_lora(X.to(dev), W.to(dev), Ad, Bd, 0.5, sei.to(dev), ssi.to(dev), 1, None)
+        ref = oracle.scatter2scatter_lora(X, W, A, B, 0.5, sei, ssi, 1)
+        assert rel(y, ref) < TOL[torch.bfloat16]
