@@ -107,7 +107,8 @@ int moe_launch_generic_xty(const void* X, int64_t sxm, int64_t sxk, const void* 
                            int64_t N, float scale, int dtype, hipStream_t stream);
 
 // low-rank helpers (16-bit storage: bf16, or IEEE half when f16 != 0; rank <= 16)
-// a batch of pack jobs sharing E: src strides {expert, k, r}, dst as moe_launch_pack_lora
+// a batch of pack jobs sharing E: src strides {expert, k, r}; dst [E][K][16], or with transpose the 16x16x32 operand fragments
+// (K rounded up to 32) one after the other
 constexpr int MOE_PACK_MAX_JOBS = 12;
 struct MoePackJob { const uint16_t* src; int64_t se, sk, sr; uint16_t* dst; int64_t K; int transpose; int rank; };   // rank <= 16 columns, zero padded to 16
 struct MoePackBatch { MoePackJob job[MOE_PACK_MAX_JOBS]; int njobs; int E; int* zero_ptr; int zero_n; };   // zero_ptr[0..zero_n) is cleared by the launch
