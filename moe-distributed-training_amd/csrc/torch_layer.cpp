@@ -410,7 +410,6 @@ Tensor linear_checked(const Tensor& x_, const Tensor& W, const Tensor& A, const 
                       const Tensor& eo_, const Tensor& gates_, bool grouped_in, bool grouped_out)
 {
     require_gpu({&x_, &W, &A, &B, &sei, &ssi_, &eo_, &gates_});
-    const c10::DeviceGuard guard(x_.device());
     MOE_ASSERT(ssi_.size(0) == sei.size(0), "sorted_scattered_idxs and sorted_expert_idxs differ in length");
     MOE_ASSERT(ssi_.size(0) == x_.size(0) * k, "the number of assignments is not rows of X times k");
     MOE_ASSERT(x_.dim() == 2 && W.dim() == 3 && x_.size(1) == W.size(1), "X and W have inconsistent inner dims.");
@@ -421,6 +420,7 @@ Tensor linear_checked(const Tensor& x_, const Tensor& W, const Tensor& A, const 
         MOE_ASSERT(A.size(2) == B.size(1), "A and B have inconsistent inner dims.");
         MOE_ASSERT(A.scalar_type() == x_.scalar_type() && B.scalar_type() == x_.scalar_type(), "A, B and X must share a dtype");
     }
+    const c10::DeviceGuard guard(x_.device());
     Tensor x = unit_inner(x_), ssi = ssi_.contiguous(), eo = eo_.defined() ? eo_.contiguous() : offsets_from_sorted(sei, W.size(0));
     Tensor gates = gates_.defined() ? gates_.contiguous() : Tensor();
     const LinearCfg c{scaling, scaling_ab, k, grouped_in, grouped_out};
@@ -572,14 +572,15 @@ bool mlp_fast_path(const Tensor& x, const Tensor& w1, const Tensor& w2, const Te
 Tensor expert_mlp(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& w3, int64_t fan_out, const Tensor& ssi_, const Tensor& offsets_,
                   const std::vector<Tensor>& lora, double lora_alpha, const OptTensor& gates_, bool grouped_out)
 {
-    require_gpu({&x, &w1, &w2, &w3, &ssi_, &offsets_});
-    const c10::DeviceGuard guard(x.device());
+    const Tensor gates_in = val(gates_);
     Tensor lt[6];
     for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
+    require_gpu({&x, &w1, &w2, &w3, &ssi_, &offsets_, &gates_in, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]});
+    const c10::DeviceGuard guard(x.device());
     TORCH_CHECK(fast_path_ok(x, w1, w2, w3, lt, false, w1.size(0), w1.size(2), w1.size(1)),
                 "fused_expert_mlp needs bf16, contiguous (E,f,d) weights, d and f multiples of 64 and rank <= 128; use scattermoe_permute_and_compute for "
                 "other cases");
-    Tensor ssi = ssi_.contiguous(), offsets = offsets_.contiguous(), gates = gates_.has_value() ? gates_->contiguous() : Tensor();
+    Tensor ssi = ssi_.contiguous(), offsets = offsets_.contiguous(), gates = gates_in.defined() ? gates_in.contiguous() : Tensor();
     const MlpCfg c{lt[0].defined() ? lora_alpha / (double)lt[0].size(2) : 0.0, fan_out, grouped_out && !gates.defined()};
     if (needs_node({&x, &w1, &w2, &w3, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5], &gates}))
         return ExpertMlpFn::apply(x, w1, w3, w2, opt(lt[0]), opt(lt[1]), opt(lt[2]), opt(lt[3]), opt(lt[4]), opt(lt[5]), opt(gates), ssi, offsets, c);
@@ -670,7 +671,9 @@ void lora_storage_to_views(Tensor* lt, int64_t E, int64_t d, int64_t f, int64_t 
 variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const Tensor& w2_, const Tensor& w3_, int64_t E, int64_t f, int64_t k,
                     const std::vector<Tensor>& lora, double lora_alpha, bool normalize, bool storage)
 {
-    require_gpu({&x, &wg, &w1_, &w2_, &w3_});
+    Tensor lt[6];
+    for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
+    require_gpu({&x, &wg, &w1_, &w2_, &w3_, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]});
     const c10::DeviceGuard guard(x.device());
     const int64_t d = x.size(1);
     // (the fused launches take sizes from E, f and the input's columns, so every weight is held against them here)
@@ -680,8 +683,6 @@ variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const 
         return w.contiguous();
     };
     const Tensor w1 = whole(w1_), w2 = whole(w2_), w3 = whole(w3_);
-    Tensor lt[6];
-    for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
     const int64_t rank = lt[0].defined() ? lt[0].size(storage ? 1 : 2) : 0;
     const double scaling = rank ? lora_alpha / (double)rank : 0.0;
     if (rank && storage) {

@@ -1,0 +1,73 @@
+"""Calls that the entry points refuse on the host, before anything is enqueued.  The tensors are fakes that only claim to lie on a GPU, so
+every check runs without one; a call that got past its checks would fail differently (no device here)."""
+import warnings
+
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+T, D, F, E, K, R = 24, 64, 128, 4, 2, 16
+BF16, F32, I32 = torch.bfloat16, torch.float32, torch.int32
+_MODE = FakeTensorMode(allow_non_fake_inputs=True)
+
+
+def _fake(*shape, dtype=BF16, device="cuda:0"):
+    with _MODE:
+        return torch.empty(shape, dtype=dtype, device=device)
+
+
+def _mlp_args(**changed):
+    args = dict(x=_fake(T, D), w1=_fake(E, F, D), w2=_fake(E, F, D), w3=_fake(E, F, D), k=K, sorted_scattered_idxs=_fake(T * K, dtype=I32),
+                expert_offsets=_fake(E, dtype=I32))
+    return {**args, **changed}
+
+
+def _linear_args(**changed):
+    args = dict(inputs=_fake(T, D), expert_weights=_fake(E, D, F), k=K, sorted_expert_idxs=_fake(T * K, dtype=I32),
+                sorted_scattered_idxs=_fake(T * K, dtype=I32), padded_block_idxs=None, expert_offsets=_fake(E, dtype=I32))
+    return {**args, **changed}
+
+
+def _refused(match, fn, *args, **kw):
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")   # (a fake's data pointer)
+        with pytest.raises((RuntimeError, AssertionError), match=match):
+            fn(*args, **kw)
+
+
+def _factors(**changed):
+    """a1, b1, a3, b3, a2, b2 as views (E, K, r) / (E, r, N)"""
+    from moe_distributed_training_amd.megablocks_utils.moe_mlp import LoraViews
+    v = dict(a1=_fake(E, D, R), b1=_fake(E, R, F), a3=_fake(E, D, R), b3=_fake(E, R, F), a2=_fake(E, F, R), b2=_fake(E, R, D))
+    return LoraViews(**{**v, **changed})
+
+
+def _layer_args(**changed):
+    args = dict(x=_fake(T, D), wg=_fake(E, D), w1=_fake(E, F, D), w2=_fake(E, F, D), w3=_fake(E, F, D), top_k=K)
+    return {**args, **changed}
+
+
+ELSEWHERE = [("GPU only", "cpu"), ("same device", "cuda:1")]
+
+
+@pytest.mark.parametrize("match,device", ELSEWHERE)
+def test_gates_elsewhere_are_refused(match, device):
+    import moe_distributed_training_amd as moe
+    gates = _fake(T, K, dtype=F32, device=device)
+    _refused(match, moe.fused_expert_mlp, **_mlp_args(gates=gates))
+    _refused(match, moe.parallel_linear, **_linear_args(gates=gates))
+
+
+@pytest.mark.parametrize("match,device", ELSEWHERE)
+@pytest.mark.parametrize("name", ["a1", "b1", "a3", "b3", "a2", "b2"])
+def test_adapter_factors_elsewhere_are_refused(match, device, name):
+    import moe_distributed_training_amd as moe
+    shape = getattr(_factors(), name).shape
+    lora = _factors(**{name: _fake(*shape, device=device)})
+    _refused(match, moe.fused_expert_mlp, **_mlp_args(lora=lora))
+    _refused(match, moe.moe_layer_forward, **_layer_args(lora=lora))
+    block = moe.ScatterMoEBlock(D, F, E, top_k=K, lora_r=R, dtype=BF16, device="meta")
+    for n, p in list(block.named_parameters()):
+        where = device if n == "lora_" + {"a2": "B_w2", "b2": "A_w2"}.get(name, name[0].upper() + "_w" + name[1]) else "cuda:0"
+        setattr(block, n, torch.nn.Parameter(_fake(*p.shape, device=where), requires_grad=False))
+    _refused(match, block, _fake(T, D))
