@@ -64,6 +64,13 @@ inline void require_gpu(std::initializer_list<const Tensor*> ts)
     }
 }
 
+// gates (T, k): one weight per row of the product; the combine takes its sizes from them
+inline void check_gates(const Tensor& gates, int64_t rows)
+{
+    TORCH_CHECK(!gates.defined() || (gates.dim() == 2 && gates.numel() == rows), "gates of ", gates.defined() ? gates.sizes() : at::IntArrayRef(),
+                " must be (tokens, experts per token) with one weight for each of the ", rows, " assignments");
+}
+
 inline Tensor bytes_on(const Tensor& like, size_t n)
 {
     return at::empty({(int64_t)(n < 256 ? 256 : n)}, like.options().dtype(at::kByte));
@@ -332,6 +339,7 @@ struct RouterFn : Function<RouterFn> {
 variable_list router(const Tensor& x_, const Tensor& wg_, int64_t k, bool normalize)
 {
     require_gpu({&x_, &wg_});
+    TORCH_CHECK(x_.dim() == 2 && wg_.dim() == 2, "the router takes (tokens, hidden size) and a weight of (experts, hidden size), got ", x_.sizes(), " and ", wg_.sizes());
     const c10::DeviceGuard guard(x_.device());
     Tensor x = unit_inner(x_), wg = unit_inner(wg_);
     if (needs_node({&x, &wg})) return RouterFn::apply(x, wg, k, normalize);
@@ -420,6 +428,7 @@ Tensor linear_checked(const Tensor& x_, const Tensor& W, const Tensor& A, const 
         MOE_ASSERT(A.size(2) == B.size(1), "A and B have inconsistent inner dims.");
         MOE_ASSERT(A.scalar_type() == x_.scalar_type() && B.scalar_type() == x_.scalar_type(), "A, B and X must share a dtype");
     }
+    check_gates(gates_, ssi_.size(0));
     const c10::DeviceGuard guard(x_.device());
     Tensor x = unit_inner(x_), ssi = ssi_.contiguous(), eo = eo_.defined() ? eo_.contiguous() : offsets_from_sorted(sei, W.size(0));
     Tensor gates = gates_.defined() ? gates_.contiguous() : Tensor();
@@ -576,6 +585,7 @@ Tensor expert_mlp(const Tensor& x, const Tensor& w1, const Tensor& w2, const Ten
     Tensor lt[6];
     for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
     require_gpu({&x, &w1, &w2, &w3, &ssi_, &offsets_, &gates_in, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]});
+    check_gates(gates_in, ssi_.numel());
     const c10::DeviceGuard guard(x.device());
     TORCH_CHECK(fast_path_ok(x, w1, w2, w3, lt, false, w1.size(0), w1.size(2), w1.size(1)),
                 "fused_expert_mlp needs bf16, contiguous (E,f,d) weights, d and f multiples of 64 and rank <= 128; use scattermoe_permute_and_compute for "
@@ -674,6 +684,7 @@ variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const 
     Tensor lt[6];
     for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
     require_gpu({&x, &wg, &w1_, &w2_, &w3_, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]});
+    TORCH_CHECK(x.dim() == 2, "the layer takes (tokens, hidden size), got ", x.sizes());
     const c10::DeviceGuard guard(x.device());
     const int64_t d = x.size(1);
     // (the fused launches take sizes from E, f and the input's columns, so every weight is held against them here)

@@ -71,3 +71,21 @@ def test_adapter_factors_elsewhere_are_refused(match, device, name):
         where = device if n == "lora_" + {"a2": "B_w2", "b2": "A_w2"}.get(name, name[0].upper() + "_w" + name[1]) else "cuda:0"
         setattr(block, n, torch.nn.Parameter(_fake(*p.shape, device=where), requires_grad=False))
     _refused(match, block, _fake(T, D))
+
+
+@pytest.mark.parametrize("shape", [(T, K, 2), (T * K,), (T + 1, K), (T // 2, K), (K, T, 1)])
+def test_gates_of_another_shape_are_refused(shape):
+    import moe_distributed_training_amd as moe
+    gates = _fake(*shape, dtype=F32)
+    _refused("gates of", moe.fused_expert_mlp, **_mlp_args(gates=gates))
+    _refused("gates of", moe.parallel_linear, **_linear_args(gates=gates))
+    _refused("gates of", moe.parallel_linear_lora, **_linear_args(gates=gates), expert_lora_A=_fake(E, D, R), expert_lora_B=_fake(E, R, F), lora_r=R,
+             lora_alp=32.0)
+
+
+@pytest.mark.parametrize("shape", [(T, D, 2), (2, T, D), (D,)])
+def test_inputs_that_are_no_matrix_are_refused(shape):
+    import moe_distributed_training_amd as moe
+    from moe_distributed_training_amd._lib import native
+    _refused("takes", moe.moe_layer_forward, **_layer_args(x=_fake(*shape)))
+    _refused("takes", native.router, _fake(*shape), _fake(E, D), K, True)
