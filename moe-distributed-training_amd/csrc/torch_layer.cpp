@@ -184,13 +184,20 @@ Lora describe_lora(const Tensor* t, bool storage, int64_t d, int64_t f)
     return l;
 }
 
+// (E, f, d), or in the storage of the block module (E*f, d): the launches take the sizes of all three from E, f and d
+void check_expert_weight(const Tensor& w, int64_t E, int64_t f, int64_t d)
+{
+    const bool fits = w.dim() == 3 ? w.size(0) == E && w.size(1) == f && w.size(2) == d : w.dim() == 2 && w.size(0) == E * f && w.size(1) == d;
+    TORCH_CHECK(fits, "expert weights of ", w.sizes(), " do not fit ", E, " experts of ", f, " x ", d);
+}
+
 // what the fused launches take (the same limits the library checks before it enqueues anything)
 bool fast_path_ok(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor* lora, bool storage, int64_t E, int64_t d,
                   int64_t f)
 {
     (void)E;
     if (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf) return false;
-    if (w1.scalar_type() != x.scalar_type()) return false;
+    if (w1.scalar_type() != x.scalar_type() || w2.scalar_type() != x.scalar_type() || w3.scalar_type() != x.scalar_type()) return false;
     const bool has = lora[0].defined();
     for (int i = 0; i < 6 && has; ++i)
         if (lora[i].scalar_type() != x.scalar_type() || (storage && !lora[i].is_contiguous())) return false;
@@ -586,10 +593,12 @@ Tensor expert_mlp(const Tensor& x, const Tensor& w1, const Tensor& w2, const Ten
     for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
     require_gpu({&x, &w1, &w2, &w3, &ssi_, &offsets_, &gates_in, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]});
     check_gates(gates_in, ssi_.numel());
-    const c10::DeviceGuard guard(x.device());
+    TORCH_CHECK(x.dim() == 2 && w1.dim() == 3 && x.size(1) == w1.size(2), "rows of ", x.sizes(), " do not fit expert weights of ", w1.sizes());
+    for (const Tensor* w : {&w2, &w3}) check_expert_weight(*w, w1.size(0), w1.size(1), w1.size(2));
     TORCH_CHECK(fast_path_ok(x, w1, w2, w3, lt, false, w1.size(0), w1.size(2), w1.size(1)),
-                "fused_expert_mlp needs bf16, contiguous (E,f,d) weights, d and f multiples of 64 and rank <= 128; use scattermoe_permute_and_compute for "
-                "other cases");
+                "fused_expert_mlp needs bf16 or fp16 throughout, contiguous (E,f,d) weights, d and f multiples of 64 and rank <= 128; use "
+                "scattermoe_permute_and_compute for other cases");
+    const c10::DeviceGuard guard(x.device());
     Tensor ssi = ssi_.contiguous(), offsets = offsets_.contiguous(), gates = gates_in.defined() ? gates_in.contiguous() : Tensor();
     const MlpCfg c{lt[0].defined() ? lora_alpha / (double)lt[0].size(2) : 0.0, fan_out, grouped_out && !gates.defined()};
     if (needs_node({&x, &w1, &w2, &w3, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5], &gates}))
@@ -685,15 +694,14 @@ variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const 
     for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
     require_gpu({&x, &wg, &w1_, &w2_, &w3_, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]});
     TORCH_CHECK(x.dim() == 2, "the layer takes (tokens, hidden size), got ", x.sizes());
-    const c10::DeviceGuard guard(x.device());
     const int64_t d = x.size(1);
-    // (the fused launches take sizes from E, f and the input's columns, so every weight is held against them here)
     TORCH_CHECK(wg.dim() == 2 && wg.size(0) == E, "router weight of ", wg.sizes(), " does not fit ", E, " experts");
-    auto whole = [&](const Tensor& w) {   // storage order, as the launches address it
-        TORCH_CHECK(w.size(-1) == d && (storage ? w.numel() == E * f * d : w.numel() >= E * f * d), "expert weights of ", w.sizes(), " do not fit ", E, " experts of ", f, " x ", d);
-        return w.contiguous();
-    };
-    const Tensor w1 = whole(w1_), w2 = whole(w2_), w3 = whole(w3_);
+    for (const Tensor* w : {&w1_, &w2_, &w3_}) {
+        check_expert_weight(*w, E, f, d);
+        MOE_ASSERT(w->scalar_type() == x.scalar_type(), "X and W must share a dtype");
+    }
+    const c10::DeviceGuard guard(x.device());
+    const Tensor w1 = w1_.contiguous(), w2 = w2_.contiguous(), w3 = w3_.contiguous();   // storage order, as the launches address it
     const int64_t rank = lt[0].defined() ? lt[0].size(storage ? 1 : 2) : 0;
     const double scaling = rank ? lora_alpha / (double)rank : 0.0;
     if (rank && storage) {

@@ -89,3 +89,26 @@ def test_inputs_that_are_no_matrix_are_refused(shape):
     from moe_distributed_training_amd._lib import native
     _refused("takes", moe.moe_layer_forward, **_layer_args(x=_fake(*shape)))
     _refused("takes", native.router, _fake(*shape), _fake(E, D), K, True)
+
+
+@pytest.mark.parametrize("name", ["w1", "w2", "w3"])
+@pytest.mark.parametrize("shape", [(E, 2 * F, D), (E, F // 2, D), (E + 1, F, D), (E - 1, F, D), (E * F // 2, D), (E, F, D // 2), (E, F * D)])
+def test_expert_weights_that_do_not_fit_are_refused(name, shape):
+    import moe_distributed_training_amd as moe
+    if name != "w1":   # (sizes are those of w1; its own misfits show in the others, or in the input's columns)
+        _refused("do not fit", moe.fused_expert_mlp, **_mlp_args(**{name: _fake(*shape)}))
+    _refused("fit", moe.moe_layer_forward, **_layer_args(**{name: _fake(*shape)}))
+
+
+@pytest.mark.parametrize("name", ["w1", "w2", "w3"])
+def test_expert_weights_of_another_type_are_refused(name):
+    """Two 2-byte types in one call would be read bit for bit as one of them."""
+    import moe_distributed_training_amd as moe
+    _refused("throughout", moe.fused_expert_mlp, **_mlp_args(**{name: _fake(E, F, D, dtype=torch.float16)}))
+    _refused("dtype", moe.moe_layer_forward, **_layer_args(**{name: _fake(E, F, D, dtype=torch.float16)}))
+
+
+def test_rows_of_another_width_are_refused():
+    import moe_distributed_training_amd as moe
+    _refused("rows of", moe.fused_expert_mlp, **_mlp_args(x=_fake(T, 2 * D)))
+    _refused("rows of", moe.fused_expert_mlp, **_mlp_args(x=_fake(T, D, 1)))
