@@ -169,7 +169,7 @@ Lora describe_lora(const Tensor* t, bool storage, int64_t d, int64_t f)
 {
     Lora l;
     if (!t[0].defined()) return l;
-    l.rank = (int)(storage ? t[0].size(1) : t[0].size(2));
+    l.rank = (int)t[0].size(-1);
     const int64_t r = l.rank;
     for (int i = 0; i < 6; ++i) {
         int64_t* s = l.s + 3 * i;
@@ -191,6 +191,22 @@ void check_expert_weight(const Tensor& w, int64_t E, int64_t f, int64_t d)
     TORCH_CHECK(fits, "expert weights of ", w.sizes(), " do not fit ", E, " experts of ", f, " x ", d);
 }
 
+// The six factors, all of the rank of the first: views (E, K, r) / (E, r, N), or the block's storage.  The launches take every extent
+// from E, f, d and that rank, and the gradients are allocated like the factors.
+void check_factors(const Tensor* t, bool storage, int64_t E, int64_t f, int64_t d)
+{
+    if (!t[0].defined()) return;
+    const int64_t rank = t[0].dim() ? t[0].size(-1) : 0;
+    for (int i = 0; i < 6; ++i) {
+        const bool on_ffn = i == 1 || i == 3 || i == 4, a_like = i % 2 == 0;
+        const int64_t rows = on_ffn ? f : d;
+        const bool fits = t[i].defined() && (storage ? t[i].dim() >= 2 && t[i].size(-1) == rank && t[i].numel() == E * rows * rank
+                                                     : t[i].dim() == 3 && t[i].size(0) == E && t[i].size(a_like ? 1 : 2) == rows && t[i].size(a_like ? 2 : 1) == rank);
+        TORCH_CHECK(fits, "adapter factor of ", t[i].defined() ? t[i].sizes() : at::IntArrayRef(), " does not fit ", E, " experts of ", rows,
+                    " rows and rank ", rank);
+    }
+}
+
 // what the fused launches take (the same limits the library checks before it enqueues anything)
 bool fast_path_ok(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& w3, const Tensor* lora, bool storage, int64_t E, int64_t d,
                   int64_t f)
@@ -203,9 +219,16 @@ bool fast_path_ok(const Tensor& x, const Tensor& w1, const Tensor& w2, const Ten
         if (lora[i].scalar_type() != x.scalar_type() || (storage && !lora[i].is_contiguous())) return false;
     if (d % 64 || f % 64 || x.stride(-1) != 1 || x.stride(0) % 8) return false;
     if (!w1.is_contiguous() || !w2.is_contiguous() || !w3.is_contiguous()) return false;
-    if (has && (storage ? lora[0].size(1) : lora[0].size(2)) > 128) return false;   // up to eight 16-wide rank chunks
+    if (has && lora[0].size(-1) > 128) return false;   // up to eight 16-wide rank chunks
     // gathered activation rows and one expert's matrix are addressed with 32-bit byte offsets
     return (x.size(0) * x.stride(0) + d) * 2 < ((int64_t)1 << 32) && (f * d + d) * 2 < ((int64_t)1 << 32);
+}
+
+// lora: empty, or six factors in the order a1, b1, a3, b3, a2, b2
+void take_factors(const std::vector<Tensor>& lora, Tensor* t)
+{
+    TORCH_CHECK(lora.empty() || lora.size() == 6, "an expert MLP has six adapter factors, got ", lora.size());
+    for (size_t i = 0; i < lora.size(); ++i) t[i] = lora[i];
 }
 
 struct MlpShape { int64_t E, d, f, R; int fan_out; double scaling; };
@@ -433,6 +456,7 @@ Tensor linear_checked(const Tensor& x_, const Tensor& W, const Tensor& A, const 
         MOE_ASSERT(W.size(1) == A.size(1), "A has incorrect input size.");
         MOE_ASSERT(W.size(2) == B.size(2), "B has incorrect output size.");
         MOE_ASSERT(A.size(2) == B.size(1), "A and B have inconsistent inner dims.");
+        MOE_ASSERT(A.dim() == 3 && B.dim() == 3 && A.size(0) >= W.size(0) && B.size(0) >= W.size(0), "A and B must hold a factor for every expert.");
         MOE_ASSERT(A.scalar_type() == x_.scalar_type() && B.scalar_type() == x_.scalar_type(), "A, B and X must share a dtype");
     }
     check_gates(gates_, ssi_.size(0));
@@ -580,7 +604,7 @@ struct ExpertMlpFn : Function<ExpertMlpFn> {
 bool mlp_fast_path(const Tensor& x, const Tensor& w1, const Tensor& w2, const Tensor& w3, const std::vector<Tensor>& lora)
 {
     Tensor lt[6];
-    for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
+    take_factors(lora, lt);
     return fast_path_ok(x, w1, w2, w3, lt, false, w1.size(0), w1.size(2), w1.size(1));
 }
 
@@ -590,11 +614,12 @@ Tensor expert_mlp(const Tensor& x, const Tensor& w1, const Tensor& w2, const Ten
 {
     const Tensor gates_in = val(gates_);
     Tensor lt[6];
-    for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
+    take_factors(lora, lt);
     require_gpu({&x, &w1, &w2, &w3, &ssi_, &offsets_, &gates_in, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]});
     check_gates(gates_in, ssi_.numel());
     TORCH_CHECK(x.dim() == 2 && w1.dim() == 3 && x.size(1) == w1.size(2), "rows of ", x.sizes(), " do not fit expert weights of ", w1.sizes());
     for (const Tensor* w : {&w2, &w3}) check_expert_weight(*w, w1.size(0), w1.size(1), w1.size(2));
+    check_factors(lt, false, w1.size(0), w1.size(1), w1.size(2));
     TORCH_CHECK(fast_path_ok(x, w1, w2, w3, lt, false, w1.size(0), w1.size(2), w1.size(1)),
                 "fused_expert_mlp needs bf16 or fp16 throughout, contiguous (E,f,d) weights, d and f multiples of 64 and rank <= 128; use "
                 "scattermoe_permute_and_compute for other cases");
@@ -691,7 +716,7 @@ variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const 
                     const std::vector<Tensor>& lora, double lora_alpha, bool normalize, bool storage)
 {
     Tensor lt[6];
-    for (size_t i = 0; i < 6 && i < lora.size(); ++i) lt[i] = lora[i];
+    take_factors(lora, lt);
     require_gpu({&x, &wg, &w1_, &w2_, &w3_, &lt[0], &lt[1], &lt[2], &lt[3], &lt[4], &lt[5]});
     TORCH_CHECK(x.dim() == 2, "the layer takes (tokens, hidden size), got ", x.sizes());
     const int64_t d = x.size(1);
@@ -700,18 +725,14 @@ variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const 
         check_expert_weight(*w, E, f, d);
         MOE_ASSERT(w->scalar_type() == x.scalar_type(), "X and W must share a dtype");
     }
+    check_factors(lt, storage, E, f, d);
     const c10::DeviceGuard guard(x.device());
     const Tensor w1 = w1_.contiguous(), w2 = w2_.contiguous(), w3 = w3_.contiguous();   // storage order, as the launches address it
-    const int64_t rank = lt[0].defined() ? lt[0].size(storage ? 1 : 2) : 0;
+    const int64_t rank = lt[0].defined() ? lt[0].size(-1) : 0;
     const double scaling = rank ? lora_alpha / (double)rank : 0.0;
     if (rank && storage) {
         bool contiguous = true;
-        for (int i = 0; i < 6; ++i) {
-            const bool on_ffn = i == 1 || i == 3 || i == 4;
-            TORCH_CHECK(lt[i].numel() == E * (on_ffn ? f : d) * rank, "adapter factor of ", lt[i].sizes(), " does not fit ", E, " experts of ",
-                        on_ffn ? f : d, " rows and rank ", rank);
-            contiguous = contiguous && lt[i].is_contiguous();
-        }
+        for (int i = 0; i < 6; ++i) contiguous = contiguous && lt[i].is_contiguous();
         if (!contiguous) {
             lora_storage_to_views(lt, E, d, f, rank);
             storage = false;

@@ -112,3 +112,31 @@ def test_rows_of_another_width_are_refused():
     import moe_distributed_training_amd as moe
     _refused("rows of", moe.fused_expert_mlp, **_mlp_args(x=_fake(T, 2 * D)))
     _refused("rows of", moe.fused_expert_mlp, **_mlp_args(x=_fake(T, D, 1)))
+
+
+@pytest.mark.parametrize("name", ["a1", "b1", "a3", "b3", "a2", "b2"])
+@pytest.mark.parametrize("change", ["experts", "fewer_experts", "rows", "rank", "dims"])
+def test_adapter_factors_that_do_not_fit_are_refused(name, change):
+    import moe_distributed_training_amd as moe
+    shape = list(getattr(_factors(), name).shape)
+    a_like = name[0] == "a"
+    if change == "experts":
+        shape[0] += 1
+    elif change == "fewer_experts":
+        shape[0] -= 1
+    elif change == "rows":
+        shape[1 if a_like else 2] //= 2
+    elif change == "rank":
+        shape[2 if a_like else 1] //= 2
+    else:
+        shape = [shape[0] * shape[1], shape[2]]
+    lora = _factors(**{name: _fake(*shape)})
+    _refused("adapter factor", moe.fused_expert_mlp, **_mlp_args(lora=lora))
+    _refused("adapter factor", moe.moe_layer_forward, **_layer_args(lora=lora))
+    _refused("six adapter", moe.fused_expert_mlp, **_mlp_args(lora=list(_factors())[:5]))
+
+
+@pytest.mark.parametrize("a,b", [((E - 1, D, R), (E, R, F)), ((E, D, R), (E - 1, R, F)), ((E, D, R), (E, R, F, 1))])
+def test_factors_of_a_projection_cover_every_expert(a, b):
+    import moe_distributed_training_amd as moe
+    _refused("every expert", moe.parallel_linear_lora, **_linear_args(), expert_lora_A=_fake(*a), expert_lora_B=_fake(*b), lora_r=R, lora_alp=32.0)
