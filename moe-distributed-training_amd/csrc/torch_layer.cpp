@@ -71,6 +71,12 @@ inline void check_gates(const Tensor& gates, int64_t rows)
                 " must be (tokens, experts per token) with one weight for each of the ", rows, " assignments");
 }
 
+// inclusive row counts: the kernels read one per expert
+inline void check_offsets(const Tensor& offsets, int64_t E)
+{
+    TORCH_CHECK(offsets.numel() >= E, "expert offsets of ", offsets.sizes(), " do not cover ", E, " experts");
+}
+
 inline Tensor bytes_on(const Tensor& like, size_t n)
 {
     return at::empty({(int64_t)(n < 256 ? 256 : n)}, like.options().dtype(at::kByte));
@@ -459,6 +465,7 @@ Tensor linear_checked(const Tensor& x_, const Tensor& W, const Tensor& A, const 
         MOE_ASSERT(A.dim() == 3 && B.dim() == 3 && A.size(0) >= W.size(0) && B.size(0) >= W.size(0), "A and B must hold a factor for every expert.");
         MOE_ASSERT(A.scalar_type() == x_.scalar_type() && B.scalar_type() == x_.scalar_type(), "A, B and X must share a dtype");
     }
+    if (eo_.defined()) check_offsets(eo_, W.size(0));
     check_gates(gates_, ssi_.size(0));
     const c10::DeviceGuard guard(x_.device());
     Tensor x = unit_inner(x_), ssi = ssi_.contiguous(), eo = eo_.defined() ? eo_.contiguous() : offsets_from_sorted(sei, W.size(0));
@@ -620,6 +627,11 @@ Tensor expert_mlp(const Tensor& x, const Tensor& w1, const Tensor& w2, const Ten
     TORCH_CHECK(x.dim() == 2 && w1.dim() == 3 && x.size(1) == w1.size(2), "rows of ", x.sizes(), " do not fit expert weights of ", w1.sizes());
     for (const Tensor* w : {&w2, &w3}) check_expert_weight(*w, w1.size(0), w1.size(1), w1.size(2));
     check_factors(lt, false, w1.size(0), w1.size(1), w1.size(2));
+    check_offsets(offsets_, w1.size(0));
+    // Positions name rows of x (position / fan_out) and, unless the output stays grouped, its rows as well: there they are a permutation.
+    // (A grouped output may hold a row of x any number of times.)
+    TORCH_CHECK(fan_out >= 1 && ((grouped_out && !gates_in.defined()) || ssi_.numel() <= x.size(0) * fan_out), "positions of ",
+                ssi_.sizes(), " do not fit ", x.size(0), " rows with a fan-out of ", fan_out);
     TORCH_CHECK(fast_path_ok(x, w1, w2, w3, lt, false, w1.size(0), w1.size(2), w1.size(1)),
                 "fused_expert_mlp needs bf16 or fp16 throughout, contiguous (E,f,d) weights, d and f multiples of 64 and rank <= 128; use "
                 "scattermoe_permute_and_compute for other cases");

@@ -140,3 +140,18 @@ def test_adapter_factors_that_do_not_fit_are_refused(name, change):
 def test_factors_of_a_projection_cover_every_expert(a, b):
     import moe_distributed_training_amd as moe
     _refused("every expert", moe.parallel_linear_lora, **_linear_args(), expert_lora_A=_fake(*a), expert_lora_B=_fake(*b), lora_r=R, lora_alp=32.0)
+
+
+@pytest.mark.parametrize("shape", [(E - 1,), (0,), ()])
+def test_offsets_that_do_not_cover_the_experts_are_refused(shape):
+    import moe_distributed_training_amd as moe
+    eo = _fake(*shape, dtype=I32)
+    _refused("expert offsets", moe.fused_expert_mlp, **_mlp_args(expert_offsets=eo))
+    _refused("expert offsets", moe.parallel_linear, **_linear_args(expert_offsets=eo))
+
+
+@pytest.mark.parametrize("changed", [dict(sorted_scattered_idxs=(T * K + 1,)), dict(k=1), dict(k=0)])
+def test_positions_beyond_the_rows_are_refused(changed):
+    import moe_distributed_training_amd as moe
+    args = {n: _fake(*v, dtype=I32) if isinstance(v, tuple) else v for n, v in changed.items()}
+    _refused("positions of", moe.fused_expert_mlp, **_mlp_args(**args))
