@@ -418,6 +418,8 @@ struct LinearFn : Function<LinearFn> {
         const double scaling = ctx->saved_data["scaling"].toDouble();
         const int64_t k = ctx->saved_data["k"].toInt(), flags = ctx->saved_data["flags"].toInt(), E = W.size(0), L = ssi.size(0);
         const bool grouped_in = flags & 1, grouped_out = flags & 2;
+        MOE_ASSERT(k >= 1, "no gradients without assignments per row of X");
+        MOE_ASSERT(!grouped_out || g[0].size(0) == L, "gates combine rows in token order: no gradients for them with a grouped output");
         Tensor dout = g[0].contiguous(), d_gates, coeff, dA, dB, dW;
         int64_t gate_fan = 1;
         if (gates.defined()) {
@@ -457,6 +459,7 @@ Tensor linear_checked(const Tensor& x_, const Tensor& W, const Tensor& A, const 
     MOE_ASSERT(ssi_.size(0) == sei.size(0), "sorted_scattered_idxs and sorted_expert_idxs differ in length");
     MOE_ASSERT(ssi_.size(0) == x_.size(0) * k, "the number of assignments is not rows of X times k");
     MOE_ASSERT(x_.dim() == 2 && W.dim() == 3 && x_.size(1) == W.size(1), "X and W have inconsistent inner dims.");
+    MOE_ASSERT(!grouped_in || k == 1, "grouped rows of X are one for each assignment: k is 1 with them");
     MOE_ASSERT(W.scalar_type() == x_.scalar_type(), "X and W must share a dtype");
     if (A.defined()) {
         MOE_ASSERT(W.size(1) == A.size(1), "A has incorrect input size.");

@@ -106,6 +106,7 @@ def _scatter2scatter(X, W, A, B, lora_alp, sorted_expert_idxs, sorted_scattered_
     assert sorted_scattered_idxs.size(0) == X.size(0) * k
     assert X.dim() == 2 and W.dim() == 3 and X.size(1) == W.size(1), "X and W have inconsistent inner dims."
     assert W.dtype == X.dtype, "X and W must share a dtype"
+    assert not x_grouped or k == 1, "grouped rows of X are one for each assignment: k is 1 with them"
     rank = 0
     scaling = 0.0
     if A is not None:

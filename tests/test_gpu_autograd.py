@@ -107,3 +107,37 @@ def test_weights_and_factors_in_other_layouts_take_the_same_route(dev):
         if name != "router":
             setattr(block, name, torch.nn.Parameter(wide[:, ::2], requires_grad=p.requires_grad))
     assert _same(_step(lambda v: block(v)[0], block, x, dout), want)
+
+
+def _routing(dev, t=T, k=K):
+    import moe_distributed_training_amd as moe
+    idx = torch.randint(0, E, (t, k), generator=torch.Generator().manual_seed(3)).to(dev)
+    sei, ssi = moe.flatten_and_sort(idx, E)
+    return (sei, ssi) + moe.padded_block_indices(sei, E)
+
+
+def _factor(dev, *shape):
+    return (torch.randn(shape, device=dev) * 0.05).bfloat16().requires_grad_(True)
+
+
+@pytest.mark.parametrize("lora", [True, False])
+def test_gradients_of_gates_over_a_grouped_output_are_refused(dev, lora):
+    """The gradient of the combined output has one row per token; a grouped output has one per assignment."""
+    import moe_distributed_training_amd as moe
+    sei, ssi, pbi, eo = _routing(dev)
+    x, w, gates = _factor(dev, T, D), (torch.randn(E, D, F, device=dev) * 0.05).bfloat16(), torch.rand(T, K, device=dev)
+    if lora:
+        y = moe.parallel_linear_lora(x, w, _factor(dev, E, D, R), _factor(dev, E, R, F), R, 32.0, K, sei, ssi, pbi, eo, gates, False, True)
+    else:
+        y = moe.parallel_linear(x, w, K, sei, ssi, pbi, eo, gates, False, True)
+    with pytest.raises(AssertionError, match="token order"):
+        y.sum().backward()
+
+
+def test_gradients_without_assignments_are_refused(dev):
+    import moe_distributed_training_amd as moe
+    x, w, none = _factor(dev, T, D), (torch.randn(E, D, F, device=dev) * 0.05).bfloat16(), torch.zeros(0, dtype=torch.int64, device=dev)
+    y = moe.parallel_linear(x, w, 0, none, none, None, torch.zeros(E, dtype=torch.int64, device=dev))
+    assert y.shape == (0, F)
+    with pytest.raises(AssertionError, match="assignments"):
+        y.sum().backward()

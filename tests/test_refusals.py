@@ -155,3 +155,10 @@ def test_positions_beyond_the_rows_are_refused(changed):
     import moe_distributed_training_amd as moe
     args = {n: _fake(*v, dtype=I32) if isinstance(v, tuple) else v for n, v in changed.items()}
     _refused("positions of", moe.fused_expert_mlp, **_mlp_args(**args))
+
+
+def test_grouped_rows_take_no_fan_out():
+    """One row per assignment: with k of them for each row of X, most would be read past its end."""
+    import moe_distributed_training_amd as moe
+    _refused("grouped rows", moe.parallel_linear, **_linear_args(grouped_in=True))
+    _refused("grouped rows", moe.scatter2scatter, _fake(T, D), _fake(E, D, F), _fake(T * K, dtype=I32), _fake(T * K, dtype=I32), K, x_grouped=True)
