@@ -58,6 +58,7 @@ inline void require_gpu(std::initializer_list<const Tensor*> ts)
     const Tensor* first = nullptr;
     for (const Tensor* t : ts) {
         if (!t->defined()) continue;
+        TORCH_CHECK(t->has_storage(), "function transforms (torch.func, vmap) are not supported: their tensors hold no memory that a kernel could read");
         TORCH_CHECK(t->is_cuda(), "moe_distributed_training_amd runs on the GPU only (got a CPU tensor); there is no host fallback");
         if (!first) first = t;
         TORCH_CHECK(t->device() == first->device(), "all tensors must live on the same device");

@@ -162,3 +162,17 @@ def test_grouped_rows_take_no_fan_out():
     import moe_distributed_training_amd as moe
     _refused("grouped rows", moe.parallel_linear, **_linear_args(grouped_in=True))
     _refused("grouped rows", moe.scatter2scatter, _fake(T, D), _fake(E, D, F), _fake(T * K, dtype=I32), _fake(T * K, dtype=I32), K, x_grouped=True)
+
+
+@pytest.mark.parametrize("transform", ["vmap", "grad", "jvp"])
+def test_function_transforms_are_refused(transform):
+    """Their tensors are wrappers without memory (plain CPU tensors inside here: the refusal comes before that matters)."""
+    import moe_distributed_training_amd as moe
+    x, wg, w, wt = torch.randn(3, T, D), torch.randn(E, D), torch.randn(E, F, D), torch.randn(E, D, F)
+    i, o = torch.zeros(T * K, dtype=I32), torch.zeros(E, dtype=I32)
+    calls = [lambda v: moe.moe_layer_forward(v, wg, w, w, w, K)[0], lambda v: moe.forward_router(v, wg, K)[0],
+             lambda v: moe.fused_expert_mlp(v, w, w, w, K, i, o), lambda v: moe.parallel_linear(v, wt, K, i, i, None, o)]
+    for f in calls:
+        run = {"vmap": lambda: torch.vmap(f)(x), "grad": lambda: torch.func.grad(lambda v: f(v).sum())(x[0]),
+               "jvp": lambda: torch.func.jvp(f, (x[0],), (x[0],))}[transform]
+        _refused("function transforms", run)
