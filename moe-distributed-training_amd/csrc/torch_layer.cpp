@@ -137,11 +137,11 @@ Tensor group_bwd_w(const Tensor& dy, const Tensor& x, const void* offsets, int o
 }
 
 Tensor scatter2scatter(const Tensor& X, const Tensor& W, const Tensor& A, const Tensor& B, double scaling, const Tensor& ssi, const Tensor& eo,
-                       int64_t k, bool x_grouped, bool y_grouped)
+                       int64_t k, bool x_grouped, bool y_grouped, const Tensor& into = Tensor())
 {
     const int64_t L = ssi.size(0), E = W.size(0), K = W.size(1), N = W.size(2);
     const int rank = A.defined() ? (int)A.size(2) : 0;
-    Tensor out = at::empty({L, N}, X.options());
+    Tensor out = into.defined() ? into : at::empty({L, N}, X.options());
     if (L == 0) return out;
     Tensor ws = bytes_on(X, moe_scatter2scatter_workspace_bytes(L, (int)E, K, N, rank));
     auto st = [](const Tensor& t, int i) { return t.defined() ? t.stride(i) : (int64_t)0; };
@@ -428,9 +428,10 @@ struct LinearFn : Function<LinearFn> {
             coeff = gates.reshape({-1});
             gate_fan = gates.size(1);
         }
-        // gradients of adapters and weights need dY and X in expert-grouped order (reference :83-99)
+        // Gradients of adapters and weights need dY and X in expert-grouped order (reference :83-99); nobody else reads the latter.
+        // (dY does not go into the saved rows of Y: a second backward pass over the same graph reads those again.)
         Tensor dy_g = grouped_out ? dout : group_rows(dout, ptr(ssi), is64(ssi), L, gate_fan, coeff);
-        Tensor x_g = grouped_in ? x : group_rows(x, ptr(ssi), is64(ssi), L, k);
+        Tensor x_g = grouped_in ? x : A.defined() || ctx->needs_input_grad(1) ? group_rows(x, ptr(ssi), is64(ssi), L, k) : Tensor();
         if (A.defined()) {
             const int64_t K = x_g.size(1), N = dy_g.size(1), r = A.size(2);
             dA = at::empty({E, K, r}, dy_g.options());
@@ -445,9 +446,10 @@ struct LinearFn : Function<LinearFn> {
         } else if (ctx->needs_input_grad(1)) {
             dW = group_bwd_w(dy_g, x_g, ptr(eo), is64(eo), E);
         }
-        // dX = dY W^T + s (dY B^T) A^T: the same grouped GEMM on transposed views (reference :116-128), then the fan-out sum (:134)
+        // dX = dY W^T + s (dY B^T) A^T: the same grouped GEMM on transposed views (reference :116-128), then the fan-out sum (:134).  Its rows
+        // take the place of the gathered X, which has had its readers: as large as dX before that sum, and freed with it
         Tensor dx = scatter2scatter(dy_g, W.transpose(1, 2), A.defined() ? B.transpose(1, 2) : Tensor(), A.defined() ? A.transpose(1, 2) : Tensor(), scaling,
-                                    ssi, eo, 1, true, grouped_in);
+                                    ssi, eo, 1, true, grouped_in, grouped_in ? Tensor() : x_g);
         if (k != 1) dx = combine(dx, Tensor(), nullptr, k, dx.size(0) / k);
         return {dx, dW, dA, dB, d_gates, Tensor(), Tensor(), Tensor()};
     }

@@ -141,3 +141,30 @@ def test_gradients_without_assignments_are_refused(dev):
     assert y.shape == (0, F)
     with pytest.raises(AssertionError, match="assignments"):
         y.sum().backward()
+
+
+@pytest.mark.parametrize("lora,weight_grad", [(True, False), (False, True), (False, False)])
+def test_backward_of_a_projection_holds_one_copy_of_its_rows(dev, lora, weight_grad):
+    """Peak memory: gathered X and the rows of dX share a buffer, and without adapters and weight gradients X is not gathered at all."""
+    import moe_distributed_training_amd as moe
+    from moe_distributed_training_amd._lib import MOE_BF16, lib
+    t, d, n = 4096, 4096, 256
+    L = t * K
+    sei, ssi, pbi, eo = _routing(dev, t)
+    x, w = _factor(dev, t, d), (torch.randn(E, d, n, device=dev) * 0.02).bfloat16().requires_grad_(weight_grad)
+    if lora:
+        y = moe.parallel_linear_lora(x, w, _factor(dev, E, d, R), _factor(dev, E, R, n), R, 32.0, K, sei, ssi, pbi, eo)
+    else:
+        y = moe.parallel_linear(x, w, K, sei, ssi, pbi, eo)
+    dout = torch.ones_like(y)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated(dev)
+    torch.cuda.reset_peak_memory_stats(dev)
+    y.backward(dout)
+    grown = torch.cuda.max_memory_allocated(dev) - before
+    workspaces = [lib.moe_scatter2scatter_workspace_bytes(L, E, n, d, R if lora else 0), t * d * 2]   # of the dX product, or its fan-out sum
+    if lora:
+        workspaces.append(lib.moe_group_bwd_ab_workspace_bytes(L, E, d, n, R, MOE_BF16))
+    grads = (E * R * (d + n) * 2 if lora else 0) + (E * d * n * 2 if weight_grad else 0)
+    rows = L * n * 2 + L * d * 2          # grouped dY; gathered X, then the rows of dX
+    assert grown <= rows + max(workspaces) + grads + (4 << 20), (grown, rows, workspaces, grads)
