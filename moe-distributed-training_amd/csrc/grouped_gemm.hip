@@ -503,7 +503,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     // than on its MFMAs.  Blocks inside the count that lie past the group work on whatever their LDS rows hold; every
     // consumer of the accumulators masks rows past the group.  FULL: all activation loads are issued, those of rows past
     // the tile re-read its last row (branches around loads split the loop body, which costs a tile of many blocks more
-    // than the loads do); without it, for tiles of at most half the blocks, loads of dead rows are dropped.
+    // than the loads do); without it, for groups of at most half a tile's blocks, loads of dead rows are dropped.
     auto mainloop = [&](auto nblk_tag, auto full_tag, auto once) {
         constexpr int NBLK = decltype(nblk_tag)::value;
         constexpr bool FULL = decltype(full_tag)::value;
@@ -606,10 +606,12 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     // (one scalar compare chain per wave; the counts of a tile's two rows of waves differ by at most one)
     // The only tile of its group is also the only reader of its weight tiles: their loads are non-temporal (a streaming read
     // reaches 7.0 TB/s that way, 6.1 without; 24 tokens over 8 experts: 589 -> 539 us forward.  Where several row tiles share the
-    // weight tiles the hint costs 2 %: it works against the sharing in L2).
+    // weight tiles the hint costs 2 %: it works against the sharing in L2).  A tile of eight blocks can be either: 17 blocks are
+    // dealt 9 and 8, and those two walk K alike (the smaller one through the loop of MBH blocks that the larger one's second row of
+    // waves takes as well); fewer blocks than that are always a whole group.
     using T_ = std::true_type;
     using F_ = std::false_type;
-    if (nblocks > MB) {
+    if (nblocks > MB || !item.only_tile) {
         if (item.only_tile) {
             if (mb_cnt > 6) mainloop(std::integral_constant<int, MB>{}, T_{}, T_{});
             else mainloop(std::integral_constant<int, 6>{}, T_{}, T_{});

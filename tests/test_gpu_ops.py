@@ -463,6 +463,26 @@ def test_grouped_gemm_rows_dealt_evenly_to_tiles(dev, oracle, counts, layout):
     assert float((y.float().cpu() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("rows", [257, 272, 300, 513, 544])
+@pytest.mark.parametrize("layout", ["k_contiguous", "n_contiguous"])
+def test_grouped_gemm_tiles_of_a_group_walk_the_same_way(dev, rows, layout):
+    """Equal rows of a group have equal bits whichever of its row tiles they fall into: tiles that share their weights take them in one
+    order (a tile of half the row blocks among them: 257..272 rows are 9 and 8 blocks)."""
+    ops = _ops()
+    torch.manual_seed(24)
+    E, K, N = 3, 512, 4096
+    sei = torch.repeat_interleave(torch.arange(E), torch.tensor([rows, 5, rows])).to(dev)
+    ssi = torch.arange(len(sei), device=dev)
+    X = torch.randn(1, K, device=dev, dtype=torch.float16).expand(len(sei), K).contiguous()
+    W = torch.randn(E, K, N, device=dev, dtype=torch.float16)
+    if layout == "k_contiguous":
+        W = W.permute(0, 2, 1).contiguous().permute(0, 2, 1)
+    y = ops.scatter2scatter(X, W, sei, ssi, 1)
+    for e in (0, 2):
+        group = y[sei == e]
+        assert torch.equal(group, group[:1].expand_as(group)), e
+
+
 @pytest.mark.parametrize("rows", [1, 33, 128, 129, 176, 255, 256])
 @pytest.mark.parametrize("layout,K,N", [("k_contiguous", 1024, 1280), ("n_contiguous", 1024, 1280), ("k_contiguous", 64, 8), ("k_contiguous", 1000, 264)])
 def test_grouped_gemm_single_tile_groups(dev, oracle, rows, layout, K, N):
