@@ -2,7 +2,7 @@
 //
 //   Y[out_row(m)][n] = sum_seg sum_k X_seg[in_row(m)][k] * W_seg[e(m)][k][n]  +  sum_slab Q_slab[m][0:16] . LB_slab[e(m)][n][0:16]
 //
-// m runs over expert-sorted positions; row tiles of BM positions never straddle two experts (derived from the
+// m runs over expert-sorted positions; row tiles of up to BM positions never straddle two experts (derived from the
 // inclusive expert offsets), rows past the end of a group are computed on clamped addresses and never stored,
 // so no token is dropped and no padding is materialised.  The low-rank (LoRA) branch enters as one extra
 // 16-wide K slab per adapter: Q = bf16(scaling * X A) is produced once per row by the skinny kernel in
@@ -100,7 +100,7 @@ struct WorkItem {
     int split_item;            // exchange slot of this part (the slots of a tile are consecutive, in part order)
     int split_tile;            // counter of the split tile
     bool only_tile;            // the group fits in this one row tile
-    int mtile;                 // number of the row tile among all row tiles (experts in order, BM rows each)
+    int mtile;                 // number of the row tile among all row tiles (experts in order)
 };
 
 // Rows of row tile mt of a group's mte tiles: the group's 16-row blocks are dealt evenly to its tiles (mte = the number of
@@ -117,8 +117,6 @@ __device__ __forceinline__ void even_rows(int64_t start, int64_t end, int64_t mt
     *row1 = r1 < end ? r1 : end;
 }
 
-// EVEN: rows as the GEMM deals them to the tiles of a group (even_rows); otherwise those of the tile's 256-row slot
-template <bool EVEN>
 __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int off64, int E, int ntiles_n, int ktiles,
                                                      int max_split, int ncu)
 {
@@ -183,8 +181,8 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
         const int64_t local = t - before * ntiles_n;
         const int nt = (int)(local / mte);
         const int64_t mt = local % mte;
-        int64_t row0 = start + mt * BM, row1 = (row0 + BM < end) ? row0 + BM : end;
-        if (EVEN) even_rows(start, end, mt, mte, &row0, &row1);
+        int64_t row0, row1;
+        even_rows(start, end, mt, mte, &row0, &row1);
         // the shuffles return per-lane values; everything derived from the item is uniform and belongs in scalar registers
         w.expert = __builtin_amdgcn_readfirstlane(expert);
         w.nt = __builtin_amdgcn_readfirstlane(nt);
@@ -207,9 +205,7 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
             const int64_t mt = local % mte;
             w.expert = base + hl;
             w.nt = (int)(local / mte);
-            w.row0 = start + mt * BM;
-            w.row1 = (w.row0 + BM < end) ? w.row0 + BM : end;
-            if (EVEN) even_rows(start, end, mt, mte, &w.row0, &w.row1);
+            even_rows(start, end, mt, mte, &w.row0, &w.row1);
             w.mtile = (int)(mtiles_before + before + mt);
             w.only_tile = mte == 1;
             w.valid = true;
@@ -227,7 +223,7 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
 // (valid, expert, n tile, first row, one-past-last row, part, parts, exchange slot), the split tile's counter in the 9th.
 __global__ void gemm_plan_kernel(const void* offsets, int off64, int E, int ntiles_n, int ktiles, int max_split, int ncu, int* out)
 {
-    const WorkItem w = decode_work_item<false>(offsets, off64, E, ntiles_n, ktiles, max_split, ncu);
+    const WorkItem w = decode_work_item(offsets, off64, E, ntiles_n, ktiles, max_split, ncu);
     if (threadIdx.x == 0) {
         int* o = out + (int64_t)blockIdx.x * 9;
         o[0] = w.valid; o[1] = w.expert; o[2] = w.nt; o[3] = (int)w.row0; o[4] = (int)w.row1;
@@ -254,7 +250,7 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     const int ktiles_seg = KTAIL ? (int)((p.K + BK - 1) / BK) : (int)(p.K / BK);
     constexpr bool TWO_SEG = EPI == MOE_EPI_STORE;   // (the only epilogue that launches with two K segments)
     const int ktiles = TWO_SEG ? ktiles_seg * p.nseg : ktiles_seg;
-    const WorkItem item = decode_work_item<true>(p.offsets, p.off64, p.E, ntiles_n, ktiles, p.max_split, p.num_cus);
+    const WorkItem item = decode_work_item(p.offsets, p.off64, p.E, ntiles_n, ktiles, p.max_split, p.num_cus);
     if (!item.valid) return;
     const int expert = item.expert, nt = item.nt, part = item.part, nparts = item.nparts, split_item = item.split_item;
     const int64_t row0 = item.row0, row1 = item.row1;
@@ -1222,8 +1218,7 @@ __global__ void zero_i32_kernel(int* p, int64_t n)
 }
 
 // Workgroups of a launch: an upper bound on the output tiles plus one round for the split items.  Surplus workgroups
-// leave at once.  (The cost-balanced ranges of a launch of few rounds differ in tile count; a plan whose largest range
-// does not fit this grid falls back to ranges of equal counts.)
+// leave at once.
 int64_t plan_grid(int64_t R, int E, int ntiles_n, int ncu)
 {
     const int64_t grid = (R / BM + E) * ntiles_n + ncu;

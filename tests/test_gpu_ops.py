@@ -374,15 +374,16 @@ def _plan(dev, counts, K, N, pair, nseg=1):
     return out.cpu().numpy(), blocks
 
 
-@pytest.mark.parametrize("case", range(24))
+@pytest.mark.parametrize("case", range(32))
 def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case):
     """The work items the grouped GEMM's workgroups decode for themselves, for seeded group sizes (even, ragged, skewed,
-    empty groups, few and many rounds of tiles, both tile widths): every output tile appears exactly once, either whole
-    or as K parts 0..n-1 with consecutive exchange slots and one counter, and slots and counters are unique and within
-    the exchange area's size."""
+    empty groups, few and many rounds of tiles, both tile widths, more experts than one wave looks up at once): the rows of a
+    group are cut into as many tiles as it needs, without a gap, at 16-row blocks and to within one block evenly; every output
+    tile appears exactly once, either whole or as K parts 0..n-1 with consecutive exchange slots and one counter, and slots and
+    counters are unique and within the exchange area's size."""
     import random
     rng = random.Random(500 + case)
-    E = rng.choice([1, 2, 3, 8, 8, 8, 17, 64])
+    E = rng.choice([1, 2, 3, 8, 8, 8, 17, 64]) if case < 24 else rng.choice([65, 96, 130])
     kind = rng.choice(["even", "ragged", "skewed", "tiny"])
     R = rng.choice([300, 2000, 8192, 8192, 20000])
     if kind == "even":
@@ -397,6 +398,9 @@ def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case):
         counts = [rng.choice([0, 0, 1, 5, 40, 130, 257]) for _ in range(E)]
     if sum(counts) == 0:
         counts[0] = 3
+    if case >= 24:   # groups of several tiles among the first and the last experts of each 64
+        for e, c in ((0, 272), (63, 1060), (64, 257), (E - 1, 600)):
+            counts[e] = c
     K = rng.choice([512, 4096, 14336])
     N = rng.choice([256, 4096, 14336, 1000])
     pair = rng.choice([False, True])
@@ -405,13 +409,6 @@ def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case):
     ncu = torch.cuda.get_device_properties(dev).multi_processor_count // 8 * 8
     bn = 128 if pair else 256
     ntn = (N + bn - 1) // bn
-    expected = {}
-    start = 0
-    for e, c in enumerate(counts):
-        for ntile in range(ntn):
-            for r0 in range(start, start + c, 256):
-                expected[(e, ntile, r0)] = min(r0 + 256, start + c)
-        start += c
     tiles_ub = (sum(counts) // 256 + E) * ((N + 255) // 256)
     slots_cap = min(4 * tiles_ub, ncu)
     seen = {}
@@ -420,11 +417,20 @@ def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case):
         assert valid in (0, 1), f"block {b} wrote nothing"
         if not valid:
             continue
-        key = (e, ntile, r0)
-        assert key in expected and expected[key] == r1, (case, key, r1)
+        key = (e, ntile, r0, r1)
         assert nparts in (1, 2, 4) and 0 <= part < nparts
         seen.setdefault(key, []).append((part, nparts, slot, counter))
-    assert set(seen) == set(expected), (case, len(seen), len(expected))
+    rows = {}
+    for e, ntile, r0, r1 in seen:
+        rows.setdefault((e, ntile), []).append((r0, r1))
+    assert set(rows) == {(e, ntile) for e, c in enumerate(counts) if c for ntile in range(ntn)}, case
+    ends = [sum(counts[:e + 1]) for e in range(E)]
+    for (e, ntile), cut in rows.items():
+        cut.sort()
+        blocks_of = [(r1 - r0 + 15) // 16 for r0, r1 in cut]
+        assert len(cut) == (counts[e] + 255) // 256 and cut[0][0] == ends[e] - counts[e] and cut[-1][1] == ends[e], (case, e, cut)
+        assert all(a[1] == b[0] and (a[1] - a[0]) % 16 == 0 for a, b in zip(cut, cut[1:])), (case, e, cut)
+        assert max(blocks_of) <= 16 and max(blocks_of) - min(blocks_of) <= 1, (case, e, cut)
     used_slots, used_counters = set(), set()
     for key, items in seen.items():
         nparts = items[0][1]
@@ -458,6 +464,24 @@ def test_grouped_gemm_rows_dealt_evenly_to_tiles(dev, oracle, counts, layout):
     X, W = torch.randn(R, K).bfloat16(), (torch.randn(E, K, N) * 0.05).bfloat16()
     Wd = W.permute(0, 2, 1).contiguous().to(dev).permute(0, 2, 1) if layout == "k_contiguous" else W.to(dev)
     y = ops.scatter2scatter(X.to(dev), Wd, sei.to(dev), ssi.to(dev), 1)
+    ref = oracle.scatter2scatter_lora(X, W, None, None, 0, sei, ssi, 1)
+    # one bf16 rounding of fp32 sums: half an ulp, 2^-9 of the value, and the sum's own error far below it
+    assert float((y.float().cpu() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("E", [65, 130])
+def test_grouped_gemm_many_experts_with_several_tiles(dev, oracle, E):
+    """Groups of several row tiles among the first and last experts of each 64 that a wave looks up at once."""
+    ops = _ops()
+    torch.manual_seed(E)
+    counts = [3 * (e % 3) for e in range(E)]
+    for e, c in ((0, 272), (63, 530), (64, 257), (E - 1, 600)):
+        counts[e] = c
+    K, N = 128, 320
+    sei = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ssi = torch.randperm(len(sei), generator=torch.Generator().manual_seed(4))
+    X, W = torch.randn(len(sei), K).bfloat16(), (torch.randn(E, K, N) * 0.05).bfloat16()
+    y = ops.scatter2scatter(X.to(dev), W.to(dev), sei.to(dev), ssi.to(dev), 1)
     ref = oracle.scatter2scatter_lora(X, W, None, None, 0, sei, ssi, 1)
     # one bf16 rounding of fp32 sums: half an ulp, 2^-9 of the value, and the sum's own error far below it
     assert float((y.float().cpu() - ref).abs().max()) <= 2.0 ** -8 * float(ref.abs().max())
