@@ -488,9 +488,19 @@ __global__ void __launch_bounds__(SORT_THREADS) sort_scatter_kernel(const void* 
 // wave per 64 entries.  Workgroup 0 also writes the per-expert counts, the inclusive offsets and the block table.  Same
 // results as the three-launch path.  Latency bound, so every step is parallel: ids are requested in batches, the scan over
 // the experts runs as prefix sums of one wave (a single thread walking 64 experts took longer than all the rest).
-constexpr int64_t SORT_ONE_LAUNCH_MAX_ROWS = 65536;
+// Rows up to which that pays: every workgroup reads all ids (6.3 us up to 8192 rows, then 0.19 us per 1000 rows whatever the number of
+// experts), the three launches take 11.5 us and grow with the experts.  One launch against three, us: 32768 rows, 1 expert 11.1 / 12.0,
+// 8 experts 10.8 / 12.6, 64 experts 11.1 / 24.7; 65536 rows, 1 expert 17.4 / 13.0, 8 experts 17.3 / 14.8, 16 experts 17.4 / 17.2, 64 experts
+// 17.7 / 31.5.  The same within 0.3 us with nine tenths of the rows on one expert.
+constexpr int64_t SORT_ONE_LAUNCH_MAX_ROWS = 65536, SORT_ONE_LAUNCH_MAX_ROWS_FEW = 32768;
+constexpr int SORT_ONE_LAUNCH_FEW_EXPERTS = 15;
 constexpr int SORT_ONE_LAUNCH_MAX_EXPERTS = 256;
 constexpr int SORT1_THREADS = SORT_CHUNK;   // one thread per entry of the chunk
+// Count rows: lane l adds into row l % SORT1_COPIES.  LDS atomics on one address are worked off a lane at a time, so with a row for all
+// lanes of a wave a batch that sends most rows to one expert took 3 us more per 4096 rows (16384 rows: 19 us, so 8); rows of an odd pitch
+// keep the copies of one expert in different banks.
+constexpr int SORT1_COPIES = 8;
+__host__ __device__ constexpr int sort1_pitch(int E) { return E | 1; }
 static_assert(SORT_CHUNK % 64 == 0, "a 64-entry group of the counting pass lies wholly before a chunk or not at all");
 __global__ void __launch_bounds__(SORT1_THREADS) sort_one_launch_kernel(const void* __restrict__ expert_idx, int in64,
                                                                         int64_t R, int E, int block_m,
@@ -501,13 +511,14 @@ __global__ void __launch_bounds__(SORT1_THREADS) sort_one_launch_kernel(const vo
                                                                         int32_t* __restrict__ num_padded, int32_t* __restrict__ inv)
 {
     constexpr int NW = SORT1_THREADS / 64;
-    constexpr int COPIES = 4;        // count rows: a wave adds into row (wave % COPIES), which thins out same-address atomics
-    extern __shared__ int32_t sh[];  // before[COPIES][E], rest[COPIES][E], cursor[NW][E]
+    constexpr int COPIES = SORT1_COPIES;
+    extern __shared__ int32_t sh[];  // before[COPIES][pitch], rest[COPIES][pitch], cursor[NW][E]
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int pitch = sort1_pitch(E);
     int32_t* before = sh;
-    int32_t* rest = sh + COPIES * E;
-    int32_t* cur = sh + 2 * COPIES * E;
-    for (int i = threadIdx.x; i < (2 * COPIES + NW) * E; i += SORT1_THREADS) sh[i] = 0;
+    int32_t* rest = sh + COPIES * pitch;
+    int32_t* cur = sh + 2 * COPIES * pitch;
+    for (int i = threadIdx.x; i < 2 * COPIES * pitch + NW * E; i += SORT1_THREADS) sh[i] = 0;
     __syncthreads();
     const int64_t chunk_base = (int64_t)blockIdx.x * SORT_CHUNK;
     // the own chunk's entry, and its per-wave histogram
@@ -517,8 +528,8 @@ __global__ void __launch_bounds__(SORT1_THREADS) sort_one_launch_kernel(const vo
     // counts over the whole array: wave w walks entries [64 (w + NW j), +64), sixteen groups' ids requested together
     // (integer counts: the order of the additions does not matter)
     constexpr int SB = 16;
-    int32_t* my_before = before + (w % COPIES) * E;
-    int32_t* my_rest = rest + (w % COPIES) * E;
+    int32_t* my_before = before + (lane % COPIES) * pitch;
+    int32_t* my_rest = rest + (lane % COPIES) * pitch;
     for (int64_t p0 = (int64_t)w * 64; p0 < R; p0 += (int64_t)NW * 64 * SB) {
         int64_t raw[SB];
         // (one branch on the index width around all the loads, so that they are in flight together; entries past the
@@ -549,7 +560,7 @@ __global__ void __launch_bounds__(SORT1_THREADS) sort_one_launch_kernel(const vo
             int32_t b = 0, t = 0;
             if (e < E) {
 #pragma unroll
-                for (int c = 0; c < COPIES; ++c) { b += before[c * E + e]; t += rest[c * E + e]; }
+                for (int c = 0; c < COPIES; ++c) { b += before[c * pitch + e]; t += rest[c * pitch + e]; }
                 before[e] = b;
                 rest[e] = b + t;
                 sum += b + t;
@@ -705,8 +716,8 @@ int moe_launch_sort(const void* expert_idx, int in64, int64_t R, int E, int bloc
     if (E < 1 || E > 4096 || R < 0 || block_m < 1) return MOE_ERR_BAD_ARG;
     if (workspace_bytes < moe_sort_ws_bytes(R, E)) return MOE_ERR_WORKSPACE;
     const int nblk = (int)((R + SORT_CHUNK - 1) / SORT_CHUNK);
-    if (nblk > 0 && R <= SORT_ONE_LAUNCH_MAX_ROWS && E <= SORT_ONE_LAUNCH_MAX_EXPERTS) {
-        hipLaunchKernelGGL(sort_one_launch_kernel, dim3(nblk), dim3(SORT1_THREADS), (8 + SORT1_THREADS / 64) * E * sizeof(int32_t), stream,
+    if (nblk > 0 && E <= SORT_ONE_LAUNCH_MAX_EXPERTS && R <= (E <= SORT_ONE_LAUNCH_FEW_EXPERTS ? SORT_ONE_LAUNCH_MAX_ROWS_FEW : SORT_ONE_LAUNCH_MAX_ROWS)) {
+        hipLaunchKernelGGL(sort_one_launch_kernel, dim3(nblk), dim3(SORT1_THREADS), (2 * SORT1_COPIES * sort1_pitch(E) + SORT1_THREADS / 64 * E) * sizeof(int32_t), stream,
                            expert_idx, in64, R, E, block_m, sorted_expert, sorted_pos, out64, counts, offsets, padded_blocks,
                            padded_cap, num_padded, inv);
         return moe_launch_status();
