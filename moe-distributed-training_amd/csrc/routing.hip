@@ -422,23 +422,37 @@ __global__ void __launch_bounds__(SORT_THREADS) sort_scan_kernel(int32_t* __rest
 }
 
 // Stores one group of 64 entries (flat positions p of consecutive lanes, expert e, -1: none) at its expert's cursor:
-// entries of one expert keep their order (stability).  A lane's rank among the earlier lanes of its expert comes from 64
-// scalar broadcasts and compares, whatever the number of experts (one ballot round per distinct expert of the group, with
-// a round trip to the cursor in each, took 2-4 times as long from 16 experts up).
-__device__ __forceinline__ void scatter_group(int e, int64_t p, int lane, int32_t* cursor, void* __restrict__ sorted_expert,
+// entries of one expert keep their order (stability).  A lane's rank among the earlier lanes of its expert takes no round trip to
+// memory: up to 16 experts one ballot per expert, beyond that 64 scalar broadcasts and compares, whatever the number of experts.
+// Sort of 262144 rows, us, ballots / broadcasts: 2 experts 21.7 / 23.8, 8 experts 26.4 / 28.5, 16 experts 33.2 / 34.4, 32 experts
+// 135.2 / 134.7, 48 experts 152.1 / 150.4.
+typedef __attribute__((address_space(3))) int32_t lds_int32_t;
+constexpr int SCATTER_BALLOT_EXPERTS = 16;
+__device__ __forceinline__ void scatter_group(int e, int64_t p, int lane, int E, int32_t* cursor_, void* __restrict__ sorted_expert,
                                               void* __restrict__ sorted_pos, int out64, int32_t* __restrict__ inv)
 {
+    lds_int32_t* cursor = (lds_int32_t*)cursor_;
     int rank = 0;
+    if (E <= SCATTER_BALLOT_EXPERTS) {
+        uint64_t mine = 0;   // lanes of this lane's expert
+#pragma unroll 1
+        for (int x = 0; x < E; ++x) {
+            const uint64_t m = __ballot(e == x);
+            mine = e == x ? m : mine;
+        }
+        rank = __popcll(mine & ((1ull << lane) - 1ull));
+    } else {
 #pragma unroll
-    for (int j = 0; j < 63; ++j) rank += (__builtin_amdgcn_readlane(e, j) == e && j < lane) ? 1 : 0;
+        for (int j = 0; j < 63; ++j) rank += (__builtin_amdgcn_readlane(e, j) == e && j < lane) ? 1 : 0;
+    }
     if (e >= 0) {
-        const int32_t dst = *(volatile int32_t*)(cursor + e) + rank;
+        const int32_t dst = *(volatile lds_int32_t*)(cursor + e) + rank;
         store_idx(sorted_expert, dst, e, out64);
         store_idx(sorted_pos, dst, p, out64);
         if (inv) inv[p] = dst;
     }
     __builtin_amdgcn_wave_barrier();
-    if (e >= 0) atomicAdd(&cursor[e], 1);   // (after every lane of the wave has read its cursor)
+    if (e >= 0) __hip_atomic_fetch_add(cursor + e, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // (after every lane of the wave has read its cursor)
     __builtin_amdgcn_wave_barrier();
 }
 
@@ -478,7 +492,7 @@ __global__ void __launch_bounds__(SORT_THREADS) sort_scatter_kernel(const void* 
         const int64_t p = wbase + i0 + lane;
         int e = -1;
         if (p < R) { const int64_t ee = load_idx(expert_idx, p, in64); e = (ee >= 0 && ee < E) ? (int)ee : -1; }
-        scatter_group(e, p, lane, sh + w * E, sorted_expert, sorted_pos, out64, inv);
+        scatter_group(e, p, lane, E, sh + w * E, sorted_expert, sorted_pos, out64, inv);
     }
 }
 
@@ -489,9 +503,9 @@ __global__ void __launch_bounds__(SORT_THREADS) sort_scatter_kernel(const void* 
 // results as the three-launch path.  Latency bound, so every step is parallel: ids are requested in batches, the scan over
 // the experts runs as prefix sums of one wave (a single thread walking 64 experts took longer than all the rest).
 // Rows up to which that pays: every workgroup reads all ids (6.3 us up to 8192 rows, then 0.19 us per 1000 rows whatever the number of
-// experts), the three launches take 11.5 us and grow with the experts.  One launch against three, us: 32768 rows, 1 expert 11.1 / 12.0,
-// 8 experts 10.8 / 12.6, 64 experts 11.1 / 24.7; 65536 rows, 1 expert 17.4 / 13.0, 8 experts 17.3 / 14.8, 16 experts 17.4 / 17.2, 64 experts
-// 17.7 / 31.5.  The same within 0.3 us with nine tenths of the rows on one expert.
+// experts), the three launches take 11.4 us and grow with the experts.  One launch against three, us: 32768 rows, 1 expert 10.1 / 12.0,
+// 8 experts 10.3 / 11.4, 64 experts 11.3 / 28.1; 65536 rows, 1 expert 17.4 / 12.3, 8 experts 17.3 / 12.9, 16 experts 17.3 / 16.8, 64 experts
+// 18.1 / 34.5.  The same within 0.3 us with nine tenths of the rows on one expert.
 constexpr int64_t SORT_ONE_LAUNCH_MAX_ROWS = 65536, SORT_ONE_LAUNCH_MAX_ROWS_FEW = 32768;
 constexpr int SORT_ONE_LAUNCH_FEW_EXPERTS = 15;
 constexpr int SORT_ONE_LAUNCH_MAX_EXPERTS = 256;
@@ -601,7 +615,7 @@ __global__ void __launch_bounds__(SORT1_THREADS) sort_one_launch_kernel(const vo
         for (int ww = 0; ww < NW; ++ww) { const int32_t c = cur[ww * E + e]; cur[ww * E + e] = run; run += c; }
     }
     __syncthreads();
-    scatter_group(eown, pown, lane, cur + w * E, sorted_expert, sorted_pos, out64, inv);
+    scatter_group(eown, pown, lane, E, cur + w * E, sorted_expert, sorted_pos, out64, inv);
 }
 
 // offsets[e] = number of entries of the non-decreasing array sorted_expert that are <= e  (inclusive running count)
