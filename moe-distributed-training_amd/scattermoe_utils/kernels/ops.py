@@ -237,20 +237,3 @@ def combine_dgates(y, dout, k, gates_dtype, inv=None):
     check(lib.moe_combine_dgates(ptr(y), y.stride(0), ptr(dout), dout.stride(0), ptr(dg), dtype_code(dg), ptr(inv), k, T,
                                  y.size(1), dtype_code(y), stream_ptr(dev)), "moe_combine_dgates")
     return dg
-
-
-def swiglu(gate, up):
-    dev = require_gpu(gate, up)
-    gate, up = gate.contiguous(), up.contiguous()
-    h = torch.empty_like(gate)
-    check(lib.moe_swiglu(ptr(gate), ptr(up), ptr(h), gate.numel(), dtype_code(gate), stream_ptr(dev)), "moe_swiglu")
-    return h
-
-
-def swiglu_bwd(gate, up, dh):
-    dev = require_gpu(gate, up, dh)
-    gate, up, dh = gate.contiguous(), up.contiguous(), dh.contiguous()
-    dg, du = torch.empty_like(gate), torch.empty_like(up)
-    check(lib.moe_swiglu_bwd(ptr(gate), ptr(up), ptr(dh), ptr(dg), ptr(du), gate.numel(), dtype_code(gate), stream_ptr(dev)),
-          "moe_swiglu_bwd")
-    return dg, du
