@@ -168,3 +168,108 @@ def test_backward_of_a_projection_holds_one_copy_of_its_rows(dev, lora, weight_g
     grads = (E * R * (d + n) * 2 if lora else 0) + (E * d * n * 2 if weight_grad else 0)
     rows = L * n * 2 + L * d * 2          # grouped dY; gathered X, then the rows of dX
     assert grown <= rows + max(workspaces) + grads + (4 << 20), (grown, rows, workspaces, grads)
+
+
+class _Call(torch.nn.Module):
+    """One call of an entry point below the block, its factors, gates and router weight as parameters."""
+
+    def __init__(self, dev, which):
+        import moe_distributed_training_amd as moe
+        super().__init__()
+        torch.manual_seed(5)
+        self.which, self.moe = which, moe
+        self.sei, self.ssi, self.pbi, self.eo = _routing(dev)
+        shapes = {"linear": [(E, D, R), (E, R, F), (T, K)], "router": [(E, D)],
+                  "mlp": [(E, D, R), (E, R, F), (E, D, R), (E, R, F), (E, F, R), (E, R, D), (T, K)]}[which]
+        self.p = torch.nn.ParameterList([torch.nn.Parameter((torch.randn(s, device=dev) * 0.05).bfloat16()) for s in shapes])
+        self.w = [(torch.randn(E, F, D, device=dev) * 0.05).bfloat16() for _ in range(3)]
+
+    def forward(self, x):
+        p = list(self.p)
+        if self.which == "linear":
+            return self.moe.parallel_linear_lora(x, self.w[0].permute(0, 2, 1), p[0], p[1], R, 32.0, K, self.sei, self.ssi, self.pbi, self.eo, p[2])
+        if self.which == "router":
+            return self.moe.forward_router(x, p[0], K)[1]
+        from moe_distributed_training_amd.megablocks_utils.moe_mlp import LoraViews
+        return self.moe.fused_expert_mlp(x, *self.w, K, self.ssi, self.eo, LoraViews(*p[:6]), 32.0, p[6])
+
+
+CALLS = ["linear", "mlp", "router"]
+
+
+def _call_case(dev, which):
+    call = _Call(dev, which)
+    x, x2 = (torch.randn(T, D, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    with torch.no_grad():
+        dout = torch.randn_like(call(x))
+    return call, x, x2, dout
+
+
+@pytest.mark.parametrize("which", CALLS)
+def test_checkpointing_and_hooks_of_single_calls_change_no_bit(dev, which):
+    from torch.utils.checkpoint import checkpoint
+    call, x, _, dout = _call_case(dev, which)
+    want = _step(call, call, x, dout)
+    for reentrant in (False, True):
+        assert _same(_step(lambda v: checkpoint(call, v, use_reentrant=reentrant), call, x, dout), want)
+    with torch.autograd.graph.save_on_cpu():
+        assert _same(_step(call, call, x, dout), want)
+    again = x.detach().requires_grad_(True)
+    out = call(again)
+    first = torch.autograd.grad(out, [again, *call.parameters()], dout, retain_graph=True)
+    assert _same(torch.autograd.grad(out, [again, *call.parameters()], dout), first) and _same(first, want[1:])   # a second pass over one graph
+
+
+@pytest.mark.parametrize("which", CALLS)
+def test_traced_single_calls_compute_on_their_inputs(dev, which):
+    call, x, x2, dout = _call_case(dev, which)
+    traced = torch.jit.trace(call, (x,), check_trace=False)
+    with torch.no_grad():
+        assert torch.equal(traced(x2), call(x2))
+    assert _same(_step(traced, call, x2, dout), _step(call, call, x2, dout))
+
+
+@pytest.mark.parametrize("which", CALLS)
+@pytest.mark.parametrize("grad", [True, False])
+def test_forward_mode_of_single_calls_is_refused(dev, which, grad):
+    import torch.autograd.forward_ad as fwad
+    call, x, _, _ = _call_case(dev, which)
+    call.requires_grad_(False)
+    with torch.set_grad_enabled(grad), fwad.dual_level(), pytest.raises(RuntimeError, match="(?i)jvp|forward"):
+        call(fwad.make_dual(x, torch.randn_like(x)))
+
+
+@pytest.mark.parametrize("gates_dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gates_of_any_type(dev, oracle, dtype, gates_dtype):
+    """Gates keep a type of their own, whatever that of the rows, and so does their gradient."""
+    import moe_distributed_training_amd as moe
+    from moe_distributed_training_amd.megablocks_utils.moe_mlp import LoraViews
+    from _metrics import rel
+    torch.manual_seed(8)
+    rn = lambda *s, std=0.05: (torch.randn(*s) * std).to(dtype)
+    f32 = lambda t: t.detach().float().clone().requires_grad_(True)
+    on = lambda t: t.detach().to(dev).requires_grad_(True)
+    x, w, gates = rn(T, D, std=1.0), [rn(E, F, D) for _ in range(3)], torch.rand(T, K).to(gates_dtype)
+    idx = torch.stack([torch.randperm(E)[:K] for _ in range(T)])
+    sei, ssi = oracle.flatten_and_sort(idx)
+    eo = torch.bincount(sei, minlength=E).cumsum(0)
+    fac = [rn(E, D, R), rn(E, R, F), rn(E, D, R), rn(E, R, F), rn(E, F, R), rn(E, R, D)]
+
+    def compare(out, xg, gg, ref, xo, go):
+        dout = torch.randn_like(ref).to(dtype)
+        ref.backward(dout.float())
+        out.backward(dout.to(dev))
+        assert gg.grad.dtype == gates_dtype
+        for got, want in ((out, ref), (xg.grad, xo.grad), (gg.grad, go.grad)):
+            assert rel(got, want) < 1e-2
+
+    xo, go, xg, gg = f32(x), f32(gates), on(x), on(gates)
+    ref = oracle.parallel_linear_lora(xo, w[0].float().permute(0, 2, 1), fac[0].float(), fac[1].float(), R, 32.0, K, sei, ssi, None, eo, go, False, False)
+    compare(moe.parallel_linear_lora(xg, w[0].to(dev).permute(0, 2, 1), fac[0].to(dev), fac[1].to(dev), R, 32.0, K, sei.to(dev), ssi.to(dev), None,
+                                     eo.to(dev), gg), xg, gg, ref, xo, go)
+    xo, go, xg, gg = f32(x), f32(gates), on(x), on(gates)
+    lo = {"w1": (fac[0].float(), fac[1].float()), "w3": (fac[2].float(), fac[3].float()), "w2": (fac[4].float(), fac[5].float())}
+    ref, _ = oracle.moe_block(xo, None, w[0].float(), w[1].float(), w[2].float(), K, lo, 32.0, routing=(go, idx))
+    compare(moe.fused_expert_mlp(xg, w[0].to(dev), w[1].to(dev), w[2].to(dev), K, ssi.to(dev), eo.to(dev), LoraViews(*(t.to(dev) for t in fac)), 32.0,
+                                 gg), xg, gg, ref, xo, go)

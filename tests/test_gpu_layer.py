@@ -124,7 +124,7 @@ def test_layer_fwd_bwd_fp16(dev, oracle, T, d, f, E, r):
 
 @pytest.mark.parametrize("E,k,r", [(96, 4, 16), (16, 8, 16), (80, 3, 0)])
 def test_layer_many_experts_and_wider_top_k(dev, oracle, E, k, r):
-    """More than 8 experts (router on the two-launch path), more than 64 (serial group lookup in every grouped kernel),
+    """More than 8 experts (router on the two-launch path), more than 64 (group lookup in blocks of 64 in every grouped kernel),
     top-k above 2 (fan-out k in the gathers and the combine); most groups hold a handful of rows, some none."""
     import moe_distributed_training_amd as moe
     T, d, f, alpha = 300, 128, 256, 32.0

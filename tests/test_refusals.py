@@ -1,10 +1,12 @@
 """Calls that the entry points refuse on the host, before anything is enqueued.  The tensors are fakes that only claim to lie on a GPU, so
-every check runs without one; a call that got past its checks would fail differently (no device here)."""
+every check runs without one; a call that got past its checks would fail differently where there is none, and not run where there is one."""
 import warnings
 
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
+
+pytestmark = pytest.mark.skipif(torch.cuda.is_available(), reason="a fake's pointer must not reach a kernel")
 
 T, D, F, E, K, R = 24, 64, 128, 4, 2, 16
 BF16, F32, I32 = torch.bfloat16, torch.float32, torch.int32
