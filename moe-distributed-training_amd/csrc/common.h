@@ -103,47 +103,51 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t v)
     return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// Row tiles of ragged expert groups: offsets[e] is the inclusive running row count, tiles of bm rows never straddle
-// two experts.  For up to 64 experts one wave looks at all groups at once -- lane e loads offsets[e], a wave-wide
-// prefix sum gives every group's first tile -- so that finding a tile costs one memory round trip instead of one per
-// expert.  Must be called with all 64 lanes of the wave active (one-dimensional workgroups).
-struct ExpertScan {
-    int64_t start, end;                   // rows of group `lane` (lanes >= E: empty)
-    int64_t tiles_before, tiles_through;  // exclusive / inclusive running tile count
-};
-__device__ __forceinline__ ExpertScan scan_expert_tiles(const void* offsets, int off64, int E, int bm)
+// The value of another lane: of lane `src` (the same in every lane) in scalar registers, and of the lane one below (lane 0: 0).
+__device__ __forceinline__ int64_t readlane_i64(int64_t v, int src)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t end = load_idx(offsets, lane < E ? lane : E - 1, off64);
-    int64_t start = __shfl_up(end, 1);
-    if (lane == 0) start = 0;
-    const int64_t nt = lane < E ? (end - start + bm - 1) / bm : 0;
-    int64_t incl = nt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int64_t t = __shfl_up(incl, d);
-        if (lane >= d) incl += t;
-    }
-    ExpertScan s;
-    s.start = start; s.end = end; s.tiles_before = incl - nt; s.tiles_through = incl;
-    return s;
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, src), hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)v >> 32), src);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+constexpr int DPP_ROW_SHR = 0x110, DPP_WAVE_SHR1 = 0x138, DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143;   // data-parallel-primitive controls of gfx9
+__device__ __forceinline__ int64_t lane_below_i64(int64_t v)
+{
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, DPP_WAVE_SHR1, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)((uint64_t)v >> 32), DPP_WAVE_SHR1, 0xf, 0xf, true);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+// inclusive running sum over the 64 lanes: within rows of 16 lanes, then from row to row
+__device__ __forceinline__ int wave_inclusive_sum(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, DPP_ROW_SHR + 1, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, DPP_ROW_SHR + 2, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, DPP_ROW_SHR + 4, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, DPP_ROW_SHR + 8, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, DPP_ROW_BCAST15, 0xa, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, DPP_ROW_BCAST31, 0xc, 0xf, true);
+    return v;
 }
 
-// The same for the 64 experts from `base` on (any E): a caller with more than 64 experts walks the blocks.
+// Row tiles of ragged expert groups: offsets[e] is the inclusive running row count, tiles of bm rows never straddle
+// two experts.  For 64 experts (from `base` on; a caller with more walks the blocks) one wave looks at all groups at once --
+// lane e loads offsets[base + e], a wave-wide prefix sum gives every group's first tile -- so that finding a tile costs one
+// memory round trip instead of one per expert.  Tile counts are 32-bit (a launch has fewer than 2^31 workgroups) and everything
+// moves between lanes by DPP or readlane: this lookup stands in front of the first load of every tile.
+// Must be called with all 64 lanes of the wave active (one-dimensional workgroups).
+struct ExpertScan {
+    int64_t start, end;               // rows of group `base + lane` (lanes past E: empty)
+    int tiles_before, tiles_through;  // exclusive / inclusive running tile count
+};
 __device__ __forceinline__ ExpertScan scan_expert_tiles_from(const void* offsets, int off64, int E, int bm, int base)
 {
     const int lane = threadIdx.x & 63;
     const int e = base + lane;
     const int64_t end = load_idx(offsets, e < E ? e : E - 1, off64);
-    int64_t start = __shfl_up(end, 1);
-    if (lane == 0) start = base > 0 ? load_idx(offsets, base - 1, off64) : 0;
-    const int64_t nt = e < E ? (end - start + bm - 1) / bm : 0;
-    int64_t incl = nt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int64_t t = __shfl_up(incl, d);
-        if (lane >= d) incl += t;
-    }
+    const int64_t before = base > 0 ? load_idx(offsets, base - 1, off64) : 0;
+    int64_t start = lane_below_i64(end);
+    if (lane == 0) start = before;
+    const int nt = e < E ? (int)((uint32_t)(end - start + bm - 1) / (uint32_t)bm) : 0;
+    const int incl = wave_inclusive_sum(nt);
     ExpertScan s;
     s.start = start; s.end = end; s.tiles_before = incl - nt; s.tiles_through = incl;
     return s;
@@ -153,19 +157,19 @@ __device__ __forceinline__ ExpertScan scan_expert_tiles_from(const void* offsets
 struct RowTile { int expert; int64_t row0; int64_t row1; };
 __device__ __forceinline__ bool find_row_tile(const void* offsets, int off64, int E, int bm, int64_t tile, RowTile* out)
 {
+    int tl = (int)tile;
     for (int base = 0; base < E; base += 64) {   // one memory round trip per 64 experts
-        const int lane = threadIdx.x & 63;
-        const ExpertScan s = E <= 64 ? scan_expert_tiles(offsets, off64, E, bm) : scan_expert_tiles_from(offsets, off64, E, bm, base);
-        const unsigned long long hit = __ballot(base + lane < E && tile >= s.tiles_before && tile < s.tiles_through);
+        const ExpertScan s = scan_expert_tiles_from(offsets, off64, E, bm, base);
+        const unsigned long long hit = __ballot(tl >= s.tiles_before && tl < s.tiles_through);   // (lanes past E hold no tiles)
         if (hit != 0) {
             const int l = __ffsll(hit) - 1;
-            const int64_t end = __shfl(s.end, l);
+            const int64_t end = readlane_i64(s.end, l);
             out->expert = base + l;
-            out->row0 = __shfl(s.start, l) + (tile - __shfl(s.tiles_before, l)) * bm;
+            out->row0 = readlane_i64(s.start, l) + (int64_t)(tl - __builtin_amdgcn_readlane(s.tiles_before, l)) * bm;
             out->row1 = (out->row0 + bm < end) ? out->row0 + bm : end;
             return true;
         }
-        tile -= uniform_i64(__shfl(s.tiles_through, 63));
+        tl -= __builtin_amdgcn_readlane(s.tiles_through, 63);
     }
     return false;
 }

@@ -108,34 +108,28 @@ struct WorkItem {
 // of 1-3 blocks behind full tiles about as much as a full one (its waves wait for the same weight tiles), so 1060 rows run
 // as five tiles of 13-14 blocks instead of four of 16 and one of 3.  8192 rows over 8 experts: gate/up launch 1630 -> 1556 us,
 // the layer's forward and backward 5029 -> 4950 us.
-__device__ __forceinline__ void even_rows(int64_t start, int64_t end, int64_t mt, int64_t mte, int64_t* row0, int64_t* row1)
+__device__ __forceinline__ void even_rows(int64_t start, int64_t end, uint32_t mt, uint32_t mte, int64_t* row0, int64_t* row1)
 {
-    const int64_t blocks = (end - start + 15) / 16, per = blocks / mte, more = blocks % mte;
-    const int64_t b0 = mt * per + (mt < more ? mt : more);
-    *row0 = start + b0 * 16;
-    const int64_t r1 = *row0 + (per + (mt < more ? 1 : 0)) * 16;
+    const uint32_t blocks = (uint32_t)((end - start + 15) >> 4), per = blocks / mte, more = blocks - per * mte;
+    const uint32_t b0 = mt * per + (mt < more ? mt : more);
+    *row0 = start + (int64_t)b0 * 16;
+    const int64_t r1 = *row0 + (int64_t)(per + (mt < more ? 1 : 0)) * 16;
     *row1 = r1 < end ? r1 : end;
 }
 
 __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int off64, int E, int ntiles_n, int ktiles,
                                                      int max_split, int ncu)
 {
+    // 32-bit throughout (a launch has fewer than 2^31 tiles): six 64-bit divisions and the shuffles of 64-bit scans made this lookup
+    // 1.6 us of every tile, 4.0 where the kernel is cold; now 0.85 and 1.3 (the four launches of a 512-token step with d=256: 92 -> 85 us)
     WorkItem w = {};
-    const int lane = threadIdx.x & 63;
-    ExpertScan sc = {};
-    int64_t T = 0;
-    if (E <= 64) {
-        // every wave sees all expert groups at once: one memory round trip for the whole lookup
-        sc = scan_expert_tiles(offsets, off64, E, BM);
-        T = uniform_i64(__shfl(sc.tiles_through, 63)) * ntiles_n;
-    } else {
-        for (int base = 0; base < E; base += 64) T += uniform_i64(__shfl(scan_expert_tiles_from(offsets, off64, E, BM, base).tiles_through, 63));
-        T *= ntiles_n;
-    }
-    const int xcd = blockIdx.x % NXCD;
-    const int64_t q = blockIdx.x / NXCD;
-    const int CH = ncu / NXCD;             // compute units per XCD
-    int64_t t = -1;                        // output tile in the list (expert, n tile, m tile fastest)
+    ExpertScan sc = scan_expert_tiles_from(offsets, off64, E, BM, 0);   // every wave sees 64 expert groups at once
+    uint32_t mtiles = __builtin_amdgcn_readlane(sc.tiles_through, 63);
+    for (int base = 64; base < E; base += 64) mtiles += __builtin_amdgcn_readlane(scan_expert_tiles_from(offsets, off64, E, BM, base).tiles_through, 63);
+    const uint32_t T = mtiles * (uint32_t)ntiles_n;
+    const uint32_t xcd = blockIdx.x % NXCD, q = blockIdx.x / NXCD;
+    const uint32_t CH = (uint32_t)ncu / NXCD;   // compute units per XCD
+    uint32_t t = 0;                             // output tile in the list (expert, n tile, m tile fastest)
     {
         // The T tiles are cut into F = (T / #CU) * #CU tiles that fill whole rounds of compute units and a remainder; the
         // remainder tiles' K ranges are split 2 or 4 ways (when that many parts still fit in one round), so that the
@@ -151,66 +145,49 @@ __device__ __forceinline__ WorkItem decode_work_item(const void* offsets, int of
         // 7-round launch with the SwiGLU-backward epilogue measured 1.5 % slower dealt out and keeps its ranges.  Measured and
         // dropped for launches of few rounds: XCD ranges cut by the running cost of the tiles (32-row blocks, at
         // least half a tile) instead of by their number -- 4-7 % slower, with either way of splitting the last tiles.
-        const int64_t F = (T / ncu) * ncu;
+        const uint32_t F = T / (uint32_t)ncu * (uint32_t)ncu;
         const int rem = (int)(T - F);
-        int split = 1;
-        while (split * 2 <= max_split && rem * split * 2 <= ncu && ktiles / (split * 2) >= 8) split *= 2;
-        const int S = rem * split;                       // items of the last round
-        const int64_t Fx = F / NXCD;
-        const int Sx = (S + NXCD - 1) / NXCD;
+        int split = 1, lg = 0;
+        while (split * 2 <= max_split && rem * split * 2 <= ncu && (ktiles >> (lg + 1)) >= 8) { split *= 2; ++lg; }
+        const uint32_t S = (uint32_t)rem * split;        // items of the last round
+        const uint32_t Fx = F / NXCD;
+        const uint32_t Sx = (S + NXCD - 1) / NXCD;
         if (q < Fx) {
-            const bool deal = F >= (int64_t)INTERLEAVE_MIN_ROUNDS * ncu || F < (int64_t)CONTIGUOUS_MIN_ROUNDS * ncu;
-            t = deal ? ((q / CH) * NXCD + xcd) * CH + q % CH : xcd * Fx + q;
+            const bool deal = F >= (uint32_t)(INTERLEAVE_MIN_ROUNDS * ncu) || F < (uint32_t)(CONTIGUOUS_MIN_ROUNDS * ncu);
+            if (deal) { const uint32_t c = q / CH; t = (c * NXCD + xcd) * CH + (q - c * CH); }
+            else t = xcd * Fx + q;
         } else {
-            const int64_t j = (int64_t)xcd * Sx + (q - Fx);
+            const uint32_t j = xcd * Sx + (q - Fx);
             if (q - Fx >= Sx || j >= S) return w;
-            t = F + j / split;
-            w.part = (int)(j % split);
+            t = F + (j >> lg);
+            w.part = (int)(j & (split - 1));
             w.nparts = split;
             w.split_item = (int)j;
-            w.split_tile = (int)(j / split);
+            w.split_tile = (int)(j >> lg);
         }
     }
     if (w.nparts == 0) w.nparts = 1;
-    if (E <= 64) {
-        const unsigned long long hit = __ballot(lane < E && t >= sc.tiles_before * ntiles_n && t < sc.tiles_through * ntiles_n);
-        if (hit == 0) return w;
-        int expert = __ffsll(hit) - 1;
-        const int64_t start = __shfl(sc.start, expert), end = __shfl(sc.end, expert), before = __shfl(sc.tiles_before, expert);
-        const int64_t mte = (end - start + BM - 1) / BM;
-        const int64_t local = t - before * ntiles_n;
-        const int nt = (int)(local / mte);
-        const int64_t mt = local % mte;
+    uint32_t before_block = 0;   // row tiles of the experts before `base`
+    for (int base = 0; base < E; base += 64) {
+        if (base > 0) sc = scan_expert_tiles_from(offsets, off64, E, BM, base);
+        const uint32_t tl = t - before_block * (uint32_t)ntiles_n;
+        const unsigned long long hit = __ballot(tl >= (uint32_t)sc.tiles_before * (uint32_t)ntiles_n && tl < (uint32_t)sc.tiles_through * (uint32_t)ntiles_n);
+        if (hit == 0) { before_block += __builtin_amdgcn_readlane(sc.tiles_through, 63); continue; }
+        // everything derived from the item is uniform and belongs in scalar registers
+        const int hl = __ffsll(hit) - 1;
+        const int64_t start = readlane_i64(sc.start, hl), end = readlane_i64(sc.end, hl);
+        const uint32_t before = __builtin_amdgcn_readlane(sc.tiles_before, hl), mte = __builtin_amdgcn_readlane(sc.tiles_through, hl) - before;
+        const uint32_t local = tl - before * (uint32_t)ntiles_n, nt = local / mte, mt = local - nt * mte;
         int64_t row0, row1;
         even_rows(start, end, mt, mte, &row0, &row1);
-        // the shuffles return per-lane values; everything derived from the item is uniform and belongs in scalar registers
-        w.expert = __builtin_amdgcn_readfirstlane(expert);
-        w.nt = __builtin_amdgcn_readfirstlane(nt);
+        w.expert = __builtin_amdgcn_readfirstlane(base + hl);
+        w.nt = __builtin_amdgcn_readfirstlane((int)nt);
         w.row0 = uniform_i64(row0);
         w.row1 = uniform_i64(row1);
-        w.mtile = __builtin_amdgcn_readfirstlane((int)(before + mt));
+        w.mtile = __builtin_amdgcn_readfirstlane((int)(before_block + before + mt));
         w.only_tile = __builtin_amdgcn_readfirstlane((int)(mte == 1)) != 0;
         w.valid = true;
-    } else {
-        int64_t mtiles_before = 0;   // row tiles of the experts before `base`
-        for (int base = 0; base < E; base += 64) {
-            sc = scan_expert_tiles_from(offsets, off64, E, BM, base);
-            const int64_t tl = t - mtiles_before * ntiles_n;
-            const unsigned long long hit = __ballot(base + lane < E && tl >= sc.tiles_before * ntiles_n && tl < sc.tiles_through * ntiles_n);
-            if (hit == 0) { mtiles_before += uniform_i64(__shfl(sc.tiles_through, 63)); continue; }
-            const int hl = __ffsll(hit) - 1;
-            const int64_t start = uniform_i64(__shfl(sc.start, hl)), end = uniform_i64(__shfl(sc.end, hl)), before = uniform_i64(__shfl(sc.tiles_before, hl));
-            const int64_t mte = (end - start + BM - 1) / BM;
-            const int64_t local = tl - before * ntiles_n;
-            const int64_t mt = local % mte;
-            w.expert = base + hl;
-            w.nt = (int)(local / mte);
-            even_rows(start, end, mt, mte, &w.row0, &w.row1);
-            w.mtile = (int)(mtiles_before + before + mt);
-            w.only_tile = mte == 1;
-            w.valid = true;
-            break;
-        }
+        break;
     }
     w.part = __builtin_amdgcn_readfirstlane(w.part);
     w.nparts = __builtin_amdgcn_readfirstlane(w.nparts);
@@ -251,6 +228,8 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
     constexpr bool TWO_SEG = EPI == MOE_EPI_STORE;   // (the only epilogue that launches with two K segments)
     const int ktiles = TWO_SEG ? ktiles_seg * p.nseg : ktiles_seg;
     const WorkItem item = decode_work_item(p.offsets, p.off64, p.E, ntiles_n, ktiles, p.max_split, p.num_cus);
+    if (EPI_IS_PAIR(EPI) && p.clear_counters && blockIdx.x == 0)   // (this launch splits no tile: the counters are the next launch's)
+        for (int i = tid; i < p.num_cus; i += NTHREADS) p.sk_counters[i] = 0;
     if (!item.valid) return;
     const int expert = item.expert, nt = item.nt, part = item.part, nparts = item.nparts, split_item = item.split_item;
     const int64_t row0 = item.row0, row1 = item.row1;
@@ -516,7 +495,8 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
         }
 #pragma unroll
         for (int i = 0; i < LPT; ++i) issue_b(kb + 1, i, 1, once);
-        __builtin_amdgcn_s_waitcnt(0x0F70 | LPT);   // everything but weight tile kb+1 has landed
+        // tile kb has landed (the loads of tile kb+1 may still be on their way; without FULL their number varies, the activations among them are waited for)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (FULL ? 2 * LPT : LPT));
         __syncthreads();                            // (also: every wave has read the row tables that share B stage 2)
         bf16x8_t af[2][MBH], bf[2][NB];
 #pragma unroll
@@ -655,24 +635,31 @@ __global__ void __launch_bounds__(NTHREADS) grouped_gemm_mfma_kernel(const MoeGe
         __syncthreads();
         if (*s_arrival != nparts - 1) return;
         if (tid == 0) __hip_atomic_store(&p.sk_counters[ti], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // clean for the next launch
+        // Two parts' loads of a row block are in flight together.
         const uint32_t first_bytes = (uint32_t)(split_item - part) * (uint32_t)(BM * BN * sizeof(float));
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
-            if (mb < mb_cnt)
+            if (mb < mb_cnt) {
+                u32x4_t v[2][NB];
+                auto fetch = [&](int x0) {
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                const uint32_t o = first_bytes + (uint32_t)(((mb * NB + nb) * NTHREADS + tid) * 16);
-                u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(xbuf, o, 0, DEVICE_SCOPE);
-                float sum[4];
+                    for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) sum[r] = __uint_as_float(v[r]);
-                for (int x = 1; x < nparts; ++x) {
-                    v = __builtin_amdgcn_raw_buffer_load_b128(xbuf, o + (uint32_t)x * (uint32_t)(BM * BN * sizeof(float)), 0, DEVICE_SCOPE);
+                        for (int nb = 0; nb < NB; ++nb)
+                            v[x][nb] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, first_bytes + (uint32_t)(x0 + x) * (uint32_t)(BM * BN * sizeof(float)) + (uint32_t)(((mb * NB + nb) * NTHREADS + tid) * 16), 0, DEVICE_SCOPE);
+                };
+                fetch(0);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) sum[r] += __uint_as_float(v[r]);
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[mb][nb][r] = __uint_as_float(v[0][nb][r]) + __uint_as_float(v[1][nb][r]);
+                if (nparts > 2) {   // four
+                    fetch(2);
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[mb][nb][r] = (acc[mb][nb][r] + __uint_as_float(v[0][nb][r])) + __uint_as_float(v[1][nb][r]);
                 }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[mb][nb][r] = sum[r];
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -1240,6 +1227,7 @@ template <bool NN, int EPI, typename Num, bool KTAIL> int launch_typed(const Moe
     q.num_cus = moe_num_cus();
     q.y_wide = (!p.y_grouped && (R * p.ldy + p.N) * 2 >= ((int64_t)1 << 31)) ? 1 : 0;
     q.max_split = moe_gemm_max_split(EPI_IS_PAIR(EPI));
+    if (q.clear_counters && !q.sk_counters) return MOE_ERR_WORKSPACE;
     if (q.max_split > 1) {
         if (!p.sk_partials || !p.sk_counters) return MOE_ERR_WORKSPACE;
         if (!p.counters_clean) hipLaunchKernelGGL(zero_i32_kernel, dim3((unsigned)((q.num_cus + 255) / 256)), dim3(256), 0, stream, p.sk_counters, (int64_t)q.num_cus);

@@ -64,6 +64,7 @@ struct MoeGemmParams {
     float* sk_partials;     // K-split exchange area, see moe_gemm_sk_bytes / moe_gemm_sk_attach
     int* sk_counters;
     int counters_clean;     // the caller guarantees sk_counters is all zero at launch (every launch leaves it so)
+    int clear_counters;     // gate/up pair (which splits no tile): clears sk_counters for the launch behind it
 };
 
 size_t moe_gemm_sk_bytes(int64_t R, int E, int64_t N);
