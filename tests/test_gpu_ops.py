@@ -554,3 +554,28 @@ def test_scatter2scatter_lora_packs_any_width_and_rank(dev, oracle, K, N, r):
         y = ops.scatter2scatter_lora(X.to(dev), W.to(dev), Ad, Bd, 0.5, sei.to(dev), ssi.to(dev), 1, None)
         ref = oracle.scatter2scatter_lora(X, W, A, B, 0.5, sei, ssi, 1)
         assert rel(y, ref) < TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("K", [1, 15, 63, 64, 65, 130])
+@pytest.mark.parametrize("layout", ["k_contiguous", "n_contiguous"])
+def test_generic_kernels_at_the_edges_of_a_contraction_step(dev, oracle, dtype, K, layout):
+    """The kernels of the sizes that the matrix cores do not take, at contractions of one step, one step more or less and a few: the
+    product with adapters, and the per-expert product over rows (whose contraction is the group: 0, 1, 63 .. 130 rows)."""
+    ops = _ops()
+    torch.manual_seed(K)
+    counts, N, r = [63, 0, 64, 1, 65, 130], 19, 3
+    E, R = len(counts), sum(counts)
+    sei = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ssi = torch.randperm(R)
+    X, W = torch.randn(R, K).to(dtype), (torch.randn(E, K, N) * 0.3).to(dtype)
+    A, B = (torch.randn(E, K, r) * 0.3).to(dtype), (torch.randn(E, r, N) * 0.3).to(dtype)
+    Wd = W.permute(0, 2, 1).contiguous().to(dev).permute(0, 2, 1) if layout == "k_contiguous" else W.to(dev)
+    y = ops.scatter2scatter_lora(X.to(dev), Wd, A.to(dev), B.to(dev), 2.0, sei.to(dev), ssi.to(dev), 1)
+    ref = oracle.scatter2scatter_lora(X, W, A, B, 2.0, sei, ssi, 1)
+    assert rel(y, ref) < TOL[dtype]
+    dy = torch.randn(R, N).to(dtype)
+    dw = ops.group_bwd_W(dy.to(dev), X.to(dev), torch.tensor(counts).cumsum(0).to(dev), E)
+    at = torch.tensor([0] + counts).cumsum(0)
+    want = torch.stack([X[a:b].float().t() @ dy[a:b].float() for a, b in zip(at[:-1], at[1:])])
+    check_expert_grads(dw, want, TOL[dtype])
