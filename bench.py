@@ -337,8 +337,8 @@ def main():
                                          T_ * d_ * 2 + T_ * E_ * 4 + 2 * R * 8)
     if "rows.combine" in stages:
         hbm["combine (per launch)"] = (stages["rows.combine"], R * d_ * 2 + T_ * k_top * 4 + T_ * d_ * 2)
-    if "rows.combine_dgates" in stages:
-        hbm["combine d_gates"] = (stages["rows.combine_dgates"], R * d_ * 2 + T_ * d_ * 2 + T_ * k_top * 4)
+    if "rows.gates_bwd" in stages:
+        hbm["gate gradients"] = (stages["rows.gates_bwd"], R * d_ * 2 + T_ * d_ * 2 + T_ * k_top * 4)
     result["hbm_stages"] = {n: {"ms": round(ms, 4), "bytes": b, "GB_per_s": round(b / (ms * 1e-3) / 1e9, 1),
                                 "frac_of_8TBps": round(b / (ms * 1e-3) / 8e12, 4)} for n, (ms, b) in hbm.items()}
     if not fp32:

@@ -88,6 +88,13 @@ int moe_router_forward(const void* x, int64_t ldx, const void* wg, int64_t ldw, 
 int moe_router_topk_bwd(const float* dtopw, const float* topw, const int32_t* topi, const float* scores,
                         float* dlogits, int64_t ntok, int E, int k, int renorm, void* stream);
 
+/* what a layer's backward pass needs from its gates, bf16 / fp16 rows: dlogits (T,E) = gradient of the logits as moe_router_topk_bwd gives it
+ * for d(topw)[t][j] = <y[t*k+j], dout[t]> (moe_combine_dgates, fp32) + d_w[t][j] (d_w: gradient of the returned weights themselves, may be null),
+ * and row_scale[inv[p]] = topw[p] for every flat assignment p = t*k+j (inv: the sort's inverse permutation). */
+int moe_gates_bwd(const void* y, int64_t ldy, const void* dout, int64_t ldd, int dtype, const float* d_w, const float* topw,
+                  const int32_t* topi, const float* scores, const int32_t* inv, float* dlogits, float* row_scale, int64_t ntok,
+                  int64_t ncols, int E, int k, int renorm, void* stream);
+
 /* gradient of the router weight: dwg[e][c] = sum_t dlogits[t][e] * x[t][c] (autograd of the F.linear at
  * config_utils.py:262), from the fp32 dlogits with fp32 accumulation and a fixed summation order; dwg (E, d) in x's
  * dtype.  The gradient with respect to the router's input, dlogits @ wg, is moe_combine with k = 0 and the dense

@@ -29,6 +29,7 @@ _SIGNATURES = {
     "moe_router_topk": ("i", "ppppliiip"),
     "moe_router_forward": ("i", "plpli" + "pppp" + "lliiip"),
     "moe_router_topk_bwd": ("i", "ppppp" + "liiip"),
+    "moe_gates_bwd": ("i", "plpli" + "ppppppp" + "ll" + "iii" + "p"),
     "moe_router_weight_grad_workspace_bytes": ("z", "lli"),
     "moe_router_weight_grad": ("i", "plppllliipzp"),
     "moe_gemm_debug_plan_blocks": ("l", "lili"),

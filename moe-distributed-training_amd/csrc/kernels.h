@@ -132,23 +132,25 @@ size_t moe_xtp_workspace_bytes(int64_t R, int E, int64_t K);
 // two products (partial2 == nullptr: one)
 int moe_launch_cc_reduce2(const float* partial, const float* partial2, int ntiles, int64_t R, float scaling, void* Q, void* Q2,
                           void* Qt, void* Qt2, int64_t ldqt, hipStream_t stream, int f16 = 0);
-// the reduction half of moe_launch_xtp2 alone, for partials [row tile of 256][K][16] that another kernel produced
-// (partial2 == nullptr: only the first)
-int moe_launch_xtp_reduce2(const float* partial, const float* partial2, void* out, void* out2, const int64_t* so,
-                           const int64_t* so2, int rank, int rank2, const void* offsets, int off64, int E, int64_t K,
-                           float scale, hipStream_t stream, int f16 = 0);
 // two reductions over the same rows in one launch pair (X2 == nullptr: only the first); so / so2: output strides
 // {expert, k, r}; rank / rank2: columns each writes; needs twice moe_xtp_workspace_bytes when X2 is given
 int moe_launch_xtp2(const void* X, const void* X2, int64_t ldx, const void* pos, int pos64, int fan_out, const void* Pt,
                     const void* Pt2, int64_t ldpt, const float* p_row_scale, void* out, void* out2, const int64_t* so,
                     const int64_t* so2, int rank, int rank2, const void* offsets, int off64, int E, int64_t R, int64_t K,
                     float scale, void* workspace, size_t workspace_bytes, hipStream_t stream, int f16 = 0);
-// up to MOE_LORA_MAX_JOBS reductions over the same row order in one launch pair; needs njobs times moe_xtp_workspace_bytes of
-// the widest job
-struct MoeXtpJob { const void* X; int64_t ldx, K; const void* Pt; void* out; int64_t so[3]; int rank; };
-int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, const void* pos, int pos64, int fan_out, int64_t ldpt, const float* p_row_scale,
-                        const void* offsets, int off64, int E, int64_t R, float scale, void* workspace, size_t workspace_bytes,
-                        hipStream_t stream, int f16);
+// up to MOE_LORA_MAX_JOBS reductions over the same row order (a job's rows: X's own, or gathered, row m of the order being row
+// pos[m] / fan_out of X); row_scale: optional factor of P's row m
+struct MoeXtpJob { const void* X; int64_t ldx, K; const void* pos; int fan_out; const void* Pt; const float* row_scale; void* out; int64_t so[3]; int rank; };
+// ... in one launch pair; needs njobs times moe_xtp_workspace_bytes of the widest job
+int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldpt, const void* offsets, int off64, int E, int64_t R, float scale,
+                        void* workspace, size_t workspace_bytes, hipStream_t stream, int f16);
+// the two launches of that pair by themselves: job j's partials [row tile of 256][K][16] at partial + j * partial_stride (out, so and rank
+// unused); and the sum of up to MOE_XTP_MAX_REDUCE sets of such partials (out strides {expert, k, r}), wherever they come from
+constexpr int MOE_XTP_MAX_REDUCE = 6;
+struct MoeXtpReduceJob { const float* partial; int64_t K; void* out; int64_t so[3]; int rank; };
+int moe_launch_xtp_partial_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldpt, const void* offsets, int off64, int E, int64_t R,
+                                float* partial, int64_t partial_stride, hipStream_t stream, int f16);
+int moe_launch_xtp_reduce_jobs(const MoeXtpReduceJob* jobs, int njobs, const void* offsets, int off64, int E, float scale, hipStream_t stream, int f16);
 
 // router + integer pipeline
 int moe_launch_router_logits(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits,
@@ -160,6 +162,10 @@ int moe_launch_router_topk(const float* logits, float* scores, float* topw, int3
                            int renorm, hipStream_t stream);
 int moe_launch_router_bwd(const float* dw, const float* w, const int32_t* topi, const float* scores, float* dlogits,
                           int64_t ntok, int E, int k, int renorm, hipStream_t stream);
+// 16-bit types: gradients of the logits and the row scales of the sorted order from a layer's gates, see gates_bwd_kernel
+int moe_launch_gates_bwd(const void* y, int64_t ldy, const void* dout, int64_t ldd, int dtype, const float* d_w, const float* w,
+                         const int32_t* topi, const float* scores, const int32_t* inv, float* dlogits, float* row_scale, int64_t ntok,
+                         int64_t d, int E, int k, int renorm, hipStream_t stream);
 size_t moe_router_wgrad_ws_bytes(int64_t ntok, int64_t d, int E);
 int moe_launch_router_wgrad(const void* x, int64_t ldx, const float* dlogits, void* dwg, int64_t ldo, int64_t ntok,
                             int64_t d, int E, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream);

@@ -219,13 +219,11 @@ constexpr int XTP_COLS = 4 * XTP_WCOLS;  // columns per workgroup
 // up to four jobs per launch (see unit_and_job): same row order, operands and outputs of their own; job j's partials start
 // at partial + j * partial_stride.  A single projection's adapter gradients are two jobs per 16 rank columns (X with P, dY
 // with Q), of 152 workgroups each at 3000 rows over 8 experts and 4096 columns: too few to fill the chip one at a time.
-struct XtpJob { const uint16_t* X; const uint16_t* Pt; uint16_t* out; int64_t soe, sok, sor; int rank; int64_t ldx, K; };   // rank: columns written (<= 16)
+// pos: gathered rows (row of X = pos[m] / fan_out), or null; row_scale: factor of P's row m, or null
+struct XtpJob { const uint16_t* X; const uint16_t* Pt; int64_t ldx, K; const void* pos; int fan_out; const float* row_scale; };
 struct XtpJobs { XtpJob job[MOE_LORA_MAX_JOBS]; };
 template <typename Num>
-__global__ void __launch_bounds__(XTP_THREADS) xtp_partial_kernel(const XtpJobs jobs,
-                                                                  const void* __restrict__ pos, int pos64, int fan_out,
-                                                                  int64_t ldpt,
-                                                                  const float* __restrict__ p_row_scale,
+__global__ void __launch_bounds__(XTP_THREADS) xtp_partial_kernel(const XtpJobs jobs, int pos64, int64_t ldpt,
                                                                   float* __restrict__ partial, int64_t partial_stride,
                                                                   const void* __restrict__ offsets, int off64, int E,
                                                                   int64_t R, int njobs)
@@ -241,6 +239,9 @@ __global__ void __launch_bounds__(XTP_THREADS) xtp_partial_kernel(const XtpJobs 
     const int64_t tile_id = unit / kblocks, kblock = unit % kblocks;
     const uint16_t* __restrict__ X = job.X;
     const uint16_t* __restrict__ Pt = job.Pt;
+    const void* __restrict__ pos = job.pos;
+    const float* __restrict__ p_row_scale = job.row_scale;
+    const int fan_out = job.fan_out;
     partial += (int64_t)job_id * partial_stride;
     RowTile rt;
     if (!find_row_tile(offsets, off64, E, XTP_RC, tile_id, &rt)) return;
@@ -320,16 +321,18 @@ __global__ void __launch_bounds__(XTP_THREADS) xtp_partial_kernel(const XtpJobs 
 
 // out[e][k][r] = scale * sum over the expert's partial tiles (ascending), zero for an empty expert.  A thread owns four
 // consecutive rank columns of one k (one 16-byte load per tile, several tiles in flight).
+struct XtpReduceJob { const float* partial; uint16_t* out; int64_t soe, sok, sor; int rank; int64_t K; };   // rank: columns written (<= 16)
+struct XtpReduceJobs { XtpReduceJob job[MOE_XTP_MAX_REDUCE]; };
 template <typename Num>
-__global__ void xtp_reduce_kernel(const float* __restrict__ partial, int64_t partial_stride, const XtpJobs jobs,
-                                  const void* __restrict__ offsets, int off64, int E, float scale)
+__global__ void xtp_reduce_kernel(const XtpReduceJobs jobs, const void* __restrict__ offsets, int off64, int E, float scale)
 {
-    const XtpJob& job = jobs.job[blockIdx.z];
+    const XtpReduceJob& job = jobs.job[blockIdx.z];
     const int64_t K = job.K;
+    if ((int64_t)blockIdx.x * blockDim.x * 4 >= K * 16) return;   // (a job narrower than the launch's widest)
     uint16_t* __restrict__ out = job.out;
+    const float* __restrict__ partial = job.partial;
     const int64_t soe = job.soe, sok = job.sok, sor = job.sor;
     const int rank = job.rank;
-    partial += (int64_t)blockIdx.z * partial_stride;
     const int e = blockIdx.y;
     int64_t tile0, start, end;
     find_group(offsets, off64, XTP_RC, e, &start, &end, &tile0);   // one round trip, not one per expert
@@ -481,34 +484,62 @@ size_t moe_xtp_workspace_bytes(int64_t R, int E, int64_t K)
     return (size_t)(R / XTP_RC + E) * (size_t)K * 16 * sizeof(float);
 }
 
-int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, const void* pos, int pos64, int fan_out, int64_t ldpt, const float* p_row_scale,
-                        const void* offsets, int off64, int E, int64_t R, float scale, void* workspace, size_t workspace_bytes,
-                        hipStream_t stream, int f16)
+int moe_launch_xtp_partial_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldpt, const void* offsets, int off64, int E, int64_t R,
+                                float* partial, int64_t partial_stride, hipStream_t stream, int f16)
 {
     if (njobs < 1 || njobs > MOE_LORA_MAX_JOBS) return MOE_ERR_UNSUPPORTED;
     XtpJobs js = {};
     int64_t kmax = 0;
     for (int j = 0; j < njobs; ++j) {
         const MoeXtpJob& q = jobs[j];
-        if (q.rank < 1 || q.rank > 16 || q.K % 8 != 0 || q.ldx % 8 != 0 || ((uintptr_t)q.X % 16) != 0 || ((uintptr_t)q.Pt % 16) != 0) return MOE_ERR_UNSUPPORTED;
-        js.job[j] = {(const uint16_t*)q.X, (const uint16_t*)q.Pt, (uint16_t*)q.out, q.so[0], q.so[1], q.so[2], q.rank, q.ldx, q.K};
+        if (q.K % 8 != 0 || q.ldx % 8 != 0 || ((uintptr_t)q.X % 16) != 0 || ((uintptr_t)q.Pt % 16) != 0) return MOE_ERR_UNSUPPORTED;
+        js.job[j] = {(const uint16_t*)q.X, (const uint16_t*)q.Pt, q.ldx, q.K, q.pos, q.fan_out, q.row_scale};
+        kmax = q.K > kmax ? q.K : kmax;
+    }
+    if (R == 0 || E == 0 || kmax == 0) return MOE_OK;
+    if (ldpt % 16 != 0 || ldpt < (R + 31) / 32 * 32) return MOE_ERR_UNSUPPORTED;
+    const int64_t units = ((kmax + XTP_COLS - 1) / XTP_COLS) * (R / XTP_RC + E);
+    if ((units + 8) * njobs >= ((int64_t)1 << 31)) return MOE_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(f16 ? xtp_partial_kernel<NumF16> : xtp_partial_kernel<NumBf16>, dim3(job_grid(units, njobs)), dim3(XTP_THREADS), 0, stream, js, pos64, ldpt,
+                       partial, partial_stride, offsets, off64, E, R, njobs);
+    return moe_launch_status();
+}
+
+int moe_launch_xtp_reduce_jobs(const MoeXtpReduceJob* jobs, int njobs, const void* offsets, int off64, int E, float scale, hipStream_t stream, int f16)
+{
+    if (njobs < 1 || njobs > MOE_XTP_MAX_REDUCE) return MOE_ERR_UNSUPPORTED;
+    XtpReduceJobs js = {};
+    int64_t kmax = 0;
+    for (int j = 0; j < njobs; ++j) {
+        const MoeXtpReduceJob& q = jobs[j];
+        if (q.rank < 1 || q.rank > 16) return MOE_ERR_UNSUPPORTED;
+        js.job[j] = {q.partial, (uint16_t*)q.out, q.so[0], q.so[1], q.so[2], q.rank, q.K};
         kmax = q.K > kmax ? q.K : kmax;
     }
     if (E == 0 || kmax == 0) return MOE_OK;
-    if (ldpt % 16 != 0 || ldpt < (R + 31) / 32 * 32) return MOE_ERR_UNSUPPORTED;
+    dim3 rgrid((unsigned)((kmax * 4 + 255) / 256), (unsigned)E, (unsigned)njobs);
+    hipLaunchKernelGGL(f16 ? xtp_reduce_kernel<NumF16> : xtp_reduce_kernel<NumBf16>, rgrid, dim3(256), 0, stream, js, offsets, off64, E, scale);
+    return moe_launch_status();
+}
+
+int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldpt, const void* offsets, int off64, int E, int64_t R, float scale,
+                        void* workspace, size_t workspace_bytes, hipStream_t stream, int f16)
+{
+    if (njobs < 1 || njobs > MOE_LORA_MAX_JOBS) return MOE_ERR_UNSUPPORTED;
+    int64_t kmax = 0;
+    for (int j = 0; j < njobs; ++j) {
+        if (jobs[j].rank < 1 || jobs[j].rank > 16) return MOE_ERR_UNSUPPORTED;
+        kmax = jobs[j].K > kmax ? jobs[j].K : kmax;
+    }
     const size_t one = moe_xtp_workspace_bytes(R, E, kmax);
     if (workspace_bytes < one * njobs) return MOE_ERR_WORKSPACE;
     const int64_t pstride = (int64_t)(one / sizeof(float));
-    if (R > 0) {
-        const int64_t units = ((kmax + XTP_COLS - 1) / XTP_COLS) * (R / XTP_RC + E);
-        if ((units + 8) * njobs >= ((int64_t)1 << 31)) return MOE_ERR_UNSUPPORTED;
-        hipLaunchKernelGGL(f16 ? xtp_partial_kernel<NumF16> : xtp_partial_kernel<NumBf16>, dim3(job_grid(units, njobs)), dim3(XTP_THREADS), 0, stream, js, pos, pos64, fan_out, ldpt,
-                           p_row_scale, (float*)workspace, pstride, offsets, off64, E, R, njobs);
-    }
-    dim3 rgrid((unsigned)((kmax * 4 + 255) / 256), (unsigned)E, (unsigned)njobs);
-    hipLaunchKernelGGL(f16 ? xtp_reduce_kernel<NumF16> : xtp_reduce_kernel<NumBf16>, rgrid, dim3(256), 0, stream, (const float*)workspace, pstride, js, offsets,
-                       off64, E, scale);
-    return moe_launch_status();
+    const int rc = moe_launch_xtp_partial_jobs(jobs, njobs, pos64, ldpt, offsets, off64, E, R, (float*)workspace, pstride, stream, f16);
+    if (rc != MOE_OK) return rc;
+    MoeXtpReduceJob red[MOE_LORA_MAX_JOBS];
+    for (int j = 0; j < njobs; ++j)
+        red[j] = {(const float*)workspace + j * pstride, jobs[j].K, jobs[j].out, {jobs[j].so[0], jobs[j].so[1], jobs[j].so[2]}, jobs[j].rank};
+    return moe_launch_xtp_reduce_jobs(red, njobs, offsets, off64, E, scale, stream, f16);
 }
 
 int moe_launch_xtp2(const void* X, const void* X2, int64_t ldx, const void* pos, int pos64, int fan_out, const void* Pt,
@@ -516,23 +547,7 @@ int moe_launch_xtp2(const void* X, const void* X2, int64_t ldx, const void* pos,
                     const int64_t* so2, int rank, int rank2, const void* offsets, int off64, int E, int64_t R, int64_t K,
                     float scale, void* workspace, size_t workspace_bytes, hipStream_t stream, int f16)
 {
-    MoeXtpJob jobs[2] = {{X, ldx, K, Pt, out, {so[0], so[1], so[2]}, rank}, {}};
-    if (X2) jobs[1] = {X2, ldx, K, Pt2, out2, {so2[0], so2[1], so2[2]}, rank2};
-    return moe_launch_xtp_jobs(jobs, X2 ? 2 : 1, pos, pos64, fan_out, ldpt, p_row_scale, offsets, off64, E, R, scale, workspace, workspace_bytes, stream, f16);
-}
-
-int moe_launch_xtp_reduce2(const float* partial, const float* partial2, void* out, void* out2, const int64_t* so,
-                           const int64_t* so2, int rank, int rank2, const void* offsets, int off64, int E, int64_t K,
-                           float scale, hipStream_t stream, int f16)
-{
-    if (E == 0 || K == 0) return MOE_OK;
-    const bool two = partial2 != nullptr;
-    if (rank < 1 || rank > 16 || (two && (rank2 < 1 || rank2 > 16))) return MOE_ERR_UNSUPPORTED;
-    XtpJobs js = {};
-    js.job[0] = {nullptr, nullptr, (uint16_t*)out, so[0], so[1], so[2], rank, 0, K};
-    if (two) js.job[1] = {nullptr, nullptr, (uint16_t*)out2, so2[0], so2[1], so2[2], rank2, 0, K};
-    dim3 rgrid((unsigned)((K * 4 + 255) / 256), (unsigned)E, two ? 2u : 1u);
-    hipLaunchKernelGGL(f16 ? xtp_reduce_kernel<NumF16> : xtp_reduce_kernel<NumBf16>, rgrid, dim3(256), 0, stream, partial, two ? (int64_t)(partial2 - partial) : 0, js,
-                       offsets, off64, E, scale);
-    return moe_launch_status();
+    MoeXtpJob jobs[2] = {{X, ldx, K, pos, fan_out, Pt, p_row_scale, out, {so[0], so[1], so[2]}, rank}, {}};
+    if (X2) jobs[1] = {X2, ldx, K, pos, fan_out, Pt2, p_row_scale, out2, {so2[0], so2[1], so2[2]}, rank2};
+    return moe_launch_xtp_jobs(jobs, X2 ? 2 : 1, pos64, ldpt, offsets, off64, E, R, scale, workspace, workspace_bytes, stream, f16);
 }

@@ -158,6 +158,18 @@ int moe_router_topk_bwd(const float* dtopw, const float* topw, const int32_t* to
     return moe_launch_router_bwd(dtopw, topw, topi, scores, dlogits, ntok, E, k, renorm, st);
 }
 
+int moe_gates_bwd(const void* y, int64_t ldy, const void* dout, int64_t ldd, int dtype, const float* d_w, const float* topw, const int32_t* topi,
+                  const float* scores, const int32_t* inv, float* dlogits, float* row_scale, int64_t ntok, int64_t ncols, int E, int k, int renorm,
+                  void* stream)
+{
+    if (ntok < 0 || ncols < 1 || E < 1 || k < 1 || k > E) return MOE_ERR_BAD_ARG;
+    if (ntok == 0) return MOE_OK;
+    if (!y || !dout || !topw || !topi || !scores || !inv || !dlogits || !row_scale) return MOE_ERR_BAD_ARG;
+    hipStream_t st = S(stream);
+    TIMED("rows.gates_bwd");
+    return moe_launch_gates_bwd(y, ldy, dout, ldd, dtype, d_w, topw, topi, scores, inv, dlogits, row_scale, ntok, ncols, E, k, renorm, st);
+}
+
 size_t moe_router_weight_grad_workspace_bytes(int64_t ntok, int64_t d, int E) { return moe_router_wgrad_ws_bytes(ntok, d, E); }
 
 int moe_router_weight_grad(const void* x, int64_t ldx, const float* dlogits, void* dwg, int64_t ldo, int64_t ntok,
@@ -357,12 +369,12 @@ int moe_group_bwd_ab(const void* DY, int64_t sdm, int64_t sdn, const void* X, in
                 pb.job[pb.njobs++] = {(const uint16_t*)B + rc * sbr, sbe, sbn, sbr, (uint16_t*)Bt[c], N, 1, rk};
                 rows[c] = {X, sxm, K, At[c], nullptr, Qt[c], nullptr};
                 rows[n + c] = {DY, sdm, N, Bt[c], nullptr, Pt[c], nullptr};
-                xtp[c] = {X, sxm, K, Pt[c], (uint16_t*)DA + rc * sdar, {sdae, sdak, sdar}, rk};
-                xtp[n + c] = {DY, sdm, N, Qt[c], (uint16_t*)DB + rc * sdbr, {sdbe, sdbn, sdbr}, rk};
+                xtp[c] = {X, sxm, K, nullptr, 1, Pt[c], nullptr, (uint16_t*)DA + rc * sdar, {sdae, sdak, sdar}, rk};
+                xtp[n + c] = {DY, sdm, N, nullptr, 1, Qt[c], nullptr, (uint16_t*)DB + rc * sdbr, {sdbe, sdbn, sdbr}, rk};
             }
             TRY(moe_launch_pack_lora_batch(pb, S(stream)));
             TRY(moe_launch_rows_lora_jobs(rows, 2 * n, ldt, nullptr, 0, offsets, off64, E, R, 1, 1, scaling, nullptr, S(stream), f16));
-            TRY(moe_launch_xtp_jobs(xtp, 2 * n, nullptr, 0, 1, ldt, nullptr, offsets, off64, E, R, 1.f, xw, xb, S(stream), f16));
+            TRY(moe_launch_xtp_jobs(xtp, 2 * n, 0, ldt, offsets, off64, E, R, 1.f, xw, xb, S(stream), f16));
         }
         return MOE_OK;
     }
@@ -456,13 +468,16 @@ static inline size_t sk_bytes_mlp(int64_t R, int E, int64_t d, int64_t f)
 // column-tile partials of the two fused column contractions of the dh GEMM: [2][ceil(f / 256)][R][16] fp32
 static inline size_t cc_bytes(int64_t R, int64_t f) { return (size_t)2 * (size_t)((f + 255) / 256) * (size_t)R * 16 * sizeof(float); }
 
+// partials of the adapter gradients: with the fused products three sets of f columns (from the dh GEMM) and three of d, all alive until one
+// launch sums them; without, two sets of either at a time
+static inline size_t mlp_xtp_bytes(int64_t R, int E, int64_t d, int64_t f) { return 3 * (moe_xtp_workspace_bytes(R, E, f) + moe_xtp_workspace_bytes(R, E, d)); }
+
 size_t moe_mlp_workspace_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
 {
     size_t n = al(sk_bytes_mlp(R, E, d, f)) + 256;
     if (rank <= 0) return n;
-    const int64_t mx = d > f ? d : f;
     const size_t C = (size_t)(rank + 15) / 16;   // 16-wide chunks per adapter
-    return n + C * (3 * pack_bytes(E, d) + 3 * pack_bytes(E, f) + 7 * q_bytes(R)) + al(3 * moe_xtp_workspace_bytes(R, E, mx)) + al(cc_bytes(R, f));
+    return n + C * (3 * pack_bytes(E, d) + 3 * pack_bytes(E, f) + 7 * q_bytes(R)) + al(mlp_xtp_bytes(R, E, d, f)) + al(cc_bytes(R, f));
 }
 
 size_t moe_mlp_saved_bytes(int64_t R, int rank) { return rank > 0 ? (size_t)((rank + 15) / 16) * 6 * q_bytes(R) : 256; }
@@ -671,8 +686,7 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         pq = (uint8_t*)ws.take((size_t)C * 6 * qb);
         if (fuse_rc) p2s = ws.take(qb);   // P2 times the row scale, row-major (the fused contraction's operand)
         if (fuse_rc) ccw = (float*)ws.take(cc_bytes(R, f));
-        const int64_t mx = d > f ? d : f;
-        xb = 3 * moe_xtp_workspace_bytes(R, E, mx);   // paired reductions keep two sets of partials, the fused ones of the dh GEMM three
+        xb = mlp_xtp_bytes(R, E, d, f);
         xw = ws.take(xb);
         TIMED("bwd.pack_lora");
         for (int c = 0; c < C; ++c) {
@@ -744,29 +758,23 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         TIMED("bwd.gemm_dh_swiglu_bwd");
         TRY(moe_launch_gemm_mfma(p, R, st));
     }
+    int64_t so[6][3] = {};   // strides {expert, k or n, rank} of the gradients, order dA1, dB1, dA3, dB3, dA2, dB2
+    for (int i = 0; i < 6 && has_lora; ++i) { so[i][0] = gs[3 * i]; so[i][1] = gs[3 * i + 1 + i % 2]; so[i][2] = gs[3 * i + 2 - i % 2]; }
     if (has_lora) {
         // dA2[e][k=f][r] = sum_m h[m][k] * (row_scale[m] P2[m][r]);  dB2[e][r][n=d] = sum_m (row_scale[m] Q2[m][r]) dy[m][n]
-        const int64_t sb1[3] = {gs[3], gs[5], gs[4]}, sb3[3] = {gs[9], gs[11], gs[10]};
-        { TIMED("bwd.xtp_w2");
-        const int64_t sa2[3] = {gs[12], gs[13], gs[14]}, sb2[3] = {gs[15], gs[17], gs[16]};
+        if (!fuse_rc) { TIMED("bwd.xtp_w2");
         uint16_t* dA2 = (uint16_t*)lg[4];
         uint16_t* dB2 = (uint16_t*)lg[5];
-        if (fuse_rc) {   // the sums over each row tile came out of the dh GEMM's epilogue: add the tiles per expert
-            const size_t one = moe_xtp_workspace_bytes(R, E, f);
-            const float* part = (const float*)xw;
-            TRY(moe_launch_xtp_reduce2(part, part + one / sizeof(float), lg[1], lg[3], sb1, sb3, rank, rank, offsets, off64, E, f, 1.f, st, f16));
-            TRY(moe_launch_xtp_reduce2(part + 2 * (one / sizeof(float)), nullptr, dA2, nullptr, sa2, nullptr, rank, 0, offsets, off64, E, f, 1.f, st, f16));
-        } else
         for (int c = 0; c < C; c += 2) {   // two chunks per launch: the twin's reads of h are served by L2
             const bool two = c + 1 < C;
             TRY(moe_launch_xtp2(h, two ? h : nullptr, f, nullptr, 0, 1, pqp(3, c), two ? pqp(3, c + 1) : nullptr, ldt, nullptr, dA2 + 16 * c * gs[14],
-                                two ? dA2 + 16 * (c + 1) * gs[14] : nullptr, sa2, sa2, chunk_rank(c), two ? chunk_rank(c + 1) : 0, offsets, off64, E, R, f,
+                                two ? dA2 + 16 * (c + 1) * gs[14] : nullptr, so[4], so[4], chunk_rank(c), two ? chunk_rank(c + 1) : 0, offsets, off64, E, R, f,
                                 1.f, xw, xb, st, f16));
         }
         for (int c = 0; c < C; c += 2) {
             const bool two = c + 1 < C;
             TRY(moe_launch_xtp2(dy, two ? dy : nullptr, lddy, dy_grouped ? nullptr : pos, pos64, dy_fan_out, svp(5, c),
-                                two ? svp(5, c + 1) : nullptr, ldt, row_scale, dB2 + 16 * c * gs[16], two ? dB2 + 16 * (c + 1) * gs[16] : nullptr, sb2, sb2,
+                                two ? svp(5, c + 1) : nullptr, ldt, row_scale, dB2 + 16 * c * gs[16], two ? dB2 + 16 * (c + 1) * gs[16] : nullptr, so[5], so[5],
                                 chunk_rank(c), two ? chunk_rank(c + 1) : 0, offsets, off64, E, R, d, 1.f, xw, xb, st, f16));
         } }
         // ---- w1 / w3 backward
@@ -803,21 +811,34 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
     if (has_lora) {
         // dA1[e][k=d][r] = sum_m x[in_row(m)][k] P1[m][r];  dB1[e][r][n=f] = sum_m Q1[m][r] dgate[m][n]
         TIMED("bwd.xtp_w1w3");
-        const int64_t sa1[3] = {gs[0], gs[1], gs[2]}, sa3[3] = {gs[6], gs[7], gs[8]};
-        const int64_t sb1[3] = {gs[3], gs[5], gs[4]}, sb3[3] = {gs[9], gs[11], gs[10]};
+        if (fuse_rc) {
+            // One launch over x and dy leaves the partials of dA1, dA3 and dB2 behind those of dB1, dB3 and dA2 that the dh GEMM's epilogue
+            // left, and one launch adds all six: six launches before (4096 tokens, d=4096, f=14336: 87 us together, 65 now; 512 tokens, d=256:
+            // 41 us, 16 now -- each of them was a few workgroups behind a gap; 2048 tokens, 64 experts: 76 and 66).
+            const size_t onef = moe_xtp_workspace_bytes(R, E, f) / sizeof(float), oned = moe_xtp_workspace_bytes(R, E, d) / sizeof(float);
+            float* part = (float*)xw;
+            float* partd = part + 3 * onef;
+            const MoeXtpJob jobs[3] = {{x, ldx, d, pos, fan_out, pqp(4, 0), nullptr, nullptr, {}, rank}, {x, ldx, d, pos, fan_out, pqp(5, 0), nullptr, nullptr, {}, rank},
+                                       {dy, lddy, d, dy_grouped ? nullptr : pos, dy_fan_out, svp(5, 0), row_scale, nullptr, {}, rank}};
+            TRY(moe_launch_xtp_partial_jobs(jobs, 3, pos64, ldt, offsets, off64, E, R, partd, (int64_t)oned, st, f16));
+            auto red = [&](const float* p, int64_t K, void* out, const int64_t* st3) { return MoeXtpReduceJob{p, K, out, {st3[0], st3[1], st3[2]}, rank}; };
+            const MoeXtpReduceJob sums[6] = {red(part, f, lg[1], so[1]), red(part + onef, f, lg[3], so[3]), red(part + 2 * onef, f, lg[4], so[4]),
+                                             red(partd, d, lg[0], so[0]), red(partd + oned, d, lg[2], so[2]), red(partd + 2 * oned, d, lg[5], so[5])};
+            TRY(moe_launch_xtp_reduce_jobs(sums, 6, offsets, off64, E, 1.f, st, f16));
+        } else
         for (int c = 0; c < C; ++c) {
             const int rk = chunk_rank(c);
             TRY(moe_launch_xtp2(x, x, ldx, pos, pos64, fan_out, pqp(4, c), pqp(5, c), ldt, nullptr, (uint16_t*)lg[0] + 16 * c * gs[2],
-                                (uint16_t*)lg[2] + 16 * c * gs[8], sa1, sa3, rk, rk, offsets, off64, E, R, d, 1.f, xw, xb, st, f16));
+                                (uint16_t*)lg[2] + 16 * c * gs[8], so[0], so[2], rk, rk, offsets, off64, E, R, d, 1.f, xw, xb, st, f16));
         }
         if (!fuse_rc)
         for (int c = 0; c < C; c += 2) {   // two chunks of one adapter per launch, so that dgate and dup are each fetched once per pair of chunks
             const bool two = c + 1 < C;
             const int rk0 = chunk_rank(c), rk1 = two ? chunk_rank(c + 1) : 0;
             TRY(moe_launch_xtp2(dgate, two ? dgate : nullptr, f, nullptr, 0, 1, svp(3, c), two ? svp(3, c + 1) : nullptr, ldt, nullptr, (uint16_t*)lg[1] + 16 * c * gs[4],
-                                two ? (uint16_t*)lg[1] + 16 * (c + 1) * gs[4] : nullptr, sb1, sb1, rk0, rk1, offsets, off64, E, R, f, 1.f, xw, xb, st, f16));
+                                two ? (uint16_t*)lg[1] + 16 * (c + 1) * gs[4] : nullptr, so[1], so[1], rk0, rk1, offsets, off64, E, R, f, 1.f, xw, xb, st, f16));
             TRY(moe_launch_xtp2(dup, two ? dup : nullptr, f, nullptr, 0, 1, svp(4, c), two ? svp(4, c + 1) : nullptr, ldt, nullptr, (uint16_t*)lg[3] + 16 * c * gs[10],
-                                two ? (uint16_t*)lg[3] + 16 * (c + 1) * gs[10] : nullptr, sb3, sb3, rk0, rk1, offsets, off64, E, R, f, 1.f, xw, xb, st, f16));
+                                two ? (uint16_t*)lg[3] + 16 * (c + 1) * gs[10] : nullptr, so[3], so[3], rk0, rk1, offsets, off64, E, R, f, 1.f, xw, xb, st, f16));
         }
     }
     return MOE_OK;

@@ -696,10 +696,11 @@ struct LayerFn : Function<LayerFn> {
         const MlpShape s{sz[0], sz[1], sz[2], T * k, (int)k, ctx->saved_data["scaling"].toDouble()};
         const Lora lora = describe_lora(&sv[5], storage, s.d, s.f);
         Tensor dout = g_[0].defined() ? g_[0].contiguous() : at::zeros_like(x);
-        Tensor d_gates = combine_dgates(y, dout, k, at::kFloat, nullptr);
-        if (g_[1].defined()) d_gates = d_gates + g_[1].to(at::kFloat);   // the caller also used the returned expert weights (e.g. in an auxiliary loss)
-        Tensor dlogits = router_topk_bwd(d_gates, weights, indices, scores, normalize);
-        Tensor row_scale = group_rows(weights.view({-1, 1}), so.ssi(), 0, s.R, 1);
+        const Tensor d_w = g_[1].defined() ? g_[1].to(at::kFloat).contiguous() : Tensor();   // the caller also used the returned expert weights (e.g. in an auxiliary loss)
+        Tensor dlogits = at::empty_like(scores), row_scale = at::empty({s.R}, scores.options());
+        check(moe_gates_bwd(ptr(y), y.stride(0), ptr(dout), dout.stride(0), dtype_code(y), (const float*)ptr(d_w), (const float*)ptr(weights),
+                            (const int32_t*)ptr(indices), (const float*)ptr(scores), so.inv(), (float*)ptr(dlogits), (float*)ptr(row_scale), T, y.size(1), (int)s.E,
+                            (int)k, normalize, stream_of(y)), "moe_gates_bwd");
         MlpGrads g = mlp_backward(dout, false, k, (const float*)ptr(row_scale), x, w1, w3, w2, &sv[5], lora, s, sv[15], sv[16], sv[17], sv[19], so.ssi(), 0,
                                   so.offsets(), 0);
         Tensor dw[3];

@@ -365,3 +365,31 @@ def test_sort_takes_no_longer_when_most_rows_go_to_one_expert(dev):
 
     even, uneven = us(0.0), us(0.9)
     assert uneven < 1.6 * even, (even, uneven)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,E,k,d,renorm", [(1, 1, 1, 8, True), (5, 3, 1, 64, True), (9, 4, 2, 520, False), (33, 8, 2, 4096, True), (7, 5, 3, 100, True),
+                                            (6, 16, 5, 512, True), (4, 40, 20, 1032, True)])
+@pytest.mark.parametrize("direct", [False, True])
+def test_gate_gradients_in_one_launch(dev, dtype, T, E, k, d, renorm, direct):
+    """moe_gates_bwd against the entry points whose sums it repeats (combine_dgates, router_topk_bwd, a gather of the weights): bit for
+    bit, for token counts and numbers of selections that do not fill its workgroups, columns that are no whole vectors, and with and
+    without a gradient that reached the weights directly."""
+    from moe_distributed_training_amd._lib import lib, check, ptr, stream_ptr, dtype_code
+    _, router, ops = _mods()
+    g = torch.Generator(device=dev).manual_seed(T * 100 + k)
+    logits = torch.randn(T, E, generator=g, device=dev)
+    s, w, i = router.router_topk(logits, k, renorm)
+    sei, ssi, _, offs, inv = router.sort_assignments(i, E)
+    y, dout = torch.randn(T * k, d, generator=g, device=dev).to(dtype), torch.randn(T, d, generator=g, device=dev).to(dtype)
+    dw = torch.randn(T, k, generator=g, device=dev) if direct else None
+    dl, scale = torch.empty_like(s), torch.full((T * k,), -7.0, device=dev)
+    check(lib.moe_gates_bwd(ptr(y), d, ptr(dout), d, dtype_code(y), ptr(dw), ptr(w), ptr(i), ptr(s), ptr(inv), ptr(dl), ptr(scale), T, d, E, k,
+                            int(renorm), stream_ptr(dev)), "moe_gates_bwd")
+    total = ops.combine_dgates(y, dout, k, torch.float32)
+    if direct:
+        total = total + dw
+    want = torch.empty_like(s)
+    check(lib.moe_router_topk_bwd(ptr(total), ptr(w), ptr(i), ptr(s), ptr(want), T, E, k, int(renorm), stream_ptr(dev)), "moe_router_topk_bwd")
+    assert torch.equal(dl, want)
+    assert torch.equal(scale, w.reshape(-1)[ssi.long()])
