@@ -230,6 +230,7 @@ __global__ void router_topk_wide_kernel(const float* __restrict__ logits, float*
 // token; the eight waves' partial sums meet in LDS and are added in wave order (fixed: the result does not depend on
 // timing).  The summation order differs from router_logits_kernel's, so the two agree to fp32 rounding, not bit for bit.
 constexpr int RM_WAVES = 8, RM_TOKENS = 16;
+constexpr int RM_MAX_EXPERTS = 96;   // beyond, a workgroup's partial sums do not fit its LDS
 constexpr int RM_BATCH = 16;   // 32-wide K steps whose loads are in flight together (16 steps x 8 waves = 4096 columns)
 template <typename T>
 __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_kernel(const T* __restrict__ x, int64_t ldx,
@@ -294,6 +295,71 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_kernel(const T* __r
     }
 }
 
+// The same for 9 to 96 experts, in EG groups of 16: a wave's activation fragment meets EG weight fragments per step, fewer steps' loads fit in
+// flight, and the eight partial sums per logit are added in wave order as above.  The two launches of the vector kernels are bound by their
+// FMAs (2048 tokens x 64 experts x 2048 columns: 26.3 + 10.2 us, this 21); the order of a logit's sum differs from theirs.
+template <typename T, int EG>
+__global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_wide_kernel(const T* __restrict__ x, int64_t ldx, const T* __restrict__ wg, int64_t ldw,
+                                                                         float* __restrict__ logits, float* __restrict__ scores,
+                                                                         float* __restrict__ topw, int32_t* __restrict__ topi, int64_t ntok, int d,
+                                                                         int E, int k, int renorm)
+{
+    constexpr int BATCH = EG == 1 ? 16 : EG == 2 ? 8 : 4;
+    constexpr int EW = EG * 16;
+    __shared__ float s_part[RM_WAVES][RM_TOKENS][EW];
+    __shared__ float s_logits[RM_TOKENS][EW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t t0 = (int64_t)blockIdx.x * RM_TOKENS;
+    const int row = lane & 15, kc = lane >> 4;
+    const int64_t tok = (t0 + row < ntok) ? t0 + row : ntok - 1;      // tokens past the end re-read the last one
+    const T* xp = x + tok * ldx + kc * 8;
+    const T* wp[EG];
+#pragma unroll
+    for (int g = 0; g < EG; ++g) wp[g] = wg + (int64_t)(g * 16 + row < E ? g * 16 + row : E - 1) * ldw + kc * 8;   // (rows past the last expert repeat it; nobody reads their logits)
+    const int nsteps = d / 32;
+    const int s_end = nsteps * (wave + 1) / RM_WAVES;
+    f32x4_t acc[EG];
+#pragma unroll
+    for (int g = 0; g < EG; ++g) acc[g] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int s0 = nsteps * wave / RM_WAVES; s0 < s_end; s0 += BATCH) {
+        uint4 xa[BATCH], wa[BATCH][EG];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int64_t st = (int64_t)((s0 + i < s_end) ? s0 + i : s_end - 1) * 32;
+            xa[i] = *(const uint4*)(xp + st);
+#pragma unroll
+            for (int g = 0; g < EG; ++g) wa[i][g] = *(const uint4*)(wp[g] + st);
+        }
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+            if (s0 + i < s_end) {
+#pragma unroll
+                for (int g = 0; g < EG; ++g) {
+                    using Num = typename std::conditional<std::is_same<T, __hip_bfloat16>::value, NumBf16, NumF16>::type;
+                    acc[g] = Num::mfma(__builtin_bit_cast(bf16x8_t, wa[i][g]), __builtin_bit_cast(bf16x8_t, xa[i]), acc[g]);
+                }
+            }
+    }
+    // acc[g][r] = partial logit of token `row`, expert 16 g + 4 kc + r
+#pragma unroll
+    for (int g = 0; g < EG; ++g) *(f32x4_t*)&s_part[wave][row][g * 16 + 4 * kc] = acc[g];
+    __syncthreads();
+    for (int i = tid; i < RM_TOKENS * EW; i += RM_WAVES * 64) {
+        const int t = i / EW, e = i % EW;
+        float sum = s_part[0][t][e];
+#pragma unroll
+        for (int w = 1; w < RM_WAVES; ++w) sum += s_part[w][t][e];
+        s_logits[t][e] = sum;
+        if (e < E && t0 + t < ntok) logits[(t0 + t) * E + e] = sum;
+    }
+    __syncthreads();
+    if (tid < RM_TOKENS * TK_LANES) {   // whole waves
+        const int tt = tid / TK_LANES;
+        const int64_t t = t0 + tt;
+        softmax_topk_token<EG>(s_logits[tt], scores + t * E, topw + t * k, topi + t * k, E, k, renorm, t < ntok);
+    }
+}
+
 // Backward of softmax -> top-k -> renormalise with respect to the logits, for one token (the pointers are its rows).
 // dwt (k): gradient of the returned weights; wt (k) the returned weights; s (E) the softmax.
 // TK_LANES lanes share a token so that its rows move coalesced; every lane computes the token's two sums over the k
@@ -353,9 +419,9 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const float* __restrict
 // wave per (token, selection) pair takes the gradient of that weight, <y[t*k+j], dout[t]> (+ d_w, a gradient that reached the returned
 // weights directly), and puts the weight at the pair's place in sorted order (the row scale of the grouped GEMMs); then the token's lanes
 // turn its k gradients into those of its logits.  The sums are those of combine_dgates and router_bwd, bit for bit.  As three launches
-// 2048 tokens, 64 experts, top-8, d=2048 took 34.6 us, this 32.8; 4096 tokens, top-2, d=4096 28.7 and 25.7; 512 tokens, d=256 9.4 and 5.1.
-constexpr int GB_WAVES = 4;
-template <typename T>
+// 2048 tokens, 64 experts, top-8, d=2048 took 34.6 us, this 25.3 (eight waves for more than four selections; four: 32.8); 4096 tokens, top-2, d=4096 28.7 and 18.8;
+// 512 tokens, d=256 9.4 and 4.7.
+template <typename T, int GB_WAVES>
 __global__ void __launch_bounds__(GB_WAVES * 64) gates_bwd_kernel(const T* __restrict__ y, int64_t ldy, const T* __restrict__ dout, int64_t ldd,
                                                                   const float* __restrict__ d_w, const float* __restrict__ w,
                                                                   const int32_t* __restrict__ topi, const float* __restrict__ scores,
@@ -372,8 +438,21 @@ __global__ void __launch_bounds__(GB_WAVES * 64) gates_bwd_kernel(const T* __res
         const T* yr = y + pair * ldy;
         const T* dr = dout + (t0 + p / k) * ldd;
         float acc = 0.f;
-#pragma unroll 4
-        for (int64_t c0 = (int64_t)lane * 8; c0 < d; c0 += 64 * 8) {
+        int64_t c0 = (int64_t)lane * 8;
+        if (vec_ok)   // whole vectors, four of each row in flight
+            for (; c0 + 3 * 512 + 8 <= d; c0 += 4 * 512) {
+                uint4 a[4], b[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    a[q] = *(const uint4*)(yr + c0 + q * 512);
+                    b[q] = *(const uint4*)(dr + c0 + q * 512);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) acc = fmaf(Elem<T>::ld((const T*)&a[q] + u), Elem<T>::ld((const T*)&b[q] + u), acc);
+            }
+        for (; c0 < d; c0 += 64 * 8) {
             const int n = d - c0 < 8 ? (int)(d - c0) : 8;
             float a[8], b[8];
             load8<T>(yr + c0, a, n, vec_ok);
@@ -721,13 +800,22 @@ int moe_launch_router_forward(const void* x, int64_t ldx, const void* wg, int64_
                               int renorm, hipStream_t stream)
 {
     if (ntok == 0) return MOE_OK;
-    const bool fused = dtype != MOE_F32 && E <= ROUTER_EXPERT_GROUP && d % 32 == 0 && d >= 32 && d < (1 << 30) &&
+    const bool fused = dtype != MOE_F32 && E <= RM_MAX_EXPERTS && d % 32 == 0 && d >= 32 && d < (1 << 30) &&
                        ((uintptr_t)x % 16 == 0) && ((uintptr_t)wg % 16 == 0) && ldx % 8 == 0 && ldw % 8 == 0;
     if (!fused) {
         const int rc = moe_launch_router_logits(x, ldx, wg, ldw, dtype, logits, ntok, d, E, stream);
         return rc != MOE_OK ? rc : moe_launch_router_topk(logits, scores, topw, topi, ntok, E, k, renorm, stream);
     }
     const unsigned grid = (unsigned)((ntok + RM_TOKENS - 1) / RM_TOKENS);
+    if (E > ROUTER_EXPERT_GROUP) {
+        auto wide = [&](auto tag) {
+            using T = decltype(tag);
+            auto kern = E <= 16 ? router_mfma_wide_kernel<T, 1> : E <= 32 ? router_mfma_wide_kernel<T, 2> : E <= 64 ? router_mfma_wide_kernel<T, 4> : router_mfma_wide_kernel<T, 6>;
+            hipLaunchKernelGGL(kern, dim3(grid), dim3(RM_WAVES * 64), 0, stream, (const T*)x, ldx, (const T*)wg, ldw, logits, scores, topw, topi, ntok, (int)d, E, k, renorm);
+        };
+        if (dtype == MOE_BF16) wide(__hip_bfloat16{}); else wide(__half{});
+        return moe_launch_status();
+    }
     if (dtype == MOE_BF16)
         hipLaunchKernelGGL(router_mfma_kernel<__hip_bfloat16>, dim3(grid), dim3(RM_WAVES * 64), 0, stream, (const __hip_bfloat16*)x, ldx,
                            (const __hip_bfloat16*)wg, ldw, logits, scores, topw, topi, ntok, (int)d, E, k, renorm);
@@ -770,16 +858,17 @@ int moe_launch_gates_bwd(const void* y, int64_t ldy, const void* dout, int64_t l
 {
     if (dtype == MOE_F32) return MOE_ERR_UNSUPPORTED;
     if (ntok == 0) return MOE_OK;
-    const int tokens = k >= GB_WAVES ? 1 : (GB_WAVES + k - 1) / k;   // at least one pair per wave; at most GB_WAVES tokens, TK_LANES lanes each
+    const int waves = k > 4 ? 8 : 4;
+    const int tokens = k >= waves ? 1 : (waves + k - 1) / k;   // at least one pair per wave; at most 4 tokens, TK_LANES lanes each
     const bool vec = (uintptr_t)y % 16 == 0 && (uintptr_t)dout % 16 == 0 && ldy % 8 == 0 && ldd % 8 == 0;
     const dim3 grid((unsigned)((ntok + tokens - 1) / tokens));
     const size_t lds = (size_t)tokens * k * sizeof(float);
-    if (dtype == MOE_BF16)
-        hipLaunchKernelGGL(gates_bwd_kernel<__hip_bfloat16>, grid, dim3(GB_WAVES * 64), lds, stream, (const __hip_bfloat16*)y, ldy, (const __hip_bfloat16*)dout, ldd, d_w,
-                           w, topi, scores, inv, dlogits, row_scale, ntok, d, E, k, renorm, tokens, vec);
-    else
-        hipLaunchKernelGGL(gates_bwd_kernel<__half>, grid, dim3(GB_WAVES * 64), lds, stream, (const __half*)y, ldy, (const __half*)dout, ldd, d_w, w, topi, scores, inv,
-                           dlogits, row_scale, ntok, d, E, k, renorm, tokens, vec);
+    auto launch = [&](auto tag) {
+        using T = decltype(tag);
+        hipLaunchKernelGGL((waves == 8 ? gates_bwd_kernel<T, 8> : gates_bwd_kernel<T, 4>), grid, dim3(waves * 64), lds, stream, (const T*)y, ldy, (const T*)dout, ldd, d_w, w,
+                           topi, scores, inv, dlogits, row_scale, ntok, d, E, k, renorm, tokens, vec);
+    };
+    if (dtype == MOE_BF16) launch(__hip_bfloat16{}); else launch(__half{});
     return moe_launch_status();
 }
 

@@ -393,3 +393,24 @@ def test_gate_gradients_in_one_launch(dev, dtype, T, E, k, d, renorm, direct):
     check(lib.moe_router_topk_bwd(ptr(total), ptr(w), ptr(i), ptr(s), ptr(want), T, E, k, int(renorm), stream_ptr(dev)), "moe_router_topk_bwd")
     assert torch.equal(dl, want)
     assert torch.equal(scale, w.reshape(-1)[ssi.long()])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,d,E,k", [(1, 32, 9, 1), (17, 96, 16, 2), (40, 544, 17, 3), (33, 2048, 32, 8), (16, 4096, 33, 2), (100, 1024, 64, 8), (31, 256, 65, 4),
+                                     (50, 8192, 96, 6), (20, 512, 97, 2)])
+def test_router_of_many_experts_on_the_matrix_cores(dev, oracle, dtype, T, d, E, k):
+    """The one-launch router at the expert counts where its groups of 16 change (and 97, which takes two launches): logits to fp32
+    rounding of sums of exact products (sqrt(d) terms of half an ulp each, far below 3e-5 here), the oracle's choices, and exactly the softmax and
+    top-k of its own logits."""
+    _, router, _ = _mods()
+    torch.manual_seed(T + d + E)
+    x, wg = torch.randn(T, d).to(dtype), (torch.randn(E, d) / d ** 0.5).to(dtype)
+    l, s, w, i = router.router_forward(x.to(dev), wg.to(dev), k)
+    lo, so, wo, io = oracle.router(x, wg, k)
+    srt = torch.sort(so, dim=-1, descending=True).values
+    assert (srt[:, k - 1] - srt[:, k]).abs().min() > 1e-7, "test data has a near tie; pick another seed"
+    assert torch.allclose(l.cpu(), lo, atol=3e-5, rtol=1e-5)
+    assert torch.equal(i.cpu().long(), io)
+    assert torch.allclose(s.cpu(), so, atol=1e-6) and torch.allclose(w.cpu(), wo, atol=1e-5)
+    s1, w1, i1 = router.router_topk(l, k)
+    assert torch.equal(s, s1) and torch.equal(w, w1) and torch.equal(i, i1)
