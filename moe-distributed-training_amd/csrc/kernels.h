@@ -117,10 +117,10 @@ int moe_launch_pack_lora_batch(const MoePackBatch& jobs, hipStream_t stream);
 // up to MOE_LORA_MAX_JOBS products in one launch over the same row order: Q = scaling * X . A in storage type, [R][16], its
 // transposed copy Qt (row pitch ldqt) and a copy of Q scaled like Qt (each optional)
 constexpr int MOE_LORA_MAX_JOBS = 4;
-struct MoeRowsLoraJob { const void* X; int64_t ldx, K; const void* At; void* Q; void* Qt; void* q_scaled; };
-int moe_launch_rows_lora_jobs(const MoeRowsLoraJob* jobs, int njobs, int64_t ldqt, const void* pos, int pos64, const void* offsets,
-                              int off64, int E, int64_t R, int fan_out, int x_grouped, float scaling, const float* qt_row_scale,
-                              hipStream_t stream, int f16);
+// (pos: gathered rows, row m of the order being row pos[m] / fan_out of X, or null; qt_row_scale: optional factor of Qt's and q_scaled's row m)
+struct MoeRowsLoraJob { const void* X; int64_t ldx, K; const void* pos; int fan_out; const void* At; void* Q; void* Qt; void* q_scaled; const float* qt_row_scale; };
+int moe_launch_rows_lora_jobs(const MoeRowsLoraJob* jobs, int njobs, int64_t ldqt, int pos64, const void* offsets, int off64, int E, int64_t R,
+                              float scaling, hipStream_t stream, int f16);
 // two products over the same rows in one launch (X2 == nullptr: only the first)
 // q_scaled (optional): a third output of the first product, [R][16] like Q but multiplied by qt_row_scale like Qt
 int moe_launch_rows_lora2(const void* X, const void* X2, int64_t ldx, const void* At, const void* At2, void* Q, void* Q2,
@@ -187,6 +187,8 @@ int moe_launch_padded_blocks(const void* offsets, int off64, int E, int block_m,
 int moe_launch_group_rows(const void* src, int64_t lds_, void* out, int64_t ldo, const void* pos, int pos64,
                           int fan_out, const void* coeff, int cdtype, int64_t nrows, int64_t ncols, int dtype,
                           hipStream_t stream);
+// out[i] = weights[pos[i]] as fp32
+int moe_launch_gather_scales(const void* weights, int wdtype, const void* pos, int pos64, int64_t n, float* out, hipStream_t stream);
 int moe_launch_combine_fwd(const void* y, int64_t ldy, void* out, int64_t ldo, const void* gates, int gdtype,
                            const int32_t* inv, int k, int64_t ntok, int64_t ncols, int dtype,
                            const float* extra_coef, const void* extra_rows, int64_t lde, int n_extra,

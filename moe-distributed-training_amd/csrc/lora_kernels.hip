@@ -95,16 +95,15 @@ static_assert(RL_KSTEPS == RL_WAVES, "one K step per wave and stage");
 // lanes touch different rows, which the memory pipeline handles one lane at a time.  All global loads of the loop are
 // inline assembly with explicit s_waitcnt: compiler-managed loads would wait for the prefetches queued behind them.
 // up to four jobs per launch (see unit_and_job): same row order and scaling, operands and outputs of their own
-struct RowsLoraJob { const uint16_t* X; const uint16_t* Af; uint16_t* Q; uint16_t* Qt; uint16_t* Qs; int64_t ldx, K; };   // Q, Qt, Qs: optional; Qs row-major like Q, scaled like Qt
+// Q, Qt, Qs: optional; Qs row-major like Q, scaled like Qt; pos: gathered rows (row of X = pos[m] / fan_out), or null
+struct RowsLoraJob { const uint16_t* X; const uint16_t* Af; uint16_t* Q; uint16_t* Qt; uint16_t* Qs; int64_t ldx, K; const void* pos; int fan_out; const float* qt_row_scale; };
 struct RowsLoraJobs { RowsLoraJob job[MOE_LORA_MAX_JOBS]; };
 // ROWS = 32 rows per workgroup, or 16 when a launch of 32-row tiles would leave most compute units with a single
 // workgroup (and so with too few loads in flight)
 template <int ROWS, typename Num>
 __global__ void __launch_bounds__(RL_THREADS) rows_lora_kernel(const RowsLoraJobs jobs,
-                                                               int64_t ldqt, const void* __restrict__ pos, int pos64,
-                                                               const void* __restrict__ offsets, int off64, int E,
-                                                               int fan_out, int x_grouped, float scaling,
-                                                               const float* __restrict__ qt_row_scale, int njobs)
+                                                               int64_t ldqt, int pos64, const void* __restrict__ offsets, int off64,
+                                                               int E, float scaling, int njobs)
 {
     int64_t tile_id;
     int job_id;
@@ -115,6 +114,8 @@ __global__ void __launch_bounds__(RL_THREADS) rows_lora_kernel(const RowsLoraJob
     const uint16_t* __restrict__ Af = job.Af;
     uint16_t* __restrict__ Q = job.Q;
     uint16_t* __restrict__ Qt = job.Qt;
+    const void* __restrict__ pos = job.pos;
+    const float* __restrict__ qt_row_scale = job.qt_row_scale;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     RowTile rt;
     if (!find_row_tile(offsets, off64, E, ROWS, tile_id, &rt)) return;
@@ -132,7 +133,7 @@ __global__ void __launch_bounds__(RL_THREADS) rows_lora_kernel(const RowsLoraJob
     for (int q = 0; q < PPW; ++q) {
         int64_t m = row0 + (wave * PPW + q) * 2 + (lane >> 5);
         if (m >= row1) m = row1 - 1;   // rows past the group re-read its last row
-        const int64_t in_row = x_grouped ? m : load_idx(pos, m, pos64) / fan_out;
+        const int64_t in_row = pos ? load_idx(pos, m, pos64) / job.fan_out : m;
         rowptr[q] = X + in_row * ldx;
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)LDS_PTR(smem));
@@ -434,9 +435,8 @@ int moe_launch_pack_lora_batch(const MoePackBatch& jobs, hipStream_t stream)
     return moe_launch_status();
 }
 
-int moe_launch_rows_lora_jobs(const MoeRowsLoraJob* jobs, int njobs, int64_t ldqt, const void* pos, int pos64, const void* offsets,
-                              int off64, int E, int64_t R, int fan_out, int x_grouped, float scaling, const float* qt_row_scale,
-                              hipStream_t stream, int f16)
+int moe_launch_rows_lora_jobs(const MoeRowsLoraJob* jobs, int njobs, int64_t ldqt, int pos64, const void* offsets, int off64, int E, int64_t R,
+                              float scaling, hipStream_t stream, int f16)
 {
     if (R == 0) return MOE_OK;
     if (njobs < 1 || njobs > MOE_LORA_MAX_JOBS) return MOE_ERR_UNSUPPORTED;
@@ -444,7 +444,7 @@ int moe_launch_rows_lora_jobs(const MoeRowsLoraJob* jobs, int njobs, int64_t ldq
     for (int j = 0; j < njobs; ++j) {
         const MoeRowsLoraJob& q = jobs[j];
         if (q.K % 8 != 0 || q.ldx % 8 != 0 || ((uintptr_t)q.X % 16) != 0 || ((uintptr_t)q.At % 16) != 0) return MOE_ERR_UNSUPPORTED;
-        js.job[j] = {(const uint16_t*)q.X, (const uint16_t*)q.At, (uint16_t*)q.Q, (uint16_t*)q.Qt, (uint16_t*)q.q_scaled, q.ldx, q.K};
+        js.job[j] = {(const uint16_t*)q.X, (const uint16_t*)q.At, (uint16_t*)q.Q, (uint16_t*)q.Qt, (uint16_t*)q.q_scaled, q.ldx, q.K, q.pos, q.fan_out, q.qt_row_scale};
     }
     static std::atomic<bool> attr_set[MOE_MAX_DEVICES];   // per device; forward and backward may call from different host threads
     const int dev = moe_current_device();
@@ -462,10 +462,10 @@ int moe_launch_rows_lora_jobs(const MoeRowsLoraJob* jobs, int njobs, int64_t ldq
     const int cus = moe_device_cus();
     if ((R / 32 + E) * njobs >= 3 * (int64_t)cus / 2) {
         hipLaunchKernelGGL((f16 ? rows_lora_kernel<32, NumF16> : rows_lora_kernel<32, NumBf16>), dim3(job_grid(R / 32 + E, njobs)), dim3(RL_THREADS), rl_lds(32), stream, js,
-                           ldqt, pos, pos64, offsets, off64, E, fan_out, x_grouped, scaling, qt_row_scale, njobs);
+                           ldqt, pos64, offsets, off64, E, scaling, njobs);
     } else {
         hipLaunchKernelGGL((f16 ? rows_lora_kernel<16, NumF16> : rows_lora_kernel<16, NumBf16>), dim3(job_grid(R / 16 + E, njobs)), dim3(RL_THREADS), rl_lds(16), stream, js,
-                           ldqt, pos, pos64, offsets, off64, E, fan_out, x_grouped, scaling, qt_row_scale, njobs);
+                           ldqt, pos64, offsets, off64, E, scaling, njobs);
     }
     return moe_launch_status();
 }
@@ -475,8 +475,9 @@ int moe_launch_rows_lora2(const void* X, const void* X2, int64_t ldx, const void
                           int E, int64_t R, int64_t K, int fan_out, int x_grouped, float scaling,
                           const float* qt_row_scale, hipStream_t stream, void* q_scaled, int f16)
 {
-    const MoeRowsLoraJob jobs[2] = {{X, ldx, K, At, Q, Qt, q_scaled}, {X2, ldx, K, At2, Q2, Qt2, nullptr}};
-    return moe_launch_rows_lora_jobs(jobs, X2 ? 2 : 1, ldqt, pos, pos64, offsets, off64, E, R, fan_out, x_grouped, scaling, qt_row_scale, stream, f16);
+    const void* const p = x_grouped ? nullptr : pos;
+    const MoeRowsLoraJob jobs[2] = {{X, ldx, K, p, fan_out, At, Q, Qt, q_scaled, qt_row_scale}, {X2, ldx, K, p, fan_out, At2, Q2, Qt2, nullptr, qt_row_scale}};
+    return moe_launch_rows_lora_jobs(jobs, X2 ? 2 : 1, ldqt, pos64, offsets, off64, E, R, scaling, stream, f16);
 }
 
 size_t moe_xtp_workspace_bytes(int64_t R, int E, int64_t K)

@@ -294,8 +294,8 @@ int moe_scatter2scatter(const void* X, int64_t sxm, int64_t sxk, const void* W, 
                 for (int hf = 0; hf < nh; hf += MOE_LORA_MAX_JOBS) {   // products over the same rows share a launch
                     MoeRowsLoraJob jobs[MOE_LORA_MAX_JOBS];
                     int n = 0;
-                    for (; n < MOE_LORA_MAX_JOBS && hf + n < nh; ++n) jobs[n] = {X, sxm, K, At[hf + n], Q[hf + n], nullptr, nullptr};
-                    TRY(moe_launch_rows_lora_jobs(jobs, n, 0, pos, pos64, offsets, off64, E, R, fan_out, x_grouped, scaling, nullptr, S(stream), f16));
+                    for (; n < MOE_LORA_MAX_JOBS && hf + n < nh; ++n) jobs[n] = {X, sxm, K, x_grouped ? nullptr : pos, fan_out, At[hf + n], Q[hf + n], nullptr, nullptr, nullptr};
+                    TRY(moe_launch_rows_lora_jobs(jobs, n, 0, pos64, offsets, off64, E, R, scaling, S(stream), f16));
                 }
                 p.nslab = nh; p.slab_mode = 0;
                 if (nh > 1) {   // the chunks' buffers were taken in turn: a fixed stride from one chunk to the next
@@ -367,13 +367,13 @@ int moe_group_bwd_ab(const void* DY, int64_t sdm, int64_t sdn, const void* X, in
                 const int rk = (rank - rc < 16) ? (int)(rank - rc) : 16;
                 pb.job[pb.njobs++] = {(const uint16_t*)A + rc * sar, sae, sak, sar, (uint16_t*)At[c], K, 1, rk};
                 pb.job[pb.njobs++] = {(const uint16_t*)B + rc * sbr, sbe, sbn, sbr, (uint16_t*)Bt[c], N, 1, rk};
-                rows[c] = {X, sxm, K, At[c], nullptr, Qt[c], nullptr};
-                rows[n + c] = {DY, sdm, N, Bt[c], nullptr, Pt[c], nullptr};
+                rows[c] = {X, sxm, K, nullptr, 1, At[c], nullptr, Qt[c], nullptr, nullptr};
+                rows[n + c] = {DY, sdm, N, nullptr, 1, Bt[c], nullptr, Pt[c], nullptr, nullptr};
                 xtp[c] = {X, sxm, K, nullptr, 1, Pt[c], nullptr, (uint16_t*)DA + rc * sdar, {sdae, sdak, sdar}, rk};
                 xtp[n + c] = {DY, sdm, N, nullptr, 1, Qt[c], nullptr, (uint16_t*)DB + rc * sdbr, {sdbe, sdbn, sdbr}, rk};
             }
             TRY(moe_launch_pack_lora_batch(pb, S(stream)));
-            TRY(moe_launch_rows_lora_jobs(rows, 2 * n, ldt, nullptr, 0, offsets, off64, E, R, 1, 1, scaling, nullptr, S(stream), f16));
+            TRY(moe_launch_rows_lora_jobs(rows, 2 * n, ldt, 0, offsets, off64, E, R, scaling, S(stream), f16));
             TRY(moe_launch_xtp_jobs(xtp, 2 * n, 0, ldt, offsets, off64, E, R, 1.f, xw, xb, S(stream), f16));
         }
         return MOE_OK;
@@ -390,6 +390,104 @@ int moe_group_bwd_ab(const void* DY, int64_t sdm, int64_t sdn, const void* X, in
     TRY(moe_launch_generic_xty(X, sxm, sxk, P, rank, 1, DA, sdae, sdak, sdar, offsets, off64, E, K, rank, scaling, dtype, S(stream)));
     TRY(moe_launch_generic_xty(Q, rank, 1, DY, sdm, sdn, DB, sdbe, sdbr, sdbn, offsets, off64, E, rank, N, scaling, dtype, S(stream)));
     return MOE_OK;
+}
+
+// Backward of a projection with adapters whose rows are gathered on both sides: the gradients of the adapters and the rows of dX without
+// the gathered copies of dY and X that moe_group_bwd_ab and moe_scatter2scatter read, with one packing and one pass over the rows instead of
+// two (8 experts, 1500 tokens, top-2, 4096 x 4096, rank 32: the launches between the gate gradients and the dX product 87 us, 64 so; forward and backward 325 -> 286).  dY's rows
+// enter unscaled; their gate weights (row_scale) multiply fp32 sums.
+static const int LINEAR_BWD_MAX_CHUNKS = MOE_MAX_SLABS;   // 16-wide rank chunks: the dX launch takes them as slabs given by pointer
+
+// The adapter gradients' partials lie where the dX launch exchanges its K-split tiles afterwards (behind the counters, which are cleared before either)
+static inline size_t linear_bwd_counter_bytes() { return al((size_t)moe_gemm_num_counters() * sizeof(int)); }
+static inline size_t linear_bwd_xtp_bytes(int64_t R, int E, int64_t K, int64_t N, int rank) { return (size_t)(rank > 16 ? 4 : 2) * moe_xtp_workspace_bytes(R, E, K > N ? K : N); }
+static inline size_t linear_bwd_shared_bytes(int64_t R, int E, int64_t K, int64_t N, int rank)
+{
+    const size_t sk = moe_gemm_sk_bytes(R, E, K), x = linear_bwd_counter_bytes() + linear_bwd_xtp_bytes(R, E, K, N, rank);
+    return sk > x ? sk : x;
+}
+
+size_t moe_linear_lora_bwd_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank)
+{
+    const size_t C = (size_t)((rank > 0 ? rank : 1) + 15) / 16;
+    return al(linear_bwd_shared_bytes(R, E, K, N, rank)) + C * (2 * pack_bytes(E, K) + pack_bytes(E, N) + 3 * q_bytes(R)) + 256;
+}
+
+int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const float* row_scale, const void* x, int64_t ldx, int fan_out,
+                        const void* W, int64_t swe, int64_t swk, int64_t swn, const void* A, int64_t sae, int64_t sak, int64_t sar,
+                        const void* B, int64_t sbe, int64_t sbr, int64_t sbn, int rank, float scaling, void* DA, int64_t sdae, int64_t sdak,
+                        int64_t sdar, void* DB, int64_t sdbe, int64_t sdbr, int64_t sdbn, void* dx_rows, int64_t lddx, const void* pos,
+                        int pos64, const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int dtype, void* workspace,
+                        size_t workspace_bytes, void* stream)
+{
+    if (!dout || !x || !W || !A || !B || !DA || !DB || !dx_rows || !pos || !offsets || rank < 1 || E < 1 || R < 0 || K < 1 || N < 1 || fan_out < 1 || dout_fan_out < 1)
+        return MOE_ERR_BAD_ARG;
+    const int C = (rank + 15) / 16;
+    const bool nt = swn == 1, nn = swk == 1 && !nt;   // of the transposed weights (E, N, K): contraction-contiguous, output-contiguous
+    if (!bwd_ab_fast(K, N, rank, dtype, ldd, 1, ldx, 1, dout, x) || C > LINEAR_BWD_MAX_CHUNKS || !(nt || nn) || R == 0) return MOE_ERR_UNSUPPORTED;
+    const int f16 = dtype == MOE_F16;
+    MoeGemmParams p = {};
+    p.X[0] = (const uint16_t*)dout; p.ldx = ldd; p.nseg = 1;
+    p.W[0] = (const uint16_t*)W; p.swe = swe; p.ldw = nt ? swk : swn; p.nn = nn ? 1 : 0;
+    p.Y[0] = (uint16_t*)dx_rows; p.ldy = lddx; p.row_scale = row_scale;
+    p.pos = pos; p.pos64 = pos64; p.offsets = offsets; p.off64 = off64;
+    p.E = E; p.K = N; p.N = K; p.fan_out = dout_fan_out; p.x_grouped = 0; p.y_grouped = 0;
+    p.epi = MOE_EPI_STORE; p.f16 = f16; p.nslab = C; p.slab_mode = 0;
+    if (!moe_gemm_mfma_supported(p, R)) return MOE_ERR_UNSUPPORTED;
+    if (!workspace || workspace_bytes < moe_linear_lora_bwd_workspace_bytes(R, E, K, N, rank)) return MOE_ERR_WORKSPACE;
+    Bump ws(workspace, workspace_bytes);
+    uint8_t* shared = (uint8_t*)ws.take(linear_bwd_shared_bytes(R, E, K, N, rank));
+    moe_gemm_sk_attach(p, shared, R, E, K);
+    p.counters_clean = 1;   // by the packing
+    void* xw = shared + linear_bwd_counter_bytes();
+    const size_t xb = linear_bwd_xtp_bytes(R, E, K, N, rank);
+    const int64_t ldt = pad_rows(R);
+    hipStream_t st = S(stream);
+    void *At[LINEAR_BWD_MAX_CHUNKS] = {}, *Bt[LINEAR_BWD_MAX_CHUNKS] = {}, *LB[LINEAR_BWD_MAX_CHUNKS] = {}, *P[LINEAR_BWD_MAX_CHUNKS] = {}, *Pt[LINEAR_BWD_MAX_CHUNKS] = {}, *Qt[LINEAR_BWD_MAX_CHUNKS] = {};
+    for (int c = 0; c < C; ++c) {
+        At[c] = ws.take(pack_bytes(E, K)); Bt[c] = ws.take(pack_bytes(E, N)); LB[c] = ws.take(pack_bytes(E, K));
+        P[c] = ws.take(q_bytes(R)); Pt[c] = ws.take(q_bytes(R)); Qt[c] = ws.take(q_bytes(R));
+        p.Q[c] = (const uint16_t*)P[c]; p.LB[c] = (const uint16_t*)LB[c];
+    }
+    if (!shared || !Qt[C - 1]) return MOE_ERR_WORKSPACE;
+    auto chunk_rank = [&](int c) { return rank - 16 * c < 16 ? rank - 16 * c : 16; };
+    static_assert(3 * LINEAR_BWD_MAX_CHUNKS <= MOE_PACK_MAX_JOBS, "one packing launch");
+    MoePackBatch pb = {};
+    pb.E = E; pb.zero_ptr = p.sk_counters; pb.zero_n = moe_gemm_num_counters();
+    for (int c = 0; c < C; ++c) {
+        const uint16_t *a = (const uint16_t*)A + 16 * c * sar, *b = (const uint16_t*)B + 16 * c * sbr;
+        pb.job[pb.njobs++] = {a, sae, sak, sar, (uint16_t*)At[c], K, 1, chunk_rank(c)};
+        pb.job[pb.njobs++] = {b, sbe, sbn, sbr, (uint16_t*)Bt[c], N, 1, chunk_rank(c)};
+        pb.job[pb.njobs++] = {a, sae, sak, sar, (uint16_t*)LB[c], K, 0, chunk_rank(c)};
+    }
+    TRY(moe_launch_pack_lora_batch(pb, st));
+    for (int c0 = 0; c0 < C; c0 += 2) {   // jobs over X first, then those over dY: neighbours share their rows in L2
+        const int n = C - c0 > 1 ? 2 : 1;
+        MoeRowsLoraJob rows[MOE_LORA_MAX_JOBS];
+        for (int i = 0; i < n; ++i) {
+            const int c = c0 + i;
+            rows[i] = {x, ldx, K, pos, fan_out, At[c], nullptr, Qt[c], nullptr, row_scale};               // (row_scale X A)^T: dB's factor
+            rows[n + i] = {dout, ldd, N, pos, dout_fan_out, Bt[c], P[c], Pt[c], nullptr, row_scale};      // dY B^T: dX's slab; (row_scale dY B^T)^T: dA's factor
+        }
+        TRY(moe_launch_rows_lora_jobs(rows, 2 * n, ldt, pos64, offsets, off64, E, R, scaling, st, f16));
+    }
+    for (int c0 = 0; c0 < C; c0 += 2) {
+        const int n = C - c0 > 1 ? 2 : 1;
+        MoeXtpJob xtp[MOE_LORA_MAX_JOBS];
+        for (int i = 0; i < n; ++i) {
+            const int c = c0 + i;
+            xtp[i] = {x, ldx, K, pos, fan_out, Pt[c], nullptr, (uint16_t*)DA + 16 * c * sdar, {sdae, sdak, sdar}, chunk_rank(c)};
+            xtp[n + i] = {dout, ldd, N, pos, dout_fan_out, Qt[c], nullptr, (uint16_t*)DB + 16 * c * sdbr, {sdbe, sdbn, sdbr}, chunk_rank(c)};
+        }
+        TRY(moe_launch_xtp_jobs(xtp, 2 * n, pos64, ldt, offsets, off64, E, R, 1.f, xw, xb, st, f16));
+    }
+    return moe_launch_gemm_mfma(p, R, st);
+}
+
+int moe_gather_scales(const void* weights, int wdtype, const void* pos, int pos64, int64_t n, float* out, void* stream)
+{
+    if (n < 0 || (n > 0 && (!weights || !pos || !out))) return MOE_ERR_BAD_ARG;
+    return moe_launch_gather_scales(weights, wdtype, pos, pos64, n, out, S(stream));
 }
 
 int moe_group_bwd_w(const void* DY, int64_t sdm, int64_t sdn, const void* X, int64_t sxm, int64_t sxk, void* DW,

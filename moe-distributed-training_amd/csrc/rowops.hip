@@ -78,6 +78,13 @@ __global__ void __launch_bounds__(ROW_THREADS) group_rows_kernel(const T* __rest
     }
 }
 
+// out[i] = weights[pos[i]] as fp32: the row scales of a sorted order (a thread per row; through group_rows a workgroup per row, 6 us for 8192 rows)
+__global__ void gather_scales_kernel(const void* __restrict__ weights, int wdtype, const void* __restrict__ pos, int pos64, int64_t n, float* __restrict__ out)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = load_gate(weights, load_idx(pos, i, pos64), wdtype);
+}
+
 // out[t][:] = sum_j gates[t*k+j] * y[row(t,j)][:],  row(t,j) = inv ? inv[t*k+j] : t*k+j.   gates may be null (=1).
 template <typename T>
 __global__ void __launch_bounds__(ROW_THREADS) combine_fwd_kernel(const T* __restrict__ y, int64_t ldy,
@@ -298,6 +305,14 @@ int moe_launch_group_rows(const void* src, int64_t lds_, void* out, int64_t ldo,
         hipLaunchKernelGGL((group_rows_kernel<T>), dim3((unsigned)nrows), dim3(ROW_THREADS), 0, stream, (const T*)src,
                            lds_, (T*)out, ldo, pos, pos64, fan_out, coeff, cdtype, nrows, ncols, vo);
     });
+    return moe_launch_status();
+}
+
+int moe_launch_gather_scales(const void* weights, int wdtype, const void* pos, int pos64, int64_t n, float* out, hipStream_t stream)
+{
+    if (wdtype != MOE_BF16 && wdtype != MOE_F16 && wdtype != MOE_F32) return MOE_ERR_BAD_ARG;
+    if (n == 0) return MOE_OK;
+    hipLaunchKernelGGL(gather_scales_kernel, dim3((unsigned)((n + ROW_THREADS - 1) / ROW_THREADS)), dim3(ROW_THREADS), 0, stream, weights, wdtype, pos, pos64, n, out);
     return moe_launch_status();
 }
 

@@ -571,7 +571,7 @@ def test_generic_kernels_at_the_edges_of_a_contraction_step(dev, oracle, dtype, 
     X, W = torch.randn(R, K).to(dtype), (torch.randn(E, K, N) * 0.3).to(dtype)
     A, B = (torch.randn(E, K, r) * 0.3).to(dtype), (torch.randn(E, r, N) * 0.3).to(dtype)
     Wd = W.permute(0, 2, 1).contiguous().to(dev).permute(0, 2, 1) if layout == "k_contiguous" else W.to(dev)
-    y = ops.scatter2scatter_lora(X.to(dev), Wd, A.to(dev), B.to(dev), 2.0, sei.to(dev), ssi.to(dev), 1)
+    y = ops.scatter2scatter_lora(X.to(dev), Wd, A.to(dev), B.to(dev), 2.0, sei.to(dev), ssi.to(dev), 1, None)
     ref = oracle.scatter2scatter_lora(X, W, A, B, 2.0, sei, ssi, 1)
     assert rel(y, ref) < TOL[dtype]
     dy = torch.randn(R, N).to(dtype)
@@ -579,3 +579,34 @@ def test_generic_kernels_at_the_edges_of_a_contraction_step(dev, oracle, dtype, 
     at = torch.tensor([0] + counts).cumsum(0)
     want = torch.stack([X[a:b].float().t() @ dy[a:b].float() for a, b in zip(at[:-1], at[1:])])
     check_expert_grads(dw, want, TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,E,k,K,N,r,gates,layout", [
+    (333, 4, 2, 256, 384, 16, True, "k_contiguous"), (100, 3, 1, 64, 96, 8, False, "k_contiguous"), (257, 5, 3, 96, 160, 24, True, "n_contiguous"),
+    (64, 2, 2, 128, 64, 33, False, "n_contiguous"), (700, 6, 4, 320, 64, 64, True, "k_contiguous"), (90, 3, 2, 64, 64, 65, True, "k_contiguous"),
+    (40, 3, 2, 48, 64, 16, True, "k_contiguous"), (50, 2, 2, 64, 32, 16, False, "k_contiguous")])
+def test_projection_backward_on_gathered_rows(dev, oracle, dtype, T, E, k, K, N, r, gates, layout):
+    """The backward pass that reads dY and X where they lie, on both sides of its rule (ranks to 64, contractions of at least 64 and multiples of
+    32; the last three take the route over gathered copies): adapter gradients, dX and the gates' against the fp32 oracle."""
+    import moe_distributed_training_amd as moe
+    torch.manual_seed(T + r)
+    _, sei, ssi, eo = _routing(oracle, T, E, k, T, skew=True)
+    X = torch.randn(T, K).to(dtype)
+    W = (torch.randn(E, N, K) * 0.05).to(dtype).permute(0, 2, 1) if layout == "k_contiguous" else (torch.randn(E, K, N) * 0.05).to(dtype)
+    A, B = (torch.randn(E, K, r) * 0.05).to(dtype), (torch.randn(E, r, N) * 0.05).to(dtype)
+    G = torch.rand(T, k).to(dtype) if gates else None
+    dY = torch.randn(T if gates else T * k, N).to(dtype)
+    f32 = lambda t: None if t is None else t.float().clone().requires_grad_(True)
+    Xo, Ao, Bo, Go = f32(X), f32(A), f32(B), f32(G)
+    oracle.parallel_linear_lora(Xo, W.float(), Ao, Bo, r, 32.0, k, sei, ssi, None, eo, Go, False, False).backward(dY.float())
+    d = lambda t: None if t is None else t.detach().to(dev).requires_grad_(True)
+    Xd, Ad, Bd, Gd = d(X), d(A), d(B), d(G)
+    Wd = W.permute(0, 2, 1).contiguous().to(dev).permute(0, 2, 1) if layout == "k_contiguous" else W.to(dev)
+    pb, eod = moe.padded_block_indices(sei.to(dev), E)
+    moe.parallel_linear_lora(Xd, Wd, Ad, Bd, r, 32.0, k, sei.to(dev), ssi.to(dev), pb, eod, Gd, False, False).backward(dY.to(dev))
+    tol = TOL[dtype] * 1.5
+    assert rel(Xd.grad, Xo.grad) < tol
+    check_expert_grads(Ad.grad, Ao.grad, tol, "dA"); check_expert_grads(Bd.grad, Bo.grad, tol, "dB")
+    if gates:
+        assert rel(Gd.grad, Go.grad) < tol
