@@ -610,3 +610,28 @@ def test_projection_backward_on_gathered_rows(dev, oracle, dtype, T, E, k, K, N,
     check_expert_grads(Ad.grad, Ao.grad, tol, "dA"); check_expert_grads(Bd.grad, Bo.grad, tol, "dB")
     if gates:
         assert rel(Gd.grad, Go.grad) < tol
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("k,n_extra,cols", [(1, 1, 64), (2, 8, 4096), (3, 9, 72), (4, 64, 1032), (8, 33, 2048), (0, 16, 256), (2, 1025, 64)])
+def test_combine_with_a_dense_tail(dev, dtype, k, n_extra, cols):
+    """The fan-out sum with the router's input gradient behind it, on the matrix instructions (16 tokens and 128 columns per wave; three tokens
+    more than a whole number of groups, columns and tail rows that fill neither): against 64 bits, and a token's sum does not depend on the
+    tokens around it."""
+    from moe_distributed_training_amd._lib import lib, check, ptr, stream_ptr, dtype_code
+    T = 4 * torch.cuda.get_device_properties(dev).multi_processor_count + 3
+    g = torch.Generator(device=dev).manual_seed(k + n_extra)
+    y = torch.randn(max(1, T * k), cols, generator=g, device=dev).to(dtype)
+    rows, coef = torch.randn(n_extra, cols, generator=g, device=dev).to(dtype), torch.randn(T, n_extra, generator=g, device=dev)
+
+    def run(t0, t1):
+        out = torch.empty(t1 - t0, cols, dtype=dtype, device=dev)
+        c = coef[t0:t1].contiguous()
+        check(lib.moe_combine(ptr(y[t0 * k:]) if k else None, cols, ptr(out), cols, None, 0, None, k, t1 - t0, cols, dtype_code(y), ptr(c), ptr(rows), cols,
+                              n_extra, stream_ptr(dev)), "moe_combine")
+        return out
+    whole = run(0, T)
+    step = 200
+    assert torch.equal(whole, torch.cat([run(t, min(T, t + step)) for t in range(0, T, step)]))
+    want = coef.double() @ rows.double() + (y.double().view(T, k, cols).sum(1) if k else 0.0)
+    assert rel(whole, want) < TOL[dtype]
+
+
