@@ -132,7 +132,10 @@ __global__ void __launch_bounds__(ROW_THREADS) combine_fwd_batched_kernel(const 
                                                                           T* __restrict__ out, int64_t ldo,
                                                                           const void* __restrict__ gates, int gdtype,
                                                                           const int32_t* __restrict__ inv, int k,
-                                                                          int64_t ncols)
+                                                                          int64_t ncols,
+                                                                          const float* __restrict__ extra_coef,
+                                                                          const T* __restrict__ extra_rows, int64_t lde,
+                                                                          int n_extra)
 {
     constexpr int N = Vec8<T>::N;
     const int64_t t = blockIdx.x;
@@ -159,6 +162,13 @@ __global__ void __launch_bounds__(ROW_THREADS) combine_fwd_batched_kernel(const 
 #pragma unroll
             for (int u = 0; u < N; ++u) acc[u] = fmaf(g[j], Elem<T>::ld(e + u), acc[u]);
         }
+        for (int e = 0; e < n_extra; ++e) {
+            const float ge = extra_coef[t * n_extra + e];
+            float v[N];
+            load_vec<T>(extra_rows + (int64_t)e * lde + c0, v, true, N);
+#pragma unroll
+            for (int u = 0; u < N; ++u) acc[u] = fmaf(ge, v[u], acc[u]);
+        }
         store_vec<T>(out + t * ldo + c0, acc, true, N);
     }
 }
@@ -184,10 +194,10 @@ template <typename T> struct Raw8 {
 // g, which are the second operand of eight v_mfma_f32_16x16x4) and one coefficient (token i).  Accumulator u holds column 8 i + u of
 // tokens 4 g .. 4 g + 3; it starts with their k rows' sum.  fp32 products and sums as before, rows first, then the tail in order.
 // One token per workgroup fetched and unpacked the whole tail for every token, one row after the other: 2048 tokens, top-8, d=2048, 64 experts
-// 51 us, this 34; 4096 tokens, top-2, d=4096, 8 experts 27.4 and 28.5, where the rows' traffic is all that counts.
+// 51 us, this 33; 4096 tokens, top-2, d=4096, 8 experts 27.4 and 27, where the rows' traffic is all that counts.
 constexpr int CT_TOKENS = 16, CT_WCOLS = 128, CT_COLS = ROW_THREADS / 64 * CT_WCOLS;
 template <typename T, int KMAX>
-__global__ void __launch_bounds__(ROW_THREADS) combine_tail_kernel(const T* __restrict__ y, int64_t ldy, T* __restrict__ out, int64_t ldo,
+__global__ void __launch_bounds__(ROW_THREADS, 4) combine_tail_kernel(const T* __restrict__ y, int64_t ldy, T* __restrict__ out, int64_t ldo,
                                                                    const void* __restrict__ gates, int gdtype, const int32_t* __restrict__ inv,
                                                                    int k, int64_t ntok, int64_t ncols, const float* __restrict__ extra_coef,
                                                                    const T* __restrict__ extra_rows, int64_t lde, int n_extra)
@@ -467,13 +477,17 @@ int moe_launch_combine_fwd(const void* y, int64_t ldy, void* out, int64_t ldo, c
     if (ntok == 0 || ncols == 0) return MOE_OK;
     MOE_DISPATCH_DTYPE(dtype, {
         const int vo = vec_aligned<T>(y, ldy) && vec_aligned<T>(out, ldo) && (!extra_rows || vec_aligned<T>(extra_rows, lde));
-        if (vo && n_extra > 0 && k <= 8 && ncols % 8 == 0 && (ncols + CT_COLS - 1) / CT_COLS <= 65535) {
+        // A tail of more than eight rows always, a shorter one where 16 tokens x 128 columns per wave give every SIMD a wave: below that one token
+        // per workgroup is done sooner (512 tokens, d=256, 8 experts: 4.0 us against 5.5; 64 experts there would take it 50).
+        const int64_t tail_waves = (ntok + CT_TOKENS - 1) / CT_TOKENS * ((ncols + CT_WCOLS - 1) / CT_WCOLS);
+        if (vo && n_extra > 0 && k <= 8 && ncols % 8 == 0 && (n_extra > 8 || k == 0 || tail_waves >= 4 * (int64_t)moe_device_cus()) && (ncols + CT_COLS - 1) / CT_COLS <= 65535) {
             auto kern = k <= 2 ? combine_tail_kernel<T, 2> : (k <= 4 ? combine_tail_kernel<T, 4> : combine_tail_kernel<T, 8>);
             hipLaunchKernelGGL(kern, dim3((unsigned)((ntok + CT_TOKENS - 1) / CT_TOKENS), (unsigned)((ncols + CT_COLS - 1) / CT_COLS)), dim3(ROW_THREADS), 0, stream,
                                (const T*)y, ldy, (T*)out, ldo, gates, gdtype, inv, k, ntok, ncols, extra_coef, (const T*)extra_rows, lde, n_extra);
-        } else if (vo && n_extra == 0 && k >= 1 && k <= 8 && ncols % Vec8<T>::N == 0) {
+        } else if (vo && k >= 1 && k <= 8 && ncols % Vec8<T>::N == 0) {
             auto kern = k <= 2 ? combine_fwd_batched_kernel<T, 2> : (k <= 4 ? combine_fwd_batched_kernel<T, 4> : combine_fwd_batched_kernel<T, 8>);
-            hipLaunchKernelGGL(kern, dim3((unsigned)ntok), dim3(ROW_THREADS), 0, stream, (const T*)y, ldy, (T*)out, ldo, gates, gdtype, inv, k, ncols);
+            hipLaunchKernelGGL(kern, dim3((unsigned)ntok), dim3(ROW_THREADS), 0, stream, (const T*)y, ldy, (T*)out, ldo, gates, gdtype, inv, k, ncols,
+                               extra_coef, (const T*)extra_rows, lde, n_extra);
         } else
         hipLaunchKernelGGL((combine_fwd_kernel<T>), dim3((unsigned)ntok), dim3(ROW_THREADS), 0, stream, (const T*)y,
                            ldy, (T*)out, ldo, gates, gdtype, inv, k, ncols, vo, extra_coef, (const T*)extra_rows, lde,
