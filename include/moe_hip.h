@@ -198,6 +198,12 @@ int moe_combine(const void* y, int64_t ldy, void* out, int64_t ldo, const void* 
 int moe_combine_dgates(const void* y, int64_t ldy, const void* dout, int64_t ldd, void* dgates, int gates_dtype,
                        const int32_t* inv, int k, int64_t ntok, int64_t ncols, int dtype, void* stream);
 
+/* fp32: h[m] = silu(x_m W_gate[e]) * (x_m W_up[e]) over expert-grouped positions m (x_m = row pos[m] / fan_out of x), bit for bit the two
+ * moe_scatter2scatter calls without adapters followed by moe_swiglu; MOE_ERR_UNSUPPORTED for other types (whose gate and up are rounded
+ * on the way). */
+int moe_swiglu_pair(const void* x, int64_t sxm, int64_t sxk, const void* w_gate, const void* w_up, int64_t swe, int64_t swk, int64_t swn,
+                    void* h, int64_t ldh, const void* pos, int pos64, const void* offsets, int off64, int E, int64_t R, int64_t K,
+                    int64_t N, int fan_out, int dtype, void* stream);
 /* ---- SwiGLU: F.silu(h1) * h3 at config_utils.py:151 and its autograd backward -------------------------------- */
 int moe_swiglu(const void* gate, const void* up, void* h, int64_t n, int dtype, void* stream);
 int moe_swiglu_bwd(const void* gate, const void* up, const void* dh, void* dgate, void* dup, int64_t n, int dtype,

@@ -52,6 +52,7 @@ _SIGNATURES = {
     "moe_group_rows": ("i", "pl" + "pl" + "pi" + "i" + "pi" + "ll" + "i" + "p"),
     "moe_combine": ("i", "pl" + "pl" + "pi" + "p" + "i" + "ll" + "i" + "p" + "pl" + "i" + "p"),
     "moe_combine_dgates": ("i", "pl" + "pl" + "pi" + "p" + "i" + "ll" + "i" + "p"),
+    "moe_swiglu_pair": ("i", "pllpplllplpipiilllii" + "p"),
     "moe_swiglu": ("i", "ppplip"),
     "moe_swiglu_bwd": ("i", "ppppplip"),
     "moe_mlp_workspace_bytes": ("z", "lilli"),

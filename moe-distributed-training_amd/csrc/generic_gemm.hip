@@ -13,11 +13,12 @@ constexpr int GT = 16;   // tile edge; workgroup is GT x GT threads
 constexpr int GK = 64;
 constexpr int GPT = GT * GK / (GT * GT);   // elements of an operand tile per thread
 
+// PAIR: two weights without adapters (gate, up) and Y = silu(gate) * up, the arithmetic of the separate launches (fp32: bit for bit).
 // Y[out_row(m)][n] = sum_k X[in_row(m)][k] * (W[e][k][n] + scaling * sum_r A[e][k][r] * B[e][r][n])
 // m runs over sorted positions; tiles of GT rows never straddle experts (find_row_tile on the offsets).
-template <typename T>
+template <typename T, bool PAIR>
 __global__ void __launch_bounds__(GT * GT) generic_grouped_gemm_kernel(
-    const T* __restrict__ X, int64_t sxm, int64_t sxk, const T* __restrict__ W, int64_t swe, int64_t swk, int64_t swn,
+    const T* __restrict__ X, int64_t sxm, int64_t sxk, const T* __restrict__ W, const T* __restrict__ W_up, int64_t swe, int64_t swk, int64_t swn,
     const T* __restrict__ A, int64_t sae, int64_t sak, int64_t sar, const T* __restrict__ B, int64_t sbe, int64_t sbr,
     int64_t sbn, T* __restrict__ Y, int64_t sym, int64_t syn, const void* __restrict__ pos, int pos64,
     const void* __restrict__ offsets, int off64, int E, int64_t K, int64_t N, int rank, int fan_out, float scaling,
@@ -25,6 +26,7 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_gemm_kernel(
 {
     __shared__ float xs[GT][GK + 1];   // [row][k]
     __shared__ float ws[GK][GT + 1];   // [k][n]
+    __shared__ float wu[PAIR ? GK : 1][GT + 1];
     __shared__ int64_t s_in[GT];
     RowTile rt;
     if (!find_row_tile(offsets, off64, E, GT, blockIdx.x, &rt)) return;
@@ -45,39 +47,48 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_gemm_kernel(
     // Which elements of an operand tile a thread loads: neighbours along the operand's own contiguous direction.
     const int tid = threadIdx.x, nrows = (int)(rt.row1 - rt.row0);
     const bool w_along_k = swk == 1;
-    auto load = [&](int64_t k0, float* xv, float* wv) {
+    const T* Wu = PAIR ? W_up + (int64_t)rt.expert * swe : nullptr;
+    auto load = [&](int64_t k0, float* xv, float* wv, float* uv) {
 #pragma unroll
         for (int i = 0; i < GPT; ++i) {
             const int xr = tid / GK + i * (GT * GT / GK);
             const int64_t xk = k0 + tid % GK;
             xv[i] = (xr < nrows && xk < K) ? Elem<T>::ld(X + s_in[xr] * sxm + xk * sxk) : 0.f;
             const int64_t k = k0 + (w_along_k ? tid % GK : tid / GT + i * GT), n = n0 + (w_along_k ? tid / GK + i * (GT * GT / GK) : tid % GT);
-            float w = 0.f;
+            float w = 0.f, u = 0.f;
             if (k < K && n < N) {   // effective weight
                 w = Elem<T>::ld(We + k * swk + n * swn);
-                if (Ae) {
+                if (PAIR) u = Elem<T>::ld(Wu + k * swk + n * swn);
+                else if (Ae) {
                     float l = 0.f;
                     for (int r = 0; r < rank; ++r) l = fmaf(Elem<T>::ld(Ae + k * sak + r * sar), Elem<T>::ld(Be + r * sbr + n * sbn), l);
                     w = fmaf(scaling, l, w);
                 }
             }
             wv[i] = w;
+            uv[i] = u;
         }
     };
-    float acc = 0.f, xv[GPT], wv[GPT];
-    load(0, xv, wv);
+    float acc = 0.f, acc_up = 0.f, xv[GPT], wv[GPT], uv[GPT];
+    load(0, xv, wv, uv);
     for (int64_t k0 = 0; k0 < K; k0 += GK) {
 #pragma unroll
         for (int i = 0; i < GPT; ++i) {
             xs[tid / GK + i * (GT * GT / GK)][tid % GK] = xv[i];
-            ws[w_along_k ? tid % GK : tid / GT + i * GT][w_along_k ? tid / GK + i * (GT * GT / GK) : tid % GT] = wv[i];
+            const int wk = w_along_k ? tid % GK : tid / GT + i * GT, wn = w_along_k ? tid / GK + i * (GT * GT / GK) : tid % GT;
+            ws[wk][wn] = wv[i];
+            if (PAIR) wu[wk][wn] = uv[i];
         }
         __syncthreads();
-        if (k0 + GK < K) load(k0 + GK, xv, wv);
+        if (k0 + GK < K) load(k0 + GK, xv, wv, uv);
 #pragma unroll
-        for (int kk = 0; kk < GK; ++kk) acc = fmaf(xs[ty][kk], ws[kk][tx], acc);
+        for (int kk = 0; kk < GK; ++kk) {
+            acc = fmaf(xs[ty][kk], ws[kk][tx], acc);
+            if (PAIR) acc_up = fmaf(xs[ty][kk], wu[kk][tx], acc_up);
+        }
         __syncthreads();
     }
+    if (PAIR) acc = acc / (1.f + __expf(-acc)) * acc_up;   // as swiglu_fwd_kernel
     if (mval && n0 + tx < N) Elem<T>::st(Y + out_row * sym + (n0 + tx) * syn, acc);
 }
 
@@ -131,10 +142,21 @@ int moe_launch_generic_gemm(const void* X, int64_t sxm, int64_t sxk, const void*
     if (R == 0 || N == 0) return MOE_OK;
     const int64_t mtiles = R / GT + E;  // upper bound on sum_e ceil(c_e / GT)
     dim3 grid((unsigned)mtiles, (unsigned)((N + GT - 1) / GT));
-    MOE_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((generic_grouped_gemm_kernel<T>), grid, dim3(GT * GT), 0, stream,
-                                                 (const T*)X, sxm, sxk, (const T*)W, swe, swk, swn, (const T*)A, sae, sak,
+    MOE_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((generic_grouped_gemm_kernel<T, false>), grid, dim3(GT * GT), 0, stream,
+                                                 (const T*)X, sxm, sxk, (const T*)W, (const T*)nullptr, swe, swk, swn, (const T*)A, sae, sak,
                                                  sar, (const T*)B, sbe, sbr, sbn, (T*)Y, sym, syn, pos, pos64, offsets,
                                                  off64, E, K, N, rank, fan_out, scaling, x_grouped, y_grouped));
+    return moe_launch_status();
+}
+
+int moe_launch_generic_swiglu_pair(const float* X, int64_t sxm, int64_t sxk, const float* W_gate, const float* W_up, int64_t swe, int64_t swk,
+                                   int64_t swn, float* H, int64_t ldh, const void* pos, int pos64, const void* offsets, int off64, int E, int64_t R,
+                                   int64_t K, int64_t N, int fan_out, hipStream_t stream)
+{
+    if (R == 0 || N == 0) return MOE_OK;
+    dim3 grid((unsigned)(R / GT + E), (unsigned)((N + GT - 1) / GT));
+    hipLaunchKernelGGL((generic_grouped_gemm_kernel<float, true>), grid, dim3(GT * GT), 0, stream, X, sxm, sxk, W_gate, W_up, swe, swk, swn, (const float*)nullptr,
+                       0, 0, 0, (const float*)nullptr, 0, 0, 0, H, ldh, 1, pos, pos64, offsets, off64, E, K, N, 0, fan_out, 0.f, 0, 1);
     return moe_launch_status();
 }
 

@@ -103,6 +103,10 @@ int moe_launch_generic_gemm(const void* X, int64_t sxm, int64_t sxk, const void*
                             int64_t sbe, int64_t sbr, int64_t sbn, void* Y, int64_t sym, int64_t syn, const void* pos,
                             int pos64, const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int rank,
                             int fan_out, float scaling, int x_grouped, int y_grouped, int dtype, hipStream_t stream);
+// fp32: H[m] = silu(X_m W_gate) * (X_m W_up) for grouped rows m of gathered X rows, without adapters
+int moe_launch_generic_swiglu_pair(const float* X, int64_t sxm, int64_t sxk, const float* W_gate, const float* W_up, int64_t swe, int64_t swk,
+                                   int64_t swn, float* H, int64_t ldh, const void* pos, int pos64, const void* offsets, int off64, int E, int64_t R,
+                                   int64_t K, int64_t N, int fan_out, hipStream_t stream);
 int moe_launch_generic_xty(const void* X, int64_t sxm, int64_t sxk, const void* Yp, int64_t sym, int64_t syn, void* O,
                            int64_t soe, int64_t sok, int64_t son, const void* offsets, int off64, int E, int64_t K,
                            int64_t N, float scale, int dtype, hipStream_t stream);

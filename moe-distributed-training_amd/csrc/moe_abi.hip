@@ -543,6 +543,16 @@ int moe_combine_dgates(const void* y, int64_t ldy, const void* dout, int64_t ldd
     return moe_launch_combine_dgates(y, ldy, dout, ldd, dgates, gates_dtype, inv, k, ntok, ncols, dtype, st);
 }
 
+int moe_swiglu_pair(const void* x, int64_t sxm, int64_t sxk, const void* w_gate, const void* w_up, int64_t swe, int64_t swk, int64_t swn, void* h,
+                    int64_t ldh, const void* pos, int pos64, const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int fan_out,
+                    int dtype, void* stream)
+{
+    if (dtype != MOE_F32) return MOE_ERR_UNSUPPORTED;
+    if (!x || !w_gate || !w_up || !h || !pos || !offsets || E < 1 || R < 0 || K < 1 || N < 1 || fan_out < 1) return MOE_ERR_BAD_ARG;
+    return moe_launch_generic_swiglu_pair((const float*)x, sxm, sxk, (const float*)w_gate, (const float*)w_up, swe, swk, swn, (float*)h, ldh, pos, pos64, offsets,
+                                          off64, E, R, K, N, fan_out, S(stream));
+}
+
 int moe_swiglu(const void* gate, const void* up, void* h, int64_t n, int dtype, void* stream)
 {
     if (n > 0 && (!gate || !up || !h)) return MOE_ERR_BAD_ARG;

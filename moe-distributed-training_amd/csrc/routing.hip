@@ -56,12 +56,20 @@ __device__ __forceinline__ void butterfly_sums(float* v, int lane)
 // hidden dimension 8 elements per lane at a time: one wave per expert group keeps every SIMD busy where one wave for all
 // groups did not (2048 tokens x 64 experts x 2048 columns: 83 -> 28 us; bound by the vector ALUs, one FMA per token,
 // expert and column plus the unpacking).  The order of the additions of a logit depends neither on TOKENS nor on the grid.
-template <typename T, int TOKENS>
+// TOPK: up to 8 experts, whose logits all lie in one wave: softmax and top-k follow in the same launch (scores .. renorm; 256 tokens fp32, 4 experts:
+// 4.4 + 3.5 us in two launches, 6.2 in one).
+constexpr int TK_LANES = 16;
+template <int PER_LANE>
+__device__ __forceinline__ void softmax_topk_token(const float* __restrict__ l, float* __restrict__ s, float* __restrict__ topw, int32_t* __restrict__ topi, int E, int k,
+                                                   int renorm, bool store);
+template <typename T, int TOKENS, bool TOPK>
 __global__ void __launch_bounds__(256) router_logits_kernel(const T* __restrict__ x, int64_t ldx,
                                                             const T* __restrict__ wg, int64_t ldw,
                                                             float* __restrict__ logits, int64_t ntok, int64_t d, int E,
-                                                            bool vec_ok)
+                                                            bool vec_ok, float* __restrict__ scores, float* __restrict__ topw,
+                                                            int32_t* __restrict__ topi, int k, int renorm)
 {
+    __shared__ float s_l[TOPK ? 4 : 1][TOKENS][ROUTER_EXPERT_GROUP];
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int64_t t0 = wave * TOKENS;
@@ -104,6 +112,18 @@ __global__ void __launch_bounds__(256) router_logits_kernel(const T* __restrict_
     const bool writer = lane % (64 / NV) == 0;
     const int i = idx / ROUTER_EXPERT_GROUP, e = e0 + idx % ROUTER_EXPERT_GROUP;
     if (writer && t0 + i < ntok && e < E) logits[(t0 + i) * E + e] = v[0];
+    if constexpr (TOPK) {
+        static_assert(TOKENS * TK_LANES <= 64, "the tokens of a wave share its lanes");
+        float (*l)[ROUTER_EXPERT_GROUP] = s_l[threadIdx.x >> 6];
+        if (writer) l[i][idx % ROUTER_EXPERT_GROUP] = v[0];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the wave's own writes, read by its other lanes
+        __builtin_amdgcn_wave_barrier();
+        const int tt = lane / TK_LANES;
+        if (tt < TOKENS) {   // whole groups of TK_LANES lanes
+            const int64_t t = t0 + tt < ntok ? t0 + tt : ntok - 1;
+            softmax_topk_token<1>(l[tt], scores + t * E, topw + t * k, topi + t * k, E, k, renorm, t0 + tt < ntok);
+        }
+    }
 }
 
 // fp32 softmax over the E logits of one token, k rounds of arg-max (the lowest expert index wins a tie), optional division
@@ -112,7 +132,6 @@ __global__ void __launch_bounds__(256) router_logits_kernel(const T* __restrict_
 // (one thread per token walking its rows in memory took 347 us for 2048 tokens x 64 experts, top-8; this takes 11).
 // The exponentials are added in expert order, the selected scores in selection order: every lane of the token adds all of
 // them, so the bits do not depend on the number of lanes.  All TK_LANES lanes of a token must be active.
-constexpr int TK_LANES = 16;
 constexpr int TK_MAX_PER_LANE = 16;   // up to TK_LANES * TK_MAX_PER_LANE = 256 experts in registers
 template <int PER_LANE>
 __device__ __forceinline__ void softmax_topk_token(const float* __restrict__ l, float* __restrict__ s,
@@ -419,10 +438,11 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const float* __restrict
 // wave per (token, selection) pair takes the gradient of that weight, <y[t*k+j], dout[t]> (+ d_w, a gradient that reached the returned
 // weights directly), and puts the weight at the pair's place in sorted order (the row scale of the grouped GEMMs); then the token's lanes
 // turn its k gradients into those of its logits.  The sums are those of combine_dgates and router_bwd, bit for bit.  As three launches
-// 2048 tokens, 64 experts, top-8, d=2048 took 34.6 us, this 25.3 (eight waves for more than four selections; four: 32.8); 4096 tokens, top-2, d=4096 28.7 and 18.8;
+// 2048 tokens, 64 experts, top-8, d=2048 took 34.6 us, this 21.4 (eight waves for more than four selections, eight per SIMD; four, and
+// as many registers as the compiler likes: 32.8); 4096 tokens, top-2, d=4096 28.7 and 18.8;
 // 512 tokens, d=256 9.4 and 4.7.
 template <typename T, int GB_WAVES>
-__global__ void __launch_bounds__(GB_WAVES * 64) gates_bwd_kernel(const T* __restrict__ y, int64_t ldy, const T* __restrict__ dout, int64_t ldd,
+__global__ void __launch_bounds__(GB_WAVES * 64, 8) gates_bwd_kernel(const T* __restrict__ y, int64_t ldy, const T* __restrict__ dout, int64_t ldd,
                                                                   const float* __restrict__ d_w, const float* __restrict__ w,
                                                                   const int32_t* __restrict__ topi, const float* __restrict__ scores,
                                                                   const int32_t* __restrict__ inv, float* __restrict__ dlogits,
@@ -774,10 +794,11 @@ __global__ void padded_blocks_kernel(const void* __restrict__ offsets, int off64
 
 }  // namespace
 
-int moe_launch_router_logits(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits,
-                             int64_t ntok, int64_t d, int E, hipStream_t stream)
+namespace {
+// topk: softmax and top-k in the same launch (E <= ROUTER_EXPERT_GROUP)
+int launch_router_logits(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits, int64_t ntok, int64_t d, int E,
+                         bool topk, float* scores, float* topw, int32_t* topi, int k, int renorm, hipStream_t stream)
 {
-    if (ntok == 0) return MOE_OK;
     const int groups = (E + ROUTER_EXPERT_GROUP - 1) / ROUTER_EXPERT_GROUP;
     // 4 tokens per wave share each weight fetch, as soon as that still leaves a wave for every SIMD; 2 for fewer tokens
     const int tokens = ((ntok + 3) / 4) * groups >= 4 * (int64_t)moe_device_cus() ? 4 : 2;
@@ -785,13 +806,20 @@ int moe_launch_router_logits(const void* x, int64_t ldx, const void* wg, int64_t
     const dim3 grid((unsigned)((waves + 3) / 4), (unsigned)groups);
     const int64_t per16 = dtype == MOE_F32 ? 4 : 8;
     const bool vec_ok = ((uintptr_t)x % 16 == 0) && ((uintptr_t)wg % 16 == 0) && ldx % per16 == 0 && ldw % per16 == 0;
-    if (tokens == 4)
-        MOE_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((router_logits_kernel<T, 4>), grid, dim3(256), 0, stream, (const T*)x, ldx,
-                                                     (const T*)wg, ldw, logits, ntok, d, E, vec_ok));
-    else
-        MOE_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((router_logits_kernel<T, 2>), grid, dim3(256), 0, stream, (const T*)x, ldx,
-                                                     (const T*)wg, ldw, logits, ntok, d, E, vec_ok));
+    MOE_DISPATCH_DTYPE(dtype, {
+        auto kern = tokens == 4 ? (topk ? router_logits_kernel<T, 4, true> : router_logits_kernel<T, 4, false>)
+                                : (topk ? router_logits_kernel<T, 2, true> : router_logits_kernel<T, 2, false>);
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, (const T*)x, ldx, (const T*)wg, ldw, logits, ntok, d, E, vec_ok, scores, topw, topi, k, renorm);
+    });
     return moe_launch_status();
+}
+}  // namespace
+
+int moe_launch_router_logits(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits,
+                             int64_t ntok, int64_t d, int E, hipStream_t stream)
+{
+    if (ntok == 0) return MOE_OK;
+    return launch_router_logits(x, ldx, wg, ldw, dtype, logits, ntok, d, E, false, nullptr, nullptr, nullptr, 0, 0, stream);
 }
 
 // logits + softmax + top-k; one launch when the router weight fits the fused kernel, otherwise the two kernels above
@@ -803,6 +831,8 @@ int moe_launch_router_forward(const void* x, int64_t ldx, const void* wg, int64_
     const bool fused = dtype != MOE_F32 && E <= RM_MAX_EXPERTS && d % 32 == 0 && d >= 32 && d < (1 << 30) &&
                        ((uintptr_t)x % 16 == 0) && ((uintptr_t)wg % 16 == 0) && ldx % 8 == 0 && ldw % 8 == 0;
     if (!fused) {
+        if (E <= ROUTER_EXPERT_GROUP)
+            return launch_router_logits(x, ldx, wg, ldw, dtype, logits, ntok, d, E, true, scores, topw, topi, k, renorm, stream);
         const int rc = moe_launch_router_logits(x, ldx, wg, ldw, dtype, logits, ntok, d, E, stream);
         return rc != MOE_OK ? rc : moe_launch_router_topk(logits, scores, topw, topi, ntok, E, k, renorm, stream);
     }

@@ -797,7 +797,12 @@ variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const 
         Tensor W = w.view({E, f, d});
         return linear_checked(in, n_contiguous ? W : W.transpose(1, 2), lt[ia], lt[ia + 1], scaling, scaling, fan, sei, ssi, offsets, Tensor(), gin, true);
     };
-    Tensor h = swiglu(proj(x, w1, false, 0, k, false), proj(x, w3, false, 2, k, false));
+    Tensor h;
+    if (!rank && x.scalar_type() == at::kFloat && !needs_node({&x, &w1, &w3})) {   // both projections and their product in one launch (three: 256 tokens, d=128, f=256: 20 us, one 10.4)
+        h = at::empty({so.R, f}, x.options());
+        check(moe_swiglu_pair(ptr(x), x.stride(0), x.stride(1), ptr(w1), ptr(w3), f * d, 1, d, ptr(h), h.stride(0), so.ssi(), 0, so.offsets(), 0, (int)E, so.R, d, f, (int)k,
+                              dtype_code(x), stream_of(x)), "moe_swiglu_pair");
+    } else h = swiglu(proj(x, w1, false, 0, k, false), proj(x, w3, false, 2, k, false));
     Tensor y = proj(h, w2, true, 4, 1, true);
     Tensor out = needs_node({&y, &rt[1]}) ? GatherCombineFn::apply(y, rt[1], inv, ssi) : combine(y, rt[1], so.inv(), k, x.size(0));
     return {out, rt[1], rt[2]};
