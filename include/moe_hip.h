@@ -151,20 +151,17 @@ int moe_scatter2scatter(const void* X, int64_t sxm, int64_t sxk, const void* W, 
                         int x_grouped, int y_grouped, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* backward of a projection with adapters, rows of X and dY gathered (bf16 / fp16, unit column strides, rank <= 64): with row m of the sorted
- * order at flat position p = pos[m], X_m = x[p / fan_out] and dY_m = row_scale[m] * dout[p / dout_fan_out] (row_scale may be null),
+ * order at flat position p = pos[m], X_m = x[p / fan_out] and dY_m = gates[p] * dout[p / dout_fan_out] (gates: one weight per flat position, may be null),
  *   DA[e] = s X_e^T (dY_e B_e^T),  DB[e] = s (X_e A_e)^T dY_e,  dx_rows[p] = dY_m W_e^T + s (dY_m B_e^T) A_e^T
  * (scattermoe_utils/parallel_linear_lora.py:83-134).  MOE_ERR_UNSUPPORTED, with nothing enqueued, for shapes outside the matrix-core paths: a
  * caller then takes moe_group_rows, moe_group_bwd_ab and moe_scatter2scatter. */
 size_t moe_linear_lora_bwd_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank);
-int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const float* row_scale, const void* x, int64_t ldx, int fan_out,
+int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const void* gates, int gates_dtype, const void* x, int64_t ldx, int fan_out,
                         const void* W, int64_t swe, int64_t swk, int64_t swn, const void* A, int64_t sae, int64_t sak, int64_t sar,
                         const void* B, int64_t sbe, int64_t sbr, int64_t sbn, int rank, float scaling, void* DA, int64_t sdae, int64_t sdak,
                         int64_t sdar, void* DB, int64_t sdbe, int64_t sdbr, int64_t sdbn, void* dx_rows, int64_t lddx, const void* pos,
                         int pos64, const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int dtype, void* workspace,
                         size_t workspace_bytes, void* stream);
-/* out[i] = weights[pos[i]] as fp32 */
-int moe_gather_scales(const void* weights, int wdtype, const void* pos, int pos64, int64_t n, float* out, void* stream);
-
 /* ---- group_bwd_AB: scattermoe_utils/kernels/ops.py:220-255, definition :284-289 ------------------------------
  * DA[e] = scaling * X_e^T (DY_e B[e]^T),  DB[e] = scaling * (X_e A[e])^T DY_e over the rows of group e (full
  * reductions over N and K), zero for empty groups.  X (R,K) and DY (R,N) in grouped order. */

@@ -44,8 +44,7 @@ _SIGNATURES = {
     "moe_scatter2scatter_workspace_bytes": ("z", "lilli"),
     "moe_scatter2scatter": ("i", "pll" + "plll" + "plll" + "plll" + "if" + "pll" + "pi" + "pi" + "i" + "lll" + "iiii" + "pzp"),
     "moe_linear_lora_bwd_workspace_bytes": ("z", "lilli"),
-    "moe_linear_lora_bwd": ("i", "pli" + "p" + "pli" + "plll" + "plll" + "plll" + "if" + "plll" + "plll" + "pl" + "pi" + "pi" + "i" + "lll" + "i" + "pzp"),
-    "moe_gather_scales": ("i", "pipilpp"),
+    "moe_linear_lora_bwd": ("i", "pli" + "pi" + "pli" + "plll" + "plll" + "plll" + "if" + "plll" + "plll" + "pl" + "pi" + "pi" + "i" + "lll" + "i" + "pzp"),
     "moe_group_bwd_ab_workspace_bytes": ("z", "lillii"),
     "moe_group_bwd_ab": ("i", "pll" + "pll" + "plll" + "plll" + "if" + "plll" + "plll" + "pi" + "i" + "lll" + "i" + "pzp"),
     "moe_group_bwd_w": ("i", "pll" + "pll" + "plll" + "pi" + "i" + "lll" + "i" + "p"),

@@ -96,6 +96,14 @@ template <> struct Elem<__half> {
     static __device__ __forceinline__ void st(__half* p, float v) { *p = __float2half(v); }
 };
 
+// element i of a weight tensor of any of the three types
+__device__ __forceinline__ float load_gate(const void* g, int64_t i, int gdtype)
+{
+    if (gdtype == MOE_F32) return ((const float*)g)[i];
+    if (gdtype == MOE_BF16) return Elem<__hip_bfloat16>::ld((const __hip_bfloat16*)g + i);
+    return Elem<__half>::ld((const __half*)g + i);
+}
+
 // a 64-bit value that is the same in every lane, moved to scalar registers
 __device__ __forceinline__ int64_t uniform_i64(int64_t v)
 {
@@ -174,20 +182,16 @@ __device__ __forceinline__ bool find_row_tile(const void* offsets, int off64, in
     return false;
 }
 
-// First and one-past-last row of group e and the number of bm-row tiles of all groups before it.  All 64 lanes active.
-__device__ __forceinline__ void find_group(const void* offsets, int off64, int bm, int e, int64_t* start, int64_t* end, int64_t* tiles_before)
+// First and one-past-last row of group e (< E) and the number of bm-row tiles of all groups before it.  All 64 lanes active.
+__device__ __forceinline__ void find_group(const void* offsets, int off64, int E, int bm, int e, int64_t* start, int64_t* end, int64_t* tiles_before)
 {
-    const int lane = threadIdx.x & 63;
     int64_t n = 0;
-    for (int ee = lane; ee < e; ee += 64) {
-        const int64_t s0 = ee > 0 ? load_idx(offsets, ee - 1, off64) : 0;
-        n += (load_idx(offsets, ee, off64) - s0 + bm - 1) / bm;
-    }
-    *start = e > 0 ? load_idx(offsets, e - 1, off64) : 0;
-    *end = load_idx(offsets, e, off64);
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d);
-    *tiles_before = n;
+    int base = 0;
+    for (; base + 64 <= e; base += 64) n += __builtin_amdgcn_readlane(scan_expert_tiles_from(offsets, off64, E, bm, base).tiles_through, 63);
+    const ExpertScan s = scan_expert_tiles_from(offsets, off64, E, bm, base);
+    *start = readlane_i64(s.start, e - base);
+    *end = readlane_i64(s.end, e - base);
+    *tiles_before = n + __builtin_amdgcn_readlane(s.tiles_before, e - base);
 }
 
 #define MOE_DISPATCH_DTYPE(dtype, ...)                                                   \

@@ -116,7 +116,8 @@ int moe_launch_generic_xty(const void* X, int64_t sxm, int64_t sxk, const void* 
 // (K rounded up to 32) one after the other
 constexpr int MOE_PACK_MAX_JOBS = 12;
 struct MoePackJob { const uint16_t* src; int64_t se, sk, sr; uint16_t* dst; int64_t K; int transpose; int rank; };   // rank <= 16 columns, zero padded to 16
-struct MoePackBatch { MoePackJob job[MOE_PACK_MAX_JOBS]; int njobs; int E; int* zero_ptr; int zero_n; };   // zero_ptr[0..zero_n) is cleared by the launch
+// side jobs of the launch: zero_ptr[0..zero_n) is cleared; scales[i] = weights[pos[i]] as fp32 for i < scales_n (the row scales of a sorted order)
+struct MoePackBatch { MoePackJob job[MOE_PACK_MAX_JOBS]; int njobs; int E; int* zero_ptr; int zero_n; const void* weights; int wdtype; const void* pos; int pos64; int64_t scales_n; float* scales; };
 int moe_launch_pack_lora_batch(const MoePackBatch& jobs, hipStream_t stream);
 // up to MOE_LORA_MAX_JOBS products in one launch over the same row order: Q = scaling * X . A in storage type, [R][16], its
 // transposed copy Qt (row pitch ldqt) and a copy of Q scaled like Qt (each optional)
@@ -191,8 +192,6 @@ int moe_launch_padded_blocks(const void* offsets, int off64, int E, int block_m,
 int moe_launch_group_rows(const void* src, int64_t lds_, void* out, int64_t ldo, const void* pos, int pos64,
                           int fan_out, const void* coeff, int cdtype, int64_t nrows, int64_t ncols, int dtype,
                           hipStream_t stream);
-// out[i] = weights[pos[i]] as fp32
-int moe_launch_gather_scales(const void* weights, int wdtype, const void* pos, int pos64, int64_t n, float* out, hipStream_t stream);
 int moe_launch_combine_fwd(const void* y, int64_t ldy, void* out, int64_t ldo, const void* gates, int gdtype,
                            const int32_t* inv, int k, int64_t ntok, int64_t ncols, int dtype,
                            const float* extra_coef, const void* extra_rows, int64_t lde, int n_extra,

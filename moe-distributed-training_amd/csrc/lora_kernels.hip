@@ -28,13 +28,15 @@ inline unsigned job_grid(int64_t units, int njobs) { return (unsigned)((units + 
 // several pack jobs in one launch (blockIdx.y selects the job): the six factors of an MLP block are a few MB in total,
 // so separate launches would cost more in launch latency than in data movement.  A thread produces 16 bytes: the 8
 // consecutive output elements of a chunk walk the source with one stride (rank stride in [K][16] order, k stride in
-// fragment order).  The launch also clears a small int array for its caller (the grouped GEMM's K-split counters),
-// which saves that caller a launch of its own.
+// fragment order).  The launch also clears a small int array for its caller (the grouped GEMM's K-split counters) and gathers the gate
+// weights into sorted order (launches with two jobs or more), which saves that caller launches of its own.
 __global__ void pack_lora_batch_kernel(const MoePackBatch jobs)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.y == 0)
         for (int64_t z = i; z < jobs.zero_n; z += (int64_t)gridDim.x * blockDim.x) jobs.zero_ptr[z] = 0;
+    else if (blockIdx.y == 1)
+        for (int64_t z = i; z < jobs.scales_n; z += (int64_t)gridDim.x * blockDim.x) jobs.scales[z] = load_gate(jobs.weights, load_idx(jobs.pos, z, jobs.pos64), jobs.wdtype);
     const MoePackJob& j = jobs.job[blockIdx.y];
     const int64_t K = j.K;
     const int rank = j.rank;
@@ -337,7 +339,7 @@ __global__ void xtp_reduce_kernel(const XtpReduceJobs jobs, const void* __restri
     const int rank = job.rank;
     const int e = blockIdx.y;
     int64_t tile0, start, end;
-    find_group(offsets, off64, XTP_RC, e, &start, &end, &tile0);   // one round trip, not one per expert
+    find_group(offsets, off64, E, XTP_RC, e, &start, &end, &tile0);   // one round trip, not one per expert (64 experts, six jobs: 22 us with 64-bit shuffles, 17.7 so)
     const int64_t ntile = (end - start + XTP_RC - 1) / XTP_RC;
     const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (idx >= K * 16) return;
@@ -448,7 +450,8 @@ int moe_launch_pack_lora_batch(const MoePackBatch& jobs, hipStream_t stream)
         kmax = k > kmax ? k : kmax;
     }
     const int64_t total = (int64_t)jobs.E * kmax * 2;   // 16-byte chunks of the largest job
-    if (total == 0 && jobs.zero_n == 0) return MOE_OK;
+    if (total == 0 && jobs.zero_n == 0 && jobs.scales_n == 0) return MOE_OK;
+    if (jobs.scales_n < 0 || (jobs.scales_n > 0 && (jobs.njobs < 2 || !jobs.weights || !jobs.pos || !jobs.scales))) return MOE_ERR_UNSUPPORTED;
     if ((total + 255) / 256 > 0x7fffffff || jobs.zero_n < 0 || (jobs.zero_n > 0 && !jobs.zero_ptr)) return MOE_ERR_UNSUPPORTED;
     for (int j = 0; j < jobs.njobs; ++j)
         if (((uintptr_t)jobs.job[j].dst % 16) != 0) return MOE_ERR_UNSUPPORTED;

@@ -395,7 +395,7 @@ int moe_group_bwd_ab(const void* DY, int64_t sdm, int64_t sdn, const void* X, in
 // Backward of a projection with adapters whose rows are gathered on both sides: the gradients of the adapters and the rows of dX without
 // the gathered copies of dY and X that moe_group_bwd_ab and moe_scatter2scatter read, with one packing and one pass over the rows instead of
 // two (8 experts, 1500 tokens, top-2, 4096 x 4096, rank 32: the launches between the gate gradients and the dX product 87 us, 64 so; forward and backward 325 -> 286).  dY's rows
-// enter unscaled; their gate weights (row_scale) multiply fp32 sums.
+// enter unscaled; their gate weights, gathered by the packing, multiply fp32 sums.
 static const int LINEAR_BWD_MAX_CHUNKS = MOE_MAX_SLABS;   // 16-wide rank chunks: the dX launch takes them as slabs given by pointer
 
 // The adapter gradients' partials lie where the dX launch exchanges its K-split tiles afterwards (behind the counters, which are cleared before either)
@@ -410,10 +410,10 @@ static inline size_t linear_bwd_shared_bytes(int64_t R, int E, int64_t K, int64_
 size_t moe_linear_lora_bwd_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank)
 {
     const size_t C = (size_t)((rank > 0 ? rank : 1) + 15) / 16;
-    return al(linear_bwd_shared_bytes(R, E, K, N, rank)) + C * (2 * pack_bytes(E, K) + pack_bytes(E, N) + 3 * q_bytes(R)) + 256;
+    return al(linear_bwd_shared_bytes(R, E, K, N, rank)) + C * (2 * pack_bytes(E, K) + pack_bytes(E, N) + 3 * q_bytes(R)) + al((size_t)R * sizeof(float)) + 256;
 }
 
-int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const float* row_scale, const void* x, int64_t ldx, int fan_out,
+int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const void* gates, int gates_dtype, const void* x, int64_t ldx, int fan_out,
                         const void* W, int64_t swe, int64_t swk, int64_t swn, const void* A, int64_t sae, int64_t sak, int64_t sar,
                         const void* B, int64_t sbe, int64_t sbr, int64_t sbn, int rank, float scaling, void* DA, int64_t sdae, int64_t sdak,
                         int64_t sdar, void* DB, int64_t sdbe, int64_t sdbr, int64_t sdbn, void* dx_rows, int64_t lddx, const void* pos,
@@ -422,6 +422,7 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const f
 {
     if (!dout || !x || !W || !A || !B || !DA || !DB || !dx_rows || !pos || !offsets || rank < 1 || E < 1 || R < 0 || K < 1 || N < 1 || fan_out < 1 || dout_fan_out < 1)
         return MOE_ERR_BAD_ARG;
+    if (gates && gates_dtype != MOE_BF16 && gates_dtype != MOE_F16 && gates_dtype != MOE_F32) return MOE_ERR_BAD_ARG;
     const int C = (rank + 15) / 16;
     const bool nt = swn == 1, nn = swk == 1 && !nt;   // of the transposed weights (E, N, K): contraction-contiguous, output-contiguous
     if (!bwd_ab_fast(K, N, rank, dtype, ldd, 1, ldx, 1, dout, x) || C > LINEAR_BWD_MAX_CHUNKS || !(nt || nn) || R == 0) return MOE_ERR_UNSUPPORTED;
@@ -429,7 +430,7 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const f
     MoeGemmParams p = {};
     p.X[0] = (const uint16_t*)dout; p.ldx = ldd; p.nseg = 1;
     p.W[0] = (const uint16_t*)W; p.swe = swe; p.ldw = nt ? swk : swn; p.nn = nn ? 1 : 0;
-    p.Y[0] = (uint16_t*)dx_rows; p.ldy = lddx; p.row_scale = row_scale;
+    p.Y[0] = (uint16_t*)dx_rows; p.ldy = lddx;
     p.pos = pos; p.pos64 = pos64; p.offsets = offsets; p.off64 = off64;
     p.E = E; p.K = N; p.N = K; p.fan_out = dout_fan_out; p.x_grouped = 0; p.y_grouped = 0;
     p.epi = MOE_EPI_STORE; p.f16 = f16; p.nslab = C; p.slab_mode = 0;
@@ -443,6 +444,8 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const f
     const size_t xb = linear_bwd_xtp_bytes(R, E, K, N, rank);
     const int64_t ldt = pad_rows(R);
     hipStream_t st = S(stream);
+    float* row_scale = gates ? (float*)ws.take((size_t)R * sizeof(float)) : nullptr;   // gate of every sorted position
+    p.row_scale = row_scale;
     void *At[LINEAR_BWD_MAX_CHUNKS] = {}, *Bt[LINEAR_BWD_MAX_CHUNKS] = {}, *LB[LINEAR_BWD_MAX_CHUNKS] = {}, *P[LINEAR_BWD_MAX_CHUNKS] = {}, *Pt[LINEAR_BWD_MAX_CHUNKS] = {}, *Qt[LINEAR_BWD_MAX_CHUNKS] = {};
     for (int c = 0; c < C; ++c) {
         At[c] = ws.take(pack_bytes(E, K)); Bt[c] = ws.take(pack_bytes(E, N)); LB[c] = ws.take(pack_bytes(E, K));
@@ -454,6 +457,7 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const f
     static_assert(3 * LINEAR_BWD_MAX_CHUNKS <= MOE_PACK_MAX_JOBS, "one packing launch");
     MoePackBatch pb = {};
     pb.E = E; pb.zero_ptr = p.sk_counters; pb.zero_n = moe_gemm_num_counters();
+    if (gates) { pb.weights = gates; pb.wdtype = gates_dtype; pb.pos = pos; pb.pos64 = pos64; pb.scales_n = R; pb.scales = row_scale; }
     for (int c = 0; c < C; ++c) {
         const uint16_t *a = (const uint16_t*)A + 16 * c * sar, *b = (const uint16_t*)B + 16 * c * sbr;
         pb.job[pb.njobs++] = {a, sae, sak, sar, (uint16_t*)At[c], K, 1, chunk_rank(c)};
@@ -482,12 +486,6 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const f
         TRY(moe_launch_xtp_jobs(xtp, 2 * n, pos64, ldt, offsets, off64, E, R, 1.f, xw, xb, st, f16));
     }
     return moe_launch_gemm_mfma(p, R, st);
-}
-
-int moe_gather_scales(const void* weights, int wdtype, const void* pos, int pos64, int64_t n, float* out, void* stream)
-{
-    if (n < 0 || (n > 0 && (!weights || !pos || !out))) return MOE_ERR_BAD_ARG;
-    return moe_launch_gather_scales(weights, wdtype, pos, pos64, n, out, S(stream));
 }
 
 int moe_group_bwd_w(const void* DY, int64_t sdm, int64_t sdn, const void* X, int64_t sxm, int64_t sxk, void* DW,

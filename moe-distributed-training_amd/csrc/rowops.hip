@@ -38,12 +38,6 @@ __device__ __forceinline__ void store_vec(T* p, const float* v, bool vec_ok, int
     }
 }
 
-__device__ __forceinline__ float load_gate(const void* g, int64_t i, int gdtype)
-{
-    if (gdtype == MOE_F32) return ((const float*)g)[i];
-    if (gdtype == MOE_BF16) return Elem<__hip_bfloat16>::ld((const __hip_bfloat16*)g + i);
-    return Elem<__half>::ld((const __half*)g + i);
-}
 __device__ __forceinline__ void store_gate(void* g, int64_t i, float v, int gdtype)
 {
     if (gdtype == MOE_F32) ((float*)g)[i] = v;
@@ -76,13 +70,6 @@ __global__ void __launch_bounds__(ROW_THREADS) group_rows_kernel(const T* __rest
         }
         store_vec<T>(o + c0, v, vo, n);
     }
-}
-
-// out[i] = weights[pos[i]] as fp32: the row scales of a sorted order (a thread per row; through group_rows a workgroup per row, 6 us for 8192 rows)
-__global__ void gather_scales_kernel(const void* __restrict__ weights, int wdtype, const void* __restrict__ pos, int pos64, int64_t n, float* __restrict__ out)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = load_gate(weights, load_idx(pos, i, pos64), wdtype);
 }
 
 // out[t][:] = sum_j gates[t*k+j] * y[row(t,j)][:],  row(t,j) = inv ? inv[t*k+j] : t*k+j.   gates may be null (=1).
@@ -276,7 +263,21 @@ __global__ void __launch_bounds__(ROW_THREADS) combine_dgates_kernel(const T* __
     const int64_t t = pair / k;
     const int64_t row = inv ? (int64_t)inv[pair] : pair;
     float acc = 0.f;
-    for (int64_t c0 = (int64_t)lane * N; c0 < ncols; c0 += 64 * N) {
+    int64_t c0 = (int64_t)lane * N;
+    if (vec_ok)   // whole vectors, four of each row in flight (3000 pairs x 4096 columns: 13.3 us one by one, 8.38 so)
+        for (; c0 + 3 * 64 * N + N <= ncols; c0 += 4 * 64 * N) {
+            uint4 a[4], b[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                a[q] = *(const uint4*)(y + row * ldy + c0 + q * 64 * N);
+                b[q] = *(const uint4*)(dout + t * ldd + c0 + q * 64 * N);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int u = 0; u < N; ++u) acc = fmaf(Elem<T>::ld((const T*)&a[q] + u), Elem<T>::ld((const T*)&b[q] + u), acc);
+        }
+    for (; c0 < ncols; c0 += 64 * N) {
         const int n = (ncols - c0 < N) ? (int)(ncols - c0) : N;
         const bool vo = vec_ok && n == N;
         float a[N], b[N];
@@ -458,14 +459,6 @@ int moe_launch_group_rows(const void* src, int64_t lds_, void* out, int64_t ldo,
         hipLaunchKernelGGL((group_rows_kernel<T>), dim3((unsigned)nrows), dim3(ROW_THREADS), 0, stream, (const T*)src,
                            lds_, (T*)out, ldo, pos, pos64, fan_out, coeff, cdtype, nrows, ncols, vo);
     });
-    return moe_launch_status();
-}
-
-int moe_launch_gather_scales(const void* weights, int wdtype, const void* pos, int pos64, int64_t n, float* out, hipStream_t stream)
-{
-    if (wdtype != MOE_BF16 && wdtype != MOE_F16 && wdtype != MOE_F32) return MOE_ERR_BAD_ARG;
-    if (n == 0) return MOE_OK;
-    hipLaunchKernelGGL(gather_scales_kernel, dim3((unsigned)((n + ROW_THREADS - 1) / ROW_THREADS)), dim3(ROW_THREADS), 0, stream, weights, wdtype, pos, pos64, n, out);
     return moe_launch_status();
 }
 

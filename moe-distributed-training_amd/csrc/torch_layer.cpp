@@ -431,22 +431,17 @@ struct LinearFn : Function<LinearFn> {
         if (A.defined() && !grouped_in && !grouped_out && scaling == ctx->saved_data["scaling_ab"].toDouble() && L > 0) {
             // all of it from the rows where they lie (shapes outside the matrix-core paths go on below)
             const int64_t K = x.size(1), N = W.size(2), r = A.size(2);
-            Tensor scales;
-            if (gates.defined()) {
-                scales = at::empty({L}, x.options().dtype(at::kFloat));
-                check(moe_gather_scales(ptr(gates), dtype_code(gates), ptr(ssi), is64(ssi), L, (float*)ptr(scales), stream_of(x)), "moe_gather_scales");
-            }
             dA = at::empty({E, K, r}, dout.options());
             dB = at::empty({E, r, N}, dout.options());
             Tensor dx = at::empty({L, K}, x.options()), ws = bytes_on(x, moe_linear_lora_bwd_workspace_bytes(L, (int)E, K, N, (int)r));
-            const int rc = moe_linear_lora_bwd(ptr(dout), dout.stride(0), (int)gate_fan, (const float*)ptr(scales), ptr(x), x.stride(0), (int)k, ptr(W), W.stride(0),
+            const int rc = moe_linear_lora_bwd(ptr(dout), dout.stride(0), (int)gate_fan, ptr(gates), gates.defined() ? dtype_code(gates) : 0, ptr(x), x.stride(0), (int)k, ptr(W), W.stride(0),
                                                W.stride(1), W.stride(2), ptr(A), A.stride(0), A.stride(1), A.stride(2), ptr(B), B.stride(0), B.stride(1), B.stride(2),
                                                (int)r, (float)scaling, ptr(dA), dA.stride(0), dA.stride(1), dA.stride(2), ptr(dB), dB.stride(0), dB.stride(1),
                                                dB.stride(2), ptr(dx), dx.stride(0), ptr(ssi), is64(ssi), ptr(eo), is64(eo), (int)E, L, K, N, dtype_code(x), ptr(ws),
                                                (size_t)ws.numel(), stream_of(x));
             if (rc != MOE_ERR_UNSUPPORTED) {
                 check(rc, "moe_linear_lora_bwd");
-                ws = scales = Tensor();   // given back before the fan-out sum takes its output
+                ws = Tensor();   // given back before the fan-out sum takes its output
                 if (k != 1) dx = combine(dx, Tensor(), nullptr, k, L / k);
                 return {dx, Tensor(), dA, dB, d_gates, Tensor(), Tensor(), Tensor()};
             }

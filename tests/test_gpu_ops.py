@@ -557,7 +557,7 @@ def test_scatter2scatter_lora_packs_any_width_and_rank(dev, oracle, K, N, r):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("K", [1, 15, 63, 64, 65, 130])
+@pytest.mark.parametrize("K", [1, 15, 63, 64, 65, 127, 128, 129, 130, 257])
 @pytest.mark.parametrize("layout", ["k_contiguous", "n_contiguous"])
 def test_generic_kernels_at_the_edges_of_a_contraction_step(dev, oracle, dtype, K, layout):
     """The kernels of the sizes that the matrix cores do not take, at contractions of one step, one step more or less and a few: the
