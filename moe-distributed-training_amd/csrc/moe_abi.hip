@@ -394,7 +394,7 @@ int moe_group_bwd_ab(const void* DY, int64_t sdm, int64_t sdn, const void* X, in
 
 // Backward of a projection with adapters whose rows are gathered on both sides: the gradients of the adapters and the rows of dX without
 // the gathered copies of dY and X that moe_group_bwd_ab and moe_scatter2scatter read, with one packing and one pass over the rows instead of
-// two (8 experts, 1500 tokens, top-2, 4096 x 4096, rank 32: the launches between the gate gradients and the dX product 87 us, 64 so; forward and backward 325 -> 286).  dY's rows
+// two (8 experts, 1500 tokens, top-2, 4096 x 4096, rank 32: the launches between the gate gradients and the dX product 87 us, 55 so; forward and backward 317 -> 269).  dY's rows
 // enter unscaled; their gate weights, gathered by the packing, multiply fp32 sums.
 static const int LINEAR_BWD_MAX_CHUNKS = MOE_MAX_SLABS;   // 16-wide rank chunks: the dX launch takes them as slabs given by pointer
 

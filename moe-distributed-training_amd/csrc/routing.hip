@@ -317,7 +317,10 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_kernel(const T* __r
 
 // The same for 9 to 96 experts, in EG groups of 16: a wave's activation fragment meets EG weight fragments per step, fewer steps' loads fit in
 // flight, and the eight partial sums per logit are added in wave order as above.  The two launches of the vector kernels are bound by their
-// FMAs (2048 tokens x 64 experts x 2048 columns: 26.3 + 10.2 us, this 21); the order of a logit's sum differs from theirs.
+// FMAs (2048 tokens x 64 experts x 2048 columns: 26.3 + 10.2 us, this 21); the order of a logit's sum differs from theirs.  A step's 32 products are
+// summed by the instruction, the steps and the waves in 64 bits: the loads hide these adds (21.1 us with fp32 accumulators too), and chained in fp32
+// the logits of 2048 bf16 columns were 1.03e-7 from 64 bits (relative 2-norm) where the vector kernels are 7.5e-8 and this 4.7e-8; 96 experts, 3072
+// columns 1.22e-7, 8.0e-8 and 4.6e-8; fp16 1.14e-7 (vector) and 5.7e-8.
 template <typename T, int EG>
 __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_wide_kernel(const T* __restrict__ x, int64_t ldx, const T* __restrict__ wg, int64_t ldw,
                                                                          float* __restrict__ logits, float* __restrict__ scores,
@@ -338,9 +341,11 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_wide_kernel(const T
     for (int g = 0; g < EG; ++g) wp[g] = wg + (int64_t)(g * 16 + row < E ? g * 16 + row : E - 1) * ldw + kc * 8;   // (rows past the last expert repeat it; nobody reads their logits)
     const int nsteps = d / 32;
     const int s_end = nsteps * (wave + 1) / RM_WAVES;
-    f32x4_t acc[EG];
+    double acc[EG][4];
 #pragma unroll
-    for (int g = 0; g < EG; ++g) acc[g] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < EG; ++g)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[g][r] = 0.0;
     for (int s0 = nsteps * wave / RM_WAVES; s0 < s_end; s0 += BATCH) {
         uint4 xa[BATCH], wa[BATCH][EG];
 #pragma unroll
@@ -356,19 +361,22 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_wide_kernel(const T
 #pragma unroll
                 for (int g = 0; g < EG; ++g) {
                     using Num = typename std::conditional<std::is_same<T, __hip_bfloat16>::value, NumBf16, NumF16>::type;
-                    acc[g] = Num::mfma(__builtin_bit_cast(bf16x8_t, wa[i][g]), __builtin_bit_cast(bf16x8_t, xa[i]), acc[g]);
+                    const f32x4_t p = Num::mfma(__builtin_bit_cast(bf16x8_t, wa[i][g]), __builtin_bit_cast(bf16x8_t, xa[i]), (f32x4_t){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[g][r] += (double)p[r];
                 }
             }
     }
     // acc[g][r] = partial logit of token `row`, expert 16 g + 4 kc + r
 #pragma unroll
-    for (int g = 0; g < EG; ++g) *(f32x4_t*)&s_part[wave][row][g * 16 + 4 * kc] = acc[g];
+    for (int g = 0; g < EG; ++g) *(f32x4_t*)&s_part[wave][row][g * 16 + 4 * kc] = (f32x4_t){(float)acc[g][0], (float)acc[g][1], (float)acc[g][2], (float)acc[g][3]};
     __syncthreads();
     for (int i = tid; i < RM_TOKENS * EW; i += RM_WAVES * 64) {
         const int t = i / EW, e = i % EW;
-        float sum = s_part[0][t][e];
+        double dsum = s_part[0][t][e];
 #pragma unroll
-        for (int w = 1; w < RM_WAVES; ++w) sum += s_part[w][t][e];
+        for (int w = 1; w < RM_WAVES; ++w) dsum += (double)s_part[w][t][e];
+        const float sum = (float)dsum;
         s_logits[t][e] = sum;
         if (e < E && t0 + t < ntok) logits[(t0 + t) * E + e] = sum;
     }

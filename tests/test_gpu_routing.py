@@ -410,6 +410,9 @@ def test_router_of_many_experts_on_the_matrix_cores(dev, oracle, dtype, T, d, E,
     srt = torch.sort(so, dim=-1, descending=True).values
     assert (srt[:, k - 1] - srt[:, k]).abs().min() > 1e-7, "test data has a near tie; pick another seed"
     assert torch.allclose(l.cpu(), lo, atol=3e-5, rtol=1e-5)
+    if d >= 256:   # and no further from 64 bits than the vector kernels' chains of fp32 sums (one rounding per wave and one per logit here)
+        ref = x.double() @ wg.double().t()
+        assert (l.cpu() - ref).norm() <= (router.router_logits(x.to(dev), wg.to(dev)).cpu() - ref).norm()
     assert torch.equal(i.cpu().long(), io)
     assert torch.allclose(s.cpu(), so, atol=1e-6) and torch.allclose(w.cpu(), wo, atol=1e-5)
     s1, w1, i1 = router.router_topk(l, k)
