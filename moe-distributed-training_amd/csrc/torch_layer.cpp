@@ -428,13 +428,15 @@ struct LinearFn : Function<LinearFn> {
             coeff = gates.reshape({-1});
             gate_fan = gates.size(1);
         }
-        if (A.defined() && !grouped_in && !grouped_out && scaling == ctx->saved_data["scaling_ab"].toDouble() && L > 0) {
-            // all of it from the rows where they lie (shapes outside the matrix-core paths go on below)
+        // All of it from the rows where they lie (shapes outside the matrix-core paths go on below).  Not for gated fp16: dY B^T is stored before its
+        // gate weight there, which can pass 65504 where the product of the weighted rows does not.
+        if (A.defined() && !grouped_in && !grouped_out && scaling == ctx->saved_data["scaling_ab"].toDouble() && L > 0 && W.numel() > 0 && A.size(2) > 0 &&
+            !(gates.defined() && x.scalar_type() == at::kHalf)) {
             const int64_t K = x.size(1), N = W.size(2), r = A.size(2);
             dA = at::empty({E, K, r}, dout.options());
             dB = at::empty({E, r, N}, dout.options());
             Tensor dx = at::empty({L, K}, x.options()), ws = bytes_on(x, moe_linear_lora_bwd_workspace_bytes(L, (int)E, K, N, (int)r));
-            const int rc = moe_linear_lora_bwd(ptr(dout), dout.stride(0), (int)gate_fan, ptr(gates), gates.defined() ? dtype_code(gates) : 0, ptr(x), x.stride(0), (int)k, ptr(W), W.stride(0),
+            const int rc = moe_linear_lora_bwd(ptr(dout), dout.stride(0), (int)gate_fan, ptr(coeff), gates.defined() ? dtype_code(gates) : 0, ptr(x), x.stride(0), (int)k, ptr(W), W.stride(0),
                                                W.stride(1), W.stride(2), ptr(A), A.stride(0), A.stride(1), A.stride(2), ptr(B), B.stride(0), B.stride(1), B.stride(2),
                                                (int)r, (float)scaling, ptr(dA), dA.stride(0), dA.stride(1), dA.stride(2), ptr(dB), dB.stride(0), dB.stride(1),
                                                dB.stride(2), ptr(dx), dx.stride(0), ptr(ssi), is64(ssi), ptr(eo), is64(eo), (int)E, L, K, N, dtype_code(x), ptr(ws),
@@ -793,7 +795,7 @@ variable_list layer(const Tensor& x, const Tensor& wg, const Tensor& w1_, const 
         return linear_checked(in, n_contiguous ? W : W.transpose(1, 2), lt[ia], lt[ia + 1], scaling, scaling, fan, sei, ssi, offsets, Tensor(), gin, true);
     };
     Tensor h;
-    if (!rank && x.scalar_type() == at::kFloat && !needs_node({&x, &w1, &w3})) {   // both projections and their product in one launch (three: 256 tokens, d=128, f=256: 20 us, one 10.4)
+    if (!rank && x.scalar_type() == at::kFloat && so.R > 0 && d > 0 && f > 0 && !needs_node({&x, &w1, &w3})) {   // both projections and their product in one launch (three: 256 tokens, d=128, f=256: 20 us, one 10.4)
         h = at::empty({so.R, f}, x.options());
         check(moe_swiglu_pair(ptr(x), x.stride(0), x.stride(1), ptr(w1), ptr(w3), f * d, 1, d, ptr(h), h.stride(0), so.ssi(), 0, so.offsets(), 0, (int)E, so.R, d, f, (int)k,
                               dtype_code(x), stream_of(x)), "moe_swiglu_pair");

@@ -782,6 +782,15 @@ def test_tiny_and_empty_batches(dev, oracle, T, r):
             assert float(lt[n][0].grad[unused].abs().max()) == 0.0 and float(lt[n][1].grad[unused].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_empty_batch_without_gradients(dev, dtype):
+    import moe_distributed_training_amd as moe
+    x, wg, w1, w2, w3, _, _ = (t.to(dev) if torch.is_tensor(t) else t for t in _make(1, 64, 128, 8, 0, dtype, seed=5))
+    with torch.no_grad():
+        out, ew, ei = moe.moe_layer_forward(x[:0], wg, w1, w2, w3, 2, None, 32.0)
+    assert out.shape == (0, 64) and ew.shape == (0, 2) and ei.shape == (0, 2)
+
+
 @pytest.mark.parametrize("seed", range(16))
 def test_layer_seeded_shape_sweep(dev, oracle, seed):
     """Seeded draws over the supported shape space of the fused layer (hidden and ffn sizes that are multiples of 64 but

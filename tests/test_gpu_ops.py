@@ -610,6 +610,33 @@ def test_projection_backward_on_gathered_rows(dev, oracle, dtype, T, E, k, K, N,
     check_expert_grads(Ad.grad, Ao.grad, tol, "dA"); check_expert_grads(Bd.grad, Bo.grad, tol, "dB")
     if gates:
         assert rel(Gd.grad, Go.grad) < tol
+
+
+@pytest.mark.parametrize("hooked", [False, True])
+def test_projection_backward_of_gated_fp16_rows_near_the_largest_number(dev, oracle, hooked):
+    """dY of up to 3e4 under gates of 1e-3: dY B^T alone passes 65504, every gradient is finite, as the product of the weighted rows is; and the same
+    where a saved-tensor hook hands the gates back with other strides."""
+    import moe_distributed_training_amd as moe
+    torch.manual_seed(3)
+    T, E, k, K, N, r = 64, 2, 2, 256, 256, 16
+    _, sei, ssi, eo = _routing(oracle, T, E, k, T)
+    h = lambda *s: torch.randn(*s)
+    X, W, A, B = h(T, K).half(), (h(E, K, N) * 0.02).half(), (h(E, K, r) * 0.1).half(), h(E, r, N).half()
+    G, dY = 1e-3 * (0.5 + torch.rand(T, k)), ((torch.rand(T, N) * 2 - 1) * 3e4).half()
+    f32 = lambda t: t.float().clone().requires_grad_(True)
+    Xo, Ao, Bo, Go = f32(X), f32(A), f32(B), f32(G)
+    oracle.parallel_linear_lora(Xo, W.float(), Ao, Bo, r, 32.0, k, sei, ssi, None, eo, Go, False, False).backward(dY.float())
+    Xd, Ad, Bd, Gd = (t.to(dev).requires_grad_(True) for t in (X, A, B, G))
+    pb, eod = moe.padded_block_indices(sei.to(dev), E)
+    turn = lambda t: t.t().contiguous().t() if hooked and t.shape == (T, k) else t   # (the gates; same values, strides (1, T))
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, turn):
+        y = moe.parallel_linear_lora(Xd, W.to(dev), Ad, Bd, r, 32.0, k, sei.to(dev), ssi.to(dev), pb, eod, Gd, False, False)
+        y.backward(dY.to(dev))
+    tol = TOL[torch.float16] * 1.5
+    for got, want in ((Xd, Xo), (Ad, Ao), (Bd, Bo), (Gd, Go)):
+        assert torch.isfinite(got.grad).all() and rel(got.grad, want.grad) < tol
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("k,n_extra,cols", [(1, 1, 64), (2, 8, 4096), (3, 9, 72), (4, 64, 1032), (8, 33, 2048), (0, 16, 256), (2, 1025, 64)])
 def test_combine_with_a_dense_tail(dev, dtype, k, n_extra, cols):
