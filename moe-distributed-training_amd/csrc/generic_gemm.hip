@@ -3,6 +3,7 @@
 // sizes, unaligned views).  fp32 accumulation, fixed summation order.
 #include "common.h"
 #include "kernels.h"
+#include <type_traits>
 
 namespace {
 
@@ -92,7 +93,9 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_gemm_kernel(
     if (mval && n0 + tx < N) Elem<T>::st(Y + out_row * sym + (n0 + tx) * syn, acc);
 }
 
-// O[e][k][n] = scale * sum_{m in group e} X[m][k] * Y[m][n];  zero for an empty group.
+// O[e][k][n] = scale * sum_{m in group e} X[m][k] * Y[m][n];  zero for an empty group.  The last step is worked through in pieces of GT rows, as far
+// as it holds rows, and a group of one piece by itself: the products are bound by their LDS reads (8 of 2048 x 2048, fp32: one row per
+// expert 82 us, 260 as a whole step; 300 rows 1214 and 1274).
 template <typename T>
 __global__ void __launch_bounds__(GT * GT) generic_grouped_xty_kernel(
     const T* __restrict__ X, int64_t sxm, int64_t sxk, const T* __restrict__ Yp, int64_t sym, int64_t syn,
@@ -106,6 +109,17 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_xty_kernel(
     const int64_t end = load_idx(offsets, e, off64);
     const int tx = threadIdx.x % GT, ty = threadIdx.x / GT;
     const int64_t k0 = (int64_t)blockIdx.x * GT, n0 = (int64_t)blockIdx.y * GT;
+    if (end - start <= GT) {
+        const int64_t m = start + ty;
+        xs[ty][tx] = (m < end && k0 + tx < K) ? Elem<T>::ld(X + m * sxm + (k0 + tx) * sxk) : 0.f;
+        ys[ty][tx] = (m < end && n0 + tx < N) ? Elem<T>::ld(Yp + m * sym + (n0 + tx) * syn) : 0.f;
+        __syncthreads();
+        float sum = 0.f;
+#pragma unroll
+        for (int q = 0; q < GT; ++q) sum = fmaf(xs[q][ty], ys[q][tx], sum);
+        if (k0 + ty < K && n0 + tx < N) Elem<T>::st(O + (int64_t)e * soe + (k0 + ty) * sok + (n0 + tx) * son, sum * scale);
+        return;
+    }
     auto load = [&](int64_t m0, float* xv, float* yv) {
 #pragma unroll
         for (int i = 0; i < GPT; ++i) {
@@ -123,9 +137,13 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_xty_kernel(
             ys[ty + i * GT][tx] = yv[i];
         }
         __syncthreads();
-        if (m0 + GK < end) load(m0 + GK, xv, yv);
+        auto multiply = [&](int first, auto length) {
 #pragma unroll
-        for (int mm = 0; mm < GK; ++mm) acc = fmaf(xs[mm][ty], ys[mm][tx], acc);
+            for (int q = 0; q < decltype(length)::value; ++q) acc = fmaf(xs[first + q][ty], ys[first + q][tx], acc);
+        };
+        if (m0 + GK < end) load(m0 + GK, xv, yv);
+        if (m0 + GK <= end) multiply(0, std::integral_constant<int, GK>{});
+        else for (int mm = 0; m0 + mm < end; mm += GT) multiply(mm, std::integral_constant<int, GT>{});
         __syncthreads();
     }
     if (k0 + ty < K && n0 + tx < N) Elem<T>::st(O + (int64_t)e * soe + (k0 + ty) * sok + (n0 + tx) * son, acc * scale);
