@@ -11,13 +11,16 @@ constexpr int GT = 16;   // tile edge; workgroup is GT x GT threads
 // Contraction elements per step.  A step costs a trip to memory and two barriers whatever its length (the tiles are small and
 // so are the launches), and the next step's operands are requested before the present one is worked through.  fp32, 512 rows over 4
 // experts: 128 x 256 9.6 -> 8.2 us, 256 x 128 12.6 -> 9.9 against steps of 16 without the request ahead (same sums, same order).
-constexpr int GK = 64;
-constexpr int GPT = GT * GK / (GT * GT);   // elements of an operand tile per thread
+// Products that steps of 64 would pad by more than a quarter take steps of 16: what a step lacks is worked through as zeros (2048 rows, K x 2048, fp32,
+// steps of 16 and of 64: K=8 27 and 46 us, 40 38 and 45, 72 54 and 76, 128 79 and 76).  Products with adapters do so too: their time is that of the
+// loads of the factors, which more elements per thread do not overlap (rank 16, K=64 137 and 143, 128 241 and 250).
+constexpr int GK = 64, GK_SHORT = 16;
+inline bool short_steps(int64_t K, bool adapters) { return adapters || (K + GK - 1) / GK * GK * 4 > 5 * K; }
 
 // PAIR: two weights without adapters (gate, up) and Y = silu(gate) * up, the arithmetic of the separate launches (fp32: bit for bit).
 // Y[out_row(m)][n] = sum_k X[in_row(m)][k] * (W[e][k][n] + scaling * sum_r A[e][k][r] * B[e][r][n])
 // m runs over sorted positions; tiles of GT rows never straddle experts (find_row_tile on the offsets).
-template <typename T, bool PAIR>
+template <typename T, bool PAIR, int GK>
 __global__ void __launch_bounds__(GT * GT) generic_grouped_gemm_kernel(
     const T* __restrict__ X, int64_t sxm, int64_t sxk, const T* __restrict__ W, const T* __restrict__ W_up, int64_t swe, int64_t swk, int64_t swn,
     const T* __restrict__ A, int64_t sae, int64_t sak, int64_t sar, const T* __restrict__ B, int64_t sbe, int64_t sbr,
@@ -25,6 +28,7 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_gemm_kernel(
     const void* __restrict__ offsets, int off64, int E, int64_t K, int64_t N, int rank, int fan_out, float scaling,
     int x_grouped, int y_grouped)
 {
+    constexpr int GPT = GT * GK / (GT * GT);   // elements of an operand tile per thread
     __shared__ float xs[GT][GK + 1];   // [row][k]
     __shared__ float ws[GK][GT + 1];   // [k][n]
     __shared__ float wu[PAIR ? GK : 1][GT + 1];
@@ -102,6 +106,7 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_xty_kernel(
     T* __restrict__ O, int64_t soe, int64_t sok, int64_t son, const void* __restrict__ offsets, int off64, int64_t K,
     int64_t N, float scale)
 {
+    constexpr int GPT = GK / GT;   // elements of an operand tile per thread
     __shared__ float xs[GK][GT + 1];  // [m][k]
     __shared__ float ys[GK][GT + 1];  // [m][n]
     const int e = blockIdx.z;
@@ -160,10 +165,11 @@ int moe_launch_generic_gemm(const void* X, int64_t sxm, int64_t sxk, const void*
     if (R == 0 || N == 0) return MOE_OK;
     const int64_t mtiles = R / GT + E;  // upper bound on sum_e ceil(c_e / GT)
     dim3 grid((unsigned)mtiles, (unsigned)((N + GT - 1) / GT));
-    MOE_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((generic_grouped_gemm_kernel<T, false>), grid, dim3(GT * GT), 0, stream,
-                                                 (const T*)X, sxm, sxk, (const T*)W, (const T*)nullptr, swe, swk, swn, (const T*)A, sae, sak,
-                                                 sar, (const T*)B, sbe, sbr, sbn, (T*)Y, sym, syn, pos, pos64, offsets,
-                                                 off64, E, K, N, rank, fan_out, scaling, x_grouped, y_grouped));
+    MOE_DISPATCH_DTYPE(dtype, {
+        auto kern = short_steps(K, A != nullptr) ? generic_grouped_gemm_kernel<T, false, GK_SHORT> : generic_grouped_gemm_kernel<T, false, GK>;
+        hipLaunchKernelGGL(kern, grid, dim3(GT * GT), 0, stream, (const T*)X, sxm, sxk, (const T*)W, (const T*)nullptr, swe, swk, swn, (const T*)A, sae, sak,
+                           sar, (const T*)B, sbe, sbr, sbn, (T*)Y, sym, syn, pos, pos64, offsets, off64, E, K, N, rank, fan_out, scaling, x_grouped, y_grouped);
+    });
     return moe_launch_status();
 }
 
@@ -173,7 +179,8 @@ int moe_launch_generic_swiglu_pair(const float* X, int64_t sxm, int64_t sxk, con
 {
     if (R == 0 || N == 0) return MOE_OK;
     dim3 grid((unsigned)(R / GT + E), (unsigned)((N + GT - 1) / GT));
-    hipLaunchKernelGGL((generic_grouped_gemm_kernel<float, true>), grid, dim3(GT * GT), 0, stream, X, sxm, sxk, W_gate, W_up, swe, swk, swn, (const float*)nullptr,
+    auto kern = short_steps(K, false) ? generic_grouped_gemm_kernel<float, true, GK_SHORT> : generic_grouped_gemm_kernel<float, true, GK>;
+    hipLaunchKernelGGL(kern, grid, dim3(GT * GT), 0, stream, X, sxm, sxk, W_gate, W_up, swe, swk, swn, (const float*)nullptr,
                        0, 0, 0, (const float*)nullptr, 0, 0, 0, H, ldh, 1, pos, pos64, offsets, off64, E, K, N, 0, fan_out, 0.f, 0, 1);
     return moe_launch_status();
 }
