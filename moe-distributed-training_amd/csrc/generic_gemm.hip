@@ -49,9 +49,11 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_gemm_kernel(
     const T* We = W + (int64_t)rt.expert * swe;
     const T* Ae = A ? A + (int64_t)rt.expert * sae : nullptr;
     const T* Be = B ? B + (int64_t)rt.expert * sbe : nullptr;
-    // Which elements of an operand tile a thread loads: neighbours along the operand's own contiguous direction.
+    // Which elements of an operand tile a thread loads: neighbours along the operand's own contiguous direction.  An adapter's factors are fetched
+    // once per rank and the weight once: a B that is contiguous along n decides, where A is not along k (rank 16, 256 x 512, 2048 rows, k-contiguous
+    // weights, fp32: 145 us along n, 584 along k, where every lane of A's loads is a row of its own).
     const int tid = threadIdx.x, nrows = (int)(rt.row1 - rt.row0);
-    const bool w_along_k = swk == 1;
+    const bool w_along_k = swk == 1 && !(Ae && sbn == 1 && sak != 1);
     const T* Wu = PAIR ? W_up + (int64_t)rt.expert * swe : nullptr;
     auto load = [&](int64_t k0, float* xv, float* wv, float* uv) {
 #pragma unroll

@@ -745,3 +745,16 @@ def test_a_projection_of_few_columns_is_not_worked_through_as_of_many(dev):
         return _us(lambda: ops.scatter2scatter(x, w, sei, ssi, 1))
     few, many = projection(8), projection(64)
     assert few < 0.8 * many, (few, many)
+
+
+def test_factors_decide_the_direction_of_the_generic_product(dev):
+    """Adapters contiguous along the output beside weights contiguous along the contraction: 145 us with loads along the output, 584 with
+    loads along the contraction, 122 with both contiguous along the output."""
+    ops = _ops()
+    E, K, N, r, T = 8, 256, 512, 16, 2048
+    x, w = torch.randn(T, K, device=dev), torch.randn(E, N, K, device=dev).permute(0, 2, 1)
+    a, b = torch.randn(E, K, r, device=dev), torch.randn(E, r, N, device=dev)
+    sei, ssi = torch.arange(E, device=dev).repeat_interleave(T // E), torch.randperm(T, device=dev)
+    time = lambda w: _us(lambda: ops.scatter2scatter_lora(x, w, a, b, 1.0, sei, ssi, 1, None))
+    along_k, along_n = time(w), time(w.contiguous())
+    assert along_k < 1.8 * along_n, (along_k, along_n)
