@@ -180,8 +180,9 @@ template <typename T> struct Raw8 {
 // tokens and 128 columns, and of every four of the tail's rows each lane fetches 8 columns of one (lane i + 16 g: columns 8 i .. 8 i + 7 of row
 // g, which are the second operand of eight v_mfma_f32_16x16x4) and one coefficient (token i).  Accumulator u holds column 8 i + u of
 // tokens 4 g .. 4 g + 3; it starts with their k rows' sum.  fp32 products and sums as before, rows first, then the tail in order.
-// One token per workgroup fetched and unpacked the whole tail for every token, one row after the other: 2048 tokens, top-8, d=2048, 64 experts
-// 51 us, this 33; 4096 tokens, top-2, d=4096, 8 experts 27.4 and 27, where the rows' traffic is all that counts.
+// One token per workgroup fetches and unpacks the whole tail for every token, one row after the other: 2048 tokens, top-8, d=2048, 64 experts
+// 39 us (51 behind the layer's other launches), this 25 (33).  Where the rows' traffic is all that counts, that kernel's whole rows are the
+// better pattern: the launcher's rule.
 constexpr int CT_TOKENS = 16, CT_WCOLS = 128, CT_COLS = ROW_THREADS / 64 * CT_WCOLS;
 template <typename T, int KMAX>
 __global__ void __launch_bounds__(ROW_THREADS, 4) combine_tail_kernel(const T* __restrict__ y, int64_t ldy, T* __restrict__ out, int64_t ldo,
@@ -470,10 +471,18 @@ int moe_launch_combine_fwd(const void* y, int64_t ldy, void* out, int64_t ldo, c
     if (ntok == 0 || ncols == 0) return MOE_OK;
     MOE_DISPATCH_DTYPE(dtype, {
         const int vo = vec_aligned<T>(y, ldy) && vec_aligned<T>(out, ldo) && (!extra_rows || vec_aligned<T>(extra_rows, lde));
-        // A tail of more than eight rows always, a shorter one where 16 tokens x 128 columns per wave give every SIMD a wave: below that one token
-        // per workgroup is done sooner (512 tokens, d=256, 8 experts: 4.0 us against 5.5; 64 experts there would take it 50).
-        const int64_t tail_waves = (ntok + CT_TOKENS - 1) / CT_TOKENS * ((ncols + CT_WCOLS - 1) / CT_WCOLS);
-        if (vo && n_extra > 0 && k <= 8 && ncols % 8 == 0 && (n_extra > 8 || k == 0 || tail_waves >= 4 * (int64_t)moe_device_cus()) && (ncols + CT_COLS - 1) / CT_COLS <= 65535) {
+        // The tail on the matrix instructions: without rows always (8192 tokens, d=4096, 8 rows of tail: 30.0 us one token per workgroup, 17.2 so).  With
+        // rows, which that kernel fetches in pieces of 256 bytes, never for a tail of up to eight (8192 tokens, d=4096, new buffers for each call:
+        // top-2 51.2 and 54.7, top-4 72 and 88), and above where the tail is what one token per workgroup takes longest for: its n_extra
+        // steps per pass over the columns or per round of workgroups (eight of them per compute unit) against the k rows' share
+        // (2048 tokens, top-8, d=2048, 16 / 32 / 64 rows: 19.3 / 25.9 / 38.9 us and 18.9 / 20.9 / 25.2; 1000 tokens, top-4, 16 / 64 / 96: 5.8 / 12.6 / 17.0
+        // and 9.5 / 15.4 / 18.8; 512 tokens, top-2, d=4096, 16 / 64: 8.1 / 22 and 5.5 / 8.7).  Rows beyond the last-level cache: more than
+        // three rows of tail per row (8192 tokens, d=4096, top-8, 16 / 32: 135 / 175 and 165 / 171; top-4, 16 / 24: 87 / 103 and 88 / 92).
+        const int64_t passes = (ncols + ROW_THREADS * Vec8<T>::N - 1) / (ROW_THREADS * Vec8<T>::N), resident = 8 * (int64_t)moe_device_cus();
+        const int64_t steps = passes * resident > ntok ? n_extra * passes : n_extra * ntok / resident;
+        const bool beyond_cache = ntok * k * ncols * (int64_t)sizeof(T) >= ((int64_t)1 << 28);
+        const bool tail = n_extra > 0 && (k == 0 || (n_extra > 8 && (beyond_cache ? n_extra > 3 * k : steps >= 6 * k + 8)));
+        if (vo && tail && k <= 8 && ncols % 8 == 0 && (ncols + CT_COLS - 1) / CT_COLS <= 65535) {
             auto kern = k <= 2 ? combine_tail_kernel<T, 2> : (k <= 4 ? combine_tail_kernel<T, 4> : combine_tail_kernel<T, 8>);
             hipLaunchKernelGGL(kern, dim3((unsigned)((ntok + CT_TOKENS - 1) / CT_TOKENS), (unsigned)((ncols + CT_COLS - 1) / CT_COLS)), dim3(ROW_THREADS), 0, stream,
                                (const T*)y, ldy, (T*)out, ldo, gates, gdtype, inv, k, ntok, ncols, extra_coef, (const T*)extra_rows, lde, n_extra);
