@@ -78,10 +78,11 @@ int moe_router_logits(const void* x, int64_t ldx, const void* wg, int64_t ldw, i
  * division by the sum of the selected scores (config_utils.py:264-270).  scores (T,E), topw (T,k) fp32, topi (T,k) int32. */
 int moe_router_topk(const float* logits, float* scores, float* topw, int32_t* topi, int64_t ntok, int E, int k,
                     int renorm, void* stream);
-/* both of the above in one call (config_utils.py:262-270): logits (T,E), scores (T,E), topw (T,k), topi (T,k); a single
- * launch when x and the router weight are a 2-byte type, E <= 8 and d is a multiple of 32 (logits on the matrix cores,
- * eight partial sums per logit added in a fixed order: the same top-k indices as moe_router_logits + moe_router_topk,
- * logits equal to theirs up to fp32 rounding, not bit for bit), the two kernels of those entry points otherwise. */
+/* both of the above in one call (config_utils.py:262-270): logits (T,E), scores (T,E), topw (T,k), topi (T,k).  With up to 96 experts, x and the
+ * router weight of a 2-byte type and d a multiple of 32 (16-byte aligned rows) the logits come from the matrix cores, eight partial sums per logit
+ * added in a fixed order: equal to those of moe_router_logits up to fp32 rounding, not bit for bit (where two logits of a token differ by no
+ * more than that, the choice may), and the same for a token in any batch.  Otherwise they are those of moe_router_logits.  scores, topw
+ * and topi are moe_router_topk of the logits in every case; one launch or two. */
 int moe_router_forward(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits, float* scores,
                        float* topw, int32_t* topi, int64_t ntok, int64_t d, int E, int k, int renorm, void* stream);
 /* gradient of moe_router_topk with respect to the logits given d(topw); the reference obtains it from autograd. */

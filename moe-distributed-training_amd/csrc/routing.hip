@@ -321,7 +321,11 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_kernel(const T* __r
 // summed by the instruction, the steps and the waves in 64 bits: the loads hide these adds (21.1 us with fp32 accumulators too), and chained in fp32
 // the logits of 2048 bf16 columns were 1.03e-7 from 64 bits (relative 2-norm) where the vector kernels are 7.5e-8 and this 4.7e-8; 96 experts, 3072
 // columns 1.22e-7, 8.0e-8 and 4.6e-8; fp16 1.14e-7 (vector) and 5.7e-8.
-template <typename T, int EG>
+// TOPK = false: the logits of one expert group per workgroup (blockIdx.y), the same sums, for few tokens of many experts: one workgroup for all of
+// them fetches every weight through one compute unit.  A batch that is not whole leaves out its loads: as repeats of the last
+// step's they made 16 experts of d=512 11.4 us where the vector kernels take 8.0 and this 5.2.  (Not with four groups and more, which
+// run for many tokens only: a loop of its own for whole batches takes registers for one wave per SIMD less, 16384 x 96 x 4096 119 -> 133 us.)
+template <typename T, int EG, bool TOPK>
 __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_wide_kernel(const T* __restrict__ x, int64_t ldx, const T* __restrict__ wg, int64_t ldw,
                                                                          float* __restrict__ logits, float* __restrict__ scores,
                                                                          float* __restrict__ topw, int32_t* __restrict__ topi, int64_t ntok, int d,
@@ -330,15 +334,16 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_wide_kernel(const T
     constexpr int BATCH = EG == 1 ? 16 : EG == 2 ? 8 : 4;
     constexpr int EW = EG * 16;
     __shared__ float s_part[RM_WAVES][RM_TOKENS][EW];
-    __shared__ float s_logits[RM_TOKENS][EW];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ float s_logits[TOPK ? RM_TOKENS : 1][EW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t t0 = (int64_t)blockIdx.x * RM_TOKENS;
+    const int e0 = TOPK ? 0 : (int)blockIdx.y * EW;
     const int row = lane & 15, kc = lane >> 4;
     const int64_t tok = (t0 + row < ntok) ? t0 + row : ntok - 1;      // tokens past the end re-read the last one
     const T* xp = x + tok * ldx + kc * 8;
     const T* wp[EG];
 #pragma unroll
-    for (int g = 0; g < EG; ++g) wp[g] = wg + (int64_t)(g * 16 + row < E ? g * 16 + row : E - 1) * ldw + kc * 8;   // (rows past the last expert repeat it; nobody reads their logits)
+    for (int g = 0; g < EG; ++g) wp[g] = wg + (int64_t)(e0 + g * 16 + row < E ? e0 + g * 16 + row : E - 1) * ldw + kc * 8;   // (rows past the last expert repeat it; nobody reads their logits)
     const int nsteps = d / 32;
     const int s_end = nsteps * (wave + 1) / RM_WAVES;
     double acc[EG][4];
@@ -346,26 +351,38 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_wide_kernel(const T
     for (int g = 0; g < EG; ++g)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[g][r] = 0.0;
-    for (int s0 = nsteps * wave / RM_WAVES; s0 < s_end; s0 += BATCH) {
+    using Num = typename std::conditional<std::is_same<T, __hip_bfloat16>::value, NumBf16, NumF16>::type;
+    // ALL: every step of the batch is the wave's.  REPEAT: loads past the wave's steps repeat the last one's.
+    auto steps = [&](int s0, auto ALL, auto REPEAT) {
+        auto mine = [&](int i) { return decltype(ALL)::value || s0 + i < s_end; };
         uint4 xa[BATCH], wa[BATCH][EG];
 #pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-            const int64_t st = (int64_t)((s0 + i < s_end) ? s0 + i : s_end - 1) * 32;
-            xa[i] = *(const uint4*)(xp + st);
+        for (int i = 0; i < BATCH; ++i)
+            if (decltype(REPEAT)::value || mine(i)) {
+                const int st = (mine(i) ? s0 + i : s_end - 1) * 32;
+                xa[i] = *(const uint4*)(xp + st);
 #pragma unroll
-            for (int g = 0; g < EG; ++g) wa[i][g] = *(const uint4*)(wp[g] + st);
-        }
+                for (int g = 0; g < EG; ++g) wa[i][g] = *(const uint4*)(wp[g] + st);
+            }
 #pragma unroll
         for (int i = 0; i < BATCH; ++i)
-            if (s0 + i < s_end) {
+            if (mine(i)) {
 #pragma unroll
                 for (int g = 0; g < EG; ++g) {
-                    using Num = typename std::conditional<std::is_same<T, __hip_bfloat16>::value, NumBf16, NumF16>::type;
                     const f32x4_t p = Num::mfma(__builtin_bit_cast(bf16x8_t, wa[i][g]), __builtin_bit_cast(bf16x8_t, xa[i]), (f32x4_t){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                     for (int r = 0; r < 4; ++r) acc[g][r] += (double)p[r];
                 }
             }
+    };
+    const int s_begin = nsteps * wave / RM_WAVES;
+    if (EG > 2) {
+        for (int s0 = s_begin; s0 < s_end; s0 += BATCH) steps(s0, std::false_type{}, std::true_type{});
+    } else {
+        for (int s0 = s_begin; s0 < s_end; s0 += BATCH) {
+            if (s0 + BATCH <= s_end) steps(s0, std::true_type{}, std::false_type{});
+            else steps(s0, std::false_type{}, std::false_type{});
+        }
     }
     // acc[g][r] = partial logit of token `row`, expert 16 g + 4 kc + r
 #pragma unroll
@@ -377,9 +394,10 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_wide_kernel(const T
 #pragma unroll
         for (int w = 1; w < RM_WAVES; ++w) dsum += (double)s_part[w][t][e];
         const float sum = (float)dsum;
-        s_logits[t][e] = sum;
-        if (e < E && t0 + t < ntok) logits[(t0 + t) * E + e] = sum;
+        if (TOPK) s_logits[t][e] = sum;
+        if (e0 + e < E && t0 + t < ntok) logits[(t0 + t) * E + e0 + e] = sum;
     }
+    if (!TOPK) return;
     __syncthreads();
     if (tid < RM_TOKENS * TK_LANES) {   // whole waves
         const int tt = tid / TK_LANES;
@@ -847,13 +865,25 @@ int moe_launch_router_forward(const void* x, int64_t ldx, const void* wg, int64_
     }
     const unsigned grid = (unsigned)((ntok + RM_TOKENS - 1) / RM_TOKENS);
     if (E > ROUTER_EXPERT_GROUP) {
+        // One launch, or one workgroup per token and expert group and top-k in a launch of its own, the same bits.  With 48 experts and more the
+        // latter is sooner while its workgroups fit the chip (16 tokens, 96 experts, d=4096: 17.7 us against 33.5, and 25.7 for the
+        // vector kernels; d=512 11.2, 12.1 and 12.5; 1024 tokens, 64 experts, d=4096 15.8 and 25.3, 2048 tokens 24.9 and 26), with more
+        // than 64, whose one launch is the slowest, also in one and a half rounds (1024 tokens, 96 experts, d=4096: 26.1 and 34).
+        const int64_t parts = (int64_t)grid * ((E + 15) / 16), cus = moe_device_cus();
+        const bool apart = E > 32 && parts <= (E > 64 ? cus * 3 / 2 : cus);
         auto wide = [&](auto tag) {
             using T = decltype(tag);
-            auto kern = E <= 16 ? router_mfma_wide_kernel<T, 1> : E <= 32 ? router_mfma_wide_kernel<T, 2> : E <= 64 ? router_mfma_wide_kernel<T, 4> : router_mfma_wide_kernel<T, 6>;
+            if (apart) {
+                hipLaunchKernelGGL((router_mfma_wide_kernel<T, 1, false>), dim3(grid, (unsigned)((E + 15) / 16)), dim3(RM_WAVES * 64), 0, stream, (const T*)x, ldx, (const T*)wg, ldw, logits,
+                                   nullptr, nullptr, nullptr, ntok, (int)d, E, 0, 0);
+                return;
+            }
+            auto kern = E <= 16 ? router_mfma_wide_kernel<T, 1, true> : E <= 32 ? router_mfma_wide_kernel<T, 2, true> : E <= 64 ? router_mfma_wide_kernel<T, 4, true> : router_mfma_wide_kernel<T, 6, true>;
             hipLaunchKernelGGL(kern, dim3(grid), dim3(RM_WAVES * 64), 0, stream, (const T*)x, ldx, (const T*)wg, ldw, logits, scores, topw, topi, ntok, (int)d, E, k, renorm);
         };
         if (dtype == MOE_BF16) wide(__hip_bfloat16{}); else wide(__half{});
-        return moe_launch_status();
+        const int rc = moe_launch_status();
+        return rc != MOE_OK || !apart ? rc : moe_launch_router_topk(logits, scores, topw, topi, ntok, E, k, renorm, stream);
     }
     auto few = [&](auto tag) {
         using T = decltype(tag);

@@ -417,3 +417,45 @@ def test_router_of_many_experts_on_the_matrix_cores(dev, oracle, dtype, T, d, E,
     assert torch.allclose(s.cpu(), so, atol=1e-6) and torch.allclose(w.cpu(), wo, atol=1e-5)
     s1, w1, i1 = router.router_topk(l, k)
     assert torch.equal(s, s1) and torch.equal(w, w1) and torch.equal(i, i1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("E,k,d", [(33, 3, 544), (48, 2, 512), (64, 8, 2048), (65, 2, 96), (96, 8, 1056)])
+def test_a_token_is_routed_the_same_in_any_batch(dev, dtype, E, k, d):
+    """The router of many experts in one launch (3000 tokens) and with top-k in a launch of its own (1 to 200), batches of steps that are
+    whole and that are not: logits, scores, weights and choices of a token are the same bits."""
+    _, router, _ = _mods()
+    g = torch.Generator(device=dev).manual_seed(E)
+    x, wg = torch.randn(3000, d, generator=g, device=dev).to(dtype), (torch.randn(E, d, generator=g, device=dev) / d ** 0.5).to(dtype)
+    whole = router.router_forward(x, wg, k)
+    for a, b in ((0, 1), (1, 18), (100, 300), (2990, 3000)):
+        for part, full in zip(router.router_forward(x[a:b], wg, k), whole):
+            assert torch.equal(part, full[a:b])
+
+
+@pytest.mark.parametrize("T,E,d", [(16, 96, 4096), (256, 64, 8192), (256, 16, 512), (1024, 96, 512)])
+def test_router_in_one_launch_is_not_slower_than_in_two(dev, T, E, d):
+    """Against the vector kernels' two launches, where one workgroup for 16 tokens and all experts took longer than those (33 us against 26, 42 and
+    36, 11.4 and 8.0, 16.0 and 14.9)."""
+    _, router, _ = _mods()
+    x, wg = torch.randn(T, d, device=dev).bfloat16(), torch.randn(E, d, device=dev).bfloat16() * 0.02
+
+    def us(fn):
+        graph = torch.cuda.CUDAGraph()   # (the kernels' own time: no host work between the calls)
+        fn()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                fn()
+        times = []
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b) * 50)
+        return min(times[1:])
+
+    one, two = us(lambda: router.router_forward(x, wg, 2)), us(lambda: router.router_topk(router.router_logits(x, wg), 2))
+    assert one < 1.05 * two, (one, two)
