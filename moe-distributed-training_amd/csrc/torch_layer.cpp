@@ -707,7 +707,8 @@ struct LayerFn : Function<LayerFn> {
     static variable_list backward(AutogradContext* ctx, variable_list g_)
     {
         const auto sv = ctx->get_saved_variables();
-        const Tensor &x = sv[0], &wg = sv[1], &w1 = sv[2], &w3 = sv[3], &w2 = sv[4], &scores = sv[11], &weights = sv[12], &indices = sv[13], &y = sv[18];
+        const Tensor &x = sv[0], &wg = sv[1], &w1 = sv[2], &w3 = sv[3], &w2 = sv[4], &y = sv[18];
+        const Tensor scores = sv[11].contiguous(), weights = sv[12].contiguous(), indices = sv[13].contiguous();   // (a saved-tensor hook may hand back other strides)
         const c10::DeviceGuard guard(x.device());
         const auto sz = ctx->saved_data["sizes"].toIntVector();
         const int64_t k = sz[3], T = x.size(0);

@@ -45,6 +45,17 @@ def test_checkpointing_and_saved_tensor_hooks_change_no_bit(dev, dtype, r):
         assert _same(_step(lambda v: block(v)[0], block, x, dout), want)
 
 
+@pytest.mark.parametrize("r", [R, 0])   # r = 0: all weights' gradients, whose rows take the gate weights again
+@pytest.mark.parametrize("turn", [lambda t: t.t().contiguous().t(), lambda t: torch.stack([t, t], -1)[..., 0]], ids=["columns", "every_other"])
+def test_saved_gates_of_other_strides_change_no_bit(dev, r, turn):
+    """A hook that hands the layer's scores, weights and choices back with other strides (same values)."""
+    block = _block(dev, torch.bfloat16, r)
+    x, dout = torch.randn(T, D, device=dev).bfloat16(), torch.randn(T, D, device=dev).bfloat16()
+    want = _step(lambda v: block(v)[0], block, x, dout)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: turn(t) if t.dim() == 2 and t.shape[0] == T and t.shape[1] <= 8 else t):
+        assert _same(_step(lambda v: block(v)[0], block, x, dout), want)
+
+
 def test_an_exception_of_a_pack_hook_arrives_as_itself(dev):
     class Stop(Exception):
         pass
