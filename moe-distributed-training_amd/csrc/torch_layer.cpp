@@ -83,6 +83,9 @@ inline Tensor bytes_on(const Tensor& like, size_t n)
     return at::empty({(int64_t)(n < 256 ? 256 : n)}, like.options().dtype(at::kByte));
 }
 
+// the gate weights one after the other, as the kernels read them (a saved-tensor hook may hand them back with strides that a reshape keeps)
+inline Tensor flat_gates(const Tensor& g) { return g.defined() ? g.reshape({-1}).contiguous() : Tensor(); }
+
 inline Tensor unit_inner(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
 
 // Whether the call has to go through its autograd node: a gradient is recorded, or an input carries a forward-mode tangent
@@ -339,8 +342,9 @@ RouterOut router_forward(const Tensor& x, const Tensor& wg, int64_t k, bool norm
     return o;
 }
 
-Tensor router_topk_bwd(const Tensor& dw, const Tensor& weights, const Tensor& indices, const Tensor& scores, bool normalize)
+Tensor router_topk_bwd(const Tensor& dw, const Tensor& weights_, const Tensor& indices_, const Tensor& scores_, bool normalize)
 {
+    const Tensor weights = weights_.contiguous(), indices = indices_.contiguous(), scores = scores_.contiguous();   // (as in flat_gates)
     Tensor d = dw.contiguous().to(at::kFloat), dl = at::empty_like(scores);
     check(moe_router_topk_bwd((const float*)ptr(d), (const float*)ptr(weights), (const int32_t*)ptr(indices), (const float*)ptr(scores), (float*)ptr(dl),
                               scores.size(0), (int)scores.size(1), (int)weights.size(1), normalize, stream_of(scores)), "moe_router_topk_bwd");
@@ -425,7 +429,7 @@ struct LinearFn : Function<LinearFn> {
         int64_t gate_fan = 1;
         if (gates.defined()) {
             d_gates = combine_dgates(y_rows, dout, gates.size(1), gates.scalar_type(), nullptr);   // reference :70-72
-            coeff = gates.reshape({-1});
+            coeff = flat_gates(gates);
             gate_fan = gates.size(1);
         }
         // All of it from the rows where they lie (shapes outside the matrix-core paths go on below).  Not for gated fp16: dY B^T is stored before its
@@ -560,7 +564,7 @@ struct GatherCombineFn : Function<GatherCombineFn> {
         Tensor dout = g[0].contiguous();
         Tensor d_w = combine_dgates(y, dout, w.size(1), w.scalar_type(), (const int32_t*)ptr(inv));
         // dy_grouped[i] = w[pos_i] * dout[pos_i // k]; pos, the inverse of inv, is the sort's own sorted_scattered_idxs
-        Tensor d_y = group_rows(dout, ptr(ssi), is64(ssi), ssi.numel(), w.size(1), w.reshape({-1}));
+        Tensor d_y = group_rows(dout, ptr(ssi), is64(ssi), ssi.numel(), w.size(1), flat_gates(w));
         return {d_y, d_w, Tensor(), Tensor()};
     }
 };
@@ -628,7 +632,7 @@ struct ExpertMlpFn : Function<ExpertMlpFn> {
         Tensor dw[3];
         const bool needs[3] = {ctx->needs_input_grad(1), ctx->needs_input_grad(2), ctx->needs_input_grad(3)};
         if (needs[0] || needs[1] || needs[2])
-            base_weight_grads(needs, x, dout, dy_grouped, dy_fan, gates.defined() ? gates.reshape({-1}) : Tensor(), g, sv[15], ptr(ssi), is64(ssi),
+            base_weight_grads(needs, x, dout, dy_grouped, dy_fan, flat_gates(gates), g, sv[15], ptr(ssi), is64(ssi),
                               ptr(offsets), is64(offsets), s, dw);
         return {d_x, dw[0], dw[1], dw[2], g.lora[0], g.lora[1], g.lora[2], g.lora[3], g.lora[4], g.lora[5], d_gates, Tensor(), Tensor(), Tensor()};
     }
