@@ -423,6 +423,8 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const v
     if (!dout || !x || !W || !A || !B || !DA || !DB || !dx_rows || !pos || !offsets || rank < 1 || E < 1 || R < 0 || K < 1 || N < 1 || fan_out < 1 || dout_fan_out < 1)
         return MOE_ERR_BAD_ARG;
     if (gates && gates_dtype != MOE_BF16 && gates_dtype != MOE_F16 && gates_dtype != MOE_F32) return MOE_ERR_BAD_ARG;
+    // dY B^T is stored before its gate weight, which in fp16 can pass 65504 where the product of the weighted rows does not
+    if (gates && dtype == MOE_F16) return MOE_ERR_UNSUPPORTED;
     const int C = (rank + 15) / 16;
     const bool nt = swn == 1, nn = swk == 1 && !nt;   // of the transposed weights (E, N, K): contraction-contiguous, output-contiguous
     if (!bwd_ab_fast(K, N, rank, dtype, ldd, 1, ldx, 1, dout, x) || C > LINEAR_BWD_MAX_CHUNKS || !(nt || nn) || R == 0) return MOE_ERR_UNSUPPORTED;

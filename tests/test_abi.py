@@ -102,3 +102,16 @@ def test_fused_layer_rank_limit_is_checked_on_the_host():
     assert saved[1] == saved[2] == 2 * saved[0] and saved[3] == 3 * saved[0] and saved[4] == 8 * saved[0]
     ws = [lib.moe_mlp_workspace_bytes(8192, 8, 4096, 14336, r) for r in (0, 16, 32, 64, 128)]
     assert ws == sorted(ws) and len(set(ws)) == 5
+
+
+def test_gated_fp16_rows_are_refused_by_the_projection_backward():
+    """dY B^T is stored before its gate weight: fp16 with gates, whose range that can pass, is refused with MOE_ERR_UNSUPPORTED before anything is
+    enqueued; bf16 with gates and fp16 without get as far as the workspace check."""
+    from moe_distributed_training_amd._lib import lib
+    one, K, N = 16, 256, 512   # (one: a non-null, 16-byte aligned stand-in, never dereferenced)
+
+    def bwd(dtype, gates):
+        return lib.moe_linear_lora_bwd(one, N, 2, gates, 2, one, K, 2, one, K * N, 1, K, one, K * 16, 16, 1, one, 16 * N, N, 1, 16, 1.0, one, K * 16, 16, 1,
+                                       one, 16 * N, N, 1, one, K, one, 0, one, 0, 4, 128, K, N, dtype, None, 0, None)
+    assert bwd(1, one) == -2
+    assert bwd(1, None) == -3 and bwd(0, one) == -3 and bwd(0, None) == -3
