@@ -156,7 +156,7 @@ int moe_scatter2scatter(const void* X, int64_t sxm, int64_t sxk, const void* W, 
  *   DA[e] = s X_e^T (dY_e B_e^T),  DB[e] = s (X_e A_e)^T dY_e,  dx_rows[p] = dY_m W_e^T + s (dY_m B_e^T) A_e^T
  * (scattermoe_utils/parallel_linear_lora.py:83-134).  MOE_ERR_UNSUPPORTED, with nothing enqueued, for shapes outside the matrix-core paths and
  * for fp16 with gates (dY B^T is stored before its gate weight, which can pass 65504 where the product of the weighted rows does not): a
- * caller then takes moe_group_rows, moe_group_bwd_ab and moe_scatter2scatter. */
+ * caller then takes moe_group_rows, moe_group_bwd_ab and moe_scatter2scatter.  The workspace query says 0 for sizes that are refused. */
 size_t moe_linear_lora_bwd_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank);
 int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const void* gates, int gates_dtype, const void* x, int64_t ldx, int fan_out,
                         const void* W, int64_t swe, int64_t swk, int64_t swn, const void* A, int64_t sae, int64_t sak, int64_t sar,

@@ -407,9 +407,16 @@ static inline size_t linear_bwd_shared_bytes(int64_t R, int E, int64_t K, int64_
     return sk > x ? sk : x;
 }
 
+// what of the sizes alone decides whether the matrix-core paths take the call
+static inline bool linear_bwd_sizes_ok(int64_t K, int64_t N, int rank)
+{
+    return rank >= 1 && (rank + 15) / 16 <= LINEAR_BWD_MAX_CHUNKS && K >= 1 && K % 32 == 0 && N >= 64 && N % 32 == 0;   // (N: the contraction of dX, a whole K tile at least)
+}
+
 size_t moe_linear_lora_bwd_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank)
 {
-    const size_t C = (size_t)((rank > 0 ? rank : 1) + 15) / 16;
+    if (!linear_bwd_sizes_ok(K, N, rank)) return 0;
+    const size_t C = (size_t)(rank + 15) / 16;
     return al(linear_bwd_shared_bytes(R, E, K, N, rank)) + C * (2 * pack_bytes(E, K) + pack_bytes(E, N) + 3 * q_bytes(R)) + al((size_t)R * sizeof(float)) + 256;
 }
 
@@ -427,7 +434,7 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const v
     if (gates && dtype == MOE_F16) return MOE_ERR_UNSUPPORTED;
     const int C = (rank + 15) / 16;
     const bool nt = swn == 1, nn = swk == 1 && !nt;   // of the transposed weights (E, N, K): contraction-contiguous, output-contiguous
-    if (!bwd_ab_fast(K, N, rank, dtype, ldd, 1, ldx, 1, dout, x) || C > LINEAR_BWD_MAX_CHUNKS || !(nt || nn) || R == 0) return MOE_ERR_UNSUPPORTED;
+    if (!bwd_ab_fast(K, N, rank, dtype, ldd, 1, ldx, 1, dout, x) || !linear_bwd_sizes_ok(K, N, rank) || !(nt || nn) || R == 0) return MOE_ERR_UNSUPPORTED;
     const int f16 = dtype == MOE_F16;
     MoeGemmParams p = {};
     p.X[0] = (const uint16_t*)dout; p.ldx = ldd; p.nseg = 1;

@@ -432,14 +432,16 @@ struct LinearFn : Function<LinearFn> {
             coeff = flat_gates(gates);
             gate_fan = gates.size(1);
         }
-        // All of it from the rows where they lie (shapes outside the matrix-core paths go on below).  Not for gated fp16: dY B^T is stored before its
-        // gate weight there, which can pass 65504 where the product of the weighted rows does not.
-        if (A.defined() && !grouped_in && !grouped_out && scaling == ctx->saved_data["scaling_ab"].toDouble() && L > 0 && W.numel() > 0 && A.size(2) > 0 &&
-            !(gates.defined() && x.scalar_type() == at::kHalf)) {
+        // All of it from the rows where they lie.  What the matrix-core paths do not take by its type or sizes goes on below before anything is
+        // allocated for them (fp16 with gates: see moe_linear_lora_bwd), what they refuse by its strides or alignment after.
+        const bool by_type = x.scalar_type() == at::kBFloat16 || (x.scalar_type() == at::kHalf && !gates.defined());
+        const size_t ws_bytes = by_type && A.defined() && !grouped_in && !grouped_out && scaling == ctx->saved_data["scaling_ab"].toDouble() && L > 0 && W.numel() > 0
+                                    ? moe_linear_lora_bwd_workspace_bytes(L, (int)E, x.size(1), W.size(2), (int)A.size(2)) : 0;
+        if (ws_bytes) {
             const int64_t K = x.size(1), N = W.size(2), r = A.size(2);
             dA = at::empty({E, K, r}, dout.options());
             dB = at::empty({E, r, N}, dout.options());
-            Tensor dx = at::empty({L, K}, x.options()), ws = bytes_on(x, moe_linear_lora_bwd_workspace_bytes(L, (int)E, K, N, (int)r));
+            Tensor dx = at::empty({L, K}, x.options()), ws = bytes_on(x, ws_bytes);
             const int rc = moe_linear_lora_bwd(ptr(dout), dout.stride(0), (int)gate_fan, ptr(coeff), gates.defined() ? dtype_code(gates) : 0, ptr(x), x.stride(0), (int)k, ptr(W), W.stride(0),
                                                W.stride(1), W.stride(2), ptr(A), A.stride(0), A.stride(1), A.stride(2), ptr(B), B.stride(0), B.stride(1), B.stride(2),
                                                (int)r, (float)scaling, ptr(dA), dA.stride(0), dA.stride(1), dA.stride(2), ptr(dB), dB.stride(0), dB.stride(1),

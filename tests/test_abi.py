@@ -115,3 +115,11 @@ def test_gated_fp16_rows_are_refused_by_the_projection_backward():
                                        one, 16 * N, N, 1, one, K, one, 0, one, 0, 4, 128, K, N, dtype, None, 0, None)
     assert bwd(1, one) == -2
     assert bwd(1, None) == -3 and bwd(0, one) == -3 and bwd(0, None) == -3
+
+
+def test_the_projection_backward_names_the_sizes_it_refuses():
+    """The workspace query is 0 for the sizes that the entry point refuses, so that a caller need not allocate to find out."""
+    from moe_distributed_training_amd._lib import lib
+    need = lambda K, N, r: lib.moe_linear_lora_bwd_workspace_bytes(128, 4, K, N, r)
+    assert all(need(*s) > 0 for s in ((32, 64, 1), (256, 512, 16), (96, 160, 64)))
+    assert all(need(*s) == 0 for s in ((256, 512, 65), (256, 512, 0), (48, 64, 16), (64, 48, 16), (64, 32, 16)))

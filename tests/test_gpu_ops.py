@@ -785,3 +785,20 @@ def test_weighted_sum_of_gathered_rows_with_a_tail(dev, dtype, gates, T, k, n_ex
     picked = y.double()[inv.long()].view(T, k, cols)
     want = (picked if w is None else picked * w.double()[:, :, None]).sum(1) + coef.double() @ rows.double()
     assert rel(got, want) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,K,N,r", [(torch.float32, 64, 96, 8), (torch.float16, 64, 96, 8), (torch.bfloat16, 64, 96, 72), (torch.bfloat16, 48, 96, 8), (torch.bfloat16, 64, 32, 8)])
+def test_projection_backward_allocates_nothing_for_the_route_that_refuses(dev, oracle, dtype, K, N, r):
+    """Gated projections that the backward on gathered rows does not take by their type or sizes: dY and X grouped, the adapters' gradients, two workspaces, the
+    gates' gradient and the fan-out sum, and no buffers of the other route."""
+    import moe_distributed_training_amd as moe
+    T, E, k = 40, 3, 2
+    _, sei, ssi, eo = _routing(oracle, T, E, k)
+    g = lambda *s: (torch.randn(*s, device=dev) * 0.1).to(dtype).requires_grad_(True)
+    x, W, A, B, G = g(T, K), g(E, K, N).detach(), g(E, K, r), g(E, r, N), g(T, k)
+    y = moe.parallel_linear_lora(x, W, A, B, r, 32.0, k, sei.to(dev), ssi.to(dev), None, eo.to(dev), gates=G)
+    dy = torch.randn_like(y)
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    n = count()
+    grads = torch.autograd.grad(y, (x, A, B, G), dy)
+    assert count() - n == 8 and len(grads) == 4
