@@ -399,11 +399,11 @@ int moe_group_bwd_ab(const void* DY, int64_t sdm, int64_t sdn, const void* X, in
 static const int LINEAR_BWD_MAX_CHUNKS = MOE_MAX_SLABS;   // 16-wide rank chunks: the dX launch takes them as slabs given by pointer
 
 // The adapter gradients' partials lie where the dX launch exchanges its K-split tiles afterwards (behind the counters, which are cleared before either)
-static inline size_t linear_bwd_counter_bytes() { return al((size_t)moe_gemm_num_counters() * sizeof(int)); }
+static inline size_t counter_bytes() { return al((size_t)moe_gemm_num_counters() * sizeof(int)); }
 static inline size_t linear_bwd_xtp_bytes(int64_t R, int E, int64_t K, int64_t N, int rank) { return (size_t)(rank > 16 ? 4 : 2) * moe_xtp_workspace_bytes(R, E, K > N ? K : N); }
 static inline size_t linear_bwd_shared_bytes(int64_t R, int E, int64_t K, int64_t N, int rank)
 {
-    const size_t sk = moe_gemm_sk_bytes(R, E, K), x = linear_bwd_counter_bytes() + linear_bwd_xtp_bytes(R, E, K, N, rank);
+    const size_t sk = moe_gemm_sk_bytes(R, E, K), x = counter_bytes() + linear_bwd_xtp_bytes(R, E, K, N, rank);
     return sk > x ? sk : x;
 }
 
@@ -449,7 +449,7 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const v
     uint8_t* shared = (uint8_t*)ws.take(linear_bwd_shared_bytes(R, E, K, N, rank));
     moe_gemm_sk_attach(p, shared, R, E, K);
     p.counters_clean = 1;   // by the packing
-    void* xw = shared + linear_bwd_counter_bytes();
+    void* xw = shared + counter_bytes();
     const size_t xb = linear_bwd_xtp_bytes(R, E, K, N, rank);
     const int64_t ldt = pad_rows(R);
     hipStream_t st = S(stream);
@@ -583,16 +583,23 @@ static inline size_t sk_bytes_mlp(int64_t R, int E, int64_t d, int64_t f)
 // column-tile partials of the two fused column contractions of the dh GEMM: [2][ceil(f / 256)][R][16] fp32
 static inline size_t cc_bytes(int64_t R, int64_t f) { return (size_t)2 * (size_t)((f + 255) / 256) * (size_t)R * 16 * sizeof(float); }
 
-// partials of the adapter gradients: with the fused products three sets of f columns (from the dh GEMM) and three of d, all alive until one
-// launch sums them; without, two sets of either at a time
-static inline size_t mlp_xtp_bytes(int64_t R, int E, int64_t d, int64_t f) { return 3 * (moe_xtp_workspace_bytes(R, E, f) + moe_xtp_workspace_bytes(R, E, d)); }
+// Partials of the adapter gradients: with the fused products (rank <= 16) three sets of f columns (from the dh GEMM) and three of d, all alive until one
+// launch sums them; without, two sets of either at a time.  The sets of d columns come when the grouped GEMMs are through: they lie
+// where those exchanged K-split tiles, behind the counters, or where that is too small in place of the column-tile partials, which have been added by then.
+static inline size_t mlp_xtp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank) { return 3 * moe_xtp_workspace_bytes(R, E, rank <= 16 || f > d ? f : d); }
+static inline bool mlp_xtp_d_in_exchange(int64_t R, int E, int64_t d, int64_t f) { return counter_bytes() + 3 * moe_xtp_workspace_bytes(R, E, d) <= sk_bytes_mlp(R, E, d, f); }
+static inline size_t mlp_cc_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
+{
+    const size_t cc = cc_bytes(R, f), x = rank <= 16 && !mlp_xtp_d_in_exchange(R, E, d, f) ? 3 * moe_xtp_workspace_bytes(R, E, d) : 0;
+    return cc > x ? cc : x;
+}
 
 size_t moe_mlp_workspace_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
 {
     size_t n = al(sk_bytes_mlp(R, E, d, f)) + 256;
     if (rank <= 0) return n;
     const size_t C = (size_t)(rank + 15) / 16;   // 16-wide chunks per adapter
-    return n + C * (3 * pack_bytes(E, d) + 3 * pack_bytes(E, f) + 7 * q_bytes(R)) + al(mlp_xtp_bytes(R, E, d, f)) + al(cc_bytes(R, f));
+    return n + C * (3 * pack_bytes(E, d) + 3 * pack_bytes(E, f) + 7 * q_bytes(R)) + al(mlp_xtp_bytes(R, E, d, f, rank)) + al(mlp_cc_bytes(R, E, d, f, rank));
 }
 
 size_t moe_mlp_saved_bytes(int64_t R, int rank) { return rank > 0 ? (size_t)((rank + 15) / 16) * 6 * q_bytes(R) : 256; }
@@ -800,8 +807,8 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
     if (has_lora) {
         pq = (uint8_t*)ws.take((size_t)C * 6 * qb);
         if (fuse_rc) p2s = ws.take(qb);   // P2 times the row scale, row-major (the fused contraction's operand)
-        if (fuse_rc) ccw = (float*)ws.take(cc_bytes(R, f));
-        xb = mlp_xtp_bytes(R, E, d, f);
+        if (fuse_rc) ccw = (float*)ws.take(mlp_cc_bytes(R, E, d, f, rank));
+        xb = mlp_xtp_bytes(R, E, d, f, rank);
         xw = ws.take(xb);
         TIMED("bwd.pack_lora");
         for (int c = 0; c < C; ++c) {
@@ -927,12 +934,12 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         // dA1[e][k=d][r] = sum_m x[in_row(m)][k] P1[m][r];  dB1[e][r][n=f] = sum_m Q1[m][r] dgate[m][n]
         TIMED("bwd.xtp_w1w3");
         if (fuse_rc) {
-            // One launch over x and dy leaves the partials of dA1, dA3 and dB2 behind those of dB1, dB3 and dA2 that the dh GEMM's epilogue
+            // One launch over x and dy leaves the partials of dA1, dA3 and dB2 beside those of dB1, dB3 and dA2 that the dh GEMM's epilogue
             // left, and one launch adds all six: six launches before (4096 tokens, d=4096, f=14336: 87 us together, 65 now; 512 tokens, d=256:
             // 41 us, 16 now -- each of them was a few workgroups behind a gap; 2048 tokens, 64 experts: 76 and 66).
             const size_t onef = moe_xtp_workspace_bytes(R, E, f) / sizeof(float), oned = moe_xtp_workspace_bytes(R, E, d) / sizeof(float);
             float* part = (float*)xw;
-            float* partd = part + 3 * onef;
+            float* partd = mlp_xtp_d_in_exchange(R, E, d, f) ? (float*)((uint8_t*)skws + counter_bytes()) : ccw;
             const MoeXtpJob jobs[3] = {{x, ldx, d, pos, fan_out, pqp(4, 0), nullptr, nullptr, {}, rank}, {x, ldx, d, pos, fan_out, pqp(5, 0), nullptr, nullptr, {}, rank},
                                        {dy, lddy, d, dy_grouped ? nullptr : pos, dy_fan_out, svp(5, 0), row_scale, nullptr, {}, rank}};
             TRY(moe_launch_xtp_partial_jobs(jobs, 3, pos64, ldt, offsets, off64, E, R, partd, (int64_t)oned, st, f16));

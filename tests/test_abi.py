@@ -123,3 +123,16 @@ def test_the_projection_backward_names_the_sizes_it_refuses():
     need = lambda K, N, r: lib.moe_linear_lora_bwd_workspace_bytes(128, 4, K, N, r)
     assert all(need(*s) > 0 for s in ((32, 64, 1), (256, 512, 16), (96, 160, 64)))
     assert all(need(*s) == 0 for s in ((256, 512, 65), (256, 512, 0), (48, 64, 16), (64, 48, 16), (64, 32, 16)))
+
+
+def test_the_mlp_workspace_holds_no_set_of_partials_twice():
+    """Rank 16: beside the packed factors, the interims, the column-tile partials of the gate/up and dh launches and three sets of row-tile
+    partials of the wider of d and f, everything shares space with the K-split exchange, whose size the query gives for rank 0."""
+    from moe_distributed_training_amd._lib import lib
+    up = lambda n, m: -(-n // m) * m
+    for R, E, d, f in ((8192, 8, 4096, 14336), (32768, 8, 4096, 14336), (16384, 64, 2048, 1024), (1024, 8, 256, 512), (2, 8, 4096, 14336)):
+        factors = 3 * 32 * E * (d + f)
+        interims = 7 * up(up(R, 32) * 32 + 1024, 256)
+        xtp = 3 * (R // 256 + E) * max(d, f) * 64
+        columns = 2 * up(f, 256) // 256 * R * 64
+        assert lib.moe_mlp_workspace_bytes(R, E, d, f, 16) <= lib.moe_mlp_workspace_bytes(R, E, d, f, 0) + factors + interims + xtp + columns + 4096
