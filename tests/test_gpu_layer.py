@@ -124,7 +124,7 @@ def test_layer_fwd_bwd_fp16(dev, oracle, T, d, f, E, r):
 
 @pytest.mark.parametrize("E,k,r", [(96, 4, 16), (16, 8, 16), (80, 3, 0)])
 def test_layer_many_experts_and_wider_top_k(dev, oracle, E, k, r):
-    """More than 8 experts (router on the two-launch path), more than 64 (group lookup in blocks of 64 in every grouped kernel),
+    """More than 8 experts (router in groups of 16), more than 64 (group lookup in blocks of 64 in every grouped kernel),
     top-k above 2 (fan-out k in the gathers and the combine); most groups hold a handful of rows, some none."""
     import moe_distributed_training_amd as moe
     T, d, f, alpha = 300, 128, 256, 32.0
@@ -152,6 +152,24 @@ def test_layer_many_experts_and_wider_top_k(dev, oracle, E, k, r):
         for n in ("w1", "w3", "w2"):
             check_expert_grads(lt[n][0].grad, lo[n][0].grad, f"dA {n}", TINY_GROUP_TOL)
             check_expert_grads(lt[n][1].grad, lo[n][1].grad, f"dB {n}", TINY_GROUP_TOL)
+
+
+@pytest.mark.parametrize("E,k", [(16, 8), (24, 2), (64, 4), (80, 3), (104, 2)])
+def test_layer_many_experts_router_gradient(dev, oracle, E, k):
+    """The router's weight with a gradient, for each width of its kernel, and above the 96 experts that the matrix-core router takes."""
+    import moe_distributed_training_amd as moe
+    T, d, f = 200, 128, 64
+    x, wg, w1, w2, w3, _, dout = _make(T, d, f, E, 0, torch.bfloat16, seed=E)
+    wg = wg * 20
+    xo, wgo = x.float().requires_grad_(True), wg.float().requires_grad_(True)
+    ref, aux = oracle.moe_block(xo, wgo, w1.float(), w2.float(), w3.float(), k, None, 32.0)
+    ref.backward(dout.float())
+    xg, wgg = x.to(dev).requires_grad_(True), wg.to(dev).requires_grad_(True)
+    out, _, ei = moe.moe_layer_forward(xg, wgg, w1.to(dev), w2.to(dev), w3.to(dev), k, None, 32.0)
+    out.backward(dout.to(dev))
+    assert torch.equal(ei.cpu().long(), aux["indices"])
+    assert rel(out, ref) < 1e-2 and rel(xg.grad, xo.grad) < 1e-2
+    assert rel(wgg.grad, wgo.grad) < 1e-2
 
 
 @pytest.mark.parametrize("r", [32, 24, 48, 64, 72, 128, 144])

@@ -223,7 +223,10 @@ def test_router_backward_matches_autograd(dev, oracle):
 
 
 @pytest.mark.parametrize("dtype,T,d,E", [(torch.float32, 1000, 260, 8), (torch.float32, 130, 77, 19), (torch.bfloat16, 4096, 4096, 8),
-                                         (torch.bfloat16, 333, 200, 3), (torch.float16, 65, 72, 16)])
+                                         (torch.bfloat16, 333, 200, 3), (torch.float16, 65, 72, 16)]
+                         # one, two and four groups of 16 experts per pass, a second and a third pass, the last group ragged; chunks of 64 tokens and columns past 128 and 512
+                         + [(dt, T, d, E) for dt in (torch.float32, torch.bfloat16, torch.float16)
+                            for T, d, E in ((67, 136, 17), (130, 520, 32), (15, 648, 33), (200, 1032, 64), (65, 72, 65), (129, 264, 96), (70, 520, 130))])
 def test_router_gradients_from_fp32_dlogits(dev, dtype, T, d, E):
     """dWg = dlogits^T x and dx = dlogits Wg computed by the library from the fp32 dlogits (several token chunks, a
     partial last chunk, expert counts off the register block, widths off the 16-byte vectors): fp32 inputs to 1e-5,
