@@ -431,7 +431,9 @@ int moe_launch_cc_reduce2(const float* partial, const float* partial2, int ntile
 {
     if (R == 0) return MOE_OK;
     const bool two = partial2 != nullptr;
-    const int parts = R * (two ? 2 : 1) < 8192 ? 4 : 1;   // (see the kernel)
+    // (see the kernel; two products, the stage with one and with four parts: 56 tiles, 256 rows 7.7 and 7.1 us, 2048 8.1 and 7.9, 3072 8.5 and 8.7, 4096 9.0 and 9.5;
+    // 112 tiles, 2048 11.2 and 9.6, 4096 15.0 and 13.8, 6144 18.6 and 18.4, 8192 21.8 and 23.0; up to 16 tiles the same)
+    const int parts = R * (two ? 2 : 1) < 8192 ? 4 : 1;
     auto kern = parts == 4 ? (f16 ? cc_reduce_kernel<NumF16, 4> : cc_reduce_kernel<NumBf16, 4>) : (f16 ? cc_reduce_kernel<NumF16, 1> : cc_reduce_kernel<NumBf16, 1>);
     const int quads = CC_THREADS / parts;
     hipLaunchKernelGGL(kern, dim3((unsigned)((R * 4 + quads - 1) / quads), two ? 2u : 1u), dim3(CC_THREADS), 0, stream, partial, partial2,

@@ -465,8 +465,7 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const float* __restrict
 // wave per (token, selection) pair takes the gradient of that weight, <y[t*k+j], dout[t]> (+ d_w, a gradient that reached the returned
 // weights directly), and puts the weight at the pair's place in sorted order (the row scale of the grouped GEMMs); then the token's lanes
 // turn its k gradients into those of its logits.  The sums are those of combine_dgates and router_bwd, bit for bit.  As three launches
-// 2048 tokens, 64 experts, top-8, d=2048 took 34.6 us, this 21.4 (eight waves for more than four selections, eight per SIMD; four, and
-// as many registers as the compiler likes: 32.8); 4096 tokens, top-2, d=4096 28.7 and 18.8;
+// 2048 tokens, 64 experts, top-8, d=2048 took 34.6 us, this 21.4 (eight waves per SIMD; as many registers as the compiler likes: 32.8); 4096 tokens, top-2, d=4096 28.7 and 18.8;
 // 512 tokens, d=256 9.4 and 4.7.
 template <typename T, int GB_WAVES>
 __global__ void __launch_bounds__(GB_WAVES * 64, 8) gates_bwd_kernel(const T* __restrict__ y, int64_t ldy, const T* __restrict__ dout, int64_t ldd,
@@ -927,7 +926,10 @@ int moe_launch_gates_bwd(const void* y, int64_t ldy, const void* dout, int64_t l
 {
     if (dtype == MOE_F32) return MOE_ERR_UNSUPPORTED;
     if (ntok == 0) return MOE_OK;
-    const int waves = k > 4 ? 8 : 4;
+    // Eight waves for more than four selections while the workgroups (one token each) are resident at once, and for wide rows; four otherwise
+    // (top-8, four and eight waves: 500 tokens, d=1536 10.9 and 9.8 us, 1000 13.0 and 12.0, 2048 17.5 and 20.2, 8192 48.5 and 56.9; 2048 tokens,
+    // d=2048 19.5 and 19.9, 4096 31.5 and 30.1; 8192 tokens, d=3072 91 and 96, 4096 117 and 111; top-5 and top-6 within 4 %).
+    const int waves = k > 4 && (ntok <= 4 * (int64_t)moe_device_cus() || d > 3072) ? 8 : 4;
     const int tokens = k >= waves ? 1 : (waves + k - 1) / k;   // at least one pair per wave; at most 4 tokens, TK_LANES lanes each
     const bool vec = (uintptr_t)y % 16 == 0 && (uintptr_t)dout % 16 == 0 && ldy % 8 == 0 && ldd % 8 == 0;
     const dim3 grid((unsigned)((ntok + tokens - 1) / tokens));
