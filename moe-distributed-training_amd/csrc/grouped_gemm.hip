@@ -1272,8 +1272,9 @@ template <bool NN, int EPI> int launch_variant(const MoeGemmParams& p, int64_t R
 }  // namespace
 
 
-// The gate/up pair kernel never splits K (its launches have many more tiles than compute units); the others may cut
-// the tiles of the last, partial round of compute units 2 or 4 ways.
+// The gate/up pair kernel never splits K: it holds two products and is at its limit of registers without an exchange (a launch of 3.5 rounds, as 8
+// experts of f = 14336 and at most 256 rows make, leaves half of the chip idle in its last).  The others may cut the tiles of the last, partial round of
+// compute units 2 or 4 ways.
 int moe_gemm_max_split(bool pair) { return pair ? 1 : 4; }
 int moe_gemm_num_counters() { return moe_num_cus(); }
 

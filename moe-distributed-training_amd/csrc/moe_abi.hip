@@ -473,6 +473,8 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const v
         pb.job[pb.njobs++] = {b, sbe, sbn, sbr, (uint16_t*)Bt[c], N, 1, chunk_rank(c)};
         pb.job[pb.njobs++] = {a, sae, sak, sar, (uint16_t*)LB[c], K, 0, chunk_rank(c)};
     }
+    {
+    TIMED("linear.bwd_adapters");
     TRY(moe_launch_pack_lora_batch(pb, st));
     for (int c0 = 0; c0 < C; c0 += 2) {   // jobs over X first, then those over dY: neighbours share their rows in L2
         const int n = C - c0 > 1 ? 2 : 1;
@@ -494,6 +496,8 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const v
         }
         TRY(moe_launch_xtp_jobs(xtp, 2 * n, pos64, ldt, offsets, off64, E, R, 1.f, xw, xb, st, f16));
     }
+    }
+    TIMED("linear.bwd_gemm_dx");
     return moe_launch_gemm_mfma(p, R, st);
 }
 
@@ -556,8 +560,10 @@ int moe_swiglu_pair(const void* x, int64_t sxm, int64_t sxk, const void* w_gate,
 {
     if (dtype != MOE_F32) return MOE_ERR_UNSUPPORTED;
     if (!x || !w_gate || !w_up || !h || !pos || !offsets || E < 1 || R < 0 || K < 1 || N < 1 || fan_out < 1) return MOE_ERR_BAD_ARG;
+    hipStream_t st = S(stream);
+    TIMED("fwd.swiglu_pair_fp32");
     return moe_launch_generic_swiglu_pair((const float*)x, sxm, sxk, (const float*)w_gate, (const float*)w_up, swe, swk, swn, (float*)h, ldh, pos, pos64, offsets,
-                                          off64, E, R, K, N, fan_out, S(stream));
+                                          off64, E, R, K, N, fan_out, st);
 }
 
 int moe_swiglu(const void* gate, const void* up, void* h, int64_t n, int dtype, void* stream)

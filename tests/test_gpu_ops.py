@@ -584,11 +584,12 @@ def test_generic_kernels_at_the_edges_of_a_contraction_step(dev, oracle, dtype, 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,E,k,K,N,r,gates,layout", [
     (333, 4, 2, 256, 384, 16, True, "k_contiguous"), (100, 3, 1, 64, 96, 8, False, "k_contiguous"), (257, 5, 3, 96, 160, 24, True, "n_contiguous"),
-    (64, 2, 2, 128, 64, 33, False, "n_contiguous"), (700, 6, 4, 320, 64, 64, True, "k_contiguous"), (90, 3, 2, 64, 64, 65, True, "k_contiguous"),
+    (64, 2, 2, 128, 64, 33, False, "n_contiguous"), (700, 6, 4, 320, 64, 64, True, "k_contiguous"), (257, 5, 3, 96, 160, 24, False, "n_contiguous"),
+    (700, 6, 4, 320, 64, 64, False, "k_contiguous"), (90, 3, 2, 64, 64, 65, True, "k_contiguous"),
     (40, 3, 2, 48, 64, 16, True, "k_contiguous"), (50, 2, 2, 64, 32, 16, False, "k_contiguous")])
 def test_projection_backward_on_gathered_rows(dev, oracle, dtype, T, E, k, K, N, r, gates, layout):
     """The backward pass that reads dY and X where they lie, on both sides of its rule (ranks to 64, contractions of at least 64 and multiples of
-    32; the last three take the route over gathered copies): adapter gradients, dX and the gates' against the fp32 oracle."""
+    32, gates with bf16 rows only; the last three, and in fp16 the gated ones, take the route over gathered copies): adapter gradients, dX and the gates' against the fp32 oracle."""
     import moe_distributed_training_amd as moe
     torch.manual_seed(T + r)
     _, sei, ssi, eo = _routing(oracle, T, E, k, T, skew=True)

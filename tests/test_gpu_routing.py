@@ -57,8 +57,8 @@ def test_router_end_to_end(dev, oracle, dtype, T, d, E):
     assert margin > 1e-6, "test data has a near tie; pick another seed"
     assert torch.equal(idx.cpu(), io)
     assert torch.allclose(w.cpu(), wo, atol=1e-5)
-    # the one-call form: two launches give the same bits as the two calls; the single fused launch (<= 8 experts of a
-    # 2-byte type, hidden size a multiple of 32) sums its logits on the matrix cores in another order -- fp32 rounding
+    # the one-call form: the vector kernels give the same bits as the two calls; a 2-byte type with a hidden size that is a
+    # multiple of 32 sums its logits on the matrix cores in another order -- fp32 rounding
     # apart, the same indices, and exactly the softmax / top-k of ITS logits
     l2, s2, w2, i2 = router.router_forward(x.to(dev), wg.to(dev), k)
     s1, w1, i1 = router.router_topk(l2, k)
@@ -402,7 +402,7 @@ def test_gate_gradients_in_one_launch(dev, dtype, T, E, k, d, renorm, direct):
 @pytest.mark.parametrize("T,d,E,k", [(1, 32, 9, 1), (17, 96, 16, 2), (40, 544, 17, 3), (33, 2048, 32, 8), (16, 4096, 33, 2), (100, 1024, 64, 8), (31, 256, 65, 4),
                                      (50, 8192, 96, 6), (20, 512, 97, 2)])
 def test_router_of_many_experts_on_the_matrix_cores(dev, oracle, dtype, T, d, E, k):
-    """The one-launch router at the expert counts where its groups of 16 change (and 97, which takes two launches): logits to fp32
+    """The matrix-core router at the expert counts where its groups of 16 change (and 97, which the vector kernels take): logits to fp32
     rounding of sums of exact products (sqrt(d) terms of half an ulp each, far below 3e-5 here), the oracle's choices, and exactly the softmax and
     top-k of its own logits."""
     _, router, _ = _mods()
