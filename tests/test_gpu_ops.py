@@ -687,14 +687,18 @@ def test_gate_and_up_in_one_launch_fp32(dev, oracle, T, E, k, K, N):
 
 
 def _us(fn, n=20):
-    """GPU time of a call in us, best of five runs of n calls (calls that are longer than the host needs to enqueue them)."""
+    """GPU time of a call in us, best of five replays of n calls in a graph (no host work between the calls)."""
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(n):
+            fn()
     times = []
     for _ in range(6):
         a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-        torch.cuda.synchronize()
         a.record()
-        for _ in range(n):
-            fn()
+        graph.replay()
         b.record()
         torch.cuda.synchronize()
         times.append(a.elapsed_time(b) / n * 1e3)
