@@ -181,7 +181,7 @@ template <typename T> struct Raw8 {
 // g, which are the second operand of eight v_mfma_f32_16x16x4) and one coefficient (token i).  Accumulator u holds column 8 i + u of
 // tokens 4 g .. 4 g + 3; it starts with their k rows' sum.  fp32 products and sums as before, rows first, then the tail in order.
 // One token per workgroup fetches and unpacks the whole tail for every token, one row after the other: 2048 tokens, top-8, d=2048, 64 experts
-// 39 us (51 behind the layer's other launches), this 25 (33).  Where the rows' traffic is all that counts, that kernel's whole rows are the
+// 39 us (51 behind the layer's other launches), this 25 (32).  Where the rows' traffic is all that counts, that kernel's whole rows are the
 // better pattern: the launcher's rule.
 constexpr int CT_TOKENS = 16, CT_WCOLS = 128, CT_COLS = ROW_THREADS / 64 * CT_WCOLS;
 template <typename T, int KMAX>
@@ -472,16 +472,16 @@ int moe_launch_combine_fwd(const void* y, int64_t ldy, void* out, int64_t ldo, c
     MOE_DISPATCH_DTYPE(dtype, {
         const int vo = vec_aligned<T>(y, ldy) && vec_aligned<T>(out, ldo) && (!extra_rows || vec_aligned<T>(extra_rows, lde));
         // The tail on the matrix instructions: without rows always (8192 tokens, d=4096, 8 rows of tail: 30.0 us one token per workgroup, 17.2 so).  With
-        // rows, which that kernel fetches in pieces of 256 bytes, never for a tail of up to eight (8192 tokens, d=4096, new buffers for each call:
-        // top-2 51.2 and 54.7, top-4 72 and 88), and above where the tail is what one token per workgroup takes longest for: its n_extra
-        // steps per pass over the columns or per round of workgroups (eight of them per compute unit) against the k rows' share
-        // (2048 tokens, top-8, d=2048, 16 / 32 / 64 rows: 19.3 / 25.9 / 38.9 us and 18.9 / 20.9 / 25.2; 1000 tokens, top-4, 16 / 64 / 96: 5.8 / 12.6 / 17.0
-        // and 9.5 / 15.4 / 18.8; 512 tokens, top-2, d=4096, 16 / 64: 8.1 / 22 and 5.5 / 8.7).  Rows beyond the last-level cache: more than
-        // three rows of tail per row (8192 tokens, d=4096, top-8, 16 / 32: 135 / 175 and 165 / 171; top-4, 16 / 24: 87 / 103 and 88 / 92).
+        // rows, which that kernel fetches in pieces of 256 bytes, where the tail is what one token per workgroup takes longest for: its n_extra steps,
+        // per pass over the columns or per round of workgroups (eight of them per compute unit), against the k rows' share; and, unless rows are
+        // no longer than eight pieces, for at least four rows of tail per row.  us with rows and buffers out of cache, one token per workgroup and so:
+        // d=4096, top-2, 8 rows: 256 tokens 10.2 and 10.4, 777 14.1 and 12.7, 4096 39.0 and 36.5, 16384 117 and 121 (behind the layer's other launches
+        // 777 tokens 12.5 and 9.5, 4096 29.5 and 27.4); top-8, 8192 tokens, 8 / 16 / 32 / 64 rows: 145 / 165 / 212 / 305 and 192 / 198 / 207 / 227;
+        // d=2048, top-8, 2048 tokens, 16 / 32 / 64: 35 / 43 / 62 and 35 / 37 / 42; d=1024, top-8, 1000 tokens, 16 / 32 / 64: 14 / 19 / 28 and 25 / 26 / 29,
+        // 16384 tokens, 8 / 16 / 32: 88 / 101 / 128 and 99 / 103 / 107.
         const int64_t passes = (ncols + ROW_THREADS * Vec8<T>::N - 1) / (ROW_THREADS * Vec8<T>::N), resident = 8 * (int64_t)moe_device_cus();
         const int64_t steps = passes * resident > ntok ? n_extra * passes : n_extra * ntok / resident;
-        const bool beyond_cache = ntok * k * ncols * (int64_t)sizeof(T) >= ((int64_t)1 << 28);
-        const bool tail = n_extra > 0 && (k == 0 || (n_extra > 8 && (beyond_cache ? n_extra > 3 * k : steps >= 6 * k + 8)));
+        const bool tail = n_extra > 0 && (k == 0 || (steps >= 5 * k + 4 && (n_extra >= 4 * k || ncols * (int64_t)sizeof(T) <= 2048)));
         if (vo && tail && k <= 8 && ncols % 8 == 0 && (ncols + CT_COLS - 1) / CT_COLS <= 65535) {
             auto kern = k <= 2 ? combine_tail_kernel<T, 2> : (k <= 4 ? combine_tail_kernel<T, 4> : combine_tail_kernel<T, 8>);
             hipLaunchKernelGGL(kern, dim3((unsigned)((ntok + CT_TOKENS - 1) / CT_TOKENS), (unsigned)((ncols + CT_COLS - 1) / CT_COLS)), dim3(ROW_THREADS), 0, stream,
