@@ -85,6 +85,11 @@ int moe_router_topk(const float* logits, float* scores, float* topw, int32_t* to
  * and topi are moe_router_topk of the logits in every case; one launch or two. */
 int moe_router_forward(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits, float* scores,
                        float* topw, int32_t* topi, int64_t ntok, int64_t d, int E, int k, int renorm, void* stream);
+/* moe_router_forward and then moe_sort_by_expert of its choices (int32 ids and outputs, inclusive offsets (E), inv the inverse permutation, the sort's workspace):
+ * the same results; one launch for up to 16 tokens of a 2-byte type and 8 experts in such rows. */
+int moe_router_forward_sorted(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits, float* scores,
+                              float* topw, int32_t* topi, int64_t ntok, int64_t d, int E, int k, int renorm, int32_t* sorted_expert,
+                              int32_t* sorted_pos, int32_t* inv, int32_t* offsets, void* workspace, size_t workspace_bytes, void* stream);
 /* gradient of moe_router_topk with respect to the logits given d(topw); the reference obtains it from autograd. */
 int moe_router_topk_bwd(const float* dtopw, const float* topw, const int32_t* topi, const float* scores,
                         float* dlogits, int64_t ntok, int E, int k, int renorm, void* stream);

@@ -28,6 +28,7 @@ _SIGNATURES = {
     "moe_router_logits": ("i", "plplipllip"),
     "moe_router_topk": ("i", "ppppliiip"),
     "moe_router_forward": ("i", "plpli" + "pppp" + "lliiip"),
+    "moe_router_forward_sorted": ("i", "plpli" + "pppp" + "lliii" + "pppp" + "pzp"),
     "moe_router_topk_bwd": ("i", "ppppp" + "liiip"),
     "moe_gates_bwd": ("i", "plpli" + "ppppppp" + "ll" + "iii" + "p"),
     "moe_router_weight_grad_workspace_bytes": ("z", "lli"),

@@ -175,6 +175,10 @@ size_t moe_router_wgrad_ws_bytes(int64_t ntok, int64_t d, int E);
 int moe_launch_router_wgrad(const void* x, int64_t ldx, const float* dlogits, void* dwg, int64_t ldo, int64_t ntok,
                             int64_t d, int E, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream);
 size_t moe_sort_ws_bytes(int64_t R, int E);
+// router and sort in one launch, where one workgroup takes all tokens (moe_router_sorts)
+bool moe_router_sorts(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, int64_t ntok, int64_t d, int E);
+int moe_launch_router_sorted(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits, float* scores, float* topw, int32_t* topi,
+                             int64_t ntok, int64_t d, int E, int k, int renorm, int32_t* sei, int32_t* ssi, int32_t* inv, int32_t* offsets, hipStream_t stream);
 int moe_launch_sort(const void* expert_idx, int in64, int64_t R, int E, int block_m, void* sorted_expert,
                     void* sorted_pos, int out64, void* counts, void* offsets, void* padded_blocks, int64_t padded_cap,
                     int32_t* num_padded, int32_t* inv, void* workspace, size_t workspace_bytes, hipStream_t stream);

@@ -147,6 +147,21 @@ int moe_router_forward(const void* x, int64_t ldx, const void* wg, int64_t ldw, 
     return moe_launch_router_forward(x, ldx, wg, ldw, dtype, logits, scores, topw, topi, ntok, d, E, k, renorm, st);
 }
 
+int moe_router_forward_sorted(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits, float* scores, float* topw, int32_t* topi,
+                              int64_t ntok, int64_t d, int E, int k, int renorm, int32_t* sorted_expert, int32_t* sorted_pos, int32_t* inv, int32_t* offsets,
+                              void* workspace, size_t workspace_bytes, void* stream)
+{
+    if (ntok < 0 || d < 1 || E < 1 || k < 1 || k > E || !offsets || !workspace) return MOE_ERR_BAD_ARG;
+    if (ntok > 0 && (!x || !wg || !logits || !scores || !topw || !topi || !sorted_expert || !sorted_pos || !inv)) return MOE_ERR_BAD_ARG;
+    if (moe_router_sorts(x, ldx, wg, ldw, dtype, ntok, d, E)) {
+        hipStream_t st = S(stream);
+        TIMED("route.router_sorted");
+        return moe_launch_router_sorted(x, ldx, wg, ldw, dtype, logits, scores, topw, topi, ntok, d, E, k, renorm, sorted_expert, sorted_pos, inv, offsets, st);
+    }
+    TRY(moe_router_forward(x, ldx, wg, ldw, dtype, logits, scores, topw, topi, ntok, d, E, k, renorm, stream));
+    return moe_sort_by_expert(topi, 0, ntok * k, E, 128, sorted_expert, sorted_pos, 0, nullptr, offsets, nullptr, 0, nullptr, inv, workspace, workspace_bytes, stream);
+}
+
 int moe_router_topk_bwd(const float* dtopw, const float* topw, const int32_t* topi, const float* scores,
                         float* dlogits, int64_t ntok, int E, int k, int renorm, void* stream)
 {

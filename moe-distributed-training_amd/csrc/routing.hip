@@ -250,16 +250,21 @@ __global__ void router_topk_wide_kernel(const float* __restrict__ logits, float*
 // timing).  The summation order differs from router_logits_kernel's, so the two agree to fp32 rounding, not bit for bit.
 constexpr int RM_WAVES = 8, RM_TOKENS = 16;
 constexpr int RM_MAX_EXPERTS = 96;   // beyond, a workgroup's partial sums do not fit its LDS
+// SORT: one workgroup holds all tokens and sorts their assignments by expert as well, as sort_one_launch_kernel would: an assignment's place is the
+// number of those before it in (expert, flat index) order, counted by a thread each.  Saves a launch and its trip to memory: one token, d = 4096, router and
+// sort 7.4 + 4.5 us in two launches.
 // RM_BATCH: 32-wide K steps whose loads are in flight together (16 steps x 8 waves = 4096 columns); a wave with fewer steps repeats the last one's
 // loads, so narrow layers take a kernel of 4 (512 tokens, d=256: 9.5 -> 5.3 us)
-template <typename T, int RM_BATCH>
+struct SortedOut { int32_t *sei, *ssi, *inv, *offsets; };
+template <typename T, int RM_BATCH, bool SORT>
 __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_kernel(const T* __restrict__ x, int64_t ldx,
                                                                     const T* __restrict__ wg, int64_t ldw,
                                                                     float* __restrict__ logits, float* __restrict__ scores,
                                                                     float* __restrict__ topw, int32_t* __restrict__ topi,
-                                                                    int64_t ntok, int d, int E, int k, int renorm)
+                                                                    int64_t ntok, int d, int E, int k, int renorm, const SortedOut so)
 {
     __shared__ float s_part[RM_WAVES][RM_TOKENS][16];
+    __shared__ int32_t s_topi[SORT ? RM_TOKENS * ROUTER_EXPERT_GROUP : 1];   // (k <= E)
     __shared__ float s_logits[RM_TOKENS][ROUTER_EXPERT_GROUP];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t t0 = (int64_t)blockIdx.x * RM_TOKENS;
@@ -311,9 +316,28 @@ __global__ void __launch_bounds__(RM_WAVES * 64) router_mfma_kernel(const T* __r
     if (tid < RM_TOKENS * TK_LANES) {   // whole waves
         const int tt = tid / TK_LANES;
         const int64_t t = t0 + tt;
-        softmax_topk_token<1>(s_logits[tt], scores + t * E, topw + t * k, topi + t * k, E, k, renorm, t < ntok);
+        softmax_topk_token<1>(s_logits[tt], scores + t * E, topw + t * k, SORT ? s_topi + t * k : topi + t * k, E, k, renorm, t < ntok);
+    }
+    if constexpr (SORT) {
+        __syncthreads();
+        const int R = (int)ntok * k;
+        if (tid < R) {
+            const int e = s_topi[tid];
+            int at = 0;
+            for (int j = 0; j < R; ++j) at += (s_topi[j] < e || (s_topi[j] == e && j < tid)) ? 1 : 0;
+            topi[tid] = e;
+            so.sei[at] = e;
+            so.ssi[at] = tid;
+            so.inv[tid] = at;
+        } else if (tid >= RM_WAVES * 64 - E) {
+            const int e = RM_WAVES * 64 - 1 - tid;
+            int n = 0;
+            for (int j = 0; j < R; ++j) n += s_topi[j] <= e ? 1 : 0;
+            so.offsets[e] = n;
+        }
     }
 }
+static_assert(RM_TOKENS * ROUTER_EXPERT_GROUP + ROUTER_EXPERT_GROUP <= RM_WAVES * 64, "a thread per assignment and one per expert");
 
 // The same for 9 to 96 experts, in EG groups of 16: a wave's activation fragment meets EG weight fragments per step, fewer steps' loads fit in
 // flight, and the eight partial sums per logit are added in wave order as above.  The two launches of the vector kernels are bound by their
@@ -849,14 +873,18 @@ int moe_launch_router_logits(const void* x, int64_t ldx, const void* wg, int64_t
 }
 
 // logits + softmax + top-k; one launch when the router weight fits the fused kernel, otherwise the two kernels above
+static bool router_mfma_ok(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, int64_t d, int E)
+{
+    return dtype != MOE_F32 && E <= RM_MAX_EXPERTS && d % 32 == 0 && d >= 32 && d < (1 << 30) &&
+           ((uintptr_t)x % 16 == 0) && ((uintptr_t)wg % 16 == 0) && ldx % 8 == 0 && ldw % 8 == 0;
+}
+
 int moe_launch_router_forward(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits,
                               float* scores, float* topw, int32_t* topi, int64_t ntok, int64_t d, int E, int k,
                               int renorm, hipStream_t stream)
 {
     if (ntok == 0) return MOE_OK;
-    const bool fused = dtype != MOE_F32 && E <= RM_MAX_EXPERTS && d % 32 == 0 && d >= 32 && d < (1 << 30) &&
-                       ((uintptr_t)x % 16 == 0) && ((uintptr_t)wg % 16 == 0) && ldx % 8 == 0 && ldw % 8 == 0;
-    if (!fused) {
+    if (!router_mfma_ok(x, ldx, wg, ldw, dtype, d, E)) {
         if (E <= ROUTER_EXPERT_GROUP)
             return launch_router_logits(x, ldx, wg, ldw, dtype, logits, ntok, d, E, true, scores, topw, topi, k, renorm, stream);
         const int rc = moe_launch_router_logits(x, ldx, wg, ldw, dtype, logits, ntok, d, E, stream);
@@ -886,10 +914,28 @@ int moe_launch_router_forward(const void* x, int64_t ldx, const void* wg, int64_
     }
     auto few = [&](auto tag) {
         using T = decltype(tag);
-        auto kern = d <= 4 * 32 * RM_WAVES ? router_mfma_kernel<T, 4> : router_mfma_kernel<T, 16>;
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(RM_WAVES * 64), 0, stream, (const T*)x, ldx, (const T*)wg, ldw, logits, scores, topw, topi, ntok, (int)d, E, k, renorm);
+        auto kern = d <= 4 * 32 * RM_WAVES ? router_mfma_kernel<T, 4, false> : router_mfma_kernel<T, 16, false>;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(RM_WAVES * 64), 0, stream, (const T*)x, ldx, (const T*)wg, ldw, logits, scores, topw, topi, ntok, (int)d, E, k, renorm, SortedOut{});
     };
     if (dtype == MOE_BF16) few(__hip_bfloat16{}); else few(__half{});
+    return moe_launch_status();
+}
+
+bool moe_router_sorts(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, int64_t ntok, int64_t d, int E)
+{
+    return ntok >= 1 && ntok <= RM_TOKENS && E <= ROUTER_EXPERT_GROUP && router_mfma_ok(x, ldx, wg, ldw, dtype, d, E);
+}
+
+int moe_launch_router_sorted(const void* x, int64_t ldx, const void* wg, int64_t ldw, int dtype, float* logits, float* scores, float* topw, int32_t* topi,
+                             int64_t ntok, int64_t d, int E, int k, int renorm, int32_t* sei, int32_t* ssi, int32_t* inv, int32_t* offsets, hipStream_t stream)
+{
+    if (!moe_router_sorts(x, ldx, wg, ldw, dtype, ntok, d, E)) return MOE_ERR_UNSUPPORTED;
+    auto go = [&](auto tag) {
+        using T = decltype(tag);
+        auto kern = d <= 4 * 32 * RM_WAVES ? router_mfma_kernel<T, 4, true> : router_mfma_kernel<T, 16, true>;
+        hipLaunchKernelGGL(kern, dim3(1), dim3(RM_WAVES * 64), 0, stream, (const T*)x, ldx, (const T*)wg, ldw, logits, scores, topw, topi, ntok, (int)d, E, k, renorm, SortedOut{sei, ssi, inv, offsets});
+    };
+    if (dtype == MOE_BF16) go(__hip_bfloat16{}); else go(__half{});
     return moe_launch_status();
 }
 

@@ -329,14 +329,20 @@ Tensor router_weight_grad(const Tensor& x, const Tensor& dlogits)
 
 struct RouterOut { Tensor scores, weights, indices; };
 
+RouterOut router_outputs(const Tensor& x, const Tensor& wg, int64_t k)
+{
+    const int64_t T = x.size(0), E = wg.size(0);
+    MOE_ASSERT(wg.scalar_type() == x.scalar_type() && wg.size(1) == x.size(1), "router weight and input do not fit");
+    MOE_ASSERT(k >= 1 && k <= E, "top_k must be between 1 and the number of experts");
+    const auto f32 = x.options().dtype(at::kFloat);
+    return {at::empty({T, E}, f32), at::empty({T, k}, f32), at::empty({T, k}, x.options().dtype(at::kInt))};
+}
+
 RouterOut router_forward(const Tensor& x, const Tensor& wg, int64_t k, bool normalize)
 {
     const int64_t T = x.size(0), d = x.size(1), E = wg.size(0);
-    MOE_ASSERT(wg.scalar_type() == x.scalar_type() && wg.size(1) == d, "router weight and input do not fit");
-    MOE_ASSERT(k >= 1 && k <= E, "top_k must be between 1 and the number of experts");
-    const auto f32 = x.options().dtype(at::kFloat);
-    Tensor logits = at::empty({T, E}, f32);
-    RouterOut o{at::empty({T, E}, f32), at::empty({T, k}, f32), at::empty({T, k}, x.options().dtype(at::kInt))};
+    RouterOut o = router_outputs(x, wg, k);
+    Tensor logits = at::empty_like(o.scores);
     check(moe_router_forward(ptr(x), x.stride(0), ptr(wg), wg.stride(0), dtype_code(x), (float*)ptr(logits), (float*)ptr(o.scores), (float*)ptr(o.weights),
                              (int32_t*)ptr(o.indices), T, d, (int)E, (int)k, normalize, stream_of(x)), "moe_router_forward");
     return o;
@@ -591,6 +597,19 @@ Sorted sort_assignments(const Tensor& indices, int64_t E)
     return s;
 }
 
+// router_forward and sort_assignments of its choices, one launch where the library has one
+void router_and_sort(const Tensor& x, const Tensor& wg, int64_t k, bool normalize, RouterOut& rt, Sorted& s)
+{
+    const int64_t T = x.size(0), E = wg.size(0), R = T * k;
+    rt = router_outputs(x, wg, k);
+    Tensor logits = at::empty_like(rt.scores);
+    s = Sorted{at::empty({3 * R + E}, rt.indices.options()), R, E};
+    Tensor ws = bytes_on(x, moe_sort_workspace_bytes(R, (int)E));
+    check(moe_router_forward_sorted(ptr(x), x.stride(0), ptr(wg), wg.stride(0), dtype_code(x), (float*)ptr(logits), (float*)ptr(rt.scores), (float*)ptr(rt.weights),
+                                    (int32_t*)ptr(rt.indices), T, x.size(1), (int)E, (int)k, normalize, s.sei(), s.ssi(), s.inv(), s.offsets(), ptr(ws),
+                                    (size_t)ws.numel(), stream_of(x)), "moe_router_forward_sorted");
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // expert MLP on expert-grouped assignments (the reference's scattermoe_permute_and_compute, config_utils.py:99-185)
 // ---------------------------------------------------------------------------------------------------------------
@@ -687,8 +706,7 @@ struct LayerOut { RouterOut rt; Sorted so; MlpOut mlp; Tensor out; };
 LayerOut layer_forward(const Tensor& x, const Tensor& wg, const Tensor& w1, const Tensor& w3, const Tensor& w2, const Tensor* lt, const LayerCfg& c, bool save)
 {
     LayerOut o;
-    o.rt = router_forward(x, unit_inner(wg), c.k, c.normalize);
-    o.so = sort_assignments(o.rt.indices, c.E);
+    router_and_sort(x, unit_inner(wg), c.k, c.normalize, o.rt, o.so);
     const MlpShape s{c.E, c.d, c.f, x.size(0) * c.k, (int)c.k, c.scaling};
     o.mlp = mlp_forward(x, w1, w3, w2, describe_lora(lt, c.storage, c.d, c.f), s, o.so.ssi(), 0, o.so.offsets(), 0, false, save);
     o.out = combine(o.mlp.y, o.rt.weights, nullptr, c.k, x.size(0));

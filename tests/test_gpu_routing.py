@@ -462,3 +462,30 @@ def test_router_in_one_launch_is_not_slower_than_in_two(dev, T, E, d):
 
     one, two = us(lambda: router.router_forward(x, wg, 2)), us(lambda: router.router_topk(router.router_logits(x, wg), 2))
     assert one < 1.05 * two, (one, two)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,d,E,k", [(1, 4096, 8, 2), (1, 32, 1, 1), (7, 96, 3, 3), (16, 1024, 8, 8), (16, 1056, 8, 1), (17, 256, 8, 2), (5, 256, 9, 2), (3, 40, 4, 2), (0, 64, 4, 2)])
+def test_router_and_sort_in_one_call(dev, dtype, T, d, E, k):
+    """moe_router_forward_sorted gives the router's and the sort's bits, up to 16 tokens of 8 experts (one launch) and beyond (two); a token whose logits
+    are NaN among them."""
+    from moe_distributed_training_amd._lib import lib, check, ptr, stream_ptr, dtype_code
+    g = torch.Generator().manual_seed(T * 100 + E)
+    x = torch.randn(T, d, generator=g).to(dtype).to(dev)
+    wg = torch.randn(E, d, generator=g).to(dtype).to(dev)
+    if T > 2:
+        x[1] = float("nan")
+    R = T * k
+    def outs():
+        return dict(logits=torch.empty(T, E, device=dev), scores=torch.empty(T, E, device=dev), w=torch.empty(T, k, device=dev), i=torch.full((T, k), -9, dtype=torch.int32, device=dev),
+                    sei=torch.full((R,), -9, dtype=torch.int32, device=dev), ssi=torch.full((R,), -9, dtype=torch.int32, device=dev),
+                    inv=torch.full((R,), -9, dtype=torch.int32, device=dev), off=torch.full((E,), -9, dtype=torch.int32, device=dev))
+    a, b = outs(), outs()
+    n = lib.moe_sort_workspace_bytes(R, E)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    check(lib.moe_router_forward(ptr(x), d, ptr(wg), d, dtype_code(x), ptr(a["logits"]), ptr(a["scores"]), ptr(a["w"]), ptr(a["i"]), T, d, E, k, 1, stream_ptr(dev)), "router")
+    check(lib.moe_sort_by_expert(ptr(a["i"]), 0, R, E, 128, ptr(a["sei"]), ptr(a["ssi"]), 0, None, ptr(a["off"]), None, 0, None, ptr(a["inv"]), ptr(ws), n, stream_ptr(dev)), "sort")
+    check(lib.moe_router_forward_sorted(ptr(x), d, ptr(wg), d, dtype_code(x), ptr(b["logits"]), ptr(b["scores"]), ptr(b["w"]), ptr(b["i"]), T, d, E, k, 1, ptr(b["sei"]), ptr(b["ssi"]),
+                                        ptr(b["inv"]), ptr(b["off"]), ptr(ws), n, stream_ptr(dev)), "router and sort")
+    for name in a:
+        assert torch.equal(a[name].view(torch.int32), b[name].view(torch.int32)), name
