@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Compiles grouped_gemm.hip with the compiler's resource-usage remarks and fails if a kernel variant of the usual shapes
+"""Compiles a grouped GEMM source with the compiler's resource-usage remarks and fails if a kernel variant of the usual shapes
 spills registers: the main loop of those variants sits at the edge of the scalar and vector register budgets, and a
 variant that spills a few scalar registers runs 1.5-2.5 % slower.  The general-shape variants (last template argument
 true) may spill scalar registers; no variant may spill vector registers.  Usage: make -C csrc check-spills"""

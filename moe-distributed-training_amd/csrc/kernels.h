@@ -70,6 +70,10 @@ struct MoeGemmParams {
 size_t moe_gemm_sk_bytes(int64_t R, int E, int64_t N);
 void moe_gemm_sk_attach(MoeGemmParams& p, void* ws, int64_t R, int E, int64_t N);
 int moe_gemm_max_split(bool pair);
+// rows and columns of a launch's output tiles: 256, one workgroup per compute unit, or 128, two (K: all segments; general-shape launches always 256)
+int moe_gemm_tile(int64_t R, int E, int64_t K, int64_t N, bool pair);
+constexpr int MOE_GEMM_MAX_WGS_PER_CU = 2;
+int moe_launch_gemm_small_tile(const MoeGemmParams& p, int64_t R, hipStream_t stream);
 int moe_gemm_num_counters();   // ints at the start of the exchange area that must be zero at launch
 // test aid: workgroups of a launch with this geometry, and each workgroup's work item (9 ints per workgroup)
 int64_t moe_gemm_plan_blocks(int64_t R, int E, int64_t N, int pair);
@@ -152,7 +156,7 @@ int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldp
 // the two launches of that pair by themselves: job j's partials [row tile of 256][K][16] at partial + j * partial_stride (out, so and rank
 // unused); and the sum of up to MOE_XTP_MAX_REDUCE sets of such partials (out strides {expert, k, r}), wherever they come from
 constexpr int MOE_XTP_MAX_REDUCE = 6;
-struct MoeXtpReduceJob { const float* partial; int64_t K; void* out; int64_t so[3]; int rank; };
+struct MoeXtpReduceJob { const float* partial; int64_t K; void* out; int64_t so[3]; int rank; int tile_rows; };   // tile_rows: rows of a partial (0: those of the passes above)
 int moe_launch_xtp_partial_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldpt, const void* offsets, int off64, int E, int64_t R,
                                 float* partial, int64_t partial_stride, hipStream_t stream, int f16);
 int moe_launch_xtp_reduce_jobs(const MoeXtpReduceJob* jobs, int njobs, const void* offsets, int off64, int E, float scale, hipStream_t stream, int f16);

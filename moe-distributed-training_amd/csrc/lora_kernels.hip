@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(XTP_THREADS, 4) xtp_partial_kernel(const XtpJo
 
 // out[e][k][r] = scale * sum over the expert's partial tiles (ascending), zero for an empty expert.  A thread owns four
 // consecutive rank columns of one k (one 16-byte load per tile, several tiles in flight).
-struct XtpReduceJob { const float* partial; uint16_t* out; int64_t soe, sok, sor; int rank; int64_t K; };   // rank: columns written (<= 16)
+struct XtpReduceJob { const float* partial; uint16_t* out; int64_t soe, sok, sor; int rank, tile_rows; int64_t K; };   // rank: columns written (<= 16)
 struct XtpReduceJobs { XtpReduceJob job[MOE_XTP_MAX_REDUCE]; };
 template <typename Num>
 __global__ void xtp_reduce_kernel(const XtpReduceJobs jobs, const void* __restrict__ offsets, int off64, int E, float scale)
@@ -339,8 +339,9 @@ __global__ void xtp_reduce_kernel(const XtpReduceJobs jobs, const void* __restri
     const int rank = job.rank;
     const int e = blockIdx.y;
     int64_t tile0, start, end;
-    find_group(offsets, off64, E, XTP_RC, e, &start, &end, &tile0);   // one round trip, not one per expert (64 experts, six jobs: 22 us with 64-bit shuffles, 17.7 so)
-    const int64_t ntile = (end - start + XTP_RC - 1) / XTP_RC;
+    const int rows = job.tile_rows;
+    find_group(offsets, off64, E, rows, e, &start, &end, &tile0);   // one round trip, not one per expert (64 experts, six jobs: 22 us with 64-bit shuffles, 17.7 so)
+    const int64_t ntile = (int64_t)((uint32_t)(end - start + rows - 1) / (uint32_t)rows);
     const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (idx >= K * 16) return;
     const int64_t k = idx >> 4;
@@ -541,7 +542,7 @@ int moe_launch_xtp_reduce_jobs(const MoeXtpReduceJob* jobs, int njobs, const voi
     for (int j = 0; j < njobs; ++j) {
         const MoeXtpReduceJob& q = jobs[j];
         if (q.rank < 1 || q.rank > 16) return MOE_ERR_UNSUPPORTED;
-        js.job[j] = {q.partial, (uint16_t*)q.out, q.so[0], q.so[1], q.so[2], q.rank, q.K};
+        js.job[j] = {q.partial, (uint16_t*)q.out, q.so[0], q.so[1], q.so[2], q.rank, q.tile_rows ? q.tile_rows : XTP_RC, q.K};
         kmax = q.K > kmax ? q.K : kmax;
     }
     if (E == 0 || kmax == 0) return MOE_OK;
@@ -566,7 +567,7 @@ int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldp
     if (rc != MOE_OK) return rc;
     MoeXtpReduceJob red[MOE_LORA_MAX_JOBS];
     for (int j = 0; j < njobs; ++j)
-        red[j] = {(const float*)workspace + j * pstride, jobs[j].K, jobs[j].out, {jobs[j].so[0], jobs[j].so[1], jobs[j].so[2]}, jobs[j].rank};
+        red[j] = {(const float*)workspace + j * pstride, jobs[j].K, jobs[j].out, {jobs[j].so[0], jobs[j].so[1], jobs[j].so[2]}, jobs[j].rank, 0};
     return moe_launch_xtp_reduce_jobs(red, njobs, offsets, off64, E, scale, stream, f16);
 }
 

@@ -601,17 +601,29 @@ static inline size_t sk_bytes_mlp(int64_t R, int E, int64_t d, int64_t f)
     const size_t a = moe_gemm_sk_bytes(R, E, d), b = moe_gemm_sk_bytes(R, E, f);
     return a > b ? a : b;
 }
-// column-tile partials of the two fused column contractions of the dh GEMM: [2][ceil(f / 256)][R][16] fp32
-static inline size_t cc_bytes(int64_t R, int64_t f) { return (size_t)2 * (size_t)((f + 255) / 256) * (size_t)R * 16 * sizeof(float); }
+// column tiles of the gate/up launch (pair) and of the dh launch, and the partials of their column contractions, one of the former's and two of the
+// latter's: [column tiles][R][16] fp32 each
+static inline int cc_tiles(int64_t R, int E, int64_t d, int64_t f, bool pair) { const int w = moe_gemm_tile(R, E, d, f, pair) / (pair ? 2 : 1); return (int)((f + w - 1) / w); }
+static inline size_t cc_bytes(int64_t R, int E, int64_t d, int64_t f)
+{
+    const int a = cc_tiles(R, E, d, f, true), b = 2 * cc_tiles(R, E, d, f, false);
+    return (size_t)(a > b ? a : b) * (size_t)R * 16 * sizeof(float);
+}
+// one set of f columns' partials of the adapter gradients from the dh launch: its row tiles, or those of the separate passes where these are more
+static inline size_t rcp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
+{
+    const size_t n = moe_xtp_workspace_bytes(R, E, f), m = rank <= 16 ? (size_t)(R / moe_gemm_tile(R, E, d, f, false) + E) * (size_t)f * 16 * sizeof(float) : 0;
+    return n > m ? n : m;
+}
 
 // Partials of the adapter gradients: with the fused products (rank <= 16) three sets of f columns (from the dh GEMM) and three of d, all alive until one
 // launch sums them; without, two sets of either at a time.  The sets of d columns come when the grouped GEMMs are through: they lie
 // where those exchanged K-split tiles, behind the counters, or where that is too small in place of the column-tile partials, which have been added by then.
-static inline size_t mlp_xtp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank) { return 3 * moe_xtp_workspace_bytes(R, E, rank <= 16 || f > d ? f : d); }
+static inline size_t mlp_xtp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank) { return rank <= 16 ? 3 * rcp_bytes(R, E, d, f, rank) : 3 * moe_xtp_workspace_bytes(R, E, f > d ? f : d); }
 static inline bool mlp_xtp_d_in_exchange(int64_t R, int E, int64_t d, int64_t f) { return counter_bytes() + 3 * moe_xtp_workspace_bytes(R, E, d) <= sk_bytes_mlp(R, E, d, f); }
 static inline size_t mlp_cc_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
 {
-    const size_t cc = cc_bytes(R, f), x = rank <= 16 && !mlp_xtp_d_in_exchange(R, E, d, f) ? 3 * moe_xtp_workspace_bytes(R, E, d) : 0;
+    const size_t cc = cc_bytes(R, E, d, f), x = rank <= 16 && !mlp_xtp_d_in_exchange(R, E, d, f) ? 3 * moe_xtp_workspace_bytes(R, E, d) : 0;
     return cc > x ? cc : x;
 }
 
@@ -687,7 +699,7 @@ int moe_mlp_fwd(const void* x, int64_t ldx, const void* w1, const void* w3, cons
     // a rank of at most 16: the w2 GEMM's low-rank operand Q2 = h A2 comes out of the pair GEMM's epilogue as per-column-tile
     // partials (h is not read again for it); more chunks take separate passes over h
     const bool fuse_q2 = has_lora && rank <= 16;
-    float* ccw = fuse_q2 ? (float*)ws.take(cc_bytes(R, f)) : nullptr;
+    float* ccw = fuse_q2 ? (float*)ws.take(cc_bytes(R, E, d, f)) : nullptr;
     if (fuse_q2 && !ccw) return MOE_ERR_WORKSPACE;
     if (has_lora) {
         // lora order a1,b1,a3,b3,a2,b2; strides {expert, dim1, dim2}
@@ -745,7 +757,7 @@ int moe_mlp_fwd(const void* x, int64_t ldx, const void* w1, const void* w3, cons
     if (has_lora) {
         TIMED("fwd.rows_lora_h");
         if (fuse_q2)   // the products over each column tile came out of the pair GEMM's epilogue: add the tiles, scale, round
-            TRY(moe_launch_cc_reduce2(ccw, nullptr, (int)((f + 127) / 128), R, scaling, svp(2, 0), nullptr, svp(5, 0), nullptr, ldt, st, f16));
+            TRY(moe_launch_cc_reduce2(ccw, nullptr, cc_tiles(R, E, d, f, true), R, scaling, svp(2, 0), nullptr, svp(5, 0), nullptr, ldt, st, f16));
         else
         for (int c = 0; c < C; c += 2) {   // two chunks per launch: the twin's reads of h are served by L2
             const bool two = c + 1 < C;
@@ -884,12 +896,12 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         p.E = E; p.K = d; p.N = f; p.fan_out = dy_fan_out; p.x_grouped = dy_grouped; p.y_grouped = 1;
         p.epi = MOE_EPI_SWIGLU_BWD; p.f16 = f16;
         if (fuse_rc) {   // dB1 = Q1^T dgate, dB3 = Q3^T dup, dA2 = h^T (row_scale P2) as per-row-tile partials from the epilogue
-            const size_t one = moe_xtp_workspace_bytes(R, E, f);
+            const size_t one = rcp_bytes(R, E, d, f, rank);
             p.RC[0] = (const uint16_t*)svp(0, 0); p.RC[1] = (const uint16_t*)svp(1, 0); p.RC[2] = (const uint16_t*)p2s;
             for (int i = 0; i < 3; ++i) p.RCP[i] = (float*)((uint8_t*)xw + i * one);
             p.nrc = 3;
             // P1 = dgate B1^T, P3 = dup B3^T (the dX GEMM's low-rank operands) as per-column-tile partials
-            const size_t cone = cc_bytes(R, f) / 2 / sizeof(float);
+            const size_t cone = (size_t)cc_tiles(R, E, d, f, false) * (size_t)R * 16;
             p.CB[0] = (const uint16_t*)bt1[0]; p.CB[1] = (const uint16_t*)bt3[0];
             p.CCP[0] = ccw; p.CCP[1] = ccw + cone;
             p.ncc = 2; p.cc_rows = R;
@@ -923,8 +935,8 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         // ---- w1 / w3 backward
         TIMED("bwd.rows_lora_dgate_dup");
         if (fuse_rc) {   // the products over each column tile came out of the dh GEMM's epilogue: add the tiles, scale, round
-            const size_t cone = cc_bytes(R, f) / 2 / sizeof(float);
-            TRY(moe_launch_cc_reduce2(ccw, ccw + cone, (int)((f + 255) / 256), R, scaling, pqp(1, 0), pqp(2, 0), pqp(4, 0), pqp(5, 0), ldt, st, f16));
+            const size_t cone = (size_t)cc_tiles(R, E, d, f, false) * (size_t)R * 16;
+            TRY(moe_launch_cc_reduce2(ccw, ccw + cone, cc_tiles(R, E, d, f, false), R, scaling, pqp(1, 0), pqp(2, 0), pqp(4, 0), pqp(5, 0), ldt, st, f16));
         } else
         for (int c = 0; c < C; c += 2) {   // two chunks of one adapter per launch, so that dgate and dup are each fetched once per pair of chunks
             const bool two = c + 1 < C;
@@ -958,14 +970,15 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
             // One launch over x and dy leaves the partials of dA1, dA3 and dB2 beside those of dB1, dB3 and dA2 that the dh GEMM's epilogue
             // left, and one launch adds all six: six launches before (4096 tokens, d=4096, f=14336: 87 us together, 65 now; 512 tokens, d=256:
             // 41 us, 16 now -- each of them was a few workgroups behind a gap; 2048 tokens, 64 experts: 76 and 66).
-            const size_t onef = moe_xtp_workspace_bytes(R, E, f) / sizeof(float), oned = moe_xtp_workspace_bytes(R, E, d) / sizeof(float);
+            const size_t onef = rcp_bytes(R, E, d, f, rank) / sizeof(float), oned = moe_xtp_workspace_bytes(R, E, d) / sizeof(float);
             float* part = (float*)xw;
             float* partd = mlp_xtp_d_in_exchange(R, E, d, f) ? (float*)((uint8_t*)skws + counter_bytes()) : ccw;
             const MoeXtpJob jobs[3] = {{x, ldx, d, pos, fan_out, pqp(4, 0), nullptr, nullptr, {}, rank}, {x, ldx, d, pos, fan_out, pqp(5, 0), nullptr, nullptr, {}, rank},
                                        {dy, lddy, d, dy_grouped ? nullptr : pos, dy_fan_out, svp(5, 0), row_scale, nullptr, {}, rank}};
             TRY(moe_launch_xtp_partial_jobs(jobs, 3, pos64, ldt, offsets, off64, E, R, partd, (int64_t)oned, st, f16));
-            auto red = [&](const float* p, int64_t K, void* out, const int64_t* st3) { return MoeXtpReduceJob{p, K, out, {st3[0], st3[1], st3[2]}, rank}; };
-            const MoeXtpReduceJob sums[6] = {red(part, f, lg[1], so[1]), red(part + onef, f, lg[3], so[3]), red(part + 2 * onef, f, lg[4], so[4]),
+            const int bm = moe_gemm_tile(R, E, d, f, false);   // the dh launch's row tiles
+            auto red = [&](const float* p, int64_t K, void* out, const int64_t* st3, int rows = 0) { return MoeXtpReduceJob{p, K, out, {st3[0], st3[1], st3[2]}, rank, rows}; };
+            const MoeXtpReduceJob sums[6] = {red(part, f, lg[1], so[1], bm), red(part + onef, f, lg[3], so[3], bm), red(part + 2 * onef, f, lg[4], so[4], bm),
                                              red(partd, d, lg[0], so[0]), red(partd + oned, d, lg[2], so[2]), red(partd + 2 * oned, d, lg[5], so[5])};
             TRY(moe_launch_xtp_reduce_jobs(sums, 6, offsets, off64, E, 1.f, st, f16));
         } else

@@ -617,6 +617,36 @@ def test_ragged_row_tiles_of_every_block_count(dev, oracle, counts):
         check_expert_grads(lt[n][1].grad, lo[n][1].grad, f"dB {n}", tol=TINY_GROUP_TOL)
 
 
+@pytest.mark.parametrize("counts", [[1, 16, 17, 32, 33, 48, 64, 65], [100, 128, 129, 144, 160, 161, 193, 224], [225, 255, 256, 257, 300, 511, 513, 0]])
+@pytest.mark.parametrize("d,f", [(1088, 2112), (192, 320)])
+def test_ragged_row_tiles_in_large_and_small_tiles(dev, oracle, counts, d, f):
+    """The row counts above where the launches take 256 x 256 tiles (1088 x 2112: the chip is more than half full) and where they take 128 x 128
+    ones with a last column tile that is not full (192 x 320); the row tiles' partials of the adapter gradients differ in number."""
+    import moe_distributed_training_amd as moe
+    r, alpha, E, R = 16, 32.0, len(counts), sum(counts)
+    g = torch.Generator().manual_seed(12)
+    rn = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).bfloat16()
+    w1, w2, w3 = rn(E, f, d, std=0.03), rn(E, f, d, std=0.03), rn(E, f, d, std=0.03)
+    lora = {"w1": (rn(E, d, r, std=0.03), rn(E, r, f, std=0.03)), "w3": (rn(E, d, r, std=0.03), rn(E, r, f, std=0.03)),
+            "w2": (rn(E, f, r, std=0.03), rn(E, r, d, std=0.03))}
+    xr, dy = rn(R, d), rn(R, d)
+    e_of_row = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(R, generator=g)]
+    sei, ssi = oracle.flatten_and_sort(e_of_row)
+    eo = torch.bincount(sei, minlength=E).cumsum(0)
+    lt, views = _views(lora, dev)
+    xg = xr.to(dev).requires_grad_(True)
+    y = moe.fused_expert_mlp(xg, w1.to(dev), w2.to(dev), w3.to(dev), 1, ssi.int().to(dev), eo.int().to(dev), views, alpha)
+    y.backward(dy.to(dev))
+    xo = xr.float().requires_grad_(True)
+    lo = {n: (a.float().requires_grad_(True), b.float().requires_grad_(True)) for n, (a, b) in lora.items()}
+    ref, _ = oracle.moe_block(xo, None, w1.float(), w2.float(), w3.float(), 1, lo, alpha, routing=(torch.ones(R, 1), e_of_row[:, None]))
+    ref.backward(dy.float())
+    assert rel(y, ref) < 1e-2 and rel(xg.grad, xo.grad) < 1e-2
+    for n in ("w1", "w3", "w2"):
+        check_expert_grads(lt[n][0].grad, lo[n][0].grad, f"dA {n}", tol=TINY_GROUP_TOL)
+        check_expert_grads(lt[n][1].grad, lo[n][1].grad, f"dB {n}", tol=TINY_GROUP_TOL)
+
+
 @pytest.mark.slow
 def test_skewed_full_size_properties(dev, oracle):
     """BASELINE configs[3] at its full size (T=16384, E=8, top-2, Zipf-skewed routing, LoRA r=16, fwd+bwd) through
