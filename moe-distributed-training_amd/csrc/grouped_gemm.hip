@@ -35,6 +35,15 @@ size_t moe_gemm_sk_bytes(int64_t R, int E, int64_t N)
     return (size_t)moe_gemm_num_counters() * sizeof(int) + 256 + bytes;
 }
 
+// what a launch of these sizes (K: all segments) writes of that area behind the counters, at most
+size_t moe_gemm_exchange_bytes(int64_t R, int E, int64_t K, int64_t N)
+{
+    const int64_t tile = moe_gemm_tile(R, E, K, N, false), tiles = (R / tile + E) * ((N + tile - 1) / tile), most = 256 / tile * moe_num_cus();
+    int64_t split = 1;
+    while (split * 2 <= moe_gemm_max_split(false) && (K + BK - 1) / BK / (split * 2) >= MIN_PART_KTILES) split *= 2;
+    return split == 1 ? 0 : (size_t)(split * tiles < most ? split * tiles : most) * tile * tile * sizeof(float);
+}
+
 void moe_gemm_sk_attach(MoeGemmParams& p, void* ws, int64_t, int, int64_t)
 {
     p.sk_counters = (int*)ws;

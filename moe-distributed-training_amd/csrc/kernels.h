@@ -69,6 +69,7 @@ struct MoeGemmParams {
 
 size_t moe_gemm_sk_bytes(int64_t R, int E, int64_t N);
 void moe_gemm_sk_attach(MoeGemmParams& p, void* ws, int64_t R, int E, int64_t N);
+size_t moe_gemm_exchange_bytes(int64_t R, int E, int64_t K, int64_t N);
 int moe_gemm_max_split(bool pair);
 // rows and columns of a launch's output tiles: 256, one workgroup per compute unit, or 128, two (K: all segments; general-shape launches always 256)
 int moe_gemm_tile(int64_t R, int E, int64_t K, int64_t N, bool pair);

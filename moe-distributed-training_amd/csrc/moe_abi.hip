@@ -619,7 +619,21 @@ static inline size_t rcp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
 // Partials of the adapter gradients: with the fused products (rank <= 16) three sets of f columns (from the dh GEMM) and three of d, all alive until one
 // launch sums them; without, two sets of either at a time.  The sets of d columns come when the grouped GEMMs are through: they lie
 // where those exchanged K-split tiles, behind the counters, or where that is too small in place of the column-tile partials, which have been added by then.
-static inline size_t mlp_xtp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank) { return rank <= 16 ? 3 * rcp_bytes(R, E, d, f, rank) : 3 * moe_xtp_workspace_bytes(R, E, f > d ? f : d); }
+// Where the dh launch takes small tiles, which leave more row-tile partials, those lie in the exchange area too: behind what it, the dX launch and the sets of d columns use of it.
+static inline size_t rcp_exchange_offset(int64_t R, int E, int64_t d, int64_t f)
+{
+    const size_t a = moe_gemm_exchange_bytes(R, E, d, f), b = moe_gemm_exchange_bytes(R, E, 2 * f, d), c = 3 * moe_xtp_workspace_bytes(R, E, d);
+    return counter_bytes() + al(a > b ? (a > c ? a : c) : (b > c ? b : c));
+}
+static inline bool rcp_in_exchange(int64_t R, int E, int64_t d, int64_t f)
+{
+    return moe_gemm_tile(R, E, d, f, false) == 128 && rcp_exchange_offset(R, E, d, f) + 3 * rcp_bytes(R, E, d, f, 16) <= sk_bytes_mlp(R, E, d, f);
+}
+static inline size_t mlp_xtp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
+{
+    if (rank > 16) return 3 * moe_xtp_workspace_bytes(R, E, f > d ? f : d);
+    return rcp_in_exchange(R, E, d, f) ? 0 : 3 * rcp_bytes(R, E, d, f, rank);
+}
 static inline bool mlp_xtp_d_in_exchange(int64_t R, int E, int64_t d, int64_t f) { return counter_bytes() + 3 * moe_xtp_workspace_bytes(R, E, d) <= sk_bytes_mlp(R, E, d, f); }
 static inline size_t mlp_cc_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
 {
@@ -842,7 +856,7 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         if (fuse_rc) p2s = ws.take(qb);   // P2 times the row scale, row-major (the fused contraction's operand)
         if (fuse_rc) ccw = (float*)ws.take(mlp_cc_bytes(R, E, d, f, rank));
         xb = mlp_xtp_bytes(R, E, d, f, rank);
-        xw = ws.take(xb);
+        xw = fuse_rc && rcp_in_exchange(R, E, d, f) ? (void*)((uint8_t*)skws + rcp_exchange_offset(R, E, d, f)) : ws.take(xb);
         TIMED("bwd.pack_lora");
         for (int c = 0; c < C; ++c) {
             bt2[c] = ws.take(pbd);  // fragment order of b2[e][r][n=d]
