@@ -99,6 +99,92 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_gemm_kernel(
     if (mval && n0 + tx < N) Elem<T>::st(Y + out_row * sym + (n0 + tx) * syn, acc);
 }
 
+// fp32 products without adapters on the fp32 matrix instructions: 16 rows x 64 columns per workgroup, a wave per 16 columns, steps of 64 along the contraction whose loads are
+// requested a step ahead.  A thread of the kernel above reads two LDS words per multiply-add, which bounds it from a few hundred rows on; here a wave reads two per 16.
+// LDS pitches: the 16 rows (or columns) x 4 k of a fragment, and the row of 64 that a wave stores, meet different banks; the weight's image is [n][k] or
+// [k][n] as the weight is contiguous.  fp32 products and sums; a step's sums run over k in another order than above.
+// (Contractions of at most 32 take steps of 16, whose loads are all of them used: 2048 rows over 8 experts, K x 2048, us with the kernel above, steps of 64 and of 16: 8 25.2, 24.3 and 15.2.)
+constexpr int FM_ROWS = 16, FM_COLS = 64, FM_K_LONG = 64, FM_K_SHORT = 16, FM_WP = FM_COLS + 16;
+template <bool PAIR, int FM_K>
+__global__ void __launch_bounds__(256) grouped_gemm_f32_kernel(
+    const float* __restrict__ X, int64_t sxm, int64_t sxk, const float* __restrict__ W, const float* __restrict__ W_up, int64_t swe, int64_t swk, int64_t swn,
+    float* __restrict__ Y, int64_t sym, int64_t syn, const void* __restrict__ pos, int pos64, const void* __restrict__ offsets, int off64, int E, int64_t K,
+    int64_t N, int fan_out, int x_grouped, int y_grouped)
+{
+    constexpr int FM_XP = FM_K + 4, STEP = 256 / FM_K;
+    constexpr int XPT = FM_ROWS * FM_K / 256, WPT = FM_COLS * FM_K / 256;   // elements per thread and step
+    __shared__ float xs[FM_ROWS * FM_XP];
+    __shared__ float ws[PAIR ? 2 : 1][FM_K * FM_WP];   // (64 columns of FM_XP fit as well)
+    static_assert(FM_COLS * FM_XP <= FM_K * FM_WP, "either image");
+    __shared__ int64_t s_in[FM_ROWS], s_out[FM_ROWS];
+    RowTile rt;
+    if (!find_row_tile(offsets, off64, E, FM_ROWS, blockIdx.x, &rt)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 15, g = lane >> 4;
+    const int nrows = (int)(rt.row1 - rt.row0);
+    const int64_t n0 = (int64_t)blockIdx.y * FM_COLS;
+    if (tid < FM_ROWS) {   // rows past the group repeat its last one and are not stored
+        const int64_t m = rt.row0 + (tid < nrows ? tid : nrows - 1);
+        const int64_t p = (x_grouped && y_grouped) ? 0 : load_idx(pos, m, pos64);
+        s_in[tid] = x_grouped ? m : p / fan_out;
+        s_out[tid] = y_grouped ? m : p;
+    }
+    __syncthreads();
+    const float* We = W + (int64_t)rt.expert * swe;
+    const float* Wu = PAIR ? W_up + (int64_t)rt.expert * swe : nullptr;
+    const bool along_k = swk == 1;   // neighbouring threads along the weight's contiguous direction
+    const int hi = tid / FM_K, lo = tid % FM_K, nhi = tid / FM_COLS, nlo = tid % FM_COLS;
+    float xv[XPT], wv[WPT], uv[PAIR ? WPT : 1];
+    auto load = [&](int64_t k0) {
+#pragma unroll
+        for (int q = 0; q < XPT; ++q) xv[q] = k0 + lo < K ? X[s_in[hi + STEP * q] * sxm + (k0 + lo) * sxk] : 0.f;
+#pragma unroll
+        for (int q = 0; q < WPT; ++q) {
+            const int64_t k = k0 + (along_k ? lo : nhi + 4 * q), n = n0 + (along_k ? hi + STEP * q : nlo);
+            const bool in = k < K && n < N;
+            wv[q] = in ? We[k * swk + n * swn] : 0.f;
+            if (PAIR) uv[q] = in ? Wu[k * swk + n * swn] : 0.f;
+        }
+    };
+    f32x4_t acc2[2] = {}, up2[2] = {};   // alternate groups of four k: half as long a chain of sums, in time and in rounding
+    load(0);
+    const int nk = along_k ? FM_XP : 1, kk1 = along_k ? 1 : FM_WP;   // strides of n and k in the weight's image
+    const bool live = n0 + wave * 16 < N;
+    for (int64_t k0 = 0; k0 < K; k0 += FM_K) {
+#pragma unroll
+        for (int q = 0; q < XPT; ++q) xs[(hi + STEP * q) * FM_XP + lo] = xv[q];
+#pragma unroll
+        for (int q = 0; q < WPT; ++q) {
+            const int at = along_k ? (hi + STEP * q) * FM_XP + lo : (nhi + 4 * q) * FM_WP + nlo;
+            ws[0][at] = wv[q];
+            if (PAIR) ws[PAIR ? 1 : 0][at] = uv[q];
+        }
+        __syncthreads();
+        if (k0 + FM_K < K) load(k0 + FM_K);
+        if (live) {
+            const float* xp = xs + i * FM_XP + g;
+            const int w0 = (wave * 16 + i) * nk + g * kk1;
+            const int left = K - k0 < FM_K ? (int)(K - k0) : FM_K;   // (what the image holds past K is zero)
+            for (int kq = 0; kq < left; kq += 16)
+#pragma unroll
+                for (int c = 0; c < 16; c += 4) {
+                    const float x = xp[kq + c];
+                    const int h = c / 4 & 1;
+                    acc2[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, ws[0][w0 + (kq + c) * kk1], acc2[h], 0, 0, 0);
+                    if (PAIR) up2[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, ws[PAIR ? 1 : 0][w0 + (kq + c) * kk1], up2[h], 0, 0, 0);
+                }
+        }
+        __syncthreads();
+    }
+    // element r: row 4 g + r, column i of the wave's 16
+    const int64_t n = n0 + wave * 16 + i;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float a = acc2[0][r] + acc2[1][r], u = up2[0][r] + up2[1][r];
+        const float v = PAIR ? a / (1.f + __expf(-a)) * u : a;   // as swiglu_fwd_kernel
+        if (4 * g + r < nrows && n < N) Y[s_out[4 * g + r] * sym + n * syn] = v;
+    }
+}
+
 // O[e][k][n] = scale * sum_{m in group e} X[m][k] * Y[m][n];  zero for an empty group.  The last step is worked through in pieces of GT rows, as far
 // as it holds rows, and a group of one piece by itself: the products are bound by their LDS reads (8 of 2048 x 2048, fp32: one row per
 // expert 82 us, 260 as a whole step; 300 rows 1214 and 1274).
@@ -156,6 +242,15 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_xty_kernel(
     if (k0 + ty < K && n0 + tx < N) Elem<T>::st(O + (int64_t)e * soe + (k0 + ty) * sok + (n0 + tx) * son, acc * scale);
 }
 
+// Few workgroups, or few columns: a thread of this kernel fetches four times the weights of the one above before it can begin.  us, above and here: 32 rows over 8 experts,
+// K = 77, N = 301 (40 tiles) 6.7 and 8.1; 64 rows, 40 x 50 6.3 and 6.8; 2048 rows, 250 x 16 10.4 and 11.4; 512 rows over 4 experts, 256 x 128 (64 tiles) 11.8 and 12.0,
+// 128 x 256 (128) 10.1 and 9.1; 1024 rows over 8 experts, 256 x 512 27.9 and 18.6; 2048 rows, 128 x 2048 83 and 41, 2048 x 512 287 and 110.
+bool f32_on_matrix_cores(int64_t R, int E, int64_t N)
+{
+    const int64_t rows16 = R / FM_ROWS, groups = R < E ? R : E;
+    return N > FM_COLS / 2 && (rows16 > groups ? rows16 : groups) * ((N + FM_COLS - 1) / FM_COLS) >= 64;
+}
+
 }  // namespace
 
 int moe_launch_generic_gemm(const void* X, int64_t sxm, int64_t sxk, const void* W, int64_t swe, int64_t swk,
@@ -167,6 +262,13 @@ int moe_launch_generic_gemm(const void* X, int64_t sxm, int64_t sxk, const void*
     if (R == 0 || N == 0) return MOE_OK;
     const int64_t mtiles = R / GT + E;  // upper bound on sum_e ceil(c_e / GT)
     dim3 grid((unsigned)mtiles, (unsigned)((N + GT - 1) / GT));
+    if (dtype == MOE_F32 && !A && f32_on_matrix_cores(R, E, N)) {
+        static_assert(FM_ROWS == GT, "the same row tiles");
+        auto f32 = K <= 2 * FM_K_SHORT ? grouped_gemm_f32_kernel<false, FM_K_SHORT> : grouped_gemm_f32_kernel<false, FM_K_LONG>;
+        hipLaunchKernelGGL(f32, dim3((unsigned)mtiles, (unsigned)((N + FM_COLS - 1) / FM_COLS)), dim3(256), 0, stream, (const float*)X, sxm, sxk, (const float*)W,
+                           (const float*)nullptr, swe, swk, swn, (float*)Y, sym, syn, pos, pos64, offsets, off64, E, K, N, fan_out, x_grouped, y_grouped);
+        return moe_launch_status();
+    }
     MOE_DISPATCH_DTYPE(dtype, {
         auto kern = short_steps(K, A != nullptr) ? generic_grouped_gemm_kernel<T, false, GK_SHORT> : generic_grouped_gemm_kernel<T, false, GK>;
         hipLaunchKernelGGL(kern, grid, dim3(GT * GT), 0, stream, (const T*)X, sxm, sxk, (const T*)W, (const T*)nullptr, swe, swk, swn, (const T*)A, sae, sak,
@@ -180,6 +282,12 @@ int moe_launch_generic_swiglu_pair(const float* X, int64_t sxm, int64_t sxk, con
                                    int64_t K, int64_t N, int fan_out, hipStream_t stream)
 {
     if (R == 0 || N == 0) return MOE_OK;
+    if (f32_on_matrix_cores(R, E, N)) {
+        auto f32 = K <= 2 * FM_K_SHORT ? grouped_gemm_f32_kernel<true, FM_K_SHORT> : grouped_gemm_f32_kernel<true, FM_K_LONG>;
+        hipLaunchKernelGGL(f32, dim3((unsigned)(R / FM_ROWS + E), (unsigned)((N + FM_COLS - 1) / FM_COLS)), dim3(256), 0, stream, X, sxm, sxk, W_gate, W_up, swe, swk,
+                           swn, H, ldh, (int64_t)1, pos, pos64, offsets, off64, E, K, N, fan_out, 0, 1);
+        return moe_launch_status();
+    }
     dim3 grid((unsigned)(R / GT + E), (unsigned)((N + GT - 1) / GT));
     auto kern = short_steps(K, false) ? generic_grouped_gemm_kernel<float, true, GK_SHORT> : generic_grouped_gemm_kernel<float, true, GK>;
     hipLaunchKernelGGL(kern, grid, dim3(GT * GT), 0, stream, X, sxm, sxk, W_gate, W_up, swe, swk, swn, (const float*)nullptr,

@@ -175,6 +175,32 @@ def test_scatter2scatter_out_argument_and_empty(dev, oracle):
     assert y0.shape == (0, N)
 
 
+@pytest.mark.parametrize("counts,K,N", [([17, 0, 1, 16, 15, 300], 64, 256), ([5, 130, 33], 63, 513), ([16] * 9, 65, 449), ([700, 324], 1, 80), ([700, 324], 31, 200), ([40, 60], 130, 1000)])
+@pytest.mark.parametrize("layout", ["k", "n", "wide"])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_fp32_products_on_the_matrix_cores(dev, counts, K, N, layout, gathered):
+    """fp32 products without adapters, edges of their 16-row, 64-column and 64-k tiles, weights contiguous along k or n or along neither, rows grouped or
+    gathered and scattered, against 64 bits.  Bound: a result is a sum of K products, each rounding at most 2^-24 of the sum of their magnitudes."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(K + N)
+    E, R = len(counts), sum(counts)
+    X = torch.randn(R, K, generator=g)
+    W = torch.randn(E, K, N, generator=g)
+    order = torch.randperm(R, generator=g) if gathered else torch.arange(R)
+    sei = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    Wd = W.to(dev)
+    if layout == "k":
+        Wd = Wd.transpose(1, 2).contiguous().transpose(1, 2)
+    elif layout == "wide":
+        Wd = torch.empty(E, K, 2 * N, device=dev)[:, :, ::2].copy_(Wd)
+    y = ops.scatter2scatter(X.to(dev), Wd, sei.to(dev), order.to(dev), 1, None, not gathered, not gathered).cpu().double()
+    rows = X[order].double() if gathered else X.double()
+    ref = torch.cat([rows[sei == e] @ W[e].double() for e in range(E)])
+    mag = torch.cat([rows[sei == e].abs() @ W[e].double().abs() for e in range(E)])
+    got = y[order] if gathered else y
+    assert bool(((got - ref).abs() <= K * 2.0 ** -24 * mag + 1e-30).all())
+
+
 @pytest.mark.parametrize("counts,K,N", [
     ([301, 0, 77, 1, 513], 256, 512),        # ragged groups: empty, one row, not a multiple of the 64-row step
     ([64, 128, 192], 512, 256),              # whole steps only
