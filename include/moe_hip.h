@@ -59,7 +59,8 @@ int moe_profile_get(int i, char* name, int name_cap, float* ms);
 /* ---- tile plan of the grouped GEMM (test aid; no counterpart in the reference) ------------------------------
  * The matrix-core grouped GEMM hands every workgroup one work item (an output tile of one expert, or one K part of a
  * tile).  moe_gemm_debug_plan_blocks() returns the number of workgroups a launch over R rows, E experts and N output
- * columns uses (pair != 0: the gate/up pair kernel with 128 columns per projection and tile);
+ * columns uses (pair != 0: the gate/up pair kernel with 128 columns per projection and tile; tiles of 256 x 256,
+ * which small launches cut smaller);
  * moe_gemm_debug_plan() writes, for each of them, 9 ints into `out` (device memory): valid, expert, n tile, first
  * row, one-past-last row, K part, K parts, exchange slot, split-tile counter.  Tests use it to check that every tile
  * is covered exactly once for any group sizes. */

@@ -7,7 +7,7 @@
 // experts of f = 14336 and at most 256 rows make, leaves half of the chip idle in its last).  The others may cut the tiles of the last, partial round of
 // compute units 2 or 4 ways.
 int moe_gemm_max_split(bool pair) { return pair ? 1 : 4; }
-int moe_gemm_num_counters() { return MOE_GEMM_MAX_WGS_PER_CU * moe_num_cus(); }
+int moe_gemm_num_counters() { return moe_num_cus(); }
 
 static int plan_ntiles_n(int64_t N, int pair) { return pair ? (int)((N + BN / 2 - 1) / (BN / 2)) : (int)((N + BN - 1) / BN); }
 int64_t moe_gemm_plan_blocks(int64_t R, int E, int64_t N, int pair) { return plan_grid(R, E, plan_ntiles_n(N, pair), moe_num_cus()); }
@@ -83,7 +83,8 @@ bool moe_gemm_mfma_supported(const MoeGemmParams& p, int64_t R)
 // an epilogue on workgroups of which most of the chip has none.  Quarter tiles spread it over up to four times as many workgroups, each with a quarter of the
 // epilogue.  Launches in us with large and small tiles: 512 tokens, d = 256, f = 512, 8 experts: gate/up (36 workgroups) 15.8 and 12.9, h W2 16.0 and 12.4, dh 24.2 and 16.3, dX 21.4
 // and 16.0; 64 rows of one expert, d = 4096, f = 14336: gate/up (112) 59.8 and 46.3, h W2 (64) 55.9 and 44.9, dh (224) 46.7 and 54.0, dX (64) 97 and 82; 500 rows: gate/up (224) 98
-// and 142, h W2 (128) 93 and 98, dX (128) 159 and 154; 2 rows of two experts: h W2 (128) 52 and 49; 4 tokens: h W2 (224) 115 and 142.  Where the chip is full the small tiles fetch
+// and 142, h W2 (128) 93 and 98, dX (128) 159 and 154 (319 rows, all of it 409 and 419); 2 rows of two experts: h W2 (128) 52 and 49; 4 tokens: h W2 (224) 115 and 142.  Groups of more than 128 rows
+// fetch their weights for more row tiles, so they take small tiles up to three eighths of the chip only.  Where the chip is full the small tiles fetch
 // twice the operand bytes per product: 2048 tokens, 64 experts, top-8 837 us and 946.
 int moe_gemm_tile(int64_t R, int E, int64_t K, int64_t N, bool pair)
 {
@@ -92,7 +93,7 @@ int moe_gemm_tile(int64_t R, int E, int64_t K, int64_t N, bool pair)
     const int64_t tiles = groups * (((R + groups - 1) / groups + BM - 1) / BM) * ((N + BN - 1) / BN * (pair ? 2 : 1));
     int64_t split = 1;
     while (split * 2 <= moe_gemm_max_split(pair) && tiles * split * 2 <= ncu && K / BK / (split * 2) >= MIN_PART_KTILES) split *= 2;
-    return tiles * split * 2 <= ncu ? 128 : 256;
+    return R <= groups * 128 ? (tiles * split * 2 <= ncu ? 128 : 256) : (tiles * split * 8 <= 3 * ncu ? 128 : 256);
 }
 
 static std::atomic<int64_t> g_mfma_launches{0};

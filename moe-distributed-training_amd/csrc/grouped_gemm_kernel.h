@@ -39,7 +39,7 @@ constexpr int BM = MOE_GEMM_TILE, BN = MOE_GEMM_TILE, BK = 64;
 constexpr int NWAVES = BM / 32;           // 2 x 4 waves of 128x64, or 2 x 2 of 64x64
 constexpr int NTHREADS = NWAVES * 64;
 constexpr int WGS_PER_CU = 256 / BM;      // workgroups that a compute unit holds (LDS)
-static_assert(WGS_PER_CU <= MOE_GEMM_MAX_WGS_PER_CU, "counters for every split tile");
+static_assert(WGS_PER_CU <= 2, "a split tile has at least two workgroups of a round: a counter per compute unit is enough");
 constexpr int WAVES_M = 2, WAVES_N = NWAVES / 2;
 constexpr int WTM = BM / WAVES_M;  // 128 or 64
 constexpr int WTN = BN / WAVES_N;  // 64
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
     const int ktiles = TWO_SEG ? ktiles_seg * p.nseg : ktiles_seg;
     const WorkItem item = decode_work_item(p.offsets, p.off64, p.E, ntiles_n, ktiles, p.max_split, p.num_cus);
     if (EPI_IS_PAIR(EPI) && p.clear_counters && blockIdx.x == 0)   // (this launch splits no tile: the counters are the next launch's)
-        for (int i = tid; i < p.num_cus / WGS_PER_CU * MOE_GEMM_MAX_WGS_PER_CU; i += NTHREADS) p.sk_counters[i] = 0;
+        for (int i = tid; i < p.num_cus / WGS_PER_CU; i += NTHREADS) p.sk_counters[i] = 0;
     if (!item.valid) return;
     const int expert = item.expert, nt = item.nt, part = item.part, nparts = item.nparts, split_item = item.split_item;
     const int64_t row0 = item.row0, row1 = item.row1;
@@ -1212,7 +1212,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
             // over this wave's 128 rows: the lower row of waves parks its sums in its own slices, the upper one adds them
             // to its own (a fixed order) and stores the tile's partial
             static_assert(WAVES_N * RC_MATS * IBLK * 1024 <= TABLE_OFF, "the exchange stays in front of the tables");
-            float* xch = (float*)(smem + (wave % WAVES_N) * (RC_MATS * IBLK * 1024));
+            // (a small tile's slices hold less than a wave parks)
+            float* xch = (float*)(smem + (BM == 256 ? ((wave % WAVES_N) + WAVES_N) * (WTM * WTN * 2) : (wave % WAVES_N) * (RC_MATS * IBLK * 1024)));
             if (wm == 1) {
 #pragma unroll
                 for (int mat = 0; mat < RC_MATS; ++mat)

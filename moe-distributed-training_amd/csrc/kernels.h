@@ -73,7 +73,6 @@ size_t moe_gemm_exchange_bytes(int64_t R, int E, int64_t K, int64_t N);
 int moe_gemm_max_split(bool pair);
 // rows and columns of a launch's output tiles: 256, one workgroup per compute unit, or 128, two (K: all segments; general-shape launches always 256)
 int moe_gemm_tile(int64_t R, int E, int64_t K, int64_t N, bool pair);
-constexpr int MOE_GEMM_MAX_WGS_PER_CU = 2;
 int moe_launch_gemm_small_tile(const MoeGemmParams& p, int64_t R, hipStream_t stream);
 int moe_gemm_num_counters();   // ints at the start of the exchange area that must be zero at launch
 // test aid: workgroups of a launch with this geometry, and each workgroup's work item (9 ints per workgroup)

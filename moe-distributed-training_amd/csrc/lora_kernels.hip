@@ -339,9 +339,10 @@ __global__ void xtp_reduce_kernel(const XtpReduceJobs jobs, const void* __restri
     const int rank = job.rank;
     const int e = blockIdx.y;
     int64_t tile0, start, end;
-    const int rows = job.tile_rows;
-    find_group(offsets, off64, E, rows, e, &start, &end, &tile0);   // one round trip, not one per expert (64 experts, six jobs: 22 us with 64-bit shuffles, 17.7 so)
-    const int64_t ntile = (int64_t)((uint32_t)(end - start + rows - 1) / (uint32_t)rows);
+    const int rows = job.tile_rows;   // (of the passes above in most jobs: a division by a constant)
+    if (rows == XTP_RC) find_group(offsets, off64, E, XTP_RC, e, &start, &end, &tile0);
+    else find_group(offsets, off64, E, rows, e, &start, &end, &tile0);   // one round trip, not one per expert (64 experts, six jobs: 22 us with 64-bit shuffles, 17.7 so)
+    const int64_t ntile = rows == XTP_RC ? (end - start + XTP_RC - 1) / XTP_RC : (int64_t)((uint32_t)(end - start + rows - 1) / (uint32_t)rows);
     const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (idx >= K * 16) return;
     const int64_t k = idx >> 4;
