@@ -156,7 +156,7 @@ int moe_launch_xtp_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldp
 // the two launches of that pair by themselves: job j's partials [row tile of 256][K][16] at partial + j * partial_stride (out, so and rank
 // unused); and the sum of up to MOE_XTP_MAX_REDUCE sets of such partials (out strides {expert, k, r}), wherever they come from
 constexpr int MOE_XTP_MAX_REDUCE = 6;
-struct MoeXtpReduceJob { const float* partial; int64_t K; void* out; int64_t so[3]; int rank; int tile_rows; };   // tile_rows: rows of a partial (0: those of the passes above)
+struct MoeXtpReduceJob { const float* partial; int64_t K; void* out; int64_t so[3]; int rank; int tile_rows; };   // tile_rows: rows of a partial, 256 or 128 (0: the 256 of the passes above)
 int moe_launch_xtp_partial_jobs(const MoeXtpJob* jobs, int njobs, int pos64, int64_t ldpt, const void* offsets, int off64, int E, int64_t R,
                                 float* partial, int64_t partial_stride, hipStream_t stream, int f16);
 int moe_launch_xtp_reduce_jobs(const MoeXtpReduceJob* jobs, int njobs, const void* offsets, int off64, int E, float scale, hipStream_t stream, int f16);

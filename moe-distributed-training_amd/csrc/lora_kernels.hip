@@ -324,10 +324,13 @@ __global__ void __launch_bounds__(XTP_THREADS, 4) xtp_partial_kernel(const XtpJo
 }
 
 // out[e][k][r] = scale * sum over the expert's partial tiles (ascending), zero for an empty expert.  A thread owns four
-// consecutive rank columns of one k (one 16-byte load per tile, several tiles in flight).
+// consecutive rank columns of one k (one 16-byte load per tile, several tiles in flight).  A launch of a few us behind a gap, bound by its chain of
+// trips to memory: the rows of a partial are constants in it.  MIXED: jobs with partials of 128 rows among them; as a number known at run time the
+// rows cost two 32-bit divisions and 290 more instructions for every launch (64 experts, six jobs: 18.3 us,
+// 17.7 so; 8 experts, 4096 x 4096, rank 32: 7.7 and 7.2).
 struct XtpReduceJob { const float* partial; uint16_t* out; int64_t soe, sok, sor; int rank, tile_rows; int64_t K; };   // rank: columns written (<= 16)
 struct XtpReduceJobs { XtpReduceJob job[MOE_XTP_MAX_REDUCE]; };
-template <typename Num>
+template <typename Num, bool MIXED>
 __global__ void xtp_reduce_kernel(const XtpReduceJobs jobs, const void* __restrict__ offsets, int off64, int E, float scale)
 {
     const XtpReduceJob& job = jobs.job[blockIdx.z];
@@ -339,10 +342,10 @@ __global__ void xtp_reduce_kernel(const XtpReduceJobs jobs, const void* __restri
     const int rank = job.rank;
     const int e = blockIdx.y;
     int64_t tile0, start, end;
-    const int rows = job.tile_rows;   // (of the passes above in most jobs: a division by a constant)
-    if (rows == XTP_RC) find_group(offsets, off64, E, XTP_RC, e, &start, &end, &tile0);
-    else find_group(offsets, off64, E, rows, e, &start, &end, &tile0);   // one round trip, not one per expert (64 experts, six jobs: 22 us with 64-bit shuffles, 17.7 so)
-    const int64_t ntile = rows == XTP_RC ? (end - start + XTP_RC - 1) / XTP_RC : (int64_t)((uint32_t)(end - start + rows - 1) / (uint32_t)rows);
+    // one round trip, not one per expert (64 experts, six jobs: 22 us with 64-bit shuffles, 17.7 so)
+    if (MIXED && job.tile_rows == XTP_RC / 2) find_group(offsets, off64, E, XTP_RC / 2, e, &start, &end, &tile0);
+    else find_group(offsets, off64, E, XTP_RC, e, &start, &end, &tile0);
+    const int64_t ntile = MIXED && job.tile_rows == XTP_RC / 2 ? (end - start + XTP_RC / 2 - 1) / (XTP_RC / 2) : (end - start + XTP_RC - 1) / XTP_RC;
     const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (idx >= K * 16) return;
     const int64_t k = idx >> 4;
@@ -540,15 +543,18 @@ int moe_launch_xtp_reduce_jobs(const MoeXtpReduceJob* jobs, int njobs, const voi
     if (njobs < 1 || njobs > MOE_XTP_MAX_REDUCE) return MOE_ERR_UNSUPPORTED;
     XtpReduceJobs js = {};
     int64_t kmax = 0;
+    bool mixed = false;
     for (int j = 0; j < njobs; ++j) {
         const MoeXtpReduceJob& q = jobs[j];
-        if (q.rank < 1 || q.rank > 16) return MOE_ERR_UNSUPPORTED;
+        if (q.rank < 1 || q.rank > 16 || (q.tile_rows != 0 && q.tile_rows != XTP_RC && q.tile_rows != XTP_RC / 2)) return MOE_ERR_UNSUPPORTED;
+        mixed |= q.tile_rows == XTP_RC / 2;
         js.job[j] = {q.partial, (uint16_t*)q.out, q.so[0], q.so[1], q.so[2], q.rank, q.tile_rows ? q.tile_rows : XTP_RC, q.K};
         kmax = q.K > kmax ? q.K : kmax;
     }
     if (E == 0 || kmax == 0) return MOE_OK;
     dim3 rgrid((unsigned)((kmax * 4 + 255) / 256), (unsigned)E, (unsigned)njobs);
-    hipLaunchKernelGGL(f16 ? xtp_reduce_kernel<NumF16> : xtp_reduce_kernel<NumBf16>, rgrid, dim3(256), 0, stream, js, offsets, off64, E, scale);
+    auto kern = mixed ? (f16 ? xtp_reduce_kernel<NumF16, true> : xtp_reduce_kernel<NumBf16, true>) : (f16 ? xtp_reduce_kernel<NumF16, false> : xtp_reduce_kernel<NumBf16, false>);
+    hipLaunchKernelGGL(kern, rgrid, dim3(256), 0, stream, js, offsets, off64, E, scale);
     return moe_launch_status();
 }
 

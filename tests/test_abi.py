@@ -136,3 +136,21 @@ def test_the_mlp_workspace_holds_no_set_of_partials_twice():
         xtp = 3 * (R // 256 + E) * max(d, f) * 64
         columns = 2 * up(f, 256) // 256 * R * 64
         assert lib.moe_mlp_workspace_bytes(R, E, d, f, 16) <= lib.moe_mlp_workspace_bytes(R, E, d, f, 0) + factors + interims + xtp + columns + 4096
+
+
+def test_the_sum_of_adapter_partials_divides_by_constants(tmp_path):
+    """The launch that adds the adapter gradients' partials is a few us of trips to memory: the rows of a partial are constants in every variant of it, and no
+    32-bit division by a number known at run time (which starts with v_rcp_iflag_f32) stands before the first load."""
+    import shutil
+    import subprocess
+    import pytest
+    if shutil.which("hipcc") is None:
+        pytest.skip("no hipcc")
+    csrc = os.path.join(ROOT, "moe-distributed-training_amd", "csrc")
+    out = str(tmp_path / "lora_kernels.s")
+    subprocess.run(["hipcc", "-O3", "-std=c++17", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-w", "--offload-device-only", "-S",
+                    os.path.join(csrc, "lora_kernels.hip"), "-o", out], check=True, timeout=300)
+    bodies = dict(re.findall(r"^(\w*xtp_reduce_kernel\w*):[^\n]*\n(.*?)^\s*s_endpgm", open(out).read(), flags=re.S | re.M))
+    assert len(bodies) >= 2
+    for name, body in bodies.items():
+        assert "v_rcp_iflag_f32" not in body, name
