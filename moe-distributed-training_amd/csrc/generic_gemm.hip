@@ -242,13 +242,20 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_xty_kernel(
     if (k0 + ty < K && n0 + tx < N) Elem<T>::st(O + (int64_t)e * soe + (k0 + ty) * sok + (n0 + tx) * son, acc * scale);
 }
 
-// Few workgroups, or few columns: a thread of this kernel fetches four times the weights of the one above before it can begin.  us, above and here: 32 rows over 8 experts,
-// K = 77, N = 301 (40 tiles) 6.7 and 8.1; 64 rows, 40 x 50 6.3 and 6.8; 2048 rows, 250 x 16 10.4 and 11.4; 512 rows over 4 experts, 256 x 128 (64 tiles) 11.8 and 12.0,
-// 128 x 256 (128) 10.1 and 9.1; 1024 rows over 8 experts, 256 x 512 27.9 and 18.6; 2048 rows, 128 x 2048 83 and 41, 2048 x 512 287 and 110.
-bool f32_on_matrix_cores(int64_t R, int E, int64_t N)
+// Which of the two: by the workgroups of the one above, a tile of 16 x 16 each.  Up to two of them per compute unit run side by side and are through after one
+// chain of K steps; a thread of the kernel here fetches four times the weights before it can begin and has as long a chain.  From there on the one
+// above takes turns.  Measured with 256 compute units, by workgroups of the one above; us above and here, of one product (and of gate and up in one launch):
+//   256: 512 rows of 4 experts, K x N = 256 x 128, 11.6 and 11.9 (11.1 and 12.0); 8 rows of 8, 512 x 512, 13.4 and 17.6 (14.5 and 20.1)
+//   512: 512 rows of 4, 128 x 256, 9.9 and 9.0 (8.8 and 7.9);  768 and 2048, 512 rows of 2, 512 x 384 and 512 x 1024: 1.42 and 1.6 times as fast here
+// One round more where tiles or columns are half empty (groups of less than 16 rows; 65 to 85 columns of 128): 512, 8 rows of 8, 256 x 1024 10.3 and 11.1;
+// 640, 2048 rows of 4, 64 x 80 0.98 times as fast (0.94);  768, 8 rows of 8, 64 x 1536 1.04 (1.05).
+// Two rounds more below 64 k, where the chain is a step or two: 768, 64 rows of 8, 40 x 1536 0.95 (0.89); 1024, 512 rows of 2, 40 x 512 1.03 (1.01).
+bool f32_on_matrix_cores(int64_t R, int E, int64_t K, int64_t N)
 {
-    const int64_t rows16 = R / FM_ROWS, groups = R < E ? R : E;
-    return N > FM_COLS / 2 && (rows16 > groups ? rows16 : groups) * ((N + FM_COLS - 1) / FM_COLS) >= 64;
+    if (N <= FM_COLS / 2) return false;   // half of the columns at least (2048 rows, 250 x 16: 10.4 and 11.4)
+    const int64_t rows16 = R / FM_ROWS, groups = R < E ? R : E, workgroups = (rows16 > groups ? rows16 : groups) * ((N + GT - 1) / GT);
+    const bool full = R >= (int64_t)FM_ROWS * E && 3 * N >= 2 * ((N + FM_COLS - 1) / FM_COLS * FM_COLS);
+    return workgroups >= ((K < 64 ? 4 : 2) + (full ? 0 : 1)) * (int64_t)moe_device_cus();
 }
 
 }  // namespace
@@ -262,7 +269,7 @@ int moe_launch_generic_gemm(const void* X, int64_t sxm, int64_t sxk, const void*
     if (R == 0 || N == 0) return MOE_OK;
     const int64_t mtiles = R / GT + E;  // upper bound on sum_e ceil(c_e / GT)
     dim3 grid((unsigned)mtiles, (unsigned)((N + GT - 1) / GT));
-    if (dtype == MOE_F32 && !A && f32_on_matrix_cores(R, E, N)) {
+    if (dtype == MOE_F32 && !A && f32_on_matrix_cores(R, E, K, N)) {
         static_assert(FM_ROWS == GT, "the same row tiles");
         auto f32 = K <= 2 * FM_K_SHORT ? grouped_gemm_f32_kernel<false, FM_K_SHORT> : grouped_gemm_f32_kernel<false, FM_K_LONG>;
         hipLaunchKernelGGL(f32, dim3((unsigned)mtiles, (unsigned)((N + FM_COLS - 1) / FM_COLS)), dim3(256), 0, stream, (const float*)X, sxm, sxk, (const float*)W,
@@ -282,7 +289,7 @@ int moe_launch_generic_swiglu_pair(const float* X, int64_t sxm, int64_t sxk, con
                                    int64_t K, int64_t N, int fan_out, hipStream_t stream)
 {
     if (R == 0 || N == 0) return MOE_OK;
-    if (f32_on_matrix_cores(R, E, N)) {
+    if (f32_on_matrix_cores(R, E, K, N)) {
         auto f32 = K <= 2 * FM_K_SHORT ? grouped_gemm_f32_kernel<true, FM_K_SHORT> : grouped_gemm_f32_kernel<true, FM_K_LONG>;
         hipLaunchKernelGGL(f32, dim3((unsigned)(R / FM_ROWS + E), (unsigned)((N + FM_COLS - 1) / FM_COLS)), dim3(256), 0, stream, X, sxm, sxk, W_gate, W_up, swe, swk,
                            swn, H, ldh, (int64_t)1, pos, pos64, offsets, off64, E, K, N, fan_out, 0, 1);

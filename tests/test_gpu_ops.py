@@ -175,12 +175,13 @@ def test_scatter2scatter_out_argument_and_empty(dev, oracle):
     assert y0.shape == (0, N)
 
 
-@pytest.mark.parametrize("counts,K,N", [([17, 0, 1, 16, 15, 300], 64, 256), ([5, 130, 33], 63, 513), ([16] * 9, 65, 449), ([700, 324], 1, 80), ([700, 324], 31, 200), ([40, 60], 130, 1000)])
+@pytest.mark.parametrize("counts,K,N", [([17, 0, 1, 16, 15, 300], 64, 256), ([5, 130, 33], 63, 513), ([16] * 9, 65, 449), ([700, 324], 1, 80), ([700, 324], 31, 200), ([40, 60], 130, 1000),
+                                        ([17, 0, 1, 16, 15, 300] * 3, 64, 512), ([50, 1030, 333], 63, 513), ([16] * 36, 65, 449), ([4700, 1324], 1, 80), ([1700, 324], 31, 200), ([40, 160], 130, 1000)])
 @pytest.mark.parametrize("layout", ["k", "n", "wide"])
 @pytest.mark.parametrize("gathered", [False, True])
 def test_fp32_products_on_the_matrix_cores(dev, counts, K, N, layout, gathered):
     """fp32 products without adapters, edges of their 16-row, 64-column and 64-k tiles, weights contiguous along k or n or along neither, rows grouped or
-    gathered and scattered, against 64 bits.  Bound: a result is a sum of K products, each rounding at most 2^-24 of the sum of their magnitudes."""
+    gathered and scattered, against 64 bits; the same edges in launches of few tiles (the vector kernel) and of more.  Bound: a result is a sum of K products, each rounding at most 2^-24 of the sum of their magnitudes."""
     ops = _ops()
     g = torch.Generator().manual_seed(K + N)
     E, R = len(counts), sum(counts)
@@ -199,6 +200,35 @@ def test_fp32_products_on_the_matrix_cores(dev, counts, K, N, layout, gathered):
     mag = torch.cat([rows[sei == e].abs() @ W[e].double().abs() for e in range(E)])
     got = y[order] if gathered else y
     assert bool(((got - ref).abs() <= K * 2.0 ** -24 * mag + 1e-30).all())
+
+
+@pytest.mark.parametrize("counts,K,N,cores", [
+    ([128] * 4, 256, 128, False), ([1] * 8, 512, 512, False), ([1] * 8, 256, 1024, False), ([512] * 4, 64, 80, False), ([512] * 4, 512, 48, False), ([256] * 2, 40, 384, False),
+    ([128] * 4, 128, 256, True), ([256] * 2, 64, 384, True), ([1] * 8, 128, 2048, True), ([256] * 2, 40, 512, True), ([2048] * 4, 64, 40, True)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_which_fp32_products_run_on_the_matrix_cores(dev, counts, K, N, cores, pair):
+    """Launches of few tiles are the vector kernel's, which is the faster one there (by up to a quarter), for one product and for gate and up.  The vector kernel adds along k whatever N is, and
+    16 columns by themselves are always its own: the bits tell which kernel a launch took."""
+    from moe_distributed_training_amd._lib import lib, check, ptr, stream_ptr
+    ncu = torch.cuda.get_device_properties(dev).multi_processor_count
+    if ncu != 256:
+        pytest.skip("the sizes are those of 256 compute units")
+    g = torch.Generator().manual_seed(K + N)
+    E, R = len(counts), sum(counts)
+    X = torch.randn(R, K, generator=g).to(dev)
+    W, U = (torch.randn(E, K, N, generator=g).to(dev) for _ in range(2))
+    eo, pos = torch.tensor(counts).cumsum(0).int().to(dev), torch.arange(R, dtype=torch.int32, device=dev)
+    ops = _ops()
+    sei = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).int().to(dev)
+
+    def product(w, u):
+        if not pair:
+            return ops.scatter2scatter(X, w, sei, pos, 1, None, True, True)
+        y = torch.empty(R, w.size(2), device=dev)
+        check(lib.moe_swiglu_pair(ptr(X), K, 1, ptr(w), ptr(u), w.stride(0), w.stride(1), 1, ptr(y), y.size(1), ptr(pos), 0, ptr(eo), 0, E, R, K, w.size(2), 1, 2, stream_ptr(dev)), "pair")
+        return y
+    pieces = torch.cat([product(W[:, :, n:n + 16], U[:, :, n:n + 16]) for n in range(0, N, 16)], 1)
+    assert torch.equal(product(W, U), pieces) is not cores
 
 
 @pytest.mark.parametrize("counts,K,N", [
