@@ -7,47 +7,52 @@
 // experts of f = 14336 and at most 256 rows make, leaves half of the chip idle in its last).  The others may cut the tiles of the last, partial round of
 // compute units 2 or 4 ways.
 int moe_gemm_max_split(bool pair) { return pair ? 1 : 4; }
-int moe_gemm_num_counters() { return moe_num_cus(); }
+int moe_gemm_cus()
+{
+    const int n = moe_device_cus() / NXCD * NXCD;
+    return n < NXCD ? NXCD : n;
+}
 
 static int plan_ntiles_n(int64_t N, int pair) { return pair ? (int)((N + BN / 2 - 1) / (BN / 2)) : (int)((N + BN - 1) / BN); }
-int64_t moe_gemm_plan_blocks(int64_t R, int E, int64_t N, int pair) { return plan_grid(R, E, plan_ntiles_n(N, pair), moe_num_cus()); }
+int64_t moe_gemm_plan_blocks(int64_t R, int E, int64_t N, int pair) { return plan_grid(R, E, plan_ntiles_n(N, pair), moe_gemm_cus()); }
 int moe_launch_gemm_plan(const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg, int* out,
                          hipStream_t stream)
 {
     if (K < BK || nseg < 1 || nseg > 2) return MOE_ERR_UNSUPPORTED;
-    const int ntiles_n = plan_ntiles_n(N, pair);
-    const int64_t grid = plan_grid(R, E, ntiles_n, moe_num_cus());
+    const int ntiles_n = plan_ntiles_n(N, pair), cus = moe_gemm_cus();
+    const int64_t grid = plan_grid(R, E, ntiles_n, cus);
     hipLaunchKernelGGL(gemm_plan_kernel, dim3((unsigned)grid), dim3(64), 0, stream, offsets, off64, E, ntiles_n,
-                       (int)((K + BK - 1) / BK) * nseg, moe_gemm_max_split(pair != 0), moe_num_cus(), out);
+                       (int)((K + BK - 1) / BK) * nseg, moe_gemm_max_split(pair != 0), cus, out);
     return moe_launch_status();
 }
 
 // exchange area of a launch: one counter per split tile and one fp32 partial tile per split item; at most one round
 // of compute units' worth of either
-size_t moe_gemm_sk_bytes(int64_t R, int E, int64_t N)
+size_t moe_gemm_sk_bytes(int cus, int64_t R, int E, int64_t N)
 {
     size_t bytes = 0;   // of the tile size that needs more
     for (int tile = 256; tile >= 128; tile /= 2) {
-        const int64_t tiles = (R / tile + E) * ((N + tile - 1) / tile), most = 256 / tile * moe_num_cus();
+        const int64_t tiles = (R / tile + E) * ((N + tile - 1) / tile), most = 256 / tile * cus;
         const size_t b = (size_t)(4 * tiles < most ? 4 * tiles : most) * tile * tile * sizeof(float);
         bytes = b > bytes ? b : bytes;
     }
-    return (size_t)moe_gemm_num_counters() * sizeof(int) + 256 + bytes;
+    return (size_t)cus * sizeof(int) + 256 + bytes;
 }
 
-// what a launch of these sizes (K: all segments) writes of that area behind the counters, at most
-size_t moe_gemm_exchange_bytes(int64_t R, int E, int64_t K, int64_t N)
+// what a launch of these sizes (K: all segments) and tiles writes of that area behind the counters, at most
+size_t moe_gemm_exchange_bytes(int cus, int tile, int64_t R, int E, int64_t K, int64_t N)
 {
-    const int64_t tile = moe_gemm_tile(R, E, K, N, false), tiles = (R / tile + E) * ((N + tile - 1) / tile), most = 256 / tile * moe_num_cus();
+    const int64_t tiles = (R / tile + E) * ((N + tile - 1) / tile), most = 256 / tile * cus;
     int64_t split = 1;
     while (split * 2 <= moe_gemm_max_split(false) && (K + BK - 1) / BK / (split * 2) >= MIN_PART_KTILES) split *= 2;
     return split == 1 ? 0 : (size_t)(split * tiles < most ? split * tiles : most) * tile * tile * sizeof(float);
 }
 
-void moe_gemm_sk_attach(MoeGemmParams& p, void* ws, int64_t, int, int64_t)
+void moe_gemm_sk_attach(MoeGemmParams& p, void* ws, int cus)
 {
+    p.num_cus = cus;
     p.sk_counters = (int*)ws;
-    p.sk_partials = (float*)((uint8_t*)ws + (((size_t)moe_gemm_num_counters() * sizeof(int) + 255) & ~(size_t)255));
+    p.sk_partials = (float*)((uint8_t*)ws + (((size_t)cus * sizeof(int) + 255) & ~(size_t)255));
 }
 
 bool moe_gemm_mfma_supported(const MoeGemmParams& p, int64_t R)
@@ -86,10 +91,10 @@ bool moe_gemm_mfma_supported(const MoeGemmParams& p, int64_t R)
 // and 142, h W2 (128) 93 and 98, dX (128) 159 and 154 (319 rows, all of it 409 and 419); 2 rows of two experts: h W2 (128) 52 and 49; 4 tokens: h W2 (224) 115 and 142.  Groups of more than 128 rows
 // fetch their weights for more row tiles, so they take small tiles up to three eighths of the chip only.  Where the chip is full the small tiles fetch
 // twice the operand bytes per product: 2048 tokens, 64 experts, top-8 837 us and 946.
-int moe_gemm_tile(int64_t R, int E, int64_t K, int64_t N, bool pair)
+int moe_gemm_tile(int cus, int64_t R, int E, int64_t K, int64_t N, bool pair)
 {
     if (R < 1 || K % BK != 0) return 256;
-    const int64_t groups = R < E ? R : E, ncu = moe_num_cus();   // (as if the rows were dealt evenly: the host does not know the groups)
+    const int64_t groups = R < E ? R : E, ncu = cus;   // (as if the rows were dealt evenly: the host does not know the groups)
     const int64_t tiles = groups * (((R + groups - 1) / groups + BM - 1) / BM) * ((N + BN - 1) / BN * (pair ? 2 : 1));
     int64_t split = 1;
     while (split * 2 <= moe_gemm_max_split(pair) && tiles * split * 2 <= ncu && K / BK / (split * 2) >= MIN_PART_KTILES) split *= 2;
@@ -104,20 +109,10 @@ int moe_launch_gemm_mfma(const MoeGemmParams& p, int64_t R, hipStream_t stream)
     if (R == 0 || p.N == 0) return MOE_OK;
     if (!moe_gemm_mfma_supported(p, R)) return MOE_ERR_UNSUPPORTED;
     ++g_mfma_launches;
-    if (p.K % BK == 0 && p.nslab <= MOE_MAX_SLABS && moe_gemm_tile(R, p.E, p.K * p.nseg, p.N, EPI_IS_PAIR(p.epi)) == 128) return moe_launch_gemm_small_tile(p, R, stream);
-    if (p.epi == MOE_EPI_STORE) return p.nn ? launch_variant<true, MOE_EPI_STORE>(p, R, stream) : launch_variant<false, MOE_EPI_STORE>(p, R, stream);
-    if (p.epi == MOE_EPI_SWIGLU) return p.nn ? MOE_ERR_UNSUPPORTED : launch_variant<false, MOE_EPI_SWIGLU>(p, R, stream);
-    if (p.epi == MOE_EPI_SWIGLU_FUSED) {
-        if (p.nn || p.ncc != 1) return MOE_ERR_UNSUPPORTED;
-        if (!p.CB[0] || !p.CCP[0] || !p.Y[0]) return MOE_ERR_BAD_ARG;
-        return launch_variant<false, MOE_EPI_SWIGLU_FUSED>(p, R, stream);
-    }
-    if (p.epi == MOE_EPI_SWIGLU_BWD) return p.nn ? launch_variant<true, MOE_EPI_SWIGLU_BWD>(p, R, stream) : launch_variant<false, MOE_EPI_SWIGLU_BWD>(p, R, stream);
-    if (p.epi == MOE_EPI_SWIGLU_BWD_FUSED) {
-        if (p.nn || p.nrc != 3 || p.ncc != 2) return MOE_ERR_UNSUPPORTED;
-        for (int i = 0; i < 3; ++i) if (!p.RC[i] || !p.RCP[i] || (i < 2 && (!p.CB[i] || !p.CCP[i]))) return MOE_ERR_BAD_ARG;
-        return launch_variant<false, MOE_EPI_SWIGLU_BWD_FUSED>(p, R, stream);
-    }
-    return MOE_ERR_BAD_ARG;
+    const bool general = p.K % BK != 0 || p.nslab > MOE_MAX_SLABS;   // (the variants for these have one tile size)
+    if (p.tile != 0 && p.tile != 128 && p.tile != 256) return MOE_ERR_BAD_ARG;
+    if (general && p.tile == 128) return MOE_ERR_UNSUPPORTED;
+    const int tile = p.tile ? p.tile : general ? 256 : moe_gemm_tile(p.num_cus ? p.num_cus : moe_gemm_cus(), R, p.E, p.K * p.nseg, p.N, EPI_IS_PAIR(p.epi));
+    if (tile == 128) return moe_launch_gemm_small_tile(p, R, stream);
+    return launch_epilogue(p, R, stream);
 }
-

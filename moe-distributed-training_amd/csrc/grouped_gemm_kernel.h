@@ -25,13 +25,6 @@
 #include <type_traits>
 
 #define EPI_IS_PAIR(e) ((e) == MOE_EPI_SWIGLU || (e) == MOE_EPI_SWIGLU_FUSED)
-constexpr int NXCD_HOST = 8;
-// compute units of the current device that the tile plan fills: a multiple of 8 (whole rounds are dealt out to the 8 XCDs)
-static int moe_num_cus()
-{
-    const int n = moe_device_cus() / NXCD_HOST * NXCD_HOST;
-    return n < NXCD_HOST ? NXCD_HOST : n;
-}
 
 namespace {
 
@@ -1264,13 +1257,14 @@ template <bool NN, int EPI, typename Num, bool KTAIL> int launch_typed(const Moe
     }
     const int ntiles_n = (EPI_IS_PAIR(EPI)) ? (int)((p.N + BN / 2 - 1) / (BN / 2)) : (int)((p.N + BN - 1) / BN);
     MoeGemmParams q = p;
-    q.num_cus = WGS_PER_CU * moe_num_cus();
+    const int cus = p.num_cus ? p.num_cus : moe_gemm_cus();
+    q.num_cus = WGS_PER_CU * cus;
     q.y_wide = (!p.y_grouped && (R * p.ldy + p.N) * 2 >= ((int64_t)1 << 31)) ? 1 : 0;
     q.max_split = moe_gemm_max_split(EPI_IS_PAIR(EPI));
     if (q.clear_counters && !q.sk_counters) return MOE_ERR_WORKSPACE;
     if (q.max_split > 1) {
         if (!p.sk_partials || !p.sk_counters) return MOE_ERR_WORKSPACE;
-        if (!p.counters_clean) hipLaunchKernelGGL(zero_i32_kernel, dim3((unsigned)((moe_gemm_num_counters() + 255) / 256)), dim3(256), 0, stream, p.sk_counters, (int64_t)moe_gemm_num_counters());
+        if (!p.counters_clean) hipLaunchKernelGGL(zero_i32_kernel, dim3((unsigned)((cus + 255) / 256)), dim3(256), 0, stream, p.sk_counters, (int64_t)cus);
     }
     const int64_t grid = plan_grid(R, p.E, ntiles_n, q.num_cus);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NTHREADS), LDS_BYTES, stream, q);
@@ -1288,6 +1282,25 @@ template <bool NN, int EPI> int launch_variant(const MoeGemmParams& p, int64_t R
             return MOE_ERR_UNSUPPORTED;
     }
     return p.f16 ? launch_typed<NN, EPI, NumF16, false>(p, R, stream) : launch_typed<NN, EPI, NumBf16, false>(p, R, stream);
+}
+
+// the kernel for the launch's epilogue and weight layout
+int launch_epilogue(const MoeGemmParams& p, int64_t R, hipStream_t stream)
+{
+    if (p.epi == MOE_EPI_STORE) return p.nn ? launch_variant<true, MOE_EPI_STORE>(p, R, stream) : launch_variant<false, MOE_EPI_STORE>(p, R, stream);
+    if (p.epi == MOE_EPI_SWIGLU) return p.nn ? MOE_ERR_UNSUPPORTED : launch_variant<false, MOE_EPI_SWIGLU>(p, R, stream);
+    if (p.epi == MOE_EPI_SWIGLU_FUSED) {
+        if (p.nn || p.ncc != 1) return MOE_ERR_UNSUPPORTED;
+        if (!p.CB[0] || !p.CCP[0] || !p.Y[0]) return MOE_ERR_BAD_ARG;
+        return launch_variant<false, MOE_EPI_SWIGLU_FUSED>(p, R, stream);
+    }
+    if (p.epi == MOE_EPI_SWIGLU_BWD) return p.nn ? launch_variant<true, MOE_EPI_SWIGLU_BWD>(p, R, stream) : launch_variant<false, MOE_EPI_SWIGLU_BWD>(p, R, stream);
+    if (p.epi == MOE_EPI_SWIGLU_BWD_FUSED) {
+        if (p.nn || p.nrc != 3 || p.ncc != 2) return MOE_ERR_UNSUPPORTED;
+        for (int i = 0; i < 3; ++i) if (!p.RC[i] || !p.RCP[i] || (i < 2 && (!p.CB[i] || !p.CCP[i]))) return MOE_ERR_BAD_ARG;
+        return launch_variant<false, MOE_EPI_SWIGLU_BWD_FUSED>(p, R, stream);
+    }
+    return MOE_ERR_BAD_ARG;
 }
 
 }  // namespace

@@ -60,27 +60,28 @@ struct MoeGemmParams {
     int f16;                // operands and outputs are IEEE half instead of bfloat16
     int y_wide;             // scattered output rows need 64-bit addresses (Y spans 2 GiB or more), set by the launcher
     int max_split;          // K parts a tile of the last round may be cut into (1, 2 or 4), set by the launcher
-    int num_cus;            // compute units the tile plan fills (a multiple of 8), set by the launcher
+    int num_cus;            // compute units (moe_gemm_cus; 0: looked up at launch); in the kernel, workgroups of a round of the tile plan
     float* sk_partials;     // K-split exchange area, see moe_gemm_sk_bytes / moe_gemm_sk_attach
     int* sk_counters;
     int counters_clean;     // the caller guarantees sk_counters is all zero at launch (every launch leaves it so)
     int clear_counters;     // gate/up pair (which splits no tile): clears sk_counters for the launch behind it
+    int tile;               // rows and columns of the output tiles (moe_gemm_tile), for callers whose buffers depend on it; 0: chosen at launch
 };
 
-size_t moe_gemm_sk_bytes(int64_t R, int E, int64_t N);
-void moe_gemm_sk_attach(MoeGemmParams& p, void* ws, int64_t R, int E, int64_t N);
-size_t moe_gemm_exchange_bytes(int64_t R, int E, int64_t K, int64_t N);
+// Compute units of the current device that the tile plan fills, a multiple of 8 (whole rounds are dealt out to the 8 XCDs).  A caller asks once and hands the number
+// to the functions below: a device look-up in each of them made a forward and backward of the fused MLP ask 200 times.
+int moe_gemm_cus();
+size_t moe_gemm_sk_bytes(int cus, int64_t R, int E, int64_t N);   // exchange area of a launch; it starts with `cus` ints that must be zero at launch
+void moe_gemm_sk_attach(MoeGemmParams& p, void* ws, int cus);
+size_t moe_gemm_exchange_bytes(int cus, int tile, int64_t R, int E, int64_t K, int64_t N);
 int moe_gemm_max_split(bool pair);
 // rows and columns of a launch's output tiles: 256, one workgroup per compute unit, or 128, two (K: all segments; general-shape launches always 256)
-int moe_gemm_tile(int64_t R, int E, int64_t K, int64_t N, bool pair);
+int moe_gemm_tile(int cus, int64_t R, int E, int64_t K, int64_t N, bool pair);
 int moe_launch_gemm_small_tile(const MoeGemmParams& p, int64_t R, hipStream_t stream);
-int moe_gemm_num_counters();   // ints at the start of the exchange area that must be zero at launch
 // test aid: workgroups of a launch with this geometry, and each workgroup's work item (9 ints per workgroup)
 int64_t moe_gemm_plan_blocks(int64_t R, int E, int64_t N, int pair);
 int moe_launch_gemm_plan(const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg, int* out,
                          hipStream_t stream);
-size_t moe_gemm_sk_bytes(int64_t R, int E, int64_t N);
-void moe_gemm_sk_attach(MoeGemmParams& p, void* ws, int64_t R, int E, int64_t N);
 bool moe_gemm_mfma_supported(const MoeGemmParams& p, int64_t R);
 int moe_launch_gemm_mfma(const MoeGemmParams& p, int64_t R, hipStream_t stream);
 int64_t moe_gemm_mfma_launch_count();   // test aid: matrix-core grouped GEMM launches enqueued by this process so far

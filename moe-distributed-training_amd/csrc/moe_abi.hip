@@ -248,13 +248,14 @@ int moe_gemm_debug_plan(const void* offsets, int off64, int E, int64_t R, int64_
 }
 
 // ---------------------------------------------------------------------------------------------------------
-size_t moe_scatter2scatter_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank)
+static inline size_t s2s_bytes(int cus, int64_t R, int E, int64_t K, int64_t N, int rank)
 {
-    const size_t sk = al(moe_gemm_sk_bytes(R, E, N));
+    const size_t sk = al(moe_gemm_sk_bytes(cus, R, E, N));
     if (rank <= 0) return sk + 256;
     const size_t chunks = (size_t)(rank + 15) / 16;   // a rank above 16 runs as several adapters of rank <= 16
     return sk + chunks * (pack_bytes(E, K) + pack_bytes(E, N) + q_bytes(R)) + 256;
 }
+size_t moe_scatter2scatter_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank) { return s2s_bytes(moe_gemm_cus(), R, E, K, N, rank); }
 
 int moe_scatter2scatter(const void* X, int64_t sxm, int64_t sxk, const void* W, int64_t swe, int64_t swk, int64_t swn,
                         const void* A, int64_t sae, int64_t sak, int64_t sar, const void* B, int64_t sbe, int64_t sbr,
@@ -282,16 +283,17 @@ int moe_scatter2scatter(const void* X, int64_t sxm, int64_t sxk, const void* W, 
         p.epi = MOE_EPI_STORE; p.f16 = f16;
         bool ok = moe_gemm_mfma_supported(p, R);
         if (ok) {
-            if (workspace_bytes < moe_scatter2scatter_workspace_bytes(R, E, K, N, A ? rank : 0) || !workspace)
+            const int cus = moe_gemm_cus();
+            if (workspace_bytes < s2s_bytes(cus, R, E, K, N, A ? rank : 0) || !workspace)
                 return MOE_ERR_WORKSPACE;
             Bump ws(workspace, workspace_bytes);
-            moe_gemm_sk_attach(p, ws.take(moe_gemm_sk_bytes(R, E, N)), R, E, N);
+            moe_gemm_sk_attach(p, ws.take(moe_gemm_sk_bytes(cus, R, E, N)), cus);
             if (A) {
                 // x A B = sum over 16-wide chunks c of x A[:, c] B[c, :]: a rank above 16 enters as several 16-wide K slabs
                 const int nh = (rank + 15) / 16;
                 void *At[MOE_MAX_STRIDED_SLABS] = {}, *LB[MOE_MAX_STRIDED_SLABS] = {}, *Q[MOE_MAX_STRIDED_SLABS] = {};
                 MoePackBatch pb = {};   // also clears the GEMM's K-split counters
-                pb.E = E; pb.zero_ptr = p.sk_counters; pb.zero_n = moe_gemm_num_counters();
+                pb.E = E; pb.zero_ptr = p.sk_counters; pb.zero_n = cus;
                 p.counters_clean = 1;
                 for (int hf = 0; hf < nh; ++hf) {
                     At[hf] = ws.take(pack_bytes(E, K));
@@ -414,11 +416,11 @@ int moe_group_bwd_ab(const void* DY, int64_t sdm, int64_t sdn, const void* X, in
 static const int LINEAR_BWD_MAX_CHUNKS = MOE_MAX_SLABS;   // 16-wide rank chunks: the dX launch takes them as slabs given by pointer
 
 // The adapter gradients' partials lie where the dX launch exchanges its K-split tiles afterwards (behind the counters, which are cleared before either)
-static inline size_t counter_bytes() { return al((size_t)moe_gemm_num_counters() * sizeof(int)); }
+static inline size_t counter_bytes(int cus) { return al((size_t)cus * sizeof(int)); }
 static inline size_t linear_bwd_xtp_bytes(int64_t R, int E, int64_t K, int64_t N, int rank) { return (size_t)(rank > 16 ? 4 : 2) * moe_xtp_workspace_bytes(R, E, K > N ? K : N); }
-static inline size_t linear_bwd_shared_bytes(int64_t R, int E, int64_t K, int64_t N, int rank)
+static inline size_t linear_bwd_shared_bytes(int cus, int64_t R, int E, int64_t K, int64_t N, int rank)
 {
-    const size_t sk = moe_gemm_sk_bytes(R, E, K), x = counter_bytes() + linear_bwd_xtp_bytes(R, E, K, N, rank);
+    const size_t sk = moe_gemm_sk_bytes(cus, R, E, K), x = counter_bytes(cus) + linear_bwd_xtp_bytes(R, E, K, N, rank);
     return sk > x ? sk : x;
 }
 
@@ -428,12 +430,13 @@ static inline bool linear_bwd_sizes_ok(int64_t K, int64_t N, int rank)
     return rank >= 1 && (rank + 15) / 16 <= LINEAR_BWD_MAX_CHUNKS && K >= 1 && K % 32 == 0 && N >= 64 && N % 32 == 0;   // (N: the contraction of dX, a whole K tile at least)
 }
 
-size_t moe_linear_lora_bwd_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank)
+static inline size_t linear_bwd_bytes(int cus, int64_t R, int E, int64_t K, int64_t N, int rank)
 {
     if (!linear_bwd_sizes_ok(K, N, rank)) return 0;
     const size_t C = (size_t)(rank + 15) / 16;
-    return al(linear_bwd_shared_bytes(R, E, K, N, rank)) + C * (2 * pack_bytes(E, K) + pack_bytes(E, N) + 3 * q_bytes(R)) + al((size_t)R * sizeof(float)) + 256;
+    return al(linear_bwd_shared_bytes(cus, R, E, K, N, rank)) + C * (2 * pack_bytes(E, K) + pack_bytes(E, N) + 3 * q_bytes(R)) + al((size_t)R * sizeof(float)) + 256;
 }
+size_t moe_linear_lora_bwd_workspace_bytes(int64_t R, int E, int64_t K, int64_t N, int rank) { return linear_bwd_bytes(moe_gemm_cus(), R, E, K, N, rank); }
 
 int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const void* gates, int gates_dtype, const void* x, int64_t ldx, int fan_out,
                         const void* W, int64_t swe, int64_t swk, int64_t swn, const void* A, int64_t sae, int64_t sak, int64_t sar,
@@ -459,12 +462,13 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const v
     p.E = E; p.K = N; p.N = K; p.fan_out = dout_fan_out; p.x_grouped = 0; p.y_grouped = 0;
     p.epi = MOE_EPI_STORE; p.f16 = f16; p.nslab = C; p.slab_mode = 0;
     if (!moe_gemm_mfma_supported(p, R)) return MOE_ERR_UNSUPPORTED;
-    if (!workspace || workspace_bytes < moe_linear_lora_bwd_workspace_bytes(R, E, K, N, rank)) return MOE_ERR_WORKSPACE;
+    const int cus = moe_gemm_cus();
+    if (!workspace || workspace_bytes < linear_bwd_bytes(cus, R, E, K, N, rank)) return MOE_ERR_WORKSPACE;
     Bump ws(workspace, workspace_bytes);
-    uint8_t* shared = (uint8_t*)ws.take(linear_bwd_shared_bytes(R, E, K, N, rank));
-    moe_gemm_sk_attach(p, shared, R, E, K);
+    uint8_t* shared = (uint8_t*)ws.take(linear_bwd_shared_bytes(cus, R, E, K, N, rank));
+    moe_gemm_sk_attach(p, shared, cus);
     p.counters_clean = 1;   // by the packing
-    void* xw = shared + counter_bytes();
+    void* xw = shared + counter_bytes(cus);
     const size_t xb = linear_bwd_xtp_bytes(R, E, K, N, rank);
     const int64_t ldt = pad_rows(R);
     hipStream_t st = S(stream);
@@ -480,7 +484,7 @@ int moe_linear_lora_bwd(const void* dout, int64_t ldd, int dout_fan_out, const v
     auto chunk_rank = [&](int c) { return rank - 16 * c < 16 ? rank - 16 * c : 16; };
     static_assert(3 * LINEAR_BWD_MAX_CHUNKS <= MOE_PACK_MAX_JOBS, "one packing launch");
     MoePackBatch pb = {};
-    pb.E = E; pb.zero_ptr = p.sk_counters; pb.zero_n = moe_gemm_num_counters();
+    pb.E = E; pb.zero_ptr = p.sk_counters; pb.zero_n = cus;
     if (gates) { pb.weights = gates; pb.wdtype = gates_dtype; pb.pos = pos; pb.pos64 = pos64; pb.scales_n = R; pb.scales = row_scale; }
     for (int c = 0; c < C; ++c) {
         const uint16_t *a = (const uint16_t*)A + 16 * c * sar, *b = (const uint16_t*)B + 16 * c * sbr;
@@ -596,58 +600,62 @@ int moe_swiglu_bwd(const void* gate, const void* up, const void* dh, void* dgate
 
 // ---------------------------------------------------------------------------------------------------------
 // fused expert MLP
-static inline size_t sk_bytes_mlp(int64_t R, int E, int64_t d, int64_t f)
+// Tiles, sizes and places of one call, made once from one device look-up by the workspace query and by either pass, so that the buffers and the
+// launches that fill them agree: a launch takes the tile that stands here or refuses.  Asked for one by one, these numbers took some 220 device look-ups and as many
+// divisions in a forward and backward, which the host of a small step cannot hide.
+struct MlpPlan {
+    int cus;
+    int pair_tile, w2_tile, dh_tile, dx_tile;   // gate/up, h W2, dh, dX
+    int pair_cols, dh_cols;                     // column tiles of the gate/up and of the dh launch: partials of their column contractions, [column tiles][R][16] fp32 each
+    size_t sk;         // K-split exchange area, any of the launches
+    size_t fwd_cc;     // partials of the gate/up launch's column contraction or of the two of the dh launch
+    size_t cc;         // ... of the backward pass, where the partials over d may follow them
+    // Partials of the adapter gradients: with the fused products (rank <= 16) three sets of f columns (from the dh GEMM) and three of d, all alive until one
+    // launch sums them; without, two sets of either at a time.  The sets of d columns come when the grouped GEMMs are through: they lie
+    // where those exchanged K-split tiles, behind the counters, or where that is too small in place of the column-tile partials, which have been added by then.
+    size_t xtp_d;      // a set of d columns
+    size_t rcp;        // a set of f columns: the dh launch's row tiles, or those of the separate passes where these are more
+    bool d_in_exchange;
+    size_t rcp_at;     // dh launches of small tiles leave more row-tile partials, which lie in the exchange area too, from here on: behind what that launch, the dX launch and the sets of d columns use of it (0: in an area of their own)
+    size_t xtp;        // that area
+    size_t total;
+};
+static MlpPlan mlp_plan(int64_t R, int E, int64_t d, int64_t f, int rank)
 {
-    const size_t a = moe_gemm_sk_bytes(R, E, d), b = moe_gemm_sk_bytes(R, E, f);
-    return a > b ? a : b;
-}
-// column tiles of the gate/up launch (pair) and of the dh launch, and the partials of their column contractions, one of the former's and two of the
-// latter's: [column tiles][R][16] fp32 each
-static inline int cc_tiles(int64_t R, int E, int64_t d, int64_t f, bool pair) { const int w = moe_gemm_tile(R, E, d, f, pair) / (pair ? 2 : 1); return (int)((f + w - 1) / w); }
-static inline size_t cc_bytes(int64_t R, int E, int64_t d, int64_t f)
-{
-    const int a = cc_tiles(R, E, d, f, true), b = 2 * cc_tiles(R, E, d, f, false);
-    return (size_t)(a > b ? a : b) * (size_t)R * 16 * sizeof(float);
-}
-// one set of f columns' partials of the adapter gradients from the dh launch: its row tiles, or those of the separate passes where these are more
-static inline size_t rcp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
-{
-    const size_t n = moe_xtp_workspace_bytes(R, E, f), m = rank <= 16 ? (size_t)(R / moe_gemm_tile(R, E, d, f, false) + E) * (size_t)f * 16 * sizeof(float) : 0;
-    return n > m ? n : m;
+    auto most = [](size_t a, size_t b) { return a > b ? a : b; };
+    MlpPlan p = {};
+    p.cus = moe_gemm_cus();
+    const int C = rank > 0 ? (rank + 15) / 16 : 0;   // 16-wide chunks per adapter
+    // (a launch of more slabs than it has pointers for is of the general variants, which have large tiles only)
+    p.pair_tile = 2 * C > MOE_MAX_SLABS ? 256 : moe_gemm_tile(p.cus, R, E, d, f, true);
+    p.w2_tile = C > MOE_MAX_SLABS ? 256 : moe_gemm_tile(p.cus, R, E, f, d, false);
+    p.dh_tile = C > MOE_MAX_SLABS ? 256 : moe_gemm_tile(p.cus, R, E, d, f, false);
+    p.dx_tile = 2 * C > MOE_MAX_SLABS ? 256 : moe_gemm_tile(p.cus, R, E, 2 * f, d, false);
+    p.sk = most(moe_gemm_sk_bytes(p.cus, R, E, d), moe_gemm_sk_bytes(p.cus, R, E, f));
+    p.total = al(p.sk) + 256;
+    if (rank <= 0) return p;
+    p.pair_cols = (int)((f + p.pair_tile / 2 - 1) / (p.pair_tile / 2));
+    p.dh_cols = (int)((f + p.dh_tile - 1) / p.dh_tile);
+    p.fwd_cc = p.cc = (size_t)(p.pair_cols > 2 * p.dh_cols ? p.pair_cols : 2 * p.dh_cols) * (size_t)R * 16 * sizeof(float);
+    p.xtp_d = moe_xtp_workspace_bytes(R, E, d);
+    const size_t xtp_f = moe_xtp_workspace_bytes(R, E, f);
+    if (rank > 16) p.xtp = 3 * most(p.xtp_d, xtp_f);
+    else {
+        p.rcp = most(xtp_f, (size_t)(R / p.dh_tile + E) * (size_t)f * 16 * sizeof(float));
+        p.d_in_exchange = counter_bytes(p.cus) + 3 * p.xtp_d <= p.sk;
+        if (!p.d_in_exchange) p.cc = most(p.cc, 3 * p.xtp_d);
+        if (p.dh_tile == 128) {
+            const size_t used = most(most(moe_gemm_exchange_bytes(p.cus, p.dh_tile, R, E, d, f), moe_gemm_exchange_bytes(p.cus, p.dx_tile, R, E, 2 * f, d)), 3 * p.xtp_d);
+            const size_t at = counter_bytes(p.cus) + al(used);
+            if (at + 3 * p.rcp <= p.sk) p.rcp_at = at;
+        }
+        if (!p.rcp_at) p.xtp = 3 * p.rcp;
+    }
+    p.total += (size_t)C * (3 * pack_bytes(E, d) + 3 * pack_bytes(E, f) + 7 * q_bytes(R)) + al(p.xtp) + al(p.cc);
+    return p;
 }
 
-// Partials of the adapter gradients: with the fused products (rank <= 16) three sets of f columns (from the dh GEMM) and three of d, all alive until one
-// launch sums them; without, two sets of either at a time.  The sets of d columns come when the grouped GEMMs are through: they lie
-// where those exchanged K-split tiles, behind the counters, or where that is too small in place of the column-tile partials, which have been added by then.
-// Where the dh launch takes small tiles, which leave more row-tile partials, those lie in the exchange area too: behind what it, the dX launch and the sets of d columns use of it.
-static inline size_t rcp_exchange_offset(int64_t R, int E, int64_t d, int64_t f)
-{
-    const size_t a = moe_gemm_exchange_bytes(R, E, d, f), b = moe_gemm_exchange_bytes(R, E, 2 * f, d), c = 3 * moe_xtp_workspace_bytes(R, E, d);
-    return counter_bytes() + al(a > b ? (a > c ? a : c) : (b > c ? b : c));
-}
-static inline bool rcp_in_exchange(int64_t R, int E, int64_t d, int64_t f)
-{
-    return moe_gemm_tile(R, E, d, f, false) == 128 && rcp_exchange_offset(R, E, d, f) + 3 * rcp_bytes(R, E, d, f, 16) <= sk_bytes_mlp(R, E, d, f);
-}
-static inline size_t mlp_xtp_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
-{
-    if (rank > 16) return 3 * moe_xtp_workspace_bytes(R, E, f > d ? f : d);
-    return rcp_in_exchange(R, E, d, f) ? 0 : 3 * rcp_bytes(R, E, d, f, rank);
-}
-static inline bool mlp_xtp_d_in_exchange(int64_t R, int E, int64_t d, int64_t f) { return counter_bytes() + 3 * moe_xtp_workspace_bytes(R, E, d) <= sk_bytes_mlp(R, E, d, f); }
-static inline size_t mlp_cc_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
-{
-    const size_t cc = cc_bytes(R, E, d, f), x = rank <= 16 && !mlp_xtp_d_in_exchange(R, E, d, f) ? 3 * moe_xtp_workspace_bytes(R, E, d) : 0;
-    return cc > x ? cc : x;
-}
-
-size_t moe_mlp_workspace_bytes(int64_t R, int E, int64_t d, int64_t f, int rank)
-{
-    size_t n = al(sk_bytes_mlp(R, E, d, f)) + 256;
-    if (rank <= 0) return n;
-    const size_t C = (size_t)(rank + 15) / 16;   // 16-wide chunks per adapter
-    return n + C * (3 * pack_bytes(E, d) + 3 * pack_bytes(E, f) + 7 * q_bytes(R)) + al(mlp_xtp_bytes(R, E, d, f, rank)) + al(mlp_cc_bytes(R, E, d, f, rank));
-}
+size_t moe_mlp_workspace_bytes(int64_t R, int E, int64_t d, int64_t f, int rank) { return mlp_plan(R, E, d, f, rank).total; }
 
 size_t moe_mlp_saved_bytes(int64_t R, int rank) { return rank > 0 ? (size_t)((rank + 15) / 16) * 6 * q_bytes(R) : 256; }
 
@@ -686,9 +694,10 @@ int moe_mlp_fwd(const void* x, int64_t ldx, const void* w1, const void* w3, cons
     uint8_t* sv = (uint8_t*)saved;
     const size_t qb = q_bytes(R);
     const int64_t ldt = pad_rows(R);
-    if (!workspace || workspace_bytes < moe_mlp_workspace_bytes(R, E, d, f, has_lora ? rank : 0)) return MOE_ERR_WORKSPACE;
+    const MlpPlan plan = mlp_plan(R, E, d, f, has_lora ? rank : 0);
+    if (!workspace || workspace_bytes < plan.total) return MOE_ERR_WORKSPACE;
     Bump ws(workspace, workspace_bytes);
-    void* skws = ws.take(sk_bytes_mlp(R, E, d, f));
+    void* skws = ws.take(plan.sk);
     bool counters_clean = has_lora;   // K-split counters: zeroed by the adapter pack launch; a GEMM launch that uses them leaves them zero
     // An adapter of rank r is worked through as C = ceil(r / 16) independent 16-wide chunks of its rank columns:
     // x A B = sum_c (x A[:, c]) B[c, :].  saved: six groups of C q_bytes blocks (one per chunk): Q1, Q3, Q2, Qt1, Qt3, Qt2.
@@ -713,7 +722,7 @@ int moe_mlp_fwd(const void* x, int64_t ldx, const void* w1, const void* w3, cons
     // a rank of at most 16: the w2 GEMM's low-rank operand Q2 = h A2 comes out of the pair GEMM's epilogue as per-column-tile
     // partials (h is not read again for it); more chunks take separate passes over h
     const bool fuse_q2 = has_lora && rank <= 16;
-    float* ccw = fuse_q2 ? (float*)ws.take(cc_bytes(R, E, d, f)) : nullptr;
+    float* ccw = fuse_q2 ? (float*)ws.take(plan.fwd_cc) : nullptr;
     if (fuse_q2 && !ccw) return MOE_ERR_WORKSPACE;
     if (has_lora) {
         // lora order a1,b1,a3,b3,a2,b2; strides {expert, dim1, dim2}
@@ -738,7 +747,7 @@ int moe_mlp_fwd(const void* x, int64_t ldx, const void* w1, const void* w3, cons
                 j[5] = {L(5) + r0 * ls[16], ls[15], ls[17], ls[16], (uint16_t*)lb2c(c), d, 0, rk};
                 pb.njobs += 6;
             }
-            if (c0 == 0) { pb.zero_ptr = (int*)skws; pb.zero_n = moe_gemm_num_counters(); }   // the K-split counters of the GEMMs below
+            if (c0 == 0) { pb.zero_ptr = (int*)skws; pb.zero_n = plan.cus; }   // the K-split counters of the GEMMs below
             TRY(moe_launch_pack_lora_batch(pb, st));
         } }
         { TIMED("fwd.rows_lora_x");
@@ -761,7 +770,8 @@ int moe_mlp_fwd(const void* x, int64_t ldx, const void* w1, const void* w3, cons
             p.epi = MOE_EPI_SWIGLU_FUSED;
             p.CB[0] = (const uint16_t*)At2c[0]; p.CCP[0] = ccw; p.ncc = 1; p.cc_rows = R;
         }
-        moe_gemm_sk_attach(p, skws, R, E, f);
+        moe_gemm_sk_attach(p, skws, plan.cus);
+        p.tile = plan.pair_tile;
         // without adapters nothing has cleared the K-split counters of the w2 launch yet: this launch does, which saves one of 4.7 us
         p.clear_counters = !counters_clean;
         counters_clean = true;
@@ -771,7 +781,7 @@ int moe_mlp_fwd(const void* x, int64_t ldx, const void* w1, const void* w3, cons
     if (has_lora) {
         TIMED("fwd.rows_lora_h");
         if (fuse_q2)   // the products over each column tile came out of the pair GEMM's epilogue: add the tiles, scale, round
-            TRY(moe_launch_cc_reduce2(ccw, nullptr, cc_tiles(R, E, d, f, true), R, scaling, svp(2, 0), nullptr, svp(5, 0), nullptr, ldt, st, f16));
+            TRY(moe_launch_cc_reduce2(ccw, nullptr, plan.pair_cols, R, scaling, svp(2, 0), nullptr, svp(5, 0), nullptr, ldt, st, f16));
         else
         for (int c = 0; c < C; c += 2) {   // two chunks per launch: the twin's reads of h are served by L2
             const bool two = c + 1 < C;
@@ -790,7 +800,8 @@ int moe_mlp_fwd(const void* x, int64_t ldx, const void* w1, const void* w3, cons
         p.Y[0] = (uint16_t*)y; p.ldy = ldy;
         p.pos = pos; p.pos64 = pos64; p.offsets = offsets; p.off64 = off64;
         p.E = E; p.K = f; p.N = d; p.fan_out = 1; p.x_grouped = 1; p.y_grouped = y_grouped; p.epi = MOE_EPI_STORE; p.f16 = f16;
-        moe_gemm_sk_attach(p, skws, R, E, d);
+        moe_gemm_sk_attach(p, skws, plan.cus);
+        p.tile = plan.w2_tile;
         p.counters_clean = counters_clean;
         if (moe_gemm_max_split(p.epi == MOE_EPI_SWIGLU || p.epi == MOE_EPI_SWIGLU_FUSED) > 1) counters_clean = true;   // zeroed by that launch if they were not, and left zero
         TIMED("fwd.gemm_w2");
@@ -847,16 +858,17 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
     // a rank of at most 16 (one chunk): the adapter gradients that sum over the rows of dgate, dup and h are produced by
     // the dh GEMM's epilogue as per-row-tile partials; more chunks take separate passes over those tensors
     const bool fuse_rc = has_lora && rank <= 16;
-    if (!workspace || workspace_bytes < moe_mlp_workspace_bytes(R, E, d, f, has_lora ? rank : 0)) return MOE_ERR_WORKSPACE;
+    const MlpPlan plan = mlp_plan(R, E, d, f, has_lora ? rank : 0);
+    if (!workspace || workspace_bytes < plan.total) return MOE_ERR_WORKSPACE;
     Bump ws(workspace, workspace_bytes);
-    void* skws = ws.take(sk_bytes_mlp(R, E, d, f));
+    void* skws = ws.take(plan.sk);
     bool counters_clean = has_lora;   // K-split counters: zeroed by the adapter pack launch; a GEMM launch that uses them leaves them zero
     if (has_lora) {
         pq = (uint8_t*)ws.take((size_t)C * 6 * qb);
         if (fuse_rc) p2s = ws.take(qb);   // P2 times the row scale, row-major (the fused contraction's operand)
-        if (fuse_rc) ccw = (float*)ws.take(mlp_cc_bytes(R, E, d, f, rank));
-        xb = mlp_xtp_bytes(R, E, d, f, rank);
-        xw = fuse_rc && rcp_in_exchange(R, E, d, f) ? (void*)((uint8_t*)skws + rcp_exchange_offset(R, E, d, f)) : ws.take(xb);
+        if (fuse_rc) ccw = (float*)ws.take(plan.cc);
+        xb = plan.xtp;
+        xw = plan.rcp_at ? (void*)((uint8_t*)skws + plan.rcp_at) : ws.take(xb);
         TIMED("bwd.pack_lora");
         for (int c = 0; c < C; ++c) {
             bt2[c] = ws.take(pbd);  // fragment order of b2[e][r][n=d]
@@ -882,7 +894,7 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
                 j[5] = {L(2) + r0 * ls[8], ls[6], ls[7], ls[8], (uint16_t*)la3(c), d, 0, rk};
                 pb.njobs += 6;
             }
-            if (c0 == 0) { pb.zero_ptr = (int*)skws; pb.zero_n = moe_gemm_num_counters(); }   // the K-split counters of the GEMMs below
+            if (c0 == 0) { pb.zero_ptr = (int*)skws; pb.zero_n = plan.cus; }   // the K-split counters of the GEMMs below
             TRY(moe_launch_pack_lora_batch(pb, st));
         }
     }
@@ -910,18 +922,18 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         p.E = E; p.K = d; p.N = f; p.fan_out = dy_fan_out; p.x_grouped = dy_grouped; p.y_grouped = 1;
         p.epi = MOE_EPI_SWIGLU_BWD; p.f16 = f16;
         if (fuse_rc) {   // dB1 = Q1^T dgate, dB3 = Q3^T dup, dA2 = h^T (row_scale P2) as per-row-tile partials from the epilogue
-            const size_t one = rcp_bytes(R, E, d, f, rank);
             p.RC[0] = (const uint16_t*)svp(0, 0); p.RC[1] = (const uint16_t*)svp(1, 0); p.RC[2] = (const uint16_t*)p2s;
-            for (int i = 0; i < 3; ++i) p.RCP[i] = (float*)((uint8_t*)xw + i * one);
+            for (int i = 0; i < 3; ++i) p.RCP[i] = (float*)((uint8_t*)xw + i * plan.rcp);
             p.nrc = 3;
             // P1 = dgate B1^T, P3 = dup B3^T (the dX GEMM's low-rank operands) as per-column-tile partials
-            const size_t cone = (size_t)cc_tiles(R, E, d, f, false) * (size_t)R * 16;
+            const size_t cone = (size_t)plan.dh_cols * (size_t)R * 16;
             p.CB[0] = (const uint16_t*)bt1[0]; p.CB[1] = (const uint16_t*)bt3[0];
             p.CCP[0] = ccw; p.CCP[1] = ccw + cone;
             p.ncc = 2; p.cc_rows = R;
             p.epi = MOE_EPI_SWIGLU_BWD_FUSED;
         }
-        moe_gemm_sk_attach(p, skws, R, E, f);
+        moe_gemm_sk_attach(p, skws, plan.cus);
+        p.tile = plan.dh_tile;
         p.counters_clean = counters_clean;
         if (moe_gemm_max_split(p.epi == MOE_EPI_SWIGLU || p.epi == MOE_EPI_SWIGLU_FUSED) > 1) counters_clean = true;   // zeroed by that launch if they were not, and left zero
         TIMED("bwd.gemm_dh_swiglu_bwd");
@@ -949,8 +961,8 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         // ---- w1 / w3 backward
         TIMED("bwd.rows_lora_dgate_dup");
         if (fuse_rc) {   // the products over each column tile came out of the dh GEMM's epilogue: add the tiles, scale, round
-            const size_t cone = (size_t)cc_tiles(R, E, d, f, false) * (size_t)R * 16;
-            TRY(moe_launch_cc_reduce2(ccw, ccw + cone, cc_tiles(R, E, d, f, false), R, scaling, pqp(1, 0), pqp(2, 0), pqp(4, 0), pqp(5, 0), ldt, st, f16));
+            const size_t cone = (size_t)plan.dh_cols * (size_t)R * 16;
+            TRY(moe_launch_cc_reduce2(ccw, ccw + cone, plan.dh_cols, R, scaling, pqp(1, 0), pqp(2, 0), pqp(4, 0), pqp(5, 0), ldt, st, f16));
         } else
         for (int c = 0; c < C; c += 2) {   // two chunks of one adapter per launch, so that dgate and dup are each fetched once per pair of chunks
             const bool two = c + 1 < C;
@@ -971,7 +983,8 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
         p.Y[0] = (uint16_t*)dx_rows; p.ldy = lddx;
         p.pos = pos; p.pos64 = pos64; p.offsets = offsets; p.off64 = off64;
         p.E = E; p.K = f; p.N = d; p.fan_out = 1; p.x_grouped = 1; p.y_grouped = dx_grouped; p.epi = MOE_EPI_STORE; p.f16 = f16;
-        moe_gemm_sk_attach(p, skws, R, E, d);
+        moe_gemm_sk_attach(p, skws, plan.cus);
+        p.tile = plan.dx_tile;
         p.counters_clean = counters_clean;
         if (moe_gemm_max_split(p.epi == MOE_EPI_SWIGLU || p.epi == MOE_EPI_SWIGLU_FUSED) > 1) counters_clean = true;   // zeroed by that launch if they were not, and left zero
         TIMED("bwd.gemm_dx_w1w3");
@@ -984,13 +997,13 @@ int moe_mlp_bwd(const void* dy, int64_t lddy, int dy_grouped, int dy_fan_out, co
             // One launch over x and dy leaves the partials of dA1, dA3 and dB2 beside those of dB1, dB3 and dA2 that the dh GEMM's epilogue
             // left, and one launch adds all six: six launches before (4096 tokens, d=4096, f=14336: 87 us together, 65 now; 512 tokens, d=256:
             // 41 us, 16 now -- each of them was a few workgroups behind a gap; 2048 tokens, 64 experts: 76 and 66).
-            const size_t onef = rcp_bytes(R, E, d, f, rank) / sizeof(float), oned = moe_xtp_workspace_bytes(R, E, d) / sizeof(float);
+            const size_t onef = plan.rcp / sizeof(float), oned = plan.xtp_d / sizeof(float);
             float* part = (float*)xw;
-            float* partd = mlp_xtp_d_in_exchange(R, E, d, f) ? (float*)((uint8_t*)skws + counter_bytes()) : ccw;
+            float* partd = plan.d_in_exchange ? (float*)((uint8_t*)skws + counter_bytes(plan.cus)) : ccw;
             const MoeXtpJob jobs[3] = {{x, ldx, d, pos, fan_out, pqp(4, 0), nullptr, nullptr, {}, rank}, {x, ldx, d, pos, fan_out, pqp(5, 0), nullptr, nullptr, {}, rank},
                                        {dy, lddy, d, dy_grouped ? nullptr : pos, dy_fan_out, svp(5, 0), row_scale, nullptr, {}, rank}};
             TRY(moe_launch_xtp_partial_jobs(jobs, 3, pos64, ldt, offsets, off64, E, R, partd, (int64_t)oned, st, f16));
-            const int bm = moe_gemm_tile(R, E, d, f, false);   // the dh launch's row tiles
+            const int bm = plan.dh_tile;   // rows of its partials
             auto red = [&](const float* p, int64_t K, void* out, const int64_t* st3, int rows = 0) { return MoeXtpReduceJob{p, K, out, {st3[0], st3[1], st3[2]}, rank, rows}; };
             const MoeXtpReduceJob sums[6] = {red(part, f, lg[1], so[1], bm), red(part + onef, f, lg[3], so[3], bm), red(part + 2 * onef, f, lg[4], so[4], bm),
                                              red(partd, d, lg[0], so[0]), red(partd + oned, d, lg[2], so[2]), red(partd + 2 * oned, d, lg[5], so[5])};
