@@ -91,14 +91,24 @@ bool moe_gemm_mfma_supported(const MoeGemmParams& p, int64_t R)
 // and 142, h W2 (128) 93 and 98, dX (128) 159 and 154 (319 rows, all of it 409 and 419); 2 rows of two experts: h W2 (128) 52 and 49; 4 tokens: h W2 (224) 115 and 142.  Groups of more than 128 rows
 // fetch their weights for more row tiles, so they take small tiles up to three eighths of the chip only.  Where the chip is full the small tiles fetch
 // twice the operand bytes per product: 2048 tokens, 64 experts, top-8 837 us and 946.
+//
+// The second condition is for rows that are not dealt evenly, which the host does not see: a group of 129 rows is two small tiles and one large one.  Two small tiles on one
+// compute unit take as long as a large one there, so of a launch that splits K the small ones must come to at most one per compute unit however the rows fall.  Of
+// 5000 drawn products (128 to 14336 columns and deep, 1 to 96 groups), small tiles by the first condition alone: those whose tiles came to one at most 0.95-1.93 times as fast as large ones,
+// those of more 0.77-1.37 and half of them slower: us, large and small, 64 groups of 121 rows on average, 1408 x 192 31.1 and 40.3; 16 of 140, 1216 x 768 30.1 and 36.6; 32 of
+// 123, 3968 x 256 57.2 and 66.7; dX of two groups of 126, 28672 x 4096, and the kernels around it 210 and 245.  Launches that never split have a longer chain of K tiles to lose on the idle half: up to
+// one and a half per compute unit (gate/up of 16 groups, 124 rows on average, 2816 x 960 and the kernels behind it 93.6 and 97.1 with 1.8; 1.05-1.6 times as fast up to 1.5).
 int moe_gemm_tile(int cus, int64_t R, int E, int64_t K, int64_t N, bool pair)
 {
     if (R < 1 || K % BK != 0) return 256;
-    const int64_t groups = R < E ? R : E, ncu = cus;   // (as if the rows were dealt evenly: the host does not know the groups)
-    const int64_t tiles = groups * (((R + groups - 1) / groups + BM - 1) / BM) * ((N + BN - 1) / BN * (pair ? 2 : 1));
-    int64_t split = 1;
+    const int64_t groups = R < E ? R : E, ncu = cus;
+    const int64_t tiles = groups * (((R + groups - 1) / groups + BM - 1) / BM) * ((N + BN - 1) / BN * (pair ? 2 : 1));   // (as if the rows were dealt evenly)
+    int64_t split = 1, parts = 1;
     while (split * 2 <= moe_gemm_max_split(pair) && tiles * split * 2 <= ncu && K / BK / (split * 2) >= MIN_PART_KTILES) split *= 2;
-    return R <= groups * 128 ? (tiles * split * 2 <= ncu ? 128 : 256) : (tiles * split * 8 <= 3 * ncu ? 128 : 256);
+    if (R <= groups * 128 ? tiles * split * 2 > ncu : tiles * split * 8 > 3 * ncu) return 256;
+    while (parts * 2 <= moe_gemm_max_split(pair) && K / BK / (parts * 2) >= MIN_PART_KTILES) parts *= 2;
+    const int64_t small = (groups + (R - groups) / 128) * (pair ? (N + 63) / 64 : (N + 127) / 128) * parts;   // at most, however the rows fall
+    return 2 * small <= (parts > 1 ? 2 : 3) * ncu ? 128 : 256;
 }
 
 static std::atomic<int64_t> g_mfma_launches{0};

@@ -90,3 +90,31 @@ def test_a_pass_looks_the_device_up_once_and_per_launch(calls, R, E, d, f, r):
     for name in ("fwd", "bwd"):
         assert res[name]["rc"] == 0 and res[name]["launches"]
         assert res[name]["lookups"] <= 1 + 2 * len(res[name]["launches"]), (name, res[name]["lookups"], len(res[name]["launches"]))
+
+
+# rows, groups, d, f: what the host sees of launches whose small tiles came to more than the compute units where rows are not dealt evenly
+UNEVEN = [(253, 2, 4096, 14336), (1988, 16, 896, 1856), (3934, 32, 512, 896), (7768, 64, 192, 1408), (2248, 16, 768, 1216), (975, 8, 1728, 1856), (1992, 16, 2816, 960), (3617, 1, 704, 1472)]
+EVEN = [(1024, 8, 256, 512), (2, 8, 4096, 14336), (64, 1, 4096, 14336), (200, 4, 512, 2048), (17, 16, 1024, 512)]
+
+
+@pytest.mark.parametrize("r", [0, 16])
+def test_small_tiles_however_the_rows_fall(calls, r):
+    """A launch that may split K takes tiles of 128 x 128 (4 waves, 80 KiB of LDS) only where these come to at most one per compute unit for any group sizes, one that never splits up to one and
+    a half; groups of a row more than 128 are two small tiles and one large one, and from there on the small ones were slower, by up to a quarter."""
+    sizes = UNEVEN + EVEN
+    small_seen = 0
+    for (R, E, d, f), res in zip(sizes, calls(*[(*s, r) for s in sizes])):
+        gemms = {n: [l for l in res[n]["launches"] if l[2] >= 80 * 1024] for n in ("fwd", "bwd")}
+        assert [len(gemms["fwd"]), len(gemms["bwd"])] == [2, 2]
+        groups = min(R, E)
+        rows = groups + (R - groups) // 128   # tiles of 128 rows, at most
+        for (_, threads, lds), K, N, pair in zip(gemms["fwd"] + gemms["bwd"], (d, f, d, 2 * f), (f, d, f, d), (True, False, False, False)):
+            assert (threads, lds) in ((256, 80 * 1024), (512, 160 * 1024))
+            parts = 1 if pair else next(p for p in (4, 2, 1) if p == 1 or K // 64 // p >= 8)
+            tiles = rows * -(-N // (64 if pair else 128)) * parts
+            if threads == 256:
+                assert 2 * tiles <= (2 if parts > 1 else 3) * 256, (R, E, d, f, K, N, pair, tiles)
+                small_seen += 1
+        if (R, E, d, f) in EVEN[:2]:   # (what small tiles are for: a narrow layer, one token of the wide one)
+            assert gemms["fwd"][1][1] == 256 and gemms["bwd"][1][1] == 256
+    assert small_seen >= 12
