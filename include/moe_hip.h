@@ -59,11 +59,16 @@ int moe_profile_get(int i, char* name, int name_cap, float* ms);
 /* ---- tile plan of the grouped GEMM (test aid; no counterpart in the reference) ------------------------------
  * The matrix-core grouped GEMM hands every workgroup one work item (an output tile of one expert, or one K part of a
  * tile).  moe_gemm_debug_plan_blocks() returns the number of workgroups a launch over R rows, E experts and N output
- * columns uses (pair != 0: the gate/up pair kernel with 128 columns per projection and tile; tiles of 256 x 256,
- * which small launches cut smaller);
+ * columns uses (pair != 0: the gate/up pair kernel with 128 columns per projection and tile);
  * moe_gemm_debug_plan() writes, for each of them, 9 ints into `out` (device memory): valid, expert, n tile, first
  * row, one-past-last row, K part, K parts, exchange slot, split-tile counter.  Tests use it to check that every tile
- * is covered exactly once for any group sizes. */
+ * is covered exactly once for any group sizes.  These two describe tiles of 256 x 256; moe_gemm_debug_tile() says
+ * which a launch of these sizes takes (256, or 128 for a small one; 256 always for K % 64 != 0 or more than four adapter
+ * slabs; nseg: segments of K), and the functions with a tile argument describe either. */
+int moe_gemm_debug_tile(int64_t R, int E, int64_t K, int64_t N, int pair, int nseg);
+int64_t moe_gemm_debug_tile_plan_blocks(int tile, int64_t R, int E, int64_t N, int pair);
+int moe_gemm_debug_tile_plan(int tile, const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg,
+                             int32_t* out, void* stream);
 int64_t moe_gemm_debug_plan_blocks(int64_t R, int E, int64_t N, int pair);
 /* number of matrix-core grouped GEMM launches this process has enqueued so far (any entry point): tests read it before
  * and after a call to tell that a shape ran on the matrix cores and not on the generic fallback kernels */

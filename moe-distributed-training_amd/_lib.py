@@ -33,6 +33,9 @@ _SIGNATURES = {
     "moe_gates_bwd": ("i", "plpli" + "ppppppp" + "ll" + "iii" + "p"),
     "moe_router_weight_grad_workspace_bytes": ("z", "lli"),
     "moe_router_weight_grad": ("i", "plppllliipzp"),
+    "moe_gemm_debug_tile": ("i", "lillii"),
+    "moe_gemm_debug_tile_plan_blocks": ("l", "ilili"),
+    "moe_gemm_debug_tile_plan": ("i", "ipiilllii" + "pp"),
     "moe_gemm_debug_plan_blocks": ("l", "lili"),
     "moe_gemm_debug_launch_count": ("l", ""),
     "moe_gemm_debug_plan": ("i", "piilllii" + "pp"),

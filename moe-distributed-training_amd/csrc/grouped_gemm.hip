@@ -13,17 +13,11 @@ int moe_gemm_cus()
     return n < NXCD ? NXCD : n;
 }
 
-static int plan_ntiles_n(int64_t N, int pair) { return pair ? (int)((N + BN / 2 - 1) / (BN / 2)) : (int)((N + BN - 1) / BN); }
-int64_t moe_gemm_plan_blocks(int64_t R, int E, int64_t N, int pair) { return plan_grid(R, E, plan_ntiles_n(N, pair), moe_gemm_cus()); }
-int moe_launch_gemm_plan(const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg, int* out,
-                         hipStream_t stream)
+int64_t moe_gemm_plan_blocks(int tile, int64_t R, int E, int64_t N, int pair) { return tile == 128 ? moe_gemm_small_plan_blocks(R, E, N, pair) : plan_blocks(R, E, N, pair); }
+int moe_launch_gemm_plan(int tile, const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg, int* out, hipStream_t stream)
 {
     if (K < BK || nseg < 1 || nseg > 2) return MOE_ERR_UNSUPPORTED;
-    const int ntiles_n = plan_ntiles_n(N, pair), cus = moe_gemm_cus();
-    const int64_t grid = plan_grid(R, E, ntiles_n, cus);
-    hipLaunchKernelGGL(gemm_plan_kernel, dim3((unsigned)grid), dim3(64), 0, stream, offsets, off64, E, ntiles_n,
-                       (int)((K + BK - 1) / BK) * nseg, moe_gemm_max_split(pair != 0), cus, out);
-    return moe_launch_status();
+    return tile == 128 ? moe_launch_gemm_small_plan(offsets, off64, E, R, K, N, pair, nseg, out, stream) : launch_plan(offsets, off64, E, R, K, N, pair, nseg, out, stream);
 }
 
 // exchange area of a launch: one counter per split tile and one fp32 partial tile per split item; at most one round

@@ -1284,6 +1284,16 @@ template <bool NN, int EPI> int launch_variant(const MoeGemmParams& p, int64_t R
     return p.f16 ? launch_typed<NN, EPI, NumF16, false>(p, R, stream) : launch_typed<NN, EPI, NumBf16, false>(p, R, stream);
 }
 
+// test aid: workgroups of a launch of these tiles, and the work item of each
+int plan_ntiles_n(int64_t N, int pair) { const int w = pair ? BN / 2 : BN; return (int)((N + w - 1) / w); }
+int64_t plan_blocks(int64_t R, int E, int64_t N, int pair) { return plan_grid(R, E, plan_ntiles_n(N, pair), WGS_PER_CU * moe_gemm_cus()); }
+int launch_plan(const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg, int* out, hipStream_t stream)
+{
+    hipLaunchKernelGGL(gemm_plan_kernel, dim3((unsigned)plan_blocks(R, E, N, pair)), dim3(64), 0, stream, offsets, off64, E, plan_ntiles_n(N, pair),
+                       (int)((K + BK - 1) / BK) * nseg, moe_gemm_max_split(pair != 0), WGS_PER_CU * moe_gemm_cus(), out);
+    return moe_launch_status();
+}
+
 // the kernel for the launch's epilogue and weight layout
 int launch_epilogue(const MoeGemmParams& p, int64_t R, hipStream_t stream)
 {

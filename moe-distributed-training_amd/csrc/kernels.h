@@ -78,10 +78,11 @@ int moe_gemm_max_split(bool pair);
 // rows and columns of a launch's output tiles: 256, one workgroup per compute unit, or 128, two (K: all segments; general-shape launches always 256)
 int moe_gemm_tile(int cus, int64_t R, int E, int64_t K, int64_t N, bool pair);
 int moe_launch_gemm_small_tile(const MoeGemmParams& p, int64_t R, hipStream_t stream);
-// test aid: workgroups of a launch with this geometry, and each workgroup's work item (9 ints per workgroup)
-int64_t moe_gemm_plan_blocks(int64_t R, int E, int64_t N, int pair);
-int moe_launch_gemm_plan(const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg, int* out,
-                         hipStream_t stream);
+// test aid: workgroups of a launch with this geometry and tile, and each workgroup's work item (9 ints per workgroup)
+int64_t moe_gemm_plan_blocks(int tile, int64_t R, int E, int64_t N, int pair);
+int64_t moe_gemm_small_plan_blocks(int64_t R, int E, int64_t N, int pair);
+int moe_launch_gemm_plan(int tile, const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg, int* out, hipStream_t stream);
+int moe_launch_gemm_small_plan(const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg, int* out, hipStream_t stream);
 bool moe_gemm_mfma_supported(const MoeGemmParams& p, int64_t R);
 int moe_launch_gemm_mfma(const MoeGemmParams& p, int64_t R, hipStream_t stream);
 int64_t moe_gemm_mfma_launch_count();   // test aid: matrix-core grouped GEMM launches enqueued by this process so far

@@ -238,13 +238,26 @@ int moe_padded_block_indices(const void* offsets, int off64, int E, int block_m,
 
 int64_t moe_gemm_debug_launch_count(void) { return moe_gemm_mfma_launch_count(); }
 
-int64_t moe_gemm_debug_plan_blocks(int64_t R, int E, int64_t N, int pair) { return moe_gemm_plan_blocks(R, E, N, pair); }
+int moe_gemm_debug_tile(int64_t R, int E, int64_t K, int64_t N, int pair, int nseg)
+{
+    if (E < 1 || R < 0 || K < 1 || N < 1 || nseg < 1 || nseg > 2) return MOE_ERR_BAD_ARG;
+    return moe_gemm_tile(moe_gemm_cus(), R, E, K * nseg, N, pair != 0);
+}
+
+int64_t moe_gemm_debug_plan_blocks(int64_t R, int E, int64_t N, int pair) { return moe_gemm_plan_blocks(256, R, E, N, pair); }
+int64_t moe_gemm_debug_tile_plan_blocks(int tile, int64_t R, int E, int64_t N, int pair) { return moe_gemm_plan_blocks(tile, R, E, N, pair); }
 
 int moe_gemm_debug_plan(const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg,
                         int32_t* out, void* stream)
 {
-    if (!offsets || !out || E < 1 || R < 0 || K < 1 || N < 1) return MOE_ERR_BAD_ARG;
-    return moe_launch_gemm_plan(offsets, off64, E, R, K, N, pair, nseg, out, S(stream));
+    return moe_gemm_debug_tile_plan(256, offsets, off64, E, R, K, N, pair, nseg, out, stream);
+}
+
+int moe_gemm_debug_tile_plan(int tile, const void* offsets, int off64, int E, int64_t R, int64_t K, int64_t N, int pair, int nseg,
+                             int32_t* out, void* stream)
+{
+    if ((tile != 128 && tile != 256) || !offsets || !out || E < 1 || R < 0 || K < 1 || N < 1) return MOE_ERR_BAD_ARG;
+    return moe_launch_gemm_plan(tile, offsets, off64, E, R, K, N, pair, nseg, out, S(stream));
 }
 
 // ---------------------------------------------------------------------------------------------------------

@@ -19,6 +19,12 @@ def check_expert_grads(got, want, tol, what=""):
     assert mx < tol and rms < tol, f"{what}: per-expert max rel err {mx:.4g}, rms rel err {rms:.4g}"
 
 
+def _tile(R, E, K, N, pair=False, nseg=1):
+    """Rows and columns of the output tiles that a launch of these sizes takes."""
+    from moe_distributed_training_amd._lib import lib
+    return lib.moe_gemm_debug_tile(R, E, K, N, int(pair), nseg)
+
+
 def _ops():
     from moe_distributed_training_amd.scattermoe_utils.kernels import ops
     return ops
@@ -59,10 +65,20 @@ CASES = [
     (torch.bfloat16, 500, 4, 2, 64, 512, 16),    # a single K tile: the adapter slabs' LDS image is requested before the loop
     (torch.bfloat16, 500, 4, 2, 192, 300, 16),   # three K tiles: ... by the first trip through the loop
 ]
+# The cases above are small and take 128 x 128 tiles where their K is a multiple of 64; the same forms in the 256 x 256 tiles of larger launches
+LARGE_TILE_CASES = [
+    (torch.bfloat16, 1500, 8, 2, 256, 2048, 16),
+    (torch.bfloat16, 1500, 8, 2, 256, 2048, 32),  # two slabs
+    (torch.bfloat16, 1500, 8, 2, 256, 2048, 40),  # three, the last one partly filled
+    (torch.float16, 1500, 8, 2, 256, 2048, 64),   # four
+    (torch.bfloat16, 1100, 4, 2, 2048, 1024, 16), # every tile cut along K
+    (torch.bfloat16, 1500, 8, 2, 64, 2048, 16),   # a single K tile
+    (torch.bfloat16, 1500, 8, 2, 192, 2056, 16),  # three, and an N tail
+]
 
 
 @pytest.mark.parametrize("layout", ["k_contiguous", "n_contiguous"])
-@pytest.mark.parametrize("dtype,T,E,k,K,N,r", CASES)
+@pytest.mark.parametrize("dtype,T,E,k,K,N,r", CASES + LARGE_TILE_CASES)
 def test_scatter2scatter_all_row_mappings(dev, oracle, layout, dtype, T, E, k, K, N, r):
     ops = _ops()
     torch.manual_seed(1)
@@ -75,6 +91,8 @@ def test_scatter2scatter_all_row_mappings(dev, oracle, layout, dtype, T, E, k, K
     # GEMM launch per call), everything else on the generic kernels
     from moe_distributed_training_amd._lib import lib
     on_matrix_cores = dtype != torch.float32 and K >= 64 and K % 8 == 0 and N % 8 == 0
+    if (dtype, T, E, k, K, N, r) in LARGE_TILE_CASES:
+        assert _tile(T * k, E, K, N) == 256
     for xg, yg in [(False, True), (False, False), (True, False), (True, True)]:
         X = torch.randn(T * k if xg else T, K).to(dtype)
         kk = 1 if xg else k
@@ -90,13 +108,13 @@ def test_scatter2scatter_all_row_mappings(dev, oracle, layout, dtype, T, E, k, K
         assert rel(y2, yo2) < TOL[dtype], (xg, yg)
 
 
-@pytest.mark.parametrize("T,E,k,K,N,layout", [(600, 4, 2, 2048, 512, "k_contiguous"), (600, 4, 2, 2048, 512, "n_contiguous"),
-                                              (4096, 8, 2, 14336, 4096, "n_contiguous")])
-def test_k_split_exchange_is_stable_over_many_launches(dev, oracle, T, E, k, K, N, layout):
+@pytest.mark.parametrize("T,E,k,K,N,layout,tile", [(600, 4, 2, 2048, 512, "k_contiguous", 128), (600, 4, 2, 2048, 512, "n_contiguous", 128),
+                                                   (1100, 4, 2, 2048, 1024, "k_contiguous", 256), (4096, 8, 2, 14336, 4096, "n_contiguous", 256)])
+def test_k_split_exchange_is_stable_over_many_launches(dev, oracle, T, E, k, K, N, layout, tile):
     """Tiles of the last, partial round are cut 2 or 4 ways along K; the parts exchange fp32 partials through memory
     that crosses the XCDs' separate L2 caches and a counter.  A stale read there would be a silent, intermittent wrong
-    sum: 2000 launches of the same problem (a small one where every tile is split, and the h W2 product at the Mixtral
-    shape) must all be bitwise equal to the first, which itself meets the oracle; stops at the first mismatch."""
+    sum: 2000 launches of the same problem (small ones where every tile is split, in tiles of either size, and the h W2 product at
+    the Mixtral shape) must all be bitwise equal to the first, which itself meets the oracle; stops at the first mismatch."""
     ops = _ops()
     torch.manual_seed(21)
     _, sei, ssi, eo = _routing(oracle, T, E, k, seed=21)
@@ -106,6 +124,7 @@ def test_k_split_exchange_is_stable_over_many_launches(dev, oracle, T, E, k, K, 
     W = (torch.randn(E, N, K, generator=g, device=dev) * 0.05).bfloat16().permute(0, 2, 1) if layout == "k_contiguous" else \
         (torch.randn(E, K, N, generator=g, device=dev) * 0.05).bfloat16()
     seid, ssid = sei.to(dev), ssi.int().to(dev)
+    assert _tile(L, E, K, N) == tile
     plan, _ = _plan(dev, torch.bincount(sei, minlength=E).tolist(), K, N, False)
     assert (plan[:, 0] == 1).any() and (plan[plan[:, 0] == 1][:, 6] > 1).any(), "the case must have K-split tiles"
     first = ops.scatter2scatter(X, W, seid, ssid, 1, None, True, True)
@@ -419,21 +438,23 @@ def test_parallel_experts_module(dev, oracle):
     assert rel(y, yo) < 1e-2
 
 
-def _plan(dev, counts, K, N, pair, nseg=1):
+def _plan(dev, counts, K, N, pair, nseg=1, tile=None):
     from moe_distributed_training_amd._lib import lib, check, ptr, stream_ptr
     E = len(counts)
     R = int(sum(counts))
     eo = torch.tensor(counts, dtype=torch.int64).cumsum(0).to(dev)
-    blocks = lib.moe_gemm_debug_plan_blocks(R, E, N, int(pair))
+    tile = tile or _tile(R, E, K, N, pair, nseg)
+    blocks = lib.moe_gemm_debug_tile_plan_blocks(tile, R, E, N, int(pair))
     out = torch.full((blocks, 9), -7, dtype=torch.int32, device=dev)
-    check(lib.moe_gemm_debug_plan(ptr(eo), 1, E, R, K, N, int(pair), nseg, ptr(out), stream_ptr(dev)), "moe_gemm_debug_plan")
+    check(lib.moe_gemm_debug_tile_plan(tile, ptr(eo), 1, E, R, K, N, int(pair), nseg, ptr(out), stream_ptr(dev)), "moe_gemm_debug_tile_plan")
     return out.cpu().numpy(), blocks
 
 
+@pytest.mark.parametrize("tile", [256, 128])
 @pytest.mark.parametrize("case", range(32))
-def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case):
+def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case, tile):
     """The work items the grouped GEMM's workgroups decode for themselves, for seeded group sizes (even, ragged, skewed,
-    empty groups, few and many rounds of tiles, both tile widths, more experts than one wave looks up at once): the rows of a
+    empty groups, few and many rounds of tiles, both tile sizes and widths, more experts than one wave looks up at once): the rows of a
     group are cut into as many tiles as it needs, without a gap, at 16-row blocks and to within one block evenly; every output
     tile appears exactly once, either whole or as K parts 0..n-1 with consecutive exchange slots and one counter, and slots and
     counters are unique and within the exchange area's size."""
@@ -461,12 +482,12 @@ def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case):
     N = rng.choice([256, 4096, 14336, 1000])
     pair = rng.choice([False, True])
     nseg = 1 if pair else rng.choice([1, 2])
-    plan, blocks = _plan(dev, counts, K, N, pair, nseg)
+    plan, blocks = _plan(dev, counts, K, N, pair, nseg, tile)
     ncu = torch.cuda.get_device_properties(dev).multi_processor_count // 8 * 8
-    bn = 128 if pair else 256
+    bn = tile // 2 if pair else tile
     ntn = (N + bn - 1) // bn
-    tiles_ub = (sum(counts) // 256 + E) * ((N + 255) // 256)
-    slots_cap = min(4 * tiles_ub, ncu)
+    tiles_ub = (sum(counts) // tile + E) * ((N + tile - 1) // tile)
+    slots_cap = min(4 * tiles_ub, 256 // tile * ncu)   # one round of workgroups; the counters, one per compute unit, are half as many with small tiles
     seen = {}
     for b in range(blocks):
         valid, e, ntile, r0, r1, part, nparts, slot, counter = (int(v) for v in plan[b])
@@ -484,9 +505,9 @@ def test_grouped_gemm_tile_plan_covers_every_tile_once(dev, case):
     for (e, ntile), cut in rows.items():
         cut.sort()
         blocks_of = [(r1 - r0 + 15) // 16 for r0, r1 in cut]
-        assert len(cut) == (counts[e] + 255) // 256 and cut[0][0] == ends[e] - counts[e] and cut[-1][1] == ends[e], (case, e, cut)
+        assert len(cut) == (counts[e] + tile - 1) // tile and cut[0][0] == ends[e] - counts[e] and cut[-1][1] == ends[e], (case, e, cut)
         assert all(a[1] == b[0] and (a[1] - a[0]) % 16 == 0 for a, b in zip(cut, cut[1:])), (case, e, cut)
-        assert max(blocks_of) <= 16 and max(blocks_of) - min(blocks_of) <= 1, (case, e, cut)
+        assert max(blocks_of) <= tile // 16 and max(blocks_of) - min(blocks_of) <= 1, (case, e, cut)
     used_slots, used_counters = set(), set()
     for key, items in seen.items():
         nparts = items[0][1]
@@ -509,12 +530,14 @@ def max_split_ok(pair):
 
 @pytest.mark.parametrize("counts", [[257, 272, 273, 1], [511, 512, 513, 15], [769, 16, 1025, 0], [144, 145, 287, 31]])
 @pytest.mark.parametrize("layout", ["k_contiguous", "n_contiguous"])
-def test_grouped_gemm_rows_dealt_evenly_to_tiles(dev, oracle, counts, layout):
-    """Groups of one block more or less than a whole number of tiles: every row exactly once, whatever tile it falls into."""
+@pytest.mark.parametrize("N,tile", [(320, 128), (8192, 256)])
+def test_grouped_gemm_rows_dealt_evenly_to_tiles(dev, oracle, counts, layout, N, tile):
+    """Groups of one block more or less than a whole number of tiles of either size: every row exactly once, whatever tile it falls into."""
     ops = _ops()
     torch.manual_seed(21)
-    E, K, N = len(counts), 512, 320
+    E, K = len(counts), 512
     R = sum(counts)
+    assert _tile(R, E, K, N) == tile
     sei = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
     ssi = torch.randperm(R, generator=torch.Generator().manual_seed(2))
     X, W = torch.randn(R, K).bfloat16(), (torch.randn(E, K, N) * 0.05).bfloat16()
