@@ -36,6 +36,12 @@ def _make(T, d, f, E, r, dtype, seed=0, lora_std=0.02):
     return x, wg, w1, w2, w3, lora, rn(T, d)
 
 
+def _tiles(R, E, d, f):
+    """Tile sizes of the layer's four grouped GEMM launches: gate/up, h W2, dh, dX."""
+    from moe_distributed_training_amd._lib import lib
+    return tuple(lib.moe_gemm_debug_tile(R, E, K, N, pair, nseg) for K, N, pair, nseg in ((d, f, 1, 1), (f, d, 0, 1), (d, f, 0, 1), (f, d, 0, 2)))
+
+
 def _views(lora, dev):
     from moe_distributed_training_amd.megablocks_utils.moe_mlp import LoraViews
     t = {n: (a.to(dev).requires_grad_(True), b.to(dev).requires_grad_(True)) for n, (a, b) in lora.items()}
@@ -172,14 +178,15 @@ def test_layer_many_experts_router_gradient(dev, oracle, E, k):
     assert rel(wgg.grad, wgo.grad) < 1e-2
 
 
-@pytest.mark.parametrize("r", [32, 24, 48, 64, 72, 128, 144])
-def test_layer_rank_above_16_adapters(dev, oracle, r):
+@pytest.mark.parametrize("T,d,f,E,r", [(384, 256, 512, 4, r) for r in (32, 24, 48, 64, 72, 128, 144)] + [(900, 512, 4096, 8, 32), (900, 512, 4096, 8, 24)])
+def test_layer_rank_above_16_adapters(dev, oracle, T, d, f, E, r):
     """Adapter rank above 16: up to 128 the fused launches take the adapter as 16-wide rank chunks (24, 72: the last
     chunk partly filled; 48, 72: an odd number of chunks; above 32 the gate/up launch finds its slabs by base and
     stride); above that the layer runs as router + sort + the three grouped calls + combine.  All gradients against
-    the oracle."""
+    the oracle.  The small layer's launches of up to four slabs take 128 x 128 tiles, the larger one's 256 x 256."""
     import moe_distributed_training_amd as moe
-    T, d, f, E, k, alpha = 384, 256, 512, 4, 2, 64.0
+    k, alpha = 2, 64.0
+    assert set(_tiles(T * k, E, d, f)) == {128 if T < 900 else 256}
     x, wg, w1, w2, w3, lora, dout = _make(T, d, f, E, r, torch.bfloat16, seed=5)
     xo = x.float().requires_grad_(True)
     lo = {n: (a.float().requires_grad_(True), b.float().requires_grad_(True)) for n, (a, b) in lora.items()}
@@ -587,7 +594,8 @@ def test_ragged_row_tiles_of_every_block_count(dev, oracle, counts):
     """Groups whose last row tile has every number of live 16-row blocks a wave can meet: each count runs its own copy
     of the grouped GEMMs' K loop, blocks inside a count but past the group compute on rows that were never loaded, and
     the fused epilogues (SwiGLU with the h A2 product; SwiGLU backward with the adapter gradients' row and column sums)
-    must keep those rows out of every sum.  Pre-dispatched rows, LoRA r=16, forward and backward against the fp32 oracle."""
+    must keep those rows out of every sum.  (The counts are those of tiles of 256 rows, which the next test's larger launches take; here the tiles have 128, and a
+    wave at most four blocks.)  Pre-dispatched rows, LoRA r=16, forward and backward against the fp32 oracle."""
     import moe_distributed_training_amd as moe
     d, f, r, alpha = 256, 512, 16, 32.0
     E, R = len(counts), sum(counts)
@@ -618,12 +626,25 @@ def test_ragged_row_tiles_of_every_block_count(dev, oracle, counts):
 
 
 @pytest.mark.parametrize("counts", [[1, 16, 17, 32, 33, 48, 64, 65], [100, 128, 129, 144, 160, 161, 193, 224], [225, 255, 256, 257, 300, 511, 513, 0]])
-@pytest.mark.parametrize("d,f", [(1088, 2112), (192, 320)])
-def test_ragged_row_tiles_in_large_and_small_tiles(dev, oracle, counts, d, f):
+@pytest.mark.parametrize("d,f,tiles", [(1088, 2112, (256, 256, 256, 256)), (192, 320, (128, 128, 128, 128)), (1024, 512, (128, 128, 128, None))])
+def test_ragged_row_tiles_in_large_and_small_tiles(dev, oracle, counts, d, f, tiles):
     """The row counts above where the launches take 256 x 256 tiles (1088 x 2112: the chip is more than half full) and where they take 128 x 128
-    ones with a last column tile that is not full (192 x 320); the row tiles' partials of the adapter gradients differ in number."""
+    ones with a last column tile that is not full (192 x 320); the row tiles' partials of the adapter gradients differ in number.  1024 x 512: the dh and dX launches cut every
+    tile along K (that of dX in tiles of either size), and the dh launch's row-tile partials lie behind what they exchange, in the same area, until the sums at the end read them."""
     import moe_distributed_training_amd as moe
     r, alpha, E, R = 16, 32.0, len(counts), sum(counts)
+    assert all(want in (None, got) for got, want in zip(_tiles(R, E, d, f), tiles))
+    if d == 1024:
+        from moe_distributed_training_amd._lib import lib
+        from test_gpu_ops import _plan
+        for K, N, nseg in ((d, f, 1), (f, d, 2)):
+            plan, _ = _plan(dev, counts, K, N, False, nseg)
+            assert (plan[plan[:, 0] == 1][:, 6] == 2).all()
+        # adapters add to the workspace their packed factors, the interims and the column-tile partials, and nothing for row tiles: those lie in the exchange area
+        up = lambda n: (n + 255) // 256 * 256
+        factors = 3 * up(E * 32 * d) + 3 * up(E * 32 * f)
+        interims, columns = 7 * up(((R + 31) // 32 * 32 + 32) * 32), up(max(f // 64, 2 * (f // 128)) * R * 64)
+        assert lib.moe_mlp_workspace_bytes(R, E, d, f, r) == lib.moe_mlp_workspace_bytes(R, E, d, f, 0) + factors + interims + columns
     g = torch.Generator().manual_seed(12)
     rn = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).bfloat16()
     w1, w2, w3 = rn(E, f, d, std=0.03), rn(E, f, d, std=0.03), rn(E, f, d, std=0.03)
