@@ -1,6 +1,6 @@
-// Shape- and dtype-generic grouped GEMM kernels (fp32 FMA through LDS tiles).  They accept any strides, any
-// K/N/rank and bf16/fp16/fp32 storage, and serve every case the MFMA kernels do not take (fp32 inputs, odd
-// sizes, unaligned views).  fp32 accumulation, fixed summation order.
+// Shape- and dtype-generic grouped GEMM kernels.  They accept any strides, any K/N/rank and bf16/fp16/fp32 storage, and serve every
+// case the 16-bit matrix-core kernels do not take (fp32 inputs, odd sizes, unaligned views): fp32 products without adapters, from a size on,
+// on the fp32 matrix instructions, the others by fp32 FMA through LDS tiles.  fp32 accumulation, fixed summation order.
 #include "common.h"
 #include "kernels.h"
 #include <type_traits>

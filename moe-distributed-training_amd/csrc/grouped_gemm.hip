@@ -89,7 +89,7 @@ bool moe_gemm_mfma_supported(const MoeGemmParams& p, int64_t R)
 // The second condition is for rows that are not dealt evenly, which the host does not see: a group of 129 rows is two small tiles and one large one.  Two small tiles on one
 // compute unit take as long as a large one there, so of a launch that splits K the small ones must come to at most one per compute unit however the rows fall.  Of
 // 5000 drawn products (128 to 14336 columns and deep, 1 to 96 groups), small tiles by the first condition alone: those whose tiles came to one at most 0.95-1.93 times as fast as large ones,
-// those of more 0.77-1.37 and half of them slower: us, large and small, 64 groups of 121 rows on average, 1408 x 192 31.1 and 40.3; 16 of 140, 1216 x 768 30.1 and 36.6; 32 of
+// those of more 0.77-1.37, 28 % of them slower by more than 1.5 %: us, large and small, 64 groups of 121 rows on average, 1408 x 192 31.1 and 40.3; 16 of 140, 1216 x 768 30.1 and 36.6; 32 of
 // 123, 3968 x 256 57.2 and 66.7; dX of two groups of 126, 28672 x 4096, and the kernels around it 210 and 245.  Launches that never split have a longer chain of K tiles to lose on the idle half: up to
 // one and a half per compute unit (gate/up of 16 groups, 124 rows on average, 2816 x 960 and the kernels behind it 93.6 and 97.1 with 1.8; 1.05-1.6 times as fast up to 1.5).
 int moe_gemm_tile(int cus, int64_t R, int E, int64_t K, int64_t N, bool pair)

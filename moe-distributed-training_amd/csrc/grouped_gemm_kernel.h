@@ -47,7 +47,7 @@ constexpr int NSTAGE_A = 2, NSTAGE_B = 3;   // the weight tile ring is one stage
 constexpr int B_REGION = NSTAGE_A * A_STAGE_BYTES;                                // weight stages follow the activation stages
 constexpr int LDS_BYTES = NSTAGE_A * A_STAGE_BYTES + NSTAGE_B * B_STAGE_BYTES;    // 160 KiB, all of a compute unit's LDS, or half of it
 // Row tables (in_row, out_row as int64) and the split tiles' arrival flag borrow the third weight stage: before the
-// main loop's first tile that stage is still empty, and after the loop the epilogue staging only needs the first 128 KiB.
+// main loop's first tile that stage is still empty, and after the loop the epilogue staging only needs what lies before it (128 or 32 KiB of 128 or 64).
 constexpr int TABLE_OFF = B_REGION + 2 * B_STAGE_BYTES;
 static_assert(TABLE_OFF >= NWAVES * (BM / 2) * (BN / (NWAVES / 2)) * 2, "epilogue staging must not reach the tables");
 // SwiGLU-backward epilogue with fused row contractions: images of three [BM][16] bf16 operands sit behind the row tables
@@ -105,7 +105,7 @@ struct WorkItem {
 };
 
 // Rows of row tile mt of a group's mte tiles: the group's 16-row blocks are dealt evenly to its tiles (mte = the number of
-// 256-row tiles the group needs).  Measured per round of tiles at K=4096: 99 us with 16 row blocks, 87 with 13, and a tail
+// tiles of BM rows the group needs; the figures are of 256 rows).  Measured per round of tiles at K=4096: 99 us with 16 row blocks, 87 with 13, and a tail
 // of 1-3 blocks behind full tiles about as much as a full one (its waves wait for the same weight tiles), so 1060 rows run
 // as five tiles of 13-14 blocks instead of four of 16 and one of 3.  8192 rows over 8 experts: gate/up launch 1630 -> 1556 us,
 // the layer's forward and backward 5029 -> 4950 us.
@@ -257,7 +257,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
     // ---- per-thread global source pointers for the direct-to-LDS loads (k offset added per tile)
     // A image: row r at r*128 B, logical 16-byte chunk c of that row at slot c ^ ((r >> 1) & 7): two rows span the
     // 64 LDS banks, so 16 consecutive rows of one chunk column hit 16 different bank groups.
-    // Wave w issues load instructions j = 0..3; instruction (j, w) fills rows [(j*8 + w)*8, +8).
+    // Wave w issues load instructions j = 0..LPT-1; instruction (j, w) fills rows [(j*NWAVES + w)*8, +8).
     // Grouped rows are addressed from the tile's first row (the descriptor is re-based there, so the 32-bit offsets
     // only span one tile whatever the number of rows); gathered rows from the start of X.
     const int64_t a_row_base = p.x_grouped ? row0 : 0;
@@ -272,7 +272,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
     // range -- with the full 32-bit range it would be a valid offset and the load would touch memory 4 GiB past the base)
     constexpr uint32_t LOAD_RANGE = KTAIL ? 0x80000000u : 0xFFFFFFFFu;
     const i32x4_t a_buf0 = make_buffer(p.X[0] + a_row_base * p.ldx, LOAD_RANGE), a_buf1 = make_buffer((TWO_SEG && p.X[1] ? p.X[1] : p.X[0]) + a_row_base * p.ldx, LOAD_RANGE);
-    // B: offsets within this expert's matrix.  For the SwiGLU pair image rows [0,128) come from W[0] and [128,256)
+    // B: offsets within this expert's matrix.  For the SwiGLU pair image rows [0, BN/2) come from W[0] and [BN/2, BN)
     // from W[1], which are whole load instructions (the first and second half of a wave's LPT); otherwise W[0] / W[1]
     // are the two K segments.
     uint32_t b_off[LPT];
@@ -305,8 +305,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
 
     // ---- low-rank slabs (up to two) ride in as the activation image of the K tile after the last: that tile's four
     // load instructions per wave fetch, instead of a re-read nobody uses, 32 rows x 16 k of Q[0], of Q[1], and 32
-    // columns x 16 k of LB[0], of LB[1] (8 KiB each over the 8 waves; for the gate/up pair the two halves of a column
-    // image hold the same 128 columns; with one slab both images of a kind hold that slab).  The slab step after the
+    // columns x 16 k of LB[0], of LB[1] (BM * 32 bytes each over the waves; for the gate/up pair the two halves of a column
+    // image hold the same BN/2 columns; with one slab both images of a kind hold that slab).  The slab step after the
     // loop then reads its fragments from LDS instead of waiting for a round trip to memory.
     static_assert(LPT == 4, "slab image: one load instruction per wave for each of Q[0], Q[1], LB[0], LB[1]");
     const bool lds_slabs = p.nslab >= 1 && p.nslab <= 2;
@@ -461,8 +461,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
     // run after the barrier that hands over the next tile, so they cover the LDS latency of that tile's first fragment
     // reads.  That barrier also frees the stages the finished tile occupied.  Neither the fragment reads nor the loads
     // that refill the stages are issued in one burst -- a burst keeps the wave's instruction stream and the LDS / load
-    // unit's queue busy while the matrix pipe idles -- but one at a time between the MFMAs: a fragment read before every
-    // second MFMA of a half step (weight blocks first, when the next half step starts a k step), the loads as below.
+    // unit's queue busy while the matrix pipe idles -- but one at a time between the MFMAs: the eight fragment reads of a half step at
+    // equal distances (before every second MFMA; every MFMA of a small tile; weight blocks first, when the next half step starts a k step), the loads as below.
     constexpr int MFMAS_PER_STEP = MBH * NB;
     constexpr int READ_GAP = MFMAS_PER_STEP / 8;     // MFMAs between two fragment reads
     static_assert((NB + MBH) * READ_GAP <= MFMAS_PER_STEP, "fragment reads are issued inside the half step");
@@ -584,8 +584,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
     // (one scalar compare chain per wave; the counts of a tile's two rows of waves differ by at most one)
     // The only tile of its group is also the only reader of its weight tiles: their loads are non-temporal (a streaming read
     // reaches 7.0 TB/s that way, 6.1 without; 24 tokens over 8 experts: 589 -> 539 us forward.  Where several row tiles share the
-    // weight tiles the hint costs 2 %: it works against the sharing in L2).  A tile of eight blocks can be either: 17 blocks are
-    // dealt 9 and 8, and those two walk K alike (the smaller one through the loop of MBH blocks that the larger one's second row of
+    // weight tiles the hint costs 2 %: it works against the sharing in L2).  A tile of half its blocks can be either: 17 blocks are
+    // dealt 9 and 8 (small tiles: 9 are dealt 5 and 4), and those two walk K alike (the smaller one through the loop of MBH blocks that the larger one's second row of
     // waves takes as well); fewer blocks than that are always a whole group.
     using T_ = std::true_type;
     using F_ = std::false_type;
@@ -747,7 +747,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
                 const int src = (upper && has_hi) ? lo + 1 : lo;
                 const bool live = !upper || has_hi;
                 if (lds_slabs) {
-                    // image of the tile after the last: Q[src] rows at src * 8 KiB, LB[src] columns 16 KiB further up
+                    // image of the tile after the last: Q[src] rows at src * BM * 32 bytes, LB[src] columns behind both
                     const uint8_t* img = smem + ((ke - kb) & 1) * A_STAGE_BYTES + src * (BM * 32) + 16 * kc;
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb) {
@@ -939,7 +939,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
         }
         if (EPI == MOE_EPI_SWIGLU_FUSED) {
             // element (row = mb*16 + 4*(lane/16) + reg, rank column lane%16) of every column wave's sums is parked in its slot;
-            // wave (wm, wn) adds the four column waves' sums (in wave order) of row blocks 2 wn, 2 wn + 1 and stores them
+            // wave (wm, wn) adds all column waves' sums (in wave order) of row blocks 2 wn, 2 wn + 1 and stores them
             __builtin_amdgcn_s_waitcnt(0xC07F);
             __syncthreads();
             const int tg = lane >> 4, ti = lane & 15;
@@ -1041,7 +1041,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
         const int trow = 8 * tg + (ti >> 2);
         constexpr int IBLK = WTN / 16;   // 16-column blocks of the wave's sub-tile
         constexpr int CC_MATS = 2, CC_KS = WTN / 32;
-        f32x4_t rcd[RC_MATS][IBLK];      // row contractions, accumulated over the wave's 128 rows
+        f32x4_t rcd[RC_MATS][IBLK];      // row contractions, accumulated over the wave's rows
         bf16x8_t cbf[CC_MATS][CC_KS];    // this wave's fragments of the two adapter factors
         if (FUSED) {
 #pragma unroll
@@ -1177,7 +1177,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
         }
         if (FUSED) {
             // column contractions: element (row = 16-row block * 16 + 4 * (lane / 16) + reg, rank column lane % 16) summed
-            // over one wave's 64 columns sits in that wave's slice; wave (wm, wn) adds the four column waves' sums (in wave
+            // over one wave's 64 columns sits in that wave's slice; wave (wm, wn) adds all column waves' sums (in wave
             // order) for the 32-row block wn of its row half and stores them
             __builtin_amdgcn_s_waitcnt(0xC07F);
             __syncthreads();
@@ -1202,10 +1202,9 @@ __global__ void __launch_bounds__(NTHREADS, 2) grouped_gemm_mfma_kernel(const Mo
             __builtin_amdgcn_s_waitcnt(0xC07F);
             __syncthreads();   // the slices are free again for the exchange below
             // row contractions: rcd[mat][ib][reg] = element (column ib*16 + 4*(lane/16) + reg, rank column lane%16) summed
-            // over this wave's 128 rows: the lower row of waves parks its sums in its own slices, the upper one adds them
-            // to its own (a fixed order) and stores the tile's partial
+            // over this wave's rows: the lower row of waves parks its sums in its own slices, in a small tile, whose slices hold less than that, side
+            // by side over all of them; the upper one adds them to its own (a fixed order) and stores the tile's partial
             static_assert(WAVES_N * RC_MATS * IBLK * 1024 <= TABLE_OFF, "the exchange stays in front of the tables");
-            // (a small tile's slices hold less than a wave parks)
             float* xch = (float*)(smem + (BM == 256 ? ((wave % WAVES_N) + WAVES_N) * (WTM * WTN * 2) : (wave % WAVES_N) * (RC_MATS * IBLK * 1024)));
             if (wm == 1) {
 #pragma unroll

@@ -34,13 +34,13 @@ struct MoeGemmParams {
     const uint16_t* H3;
     int64_t ldh;
     // MOE_EPI_SWIGLU_BWD_FUSED only: row contractions (nrc = 3).  RC[i]: bf16 [R][16] operands in grouped order;
-    // RCP[i]: fp32 partials [row tile][N][16], row tiles of 256 rows per expert in order (the layout the fixed-order
+    // RCP[i]: fp32 partials [row tile][N][16], row tiles of the launch's tile size per expert in order (the layout the fixed-order
     // reduction of the adapter gradients sums): RCP[0] = dgate^T RC[0], RCP[1] = dup^T RC[1], RCP[2] = h^T RC[2]
     const uint16_t* RC[3];
     float* RCP[3];
     int nrc;
-    // ... and column contractions (MOE_EPI_SWIGLU_BWD_FUSED: ncc = 2; MOE_EPI_SWIGLU_FUSED: ncc = 1, CCP[0] = h CB[0] per column tile of 128): CB[i]: adapter factor in fragment order [E][N/32][64][8];
-    // CCP[i]: fp32 partials [column tile of 256][cc_rows][16]: CCP[0] = dgate CB[0], CCP[1] = dup CB[1] over the tile's columns
+    // ... and column contractions (MOE_EPI_SWIGLU_BWD_FUSED: ncc = 2; MOE_EPI_SWIGLU_FUSED: ncc = 1, CCP[0] = h CB[0] per column tile of half the tile size): CB[i]: adapter factor in fragment order [E][N/32][64][8];
+    // CCP[i]: fp32 partials [column tile][cc_rows][16]: CCP[0] = dgate CB[0], CCP[1] = dup CB[1] over the tile's columns
     const uint16_t* CB[2];
     float* CCP[2];
     int ncc;
