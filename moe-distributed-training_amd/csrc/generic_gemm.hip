@@ -250,6 +250,8 @@ __global__ void __launch_bounds__(GT * GT) generic_grouped_xty_kernel(
 // One round more where tiles or columns are half empty (groups of less than 16 rows; 65 to 85 columns of 128): 512, 8 rows of 8, 256 x 1024 10.3 and 11.1;
 // 640, 2048 rows of 4, 64 x 80 0.98 times as fast (0.94);  768, 8 rows of 8, 64 x 1536 1.04 (1.05).
 // Two rounds more below 64 k, where the chain is a step or two: 768, 64 rows of 8, 40 x 1536 0.95 (0.89); 1024, 512 rows of 2, 40 x 512 1.03 (1.01).
+// Groups without rows count (the host does not see them): of 1698 drawn launches beyond these lines 20 are slower by more than 3 %, most of them of few rows over 64 or more experts and with
+// steps filled to less than 0.8 (80 rows over 64, 77 x 293 6.8 and 7.9); two rounds more for those would leave 9 and cost 111 others a tenth.
 bool f32_on_matrix_cores(int64_t R, int E, int64_t K, int64_t N)
 {
     if (N <= FM_COLS / 2) return false;   // half of the columns at least (2048 rows, 250 x 16: 10.4 and 11.4)
